@@ -15,6 +15,7 @@
 #include "elementwise.h"
 #include "group_softmax.h"
 #include "index_format.h"
+#include "row_sort.h"
 
 using namespace ts;
 
@@ -140,12 +141,11 @@ int run_csr_reduce_slice(const void *src, const int64_t *indptr, void *out, int6
                          int64_t B, int64_t N, int64_t E, int64_t K, int64_t indptr_batch_stride, int dtype,
                          int reduce, int accumulate, void *ws, size_t ws_bytes, hipStream_t stream,
                          const int32_t *perm, int64_t perm_batch_stride, bool want_perm_args, bool *perm_args_done,
-                         unsigned long long *status, bool status_reset, uint64_t status_nonce,
-                         const int *gate = nullptr, int scatter_rule = 0) {
+                         unsigned long long *status, bool status_reset, uint64_t status_nonce) {
   const bool al = aligned16(src) && aligned16(out);
-  // permuted rows always take the wide kernel (the narrow one stages consecutive entries), and so does a gated call
+  // permuted rows always take the wide kernel (the narrow one stages consecutive entries)
   const CsrPlan p = csr_plan(N, E, K, kElemBytes[dtype], al, false, reduce == TS_MIN || reduce == TS_MAX,
-                             perm == nullptr && gate == nullptr && !scatter_rule);
+                             perm == nullptr);
   const CsrWs w = csr_workspace(p, B, K, dtype, reduce);
   if (ws == nullptr || ws_bytes < w.total) return TS_ERR_WORKSPACE;
   CsrReduceArgs a;
@@ -176,9 +176,6 @@ int run_csr_reduce_slice(const void *src, const int64_t *indptr, void *out, int6
   a.carry_spin = env_int("TS_CSR_SPIN", kCarrySpin);  // test aid: -1 makes every look-back give up at once
   a.perm = perm;
   a.perm_batch_stride = perm_batch_stride;
-  a.gate = gate;
-  a.gate_want = 0;
-  a.scatter_rule = scatter_rule;
   // every row is finished inside the first kernel unless the second one runs: then the positions can leave it
   // in src's order right away;
   // when the output is large: the lookup at every row end makes the wavefront wait, a pass over [N, K]
@@ -193,7 +190,7 @@ int run_csr_reduce(const void *src, const int64_t *indptr, void *out, int64_t *a
                    int64_t B, int64_t N, int64_t E, int64_t K, int64_t indptr_batch_stride, int dtype,
                    int reduce, int accumulate, void *ws, size_t ws_bytes, unsigned long long *status,
                    hipStream_t stream, const int32_t *perm = nullptr, int64_t perm_batch_stride = 0,
-                   bool *perm_args_done = nullptr, const int *gate = nullptr, int scatter_rule = 0) {
+                   bool *perm_args_done = nullptr) {
   const int64_t s = kElemBytes[dtype];
   const bool want_perm_args = B * N * K >= ((int64_t)8 << 20);
   const uint64_t status_nonce = next_nonce();  // one for all slices: the status words describe the whole call
@@ -203,34 +200,104 @@ int run_csr_reduce(const void *src, const int64_t *indptr, void *out, int64_t *a
                                 offset_bytes(out, b0 * N * K * s), arg_out ? arg_out + b0 * N * K : nullptr,
                                 offset_bytes(count_out, b0 * N * s), nb, N, E, K, indptr_batch_stride, dtype, reduce,
                                 accumulate, ws, ws_bytes, stream, perm ? perm + b0 * perm_batch_stride : nullptr,
-                                perm_batch_stride, want_perm_args, perm_args_done, status, b0 == 0, status_nonce, gate,
-                                scatter_rule);
+                                perm_batch_stride, want_perm_args, perm_args_done, status, b0 == 0, status_nonce);
   });
 }
 
-// A scatter whose index turns out to be sorted (found by the count pass of the buckets) is finished by the
-// segmented reduction instead: sorted index -> row pointers -> one pass over src without atomics, both gated on
-// the device flag. The reduction must finish every row inside its first kernel (look-back), which needs 4- or
-// 8-byte accumulators and at most four column chunks. Extra workspace behind that of the buckets: the row
-// pointers, then the reduction's own.
-struct SortedRoute {
+// ---- scatter of wide rows: the index is sorted by row (row_sort.h), then a segmented reduction over permuted rows.
+// No atomics on out, no table misses, whatever the index; an index found in order skips the sorting passes.
+// kRowsPlan: does a call take this route, and its workspace (row sort, then the carries of the reduction).
+struct RowsRoute {
   bool ok;
-  size_t ptr_bytes, csr_bytes;
+  size_t sort_bytes, csr_bytes;
 };
-SortedRoute sorted_route_plan(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce) {
-  SortedRoute r = {false, 0, 0};
-  if (!env_int("TS_SCATTER_SORTED_ROUTE", 1) || !env_int("TS_CSR_LOOKBACK", 1)) return r;
-  if (reduce != TS_SUM && reduce != TS_MIN && reduce != TS_MAX) return r;
-  if (kAccBytes[dtype] < 4 || B < 1 || E < 1) return r;
-  const bool wa = reduce != TS_SUM;
+inline int rows_acc_bytes(int dtype, int reduce) {
+  const bool sum = reduce == TS_SUM || reduce == TS_MEAN;
+  return kElemBytes[dtype] == 8 || (sum && is_float_dtype(dtype)) ? 8 : 4;
+}
+CsrPlan rows_csr_plan(int64_t rows, int64_t n, int64_t K, int dtype, bool al, int reduce) {
+  return csr_plan(rows, n, K, kElemBytes[dtype], al, false, reduce == TS_MIN || reduce == TS_MAX, false);
+}
+inline int rows_meta_stride(const CsrPlan &p) { return p.ychunks > 4 ? p.ychunks : 4; }
+RowsRoute rows_route(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce) {
+  RowsRoute r = {false, 0, 0};
+  const int mode = env_int("TS_SCATTER_BINNED", 1);  // tuning aid: 0 never, 2 at any size
+  const int64_t row_bytes = K * kElemBytes[dtype], n = B * E, rows = B * N;
+  if (mode == 0 || B < 1 || E < 1 || N < 1 || row_bytes < 64 || !env_int("TS_CSR_LOOKBACK", 1)) return r;
+  const bool minmax = reduce == TS_MIN || reduce == TS_MAX;
+  if (!minmax && reduce != TS_SUM && reduce != TS_MEAN) return r;
+  if (!minmax && kAccBytes[dtype] < 4) return r;
+  // From where the six launches of the sort and the reduction (31-37 us on the smallest inputs) cost less than the
+  // atomics of the other kernels (us without / with, 10 entries per row, even index, 32 columns; the skewed cases gain
+  // earlier, the host does not know them):
+  //   sums of 4 bytes    32 MB 35 / 43    48 MB 54 / 48     of 8 bytes  32 MB 32 / 42   48 MB 50 / 45
+  //   sums of 2 bytes    24 MB 45 / 53    32 MB 56 / 55     with 100 entries per row  4 MB 33 / 40   8 MB 45 / 41
+  //   min / max of 4 bytes  16 MB 32 / 54   24 MB 50 / 56   32 MB 56 / 57
+  //   min / max of 2 bytes  16 MB 62 / 73   24 MB 92 / 75   of 8 bytes  16 MB 44 / 44   24 MB 55 / 45
+  // (min / max without the sort fill and walk a table of 8-byte keys as large as out: from 256 MB of keys the sort
+  // wins at any size)
+  const int es = kElemBytes[dtype];
+  const int64_t MB = 1000000;
+  // (sums of rows under 128 bytes, or with fewer than two entries per row, gain later: one entry per row, 16 / 32 / 128
+  // floats 96 MB 115 / 122, 106 / 80, 107 / 78)
+  int64_t min_bytes = minmax ? (rows * K * 8 >= 256 * MB ? MB : (es == 4 ? 28 * MB : es == 8 ? 16 * MB : 20 * MB))
+                             : (es >= 4 ? 40 * MB : (n >= 32 * rows ? 6 * MB : 32 * MB));
+  if (!minmax && row_bytes < 128) min_bytes *= 2;
+  if (!minmax && n < 2 * rows) min_bytes *= 2;
+  if (mode != 2 && n * row_bytes < min_bytes) return r;
+  const RowSortPlan sp = row_sort_plan(B, E, N, nullptr, 0);
+  if (sp.bytes == 0) return r;
   for (int al = 0; al < 2; ++al) {
-    const CsrPlan p = csr_plan(N, E, K, kElemBytes[dtype], al != 0, false, wa, false);
-    if (p.small || p.ychunks > 4) return r;
+    const CsrPlan p = rows_csr_plan(rows, n, K, dtype, al != 0, reduce);
+    if (p.ychunks > kMaxGridBatches) return r;
+    const size_t b = csr_ws_bytes(p, 1, K, rows_acc_bytes(dtype, reduce), minmax, nullptr, nullptr, rows_meta_stride(p));
+    if (b > r.csr_bytes) r.csr_bytes = b;
   }
-  r.ptr_bytes = ((size_t)B * (N + 1) * 8 + 255) & ~(size_t)255;
-  r.csr_bytes = csr_workspace_max(B, N, E, K, dtype, reduce, false) - kStatusBytes;
+  r.sort_bytes = sp.bytes;
   r.ok = true;
   return r;
+}
+// perm / ptr as launch_row_sort leaves them; ws: RowsRoute::csr_bytes
+int run_rows_reduce(const void *src, const int32_t *perm, const int64_t *ptr, void *out, int64_t *arg_out, int64_t B,
+                    int64_t E, int64_t K, int64_t N, int dtype, int reduce, int out_given, void *ws, size_t ws_bytes,
+                    hipStream_t s) {
+  const int64_t n = B * E, rows = B * N;
+  const CsrPlan p = rows_csr_plan(rows, n, K, dtype, aligned16(src) && aligned16(out), reduce);
+  CsrReduceArgs a;
+  size_t off_args = 0, off_meta = 0;
+  a.meta_stride = rows_meta_stride(p);
+  if (csr_ws_bytes(p, 1, K, rows_acc_bytes(dtype, reduce), reduce == TS_MIN || reduce == TS_MAX, &off_args, &off_meta,
+                   a.meta_stride) > ws_bytes)
+    return TS_ERR_WORKSPACE;
+  a.src = src;
+  a.indptr = ptr;
+  a.out = out;
+  a.arg_out = arg_out;
+  a.count_out = nullptr;
+  a.N = rows;
+  a.E = n;
+  a.K = K;
+  a.indptr_batch_stride = 0;
+  a.accumulate = out_given ? 1 : 0;
+  a.G = p.G;
+  a.BI = p.BI;
+  a.ipw = p.ipw;
+  a.nblk = p.nblk;
+  a.ws_vals = ws;
+  a.ws_args = reinterpret_cast<int32_t *>(static_cast<char *>(ws) + off_args);
+  a.ws_meta = reinterpret_cast<int64_t *>(static_cast<char *>(ws) + off_meta);
+  a.lookback = p.nblk > 1;
+  a.nonce = next_nonce();
+  a.perm = perm;
+  a.perm_batch_stride = 0;
+  a.perm_args = 0;
+  a.any_order = 1;
+  a.arg_E = E;
+  a.status = nullptr;
+  a.status_reset = 0;
+  a.status_nonce = 0;
+  a.carry_spin = kCarrySpin;
+  return dispatch_csr_reduce(dtype, a, p, 1, reduce, s);
 }
 
 int run_csr_gather(int dtype, const CsrGatherArgs &args, const CsrPlan &p, int64_t B, bool divide, hipStream_t s) {
@@ -261,17 +328,17 @@ int run_coo_gather(int dtype, const CooGatherArgs &args, const CooGatherPlan &p,
 
 // sorted index [B, E] -> row pointers [B, N + 1] (contiguous)
 int run_coo_to_indptr(const int64_t *index, int64_t *ptr, int64_t B, int64_t E, int64_t N, int64_t index_batch_stride,
-                      hipStream_t s, const int *gate = nullptr, int gate_want = 0) {
+                      hipStream_t s) {
   const int per = E < ((int64_t)1 << 20) ? 1 : kCooPtrPerThread;
   const int64_t per_block = (int64_t)kBlock * per;
   return for_batch_slices(B, [&](int64_t b0, int64_t nb) {
     dim3 grid((unsigned)((E + 1 + per_block - 1) / per_block), (unsigned)nb);
     if (per == 1)
       hipLaunchKernelGGL(coo_to_indptr_kernel<1>, grid, dim3(kBlock), 0, s, index + b0 * index_batch_stride,
-                         ptr + b0 * (N + 1), N, E, index_batch_stride, gate, gate_want);
+                         ptr + b0 * (N + 1), N, E, index_batch_stride);
     else
       hipLaunchKernelGGL(coo_to_indptr_kernel<kCooPtrPerThread>, grid, dim3(kBlock), 0, s,
-                         index + b0 * index_batch_stride, ptr + b0 * (N + 1), N, E, index_batch_stride, gate, gate_want);
+                         index + b0 * index_batch_stride, ptr + b0 * (N + 1), N, E, index_batch_stride);
     return hipGetLastError() == hipSuccess ? (int)TS_OK : (int)TS_ERR_LAUNCH;
   });
 }
@@ -549,24 +616,21 @@ int ts_segment_mean_coo_backward(const void *grad_out, const int64_t *index, con
 size_t ts_scatter_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce) {
   if (!valid_dtype(dtype) || !sizes_ok(B, N, E, K)) return 0;
   const bool any_size = env_int("TS_SCATTER_BINNED", 1) == 2;
+  const RowsRoute rr = reduce == TS_MEAN ? RowsRoute{false, 0, 0} : rows_route(B, E, K, N, dtype, reduce);
   if (reduce == TS_MIN || reduce == TS_MAX) {
+    if (rr.ok) return rr.sort_bytes + rr.csr_bytes;
     if (kElemBytes[dtype] > 4) return 0;  // 64-bit elements do not use packed keys
     if (env_int("TS_SCATTER_LDS_K1", 1) && env_int("TS_SCATTER_LDS", 1)) {
       const size_t k1 = k1_plan(B, E, K, N, kElemBytes[dtype], nullptr, 0, env_int("TS_SCATTER_LDS", 1) == 2).bytes;
       if (k1 != 0) return k1;
-    }
-    const size_t binned = bin_plan(B, E, K, N, kElemBytes[dtype], nullptr, 0, any_size, 8, true).bytes;
-    if (binned != 0) {
-      const SortedRoute sr = sorted_route_plan(B, E, K, N, dtype, reduce);
-      return binned + (sr.ok ? sr.ptr_bytes + sr.csr_bytes : 0);
     }
     // one flag for the sample of the index that picks the kernel when few entries meet in an output row
     const int probe = env_int("TS_SCATTER_SKEW", 1);
     return probe && skew_probe_shape(B, E, K, N, kElemBytes[dtype], probe == 2) ? 256 : 0;
   }
   if (reduce == TS_SUM && kAccBytes[dtype] >= 4) {  // table slots: int32 for int32, 8 bytes for the other types
-    const size_t binned = bin_plan(B, E, K, N, kElemBytes[dtype], nullptr, 0, any_size, dtype == TS_I32 ? 4 : 8, false, true).bytes;
-    if (binned == 0 && env_int("TS_SCATTER_LDS", 1)) {
+    if (rr.ok) return rr.sort_bytes + rr.csr_bytes;
+    if (env_int("TS_SCATTER_LDS", 1)) {
       // one 4-byte value per entry: (row in bucket, value) words, 8 bytes of scratch per entry
       const size_t payload = bin_plan_payload(B, E, K, N, kElemBytes[dtype], nullptr, 0, any_size).bytes;
       if (payload != 0) return payload;
@@ -578,14 +642,10 @@ size_t ts_scatter_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, in
         if (slabs != 0) return slabs;
       }
     }
-    if (binned == 0) {
-      // one word for the sample of the index that keeps a sorted one away from the table kernel
-      const bool table = (is_float_dtype(dtype) || dtype == TS_I32 || dtype == TS_I64) &&
-                         env_int("TS_SCATTER_LDS", 1) == 1 && sum_table_by_size(B, E, K, N, kElemBytes[dtype]);
-      return table ? 256 : 0;
-    }
-    const SortedRoute sr = sorted_route_plan(B, E, K, N, dtype, reduce);
-    return binned + (sr.ok ? sr.ptr_bytes + sr.csr_bytes : 0);
+    // one word for the sample of the index that keeps a sorted one away from the table kernel
+    const bool table = (is_float_dtype(dtype) || dtype == TS_I32 || dtype == TS_I64) &&
+                       env_int("TS_SCATTER_LDS", 1) == 1 && sum_table_by_size(B, E, K, N, kElemBytes[dtype]);
+    return table ? 256 : 0;
   }
   return 0;
 }
@@ -646,36 +706,28 @@ int scatter_ws_impl(const void *src, const int64_t *index, void *out, int64_t *a
   }
   const int full = kVecBytes / kElemBytes[dtype];
   const int vec = (full > 1 && K % full == 0 && aligned16(src)) ? full : 1;
-  // sorted index: finished by the segmented reduction (see sorted_route_plan); its workspace lies behind the buckets'
-  const int *route_flag = nullptr;
-  size_t bin_bytes = 0;
-  SortedRoute sr = {false, 0, 0};
-  if (a.bin_ws != nullptr && !out_given && index_stride_k == 0 && index_stride_e == 1 && B * E * K > 0) {
-    const bool any_size = a.bin_any_size != 0;
-    if (reduce == TS_MIN || reduce == TS_MAX)
-      bin_bytes = kElemBytes[dtype] > 4 ? 0 : bin_plan(B, E, K, N, kElemBytes[dtype], nullptr, 0, any_size, 8, true).bytes;
-    else if (reduce == TS_SUM && kAccBytes[dtype] >= 4)
-    {
-      bin_bytes = bin_plan(B, E, K, N, kElemBytes[dtype], nullptr, 0, any_size, dtype == TS_I32 ? 4 : 8, false, true).bytes;
-      if (bin_bytes == 0 && env_int("TS_SCATTER_LDS", 1))
-        bin_bytes = bin_plan_payload(B, E, K, N, kElemBytes[dtype], nullptr, 0, any_size).bytes;
-    }
-    if (bin_bytes != 0) sr = sorted_route_plan(B, E, K, N, dtype, reduce);
-    if (sr.ok && workspace_bytes >= bin_bytes + sr.ptr_bytes + sr.csr_bytes) {
-      a.sorted_route = 1;
-      a.route_flag = &route_flag;
-      a.route_ptr = reinterpret_cast<int64_t *>(static_cast<char *>(workspace) + bin_bytes);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (a.bin_ws != nullptr && index_stride_k == 0 && B * E * K > 0 && aligned16(workspace)) {
+    const RowsRoute rr = rows_route(B, E, K, N, dtype, reduce);
+    if (rr.ok && workspace_bytes >= rr.sort_bytes + rr.csr_bytes) {
+      RowSortPlan sp = row_sort_plan(B, E, N, workspace, rr.sort_bytes);
+      if (!sp.ok) return TS_ERR_WORKSPACE;
+      ts_note_scatter_route(reduce == TS_SUM ? TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED : TS_ROUTE_MINMAX_BUCKETS_OR_SEGMENTED);
+      int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, s);
+      if (rc != TS_OK) return rc;
+      rc = run_rows_reduce(src, sp.p.perm, sp.p.ptr, out, arg_out, B, E, K, N, dtype, reduce, out_given,
+                           static_cast<char *>(workspace) + rr.sort_bytes, rr.csr_bytes, s);
+      if (rc != TS_OK || count_out == nullptr) return rc;
+      hipLaunchKernelGGL(row_lengths_kernel, dim3(grid_for(B * N)), dim3(kBlock), 0, s, sp.p.ptr, count_out, B * N);
+      if (count_done != nullptr) *count_done = 1;
+      return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
     }
   }
-  if (reduce == TS_SUM && bin_bytes == 0 && workspace != nullptr && workspace_bytes >= 256 && aligned16(workspace))
+  if (reduce == TS_SUM && workspace != nullptr && workspace_bytes >= 256 && aligned16(workspace) &&
+      !(env_int("TS_SCATTER_LDS", 1) &&
+        bin_plan_payload(B, E, K, N, kElemBytes[dtype], nullptr, 0, a.bin_any_size != 0).bytes != 0))
     a.order_ws = static_cast<int *>(workspace);
-  const int rc = dispatch_scatter(dtype, a, reduce, vec, static_cast<hipStream_t>(stream));
-  if (rc != TS_OK || route_flag == nullptr) return rc;
-  // the row pointers of a sorted index come from the place pass of the buckets (bin_place_kernel)
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  return run_csr_reduce(src, a.route_ptr, out, arg_out, nullptr, B, N, E, K, N + 1, dtype, reduce, 0,
-                        static_cast<char *>(workspace) + bin_bytes + sr.ptr_bytes, sr.csr_bytes, nullptr, s, nullptr, 0,
-                        nullptr, route_flag, 1);
+  return dispatch_scatter(dtype, a, reduce, vec, s);
 }
 }  // namespace
 extern "C" {
@@ -736,7 +788,7 @@ int ts_scatter_count_with_workspace(const int64_t *index, int32_t *count, int64_
         // kernel below), even (the buckets); without the table kernel or the sample only the first and the last
         three_way = a.lds_cache == 1 && sum_table_by_size(B, E, 1, N, 4) && B * E >= 2 * kBinBlock &&
                     !getenv("TS_BIN_NO_SAMPLE");
-        launch_binned_add<int32_t, 1>(a, bp.p, 0, s, 0, three_way);
+        launch_binned_add<int32_t>(a, bp.p, s, three_way);
         a.skip_flag = bp.p.unsorted;
         binned = true;
       }
@@ -792,11 +844,8 @@ int ts_scatter_sum_count_with_workspace(const void *src, const int64_t *index, v
                   env_int("TS_SCATTER_LDS", 1) && env_int("TS_SCATTER_BINNED", 1);
   if (may_fuse) {  // only where the sum has a plan for the buckets (else count is cleared by its own call below)
     const bool any_size = env_int("TS_SCATTER_BINNED", 1) == 2;
-    bool planned = kAccBytes[dtype] >= 4 && bin_plan(B, E, K, N, kElemBytes[dtype], workspace, workspace_bytes, any_size,
-                                                     dtype == TS_I32 ? 4 : 8, false, true).ok;
-    if (!planned && K <= kBinPayloadCols && (dtype == TS_F32 || dtype == TS_I32))
-      planned = bin_plan_payload(B, E, K, N, 4, workspace, workspace_bytes, any_size).ok;
-    may_fuse = planned;
+    may_fuse = K <= kBinPayloadCols && (dtype == TS_F32 || dtype == TS_I32) &&
+               bin_plan_payload(B, E, K, N, 4, workspace, workspace_bytes, any_size).ok;
   }
   if (may_fuse)
     hipLaunchKernelGGL(fill_kernel<int32_t>, dim3(grid_for(B * N)), dim3(kBlock), 0, s, count, B * N, (int32_t)0);

@@ -345,10 +345,7 @@ constexpr int kCooPtrPerThread = 4;
 template <int PER>
 static __global__ __launch_bounds__(kBlock) void coo_to_indptr_kernel(const int64_t *__restrict__ index,
                                                                int64_t *__restrict__ ptr, int64_t N,
-                                                               int64_t E, int64_t index_batch_stride,
-                                                               const int *gate = nullptr, int gate_want = 0) {
-  // gate (optional): run only if (*gate != 0) == (gate_want != 0) -- a scatter that found its index sorted
-  if (gate != nullptr && (*gate != 0) != (gate_want != 0)) return;
+                                                               int64_t E, int64_t index_batch_stride) {
   __shared__ GapList s_gaps;
   if (threadIdx.x == 0) s_gaps.n = 0;
   __syncthreads();

@@ -73,13 +73,11 @@ struct CsrReduceArgs {
   // look-back ran out of polls ("the latest call that gave a row up"). The call gave a row up iff the two are
   // equal afterwards: no write has to be ordered against another one, and a word left by an earlier call
   // never matches.
-  // optional gate (a scatter whose index turned out to be sorted takes this reduction instead of the buckets):
-  // the kernel returns at once unless (*gate != 0) == (gate_want != 0). scatter_rule: min / max write a slot whose
-  // entries never beat the initial value of the element type as 0 with position E, as scatter does
-  // (csrc/cpu/scatter_cpu.cpp:81-82). Both need the look-back mode and a call without perm / accumulate.
-  const int *gate = nullptr;
-  int gate_want = 0;
-  int scatter_rule = 0;
+  // rows of a scatter through perm in any order inside a row (row_sort.h): B and N flattened into one list of rows;
+  // arg_E: entries per batch, so that positions come out inside their batch. accumulate: combined with out.
+  int any_order = 0;
+  int64_t arg_E = 0;
+  int meta_stride = 4;  // words of ws_meta per tile: at least one carry flag per column chunk
   unsigned long long *status;
   int status_reset;
   uint64_t status_nonce;  // never 0; the same for every slice of one call
@@ -122,29 +120,55 @@ template <typename A> __device__ __forceinline__ A carry_get(A *p) {
   return v;
 }
 
-template <typename A, int REDUCE>
+// TIES: entries come in any order; among equal values the smaller position wins
+template <typename A, int REDUCE, bool TIES = false>
 __device__ __forceinline__ void reduce_step(A &acc, int32_t &arg, A v, int32_t e) {
   if (REDUCE == TS_SUM || REDUCE == TS_MEAN) {
     acc = acc + v;
   } else if (REDUCE == TS_MIN) {
-    if (v < acc) { acc = v; arg = e; }
+    if (v < acc || (TIES && v == acc && e < arg)) { acc = v; arg = e; }
   } else {
-    if (v > acc) { acc = v; arg = e; }
+    if (v > acc || (TIES && v == acc && e < arg)) { acc = v; arg = e; }
   }
+}
+
+// The type a reduction runs in. Scatter through perm (PERM == 2): floating sums in double, as the LDS tables of the other
+// scatter kernels hold them; small integers in 32 bits, which the carries need.
+template <typename T, int REDUCE, int PERM> struct CsrAcc { typedef typename Acc<T>::type type; };
+template <typename T> struct ScatterAcc { typedef T type; };
+template <> struct ScatterAcc<float> { typedef double type; };
+template <> struct ScatterAcc<bf16_t> { typedef double type; };
+template <> struct ScatterAcc<f16_t> { typedef double type; };
+template <> struct ScatterAcc<int16_t> { typedef int32_t type; };
+template <> struct ScatterAcc<int8_t> { typedef int32_t type; };
+template <> struct ScatterAcc<uint8_t> { typedef int32_t type; };
+template <typename T> struct CsrAcc<T, TS_SUM, 2> { typedef typename ScatterAcc<T>::type type; };
+template <typename T> struct CsrAcc<T, TS_MEAN, 2> { typedef typename ScatterAcc<T>::type type; };
+template <typename T, typename A> struct MinMaxAcc { typedef A type; };
+template <typename T> struct MinMaxAcc<T, int16_t> { typedef int32_t type; };
+template <typename T> struct MinMaxAcc<T, int8_t> { typedef int32_t type; };
+template <typename T> struct MinMaxAcc<T, uint8_t> { typedef int32_t type; };
+template <typename T> struct CsrAcc<T, TS_MIN, 2> { typedef typename MinMaxAcc<T, typename Acc<T>::type>::type type; };
+template <typename T> struct CsrAcc<T, TS_MAX, 2> { typedef typename MinMaxAcc<T, typename Acc<T>::type>::type type; };
+// initial value: that of the element type (a 32-bit accumulator of bytes starts at the bytes' limits)
+template <typename T, typename A, int REDUCE> __device__ __forceinline__ A csr_acc_init() {
+  return (A)acc_init<typename Acc<T>::type, REDUCE>();
 }
 
 // Write one finished row slice. `count` is the full length of the row.
 // ACCUM: 0 = `out` is overwritten (known at compile time: the row-end code sits in divergent control flow,
 // where every instruction counts), -1 = decided by a.accumulate at run time.
-// PERM: 0 rows in place, 1 rows through a.perm, 2 rows in place under a.gate with scatter's rule for min / max
+// PERM: 0 rows in place, 1 rows through a.perm, 2 scatter through a.perm with the entries of a row in any order (arg then holds entry numbers, INT32_MAX: none)
 template <typename T, int VEC, int REDUCE, int ACCUM = -1, int PERM = 0>
 __device__ __forceinline__ void finalize_row_at(const CsrReduceArgs &a, T *op, int64_t *ap, T *count_slot,
-                                                const typename Acc<T>::type *acc, const int32_t *arg,
+                                                const typename CsrAcc<T, REDUCE, PERM>::type *acc, const int32_t *arg,
                                                 int64_t count, const int32_t *perm_b = nullptr) {
   // op / ap: the row's slice in out / arg_out; count_slot: where the row's count goes (mean with a count output)
-  typedef typename Acc<T>::type A;
+  typedef typename Acc<T>::type F;
+  typedef typename CsrAcc<T, REDUCE, PERM>::type A;
   const bool accumulate = ACCUM < 0 ? a.accumulate != 0 : ACCUM != 0;
-  if (accumulate && count == 0) return;  // rows without entries keep their content
+  constexpr bool kMinMax = REDUCE == TS_MIN || REDUCE == TS_MAX;
+  if (accumulate && count == 0 && !(PERM == 2 && kMinMax)) return;  // rows without entries keep their content
   Vec<T, VEC> o;
   int64_t oa[VEC];
   Vec<T, VEC> prev;
@@ -153,12 +177,20 @@ __device__ __forceinline__ void finalize_row_at(const CsrReduceArgs &a, T *op, i
   for (int v = 0; v < VEC; ++v) {
     A x = acc[v];
     if (REDUCE == TS_SUM || REDUCE == TS_MEAN) {
-      if (accumulate) x = to_acc<T>(prev.v[v]) + x;
-      T t = from_acc<T>(x);
+      if (accumulate) x = (A)to_acc<T>(prev.v[v]) + x;
+      T t = from_acc<T>((F)x);
       if (REDUCE == TS_MEAN && count > 1) t = div_elem<T>(t, count_as<T>(count));  // x / 1 == x
       o.v[v] = t;
     } else {
-      if (accumulate) {
+      if constexpr (PERM == 2) {
+        // an entry has to beat the previous content (none: the initial value of the element type) strictly
+        const A p = accumulate ? (A)to_acc<T>(prev.v[v])
+                               : (A)to_acc<T>(REDUCE == TS_MAX ? ElemLim<T>::lowest() : ElemLim<T>::max());
+        const bool beats = arg[v] != INT32_MAX && ((REDUCE == TS_MIN) ? (x < p) : (x > p));
+        o.v[v] = beats ? from_acc<T>((F)x) : (accumulate ? prev.v[v] : zero_elem<T>());
+        // position inside its batch
+        oa[v] = beats ? (int64_t)(a.arg_E == a.E ? (uint32_t)arg[v] : (uint32_t)arg[v] % (uint32_t)a.arg_E) : a.arg_E;
+      } else if (accumulate) {
         const A p = to_acc<T>(prev.v[v]);
         const bool beats = (REDUCE == TS_MIN) ? (x < p) : (x > p);
         o.v[v] = beats ? from_acc<T>(x) : prev.v[v];
@@ -166,14 +198,14 @@ __device__ __forceinline__ void finalize_row_at(const CsrReduceArgs &a, T *op, i
       } else {
         o.v[v] = count > 0 ? from_acc<T>(x) : zero_elem<T>();
         oa[v] = count > 0 ? (int64_t)arg[v] : a.E;
-        if constexpr (PERM != 0) {
-          if ((PERM == 2 || perm_b != nullptr) && count > 0) {
+        if constexpr (PERM == 1) {
+          if (perm_b != nullptr && count > 0) {
             // scatter's view of the slot: the position in src's order, or 0 and E if nothing beat the initial
             // value of the element type (csrc/cpu/scatter_cpu.cpp:81-82)
             const A lim = to_acc<T>(REDUCE == TS_MAX ? ElemLim<T>::lowest() : ElemLim<T>::max());
             const A xv = to_acc<T>(o.v[v]);
             if ((REDUCE == TS_MAX) ? (xv > lim) : (xv < lim)) {
-              if (PERM == 1) oa[v] = perm_b[arg[v]];
+              oa[v] = perm_b[arg[v]];
             } else {
               o.v[v] = zero_elem<T>();
               oa[v] = a.E;
@@ -194,7 +226,7 @@ __device__ __forceinline__ void finalize_row_at(const CsrReduceArgs &a, T *op, i
 template <typename T, int VEC, int REDUCE, int ACCUM = -1, int PERM = 0>
 __device__ __forceinline__ void finalize_row(const CsrReduceArgs &a, T *out_b, int64_t *arg_b,
                                              T *count_b, int64_t row, int64_t col, int lg,
-                                             const typename Acc<T>::type *acc, const int32_t *arg,
+                                             const typename CsrAcc<T, REDUCE, PERM>::type *acc, const int32_t *arg,
                                              int64_t count, bool col_ok, const int32_t *perm_b = nullptr) {
   if (!col_ok) return;
   constexpr bool kArg = REDUCE == TS_MIN || REDUCE == TS_MAX;
@@ -207,25 +239,25 @@ __device__ __forceinline__ void finalize_row(const CsrReduceArgs &a, T *out_b, i
 // mean would take 82 and drop to five, measured 7 % slower on 146 MB inputs). The other instantiations keep
 // the compiler's choice (forcing five on the 16-bit mean cost 3 % on 16 GB inputs).
 template <typename T, int VEC, int REDUCE, int PERM = 0> constexpr int csr_reduce_min_blocks() {
-  return PERM == 1 ? 1 : ((REDUCE == TS_SUM || REDUCE == TS_MEAN) && sizeof(T) >= 4 ? 6 : 1);  // PERM: 8 KB more LDS
+  return PERM == 1 || PERM == 2 ? 1 : ((REDUCE == TS_SUM || REDUCE == TS_MEAN) && sizeof(T) >= 4 ? 6 : 1);  // PERM: 8 KB more LDS
 }
 template <typename T, int VEC, int REDUCE, int ACCUM, int PERM = 0>
 __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, PERM>())) void csr_reduce_kernel(CsrReduceArgs a) {
-  typedef typename Acc<T>::type A;
+  typedef typename CsrAcc<T, REDUCE, PERM>::type A;
   constexpr bool kArg = (REDUCE == TS_MIN || REDUCE == TS_MAX);
+  constexpr bool kTies = PERM == 2;  // the entries of a row come in any order
+  constexpr bool kThrough = PERM == 1 || PERM == 2;
   constexpr int U = kLoadsInFlight;
 
-  __shared__ int32_t s_ptr[kCsrMaxItems + 4];  // row pointers of the tile + one sentinel
-  __shared__ int32_t s_perm[PERM == 1 ? kCsrMaxItems : 1];  // source rows of the tile's entries
+  // row pointers of the tile + sentinels, behind them (through perm) the source rows of the tile's entries: together
+  // one word per item of the tile
+  extern __shared__ int32_t s_ptr[];
   __shared__ A s_val[2 * kCsrBlock * VEC];
   __shared__ int32_t s_arg[kArg ? 2 * kCsrBlock * VEC : 1];
   __shared__ int32_t s_head_row[kCsrBlock];    // local row of the head partial, -1: none
   __shared__ int32_t s_head_closes[kCsrBlock];
   __shared__ int32_t s_tail_row[kCsrBlock];    // local row of the tail partial, -1: none
   __shared__ int64_t s_cut[2];
-  if constexpr (PERM == 2) {
-    if (a.gate != nullptr && (*a.gate != 0) != (a.gate_want != 0)) return;  // the same for every wavefront of the grid
-  }
 
   const int tid = threadIdx.x;
   const int G = a.G;
@@ -260,7 +292,9 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   if (a.status_reset && a.status != nullptr && tid == 0 && (blockIdx.x | blockIdx.y | blockIdx.z) == 0)
     __hip_atomic_exchange(a.status, (unsigned long long)a.status_nonce, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
-  const int64_t i0 = s_cut[0], i1 = s_cut[1];
+  const int64_t i0 = s_cut[0];
+  // (row pointers that are not monotone give cuts that cross: no more rows than the tile has items, so that LDS holds them)
+  const int64_t i1 = s_cut[1] < i0 ? i0 : (s_cut[1] > i0 + (d1 - d0) ? i0 + (d1 - d0) : s_cut[1]);
   const int64_t j0 = d0 - i0;
   const int nr = (int)(i1 - i0);         // row ends inside the tile
   const int ne = (int)((d1 - i1) - j0);  // edges inside the tile
@@ -270,8 +304,9 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   const int nload = (int)(last - i0) + 1;  // ptr[i0 .. last]
   for (int t = tid; t < nload; t += kCsrBlock) s_ptr[t] = (int32_t)(ptr[i0 + t] - j0);
   if (tid == 0) { s_ptr[nload] = INT32_MAX; s_ptr[nload + 1] = INT32_MAX; }  // rows past the last one never end
+  int32_t *const s_perm = s_ptr + nload + 2;
   const int32_t *arg_perm = nullptr;  // set: positions leave the kernel in src's order
-  if constexpr (PERM == 1) {
+  if constexpr (kThrough) {
     const int32_t *perm_b = a.perm + b * a.perm_batch_stride;
     const int32_t last_row = a.E > 0 ? (int32_t)(a.E - 1) : 0;
     for (int t = tid; t < ne; t += kCsrBlock) {
@@ -304,7 +339,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   A acc[VEC];
   int32_t arg[VEC];
 #pragma unroll
-  for (int v = 0; v < VEC; ++v) { acc[v] = acc_init<A, REDUCE>(); arg[v] = 0; }
+  for (int v = 0; v < VEC; ++v) { acc[v] = csr_acc_init<T, A, REDUCE>(); arg[v] = kTies ? INT32_MAX : 0; }
 
   const bool has_work = (ri1 > ri0) || (je1 > je0);
   // the worker's first row began before the worker's first edge
@@ -336,7 +371,10 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
                                                    (int64_t)(int32_t)(rend - rbeg), arg_perm);  // the length fits 32 bits
     }
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) acc[v] = acc_init<A, REDUCE>();
+    for (int v = 0; v < VEC; ++v) {
+      acc[v] = csr_acc_init<T, A, REDUCE>();
+      if (kTies) arg[v] = INT32_MAX;
+    }
     ++r;
     op_row += a.K;  // the slices of row r in out / arg_out / count: no 64-bit multiply per row end
     if (kArg) ap_row += a.K;
@@ -354,7 +392,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       int ee = e + u < je1 ? e + u : je1 - 1;
-      const int64_t srow = PERM == 1 ? (int64_t)s_perm[ee] : j0 + ee;
+      const int64_t srow = kThrough ? (int64_t)s_perm[ee] : j0 + ee;
       x[u] = load_vec_stream<T, VEC>(src_col + srow * a.K);
     }
   };
@@ -368,9 +406,9 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
       const int ce = e + u;
       if (ce < je1) {
         while (ce >= rend) flush();
-        const int32_t ge = (int32_t)(j0 + ce);
+        const int32_t ge = kTies && kArg ? s_perm[ce] : (int32_t)(j0 + ce);
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) reduce_step<A, REDUCE>(acc[v], arg[v], to_acc<T>(x[u].v[v]), ge);
+        for (int v = 0; v < VEC; ++v) reduce_step<A, REDUCE, kTies>(acc[v], arg[v], (A)to_acc<T>(x[u].v[v]), ge);
       }
     }
 #pragma unroll
@@ -420,7 +458,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   int64_t *meta = a.ws_meta + (b * a.nblk + blockIdx.x) * 4;
 
   // look-back mode: this tile's carry slot is the second of its two partial slots
-  uint64_t *carry_flags = reinterpret_cast<uint64_t *>(a.ws_meta) + (b * a.nblk) * 4 + blockIdx.y;
+  uint64_t *carry_flags = reinterpret_cast<uint64_t *>(a.ws_meta) + (b * a.nblk) * a.meta_stride + blockIdx.y;
   // Where element v of this lane's slice sits inside a carry row. The lanes of a worker hold VEC neighbouring
   // columns each, so instruction v of a carry written column by column would touch G addresses VEC elements apart
   // -- every 64-byte sector of the row VEC times over, and each of those atomics is a read-modify-write of a
@@ -443,7 +481,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
     }
     asm volatile("" ::"v"(sink) : "memory");  // the returns are in: the carry is in memory
     if (lg == 0)
-      __hip_atomic_exchange(carry_flags + (int64_t)blockIdx.x * 4, (a.nonce << 2) | kind, __ATOMIC_RELAXED,
+      __hip_atomic_exchange(carry_flags + (int64_t)blockIdx.x * a.meta_stride, (a.nonce << 2) | kind, __ATOMIC_RELAXED,
                             __HIP_MEMORY_SCOPE_AGENT);
     }
   };
@@ -472,7 +510,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
         uint64_t f[PF];
 #pragma unroll
         for (int q = 0; q < PF; ++q)
-          f[q] = ready[q] ? 0 : __hip_atomic_fetch_or(carry_flags + (hi - q * stride) * 4, 0ull, __ATOMIC_RELAXED,
+          f[q] = ready[q] ? 0 : __hip_atomic_fetch_or(carry_flags + (hi - q * stride) * a.meta_stride, 0ull, __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_AGENT);
         bool all = true;
 #pragma unroll
@@ -509,7 +547,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
 #pragma unroll
           for (int v = 0; v < VEC; ++v) {
             if (kArg) {
-              reduce_step<A, REDUCE>(early[q][v], early_arg[q][v], acc[v], arg[v]);  // earlier entries win ties
+              reduce_step<A, REDUCE, kTies>(early[q][v], early_arg[q][v], acc[v], arg[v]);  // earlier entries win ties
               arg[v] = early_arg[q][v];
               acc[v] = early[q][v];
             } else {
@@ -523,7 +561,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
 #pragma unroll
         for (int q = 0; q < PF; ++q)
           if (q < n)
-            __hip_atomic_exchange(carry_flags + (hi - q * stride) * 4, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_exchange(carry_flags + (hi - q * stride) * a.meta_stride, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
     }
@@ -536,7 +574,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
       if (kArg)
-        reduce_step<A, REDUCE>(acc[v], arg[v], hv[v], ha[v]);
+        reduce_step<A, REDUCE, kTies>(acc[v], arg[v], hv[v], ha[v]);
       else
         acc[v] = acc[v] + hv[v];
     }
@@ -597,7 +635,10 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
             const bool ok = walk_back(first_tile, (int64_t)blockIdx.x - 1, 1);
             if (!ok) {
 #pragma unroll
-              for (int v = 0; v < VEC; ++v) acc[v] = acc_init<A, REDUCE>();  // the row is written as empty
+              for (int v = 0; v < VEC; ++v) {  // the row is written as empty
+                acc[v] = csr_acc_init<T, A, REDUCE>();
+                if (kTies) arg[v] = INT32_MAX;
+              }
             }
             finalize_row<T, VEC, REDUCE, ACCUM, PERM>(a, out_b, arg_b, count_b, i0 + row, col, lg, acc, arg,
                                                       ok ? (int64_t)s_ptr[row + 1] - (int64_t)s_ptr[row] : 0, col_ok,
@@ -632,7 +673,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
     const int64_t first_tile = s_cut[0];
     if (first_tile < 0) return;
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) { acc[v] = acc_init<A, REDUCE>(); arg[v] = INT32_MAX; }
+    for (int v = 0; v < VEC; ++v) { acc[v] = csr_acc_init<T, A, REDUCE>(); arg[v] = INT32_MAX; }
     const bool ok = walk_back(first_tile, (int64_t)blockIdx.x - 1 - w, W);
     A *part_val = s_val + (size_t)w * CW + lg * VEC;  // the head slots: read for the last time before the barrier
     int32_t *part_arg = s_arg + (kArg ? (size_t)w * CW + lg * VEC : 0);
@@ -661,7 +702,10 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
     const int row = s_head_row[0];
     if (!all_ok) {
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) acc[v] = acc_init<A, REDUCE>();  // the row is written as empty
+      for (int v = 0; v < VEC; ++v) {  // the row is written as empty
+        acc[v] = csr_acc_init<T, A, REDUCE>();
+        if (kTies) arg[v] = INT32_MAX;
+      }
     }
     finalize_row<T, VEC, REDUCE, ACCUM, PERM>(a, out_b, arg_b, count_b, i0 + row, col, lg, acc, arg,
                                               all_ok ? (int64_t)s_ptr[row + 1] - (int64_t)s_ptr[row] : 0, col_ok,
@@ -844,11 +888,11 @@ inline CsrPlan csr_plan(int64_t N, int64_t E, int64_t K, int elem_bytes, bool al
 }
 
 inline size_t csr_ws_bytes(const CsrPlan &p, int64_t B, int64_t K, int acc_bytes, bool with_arg,
-                           size_t *off_args, size_t *off_meta) {
+                           size_t *off_args, size_t *off_meta, int meta_stride = 4) {
   auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
   size_t vals = up((size_t)B * p.nblk * 2 * K * acc_bytes);
   size_t args = with_arg ? up((size_t)B * p.nblk * 2 * K * 4) : 0;
-  size_t meta = up((size_t)B * p.nblk * 4 * 8);
+  size_t meta = up((size_t)B * p.nblk * meta_stride * 8);
   if (off_args) *off_args = vals;
   if (off_meta) *off_meta = vals + args;
   return vals + args + meta;
@@ -857,16 +901,24 @@ inline size_t csr_ws_bytes(const CsrPlan &p, int64_t B, int64_t K, int acc_bytes
 template <typename T, int VEC, int REDUCE>
 int launch_csr_reduce_t(const CsrReduceArgs &a, const CsrPlan &p, int64_t B, hipStream_t stream) {
   dim3 grid((unsigned)p.nblk, (unsigned)p.ychunks, (unsigned)B);
-  if (a.perm != nullptr) {
+  const size_t lds = ((size_t)p.BI + 8) * 4;  // row pointers (row ends of the tile + 4 words) and source rows
+  // Rows in place, a pure stream: fewer workgroups per CU suit the memory system (reads next to writes), and LDS is what
+  // sets their number: 8 KB at least (2.3 KB: max of 9 M x 128 floats 1229 against 1212 us), 16 KB above 2 GB of 4- and
+  // 8-byte elements (the same 1197 us, sum of 9 M x 64 floats 519 -> 509 us; 1 GB 271 -> 274 us, 2-byte elements lose too)
+  const bool huge = sizeof(T) >= 4 && B * a.E * a.K * (int64_t)sizeof(T) >= (int64_t)2000000000;
+  const size_t floor0 = huge ? 16000 : 8240;
+  const size_t lds0 = lds > floor0 ? lds : floor0;
+  if (a.any_order) {
+    // (every row is finished inside the kernel: always in the look-back mode)
+    if (a.perm == nullptr || !(a.lookback || p.nblk <= 1)) return TS_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL((csr_reduce_kernel<T, VEC, REDUCE, -1, 2>), grid, dim3(kCsrBlock), lds, stream, a);
+  } else if (a.perm != nullptr) {
     if (a.accumulate) return TS_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((csr_reduce_kernel<T, VEC, REDUCE, 0, 1>), grid, dim3(kCsrBlock), 0, stream, a);
-  } else if (a.gate != nullptr || a.scatter_rule) {
-    if (a.accumulate || !(a.lookback || p.nblk <= 1)) return TS_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((csr_reduce_kernel<T, VEC, REDUCE, 0, 2>), grid, dim3(kCsrBlock), 0, stream, a);
+    hipLaunchKernelGGL((csr_reduce_kernel<T, VEC, REDUCE, 0, 1>), grid, dim3(kCsrBlock), lds, stream, a);
   } else if (a.accumulate)
-    hipLaunchKernelGGL((csr_reduce_kernel<T, VEC, REDUCE, -1>), grid, dim3(kCsrBlock), 0, stream, a);
+    hipLaunchKernelGGL((csr_reduce_kernel<T, VEC, REDUCE, -1>), grid, dim3(kCsrBlock), lds0, stream, a);
   else
-    hipLaunchKernelGGL((csr_reduce_kernel<T, VEC, REDUCE, 0>), grid, dim3(kCsrBlock), 0, stream, a);
+    hipLaunchKernelGGL((csr_reduce_kernel<T, VEC, REDUCE, 0>), grid, dim3(kCsrBlock), lds0, stream, a);
   if (p.nblk > 1 && !a.lookback) {  // a single tile has no rows that cross tiles
     const int W = kBlock / p.G;
     dim3 grid2((unsigned)((p.nblk + W - 1) / W), (unsigned)p.ychunks, (unsigned)B);

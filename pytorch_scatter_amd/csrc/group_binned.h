@@ -67,8 +67,6 @@ inline GroupBinPlan group_bin_plan(int64_t B, int64_t E, int64_t K, int64_t N, i
   BinArgs &p = r.p;
   p = BinArgs();
   p.rshift = rshift;
-  p.kc = (int)K;
-  p.slices = 1;
   p.nb = (int)nb;
   {
     const int64_t rounds = (n_edges + (int64_t)512 * kBinPlaceChunk - 1) / ((int64_t)512 * kBinPlaceChunk);

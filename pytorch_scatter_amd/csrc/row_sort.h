@@ -1,0 +1,600 @@
+// An index in any order -> the entries in order of their rows: perm (entry numbers) and row pointers, the input of
+// the segmented reductions (csr_reduce.h with rows through perm). Two levels: entries are binned by bucket of R
+// consecutive rows, then every bucket is sorted by row in LDS.
+//   count : at most 512 workgroups with equal shares of the index, each a histogram over the buckets in LDS that it adds
+//           to the bucket totals; also: is the index in order and inside [0, N)? The workgroup that arrives last turns
+//           the totals into bucket starts (a launch of its own for that took 10-15 us of a single CU's latencies).
+//   place : a workgroup per tile: the tile sorted by bucket in LDS, one atomic per bucket that occurs reserves the
+//           tile's run, (row in bucket, entry) words leave in runs. An index found in order gets its row pointers and
+//           the identity from this launch instead, and the passes behind it return at once.
+//   sort  : a workgroup per bucket of up to 8192 or 16384 entries: counting sort by row in LDS, row pointers and perm out. A
+//           bucket with more entries (hubs, few rows) is taken in chunks: their row counts meet in memory, the chunk
+//           that arrives last turns them into row pointers,
+//   place chunks : ... and the chunks then write their entries, each from its offset inside every row.
+// Entries of a row come in no particular order (a reader that needs the first of equal values compares positions).
+// Entries outside [0, N) are left out.
+// What it costs: 16 bytes of index, 8 written and 8 read per entry for the words, 4 for perm; the passes are bound by the
+// latency of their chains (load, rank, reserve, store), not by that traffic. us for clear / count / place / sort / place
+// chunks: 2.3 M entries onto 268 k rows 5 / 20 / 18 / 12 / 5, 10 M even onto 1 M rows 5 / 44 / 66 / 32 / 5, 10 M under a
+// Zipf(1.2) index onto 100 k rows 5 / 47 / 67 / 43 / 34. In front of a segmented reduction this replaced tables of output
+// rows in LDS per bucket (one LDS atomic per element, bank conflicts, slabs or atomics to put chunks together):
+// 2.3 M x 128 bf16, sum 660 -> 205 us; 10 M x 64 floats onto 1 M rows, sum / max 965 / 946 -> 719 / 843 us.
+#pragma once
+
+#include "device_utils.h"
+
+namespace ts {
+
+constexpr int kRsBlock = 1024;        // count, place
+constexpr int kRsPer = 8;             // entries per lane of place
+constexpr int kRsTile = kRsPer * kRsBlock;
+// entries that one sorting workgroup holds in LDS (in registers before: 16 per lane): 512 lanes below kRsLarge entries
+// (more, shorter workgroups: 2.3 M entries 10.7 against 16.8 us), 1024 above, where fewer buckets save more in count
+// and place (10 M entries onto 1 M rows: 138 against 147 us for the three passes)
+constexpr int kRsSortPer = 16;
+constexpr int64_t kRsLarge = (int64_t)1 << 22;
+constexpr int kRsMaxBuckets = 4096;   // histogram of count and place
+constexpr int kRsMaxShift = 13;       // rows per bucket (log2): histogram of the sorting workgroup
+constexpr int kRsCountPer = 8;
+constexpr int kRsCountGroups = 256;   // (512: twice the additions to the totals)
+
+struct RowSortArgs {
+  const int64_t *index;
+  int64_t sb, se;        // element strides of the index over batches and entries
+  int64_t B, E, N;
+  int64_t n, rows;       // B * E entries, B * N rows
+  int flat;              // one batch, unit stride: entry e is index[e] (no 64-bit multiplications per entry)
+  int rshift, nb;        // rows per bucket (log2), buckets
+  int cap;               // entries that one sorting workgroup takes
+  int max_big;           // buckets above that: at most this many ...
+  int max_chunks;        // ... in at most this many chunks
+  uint32_t *totals;      // [nb] entries per bucket, cleared by the call
+  uint32_t *sync;        // [0] ticket of the count pass, [1 ...] of every large bucket: cleared with totals
+  int32_t *state;        // [0] 0: the index is in order, 1: it is not; [1] chunks of large buckets; [2] large buckets
+  uint32_t *starts;      // [nb + 1]
+  uint32_t *cursor;      // [nb]
+  int32_t *chunk_info;   // [3][max_chunks]: bucket, first chunk of the bucket, number of the large bucket
+  uint32_t *row_cnt;     // [max_big << rshift]
+  uint32_t *chunk_off;   // [max_chunks << rshift] offset of a chunk's entries inside every row
+  uint64_t *binned;      // [n] (row in bucket << 32) | entry
+  int32_t *perm;         // [n] out
+  int64_t *ptr;          // [rows + 1] out
+};
+
+struct RowSortPlan {
+  bool ok;
+  RowSortArgs p;
+  size_t bytes;
+};
+
+inline RowSortPlan row_sort_plan(int64_t B, int64_t E, int64_t N, void *ws, size_t ws_bytes) {
+  RowSortPlan r;
+  r.ok = false;
+  r.bytes = 0;
+  RowSortArgs &p = r.p;
+  if (B < 1 || E < 1 || N < 1 || B > 0x7FFFFFFFll / E || B > 0x7FFFFFFFll / N) return r;
+  p.B = B;
+  p.E = E;
+  p.N = N;
+  p.n = B * E;
+  p.rows = B * N;
+  if (p.n > 0x7FFFF000ll || p.rows >= 0x7FFFF000ll) return r;
+  // Buckets: about 1024 (the tiles of place then write runs of 8 entries, 64 bytes), fewer for small inputs, more so
+  // that a bucket of average size stays below the capacity of a sorting workgroup.
+  p.cap = kRsSortPer * (p.n < kRsLarge ? 512 : 1024);
+  int64_t want = p.n / (p.cap / 4);
+  if (want > 1024) want = 1024;
+  if (want < 16) want = 16;
+  auto buckets = [&](int s) { return (p.rows + ((int64_t)1 << s) - 1) >> s; };
+  int rs = 0;
+  while (buckets(rs) > want) ++rs;
+  while (rs > 0 && buckets(rs - 1) <= kRsMaxBuckets && p.n / buckets(rs) > p.cap * 3 / 4) --rs;
+  if (rs > kRsMaxShift) {
+    rs = kRsMaxShift;
+    if (buckets(rs) > kRsMaxBuckets) return r;  // above 33.5 M rows
+  }
+  p.rshift = rs;
+  p.nb = (int)buckets(rs);
+  p.max_big = (int)(p.n / p.cap);
+  p.max_chunks = 2 * p.max_big;
+  auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+  size_t off = 0;
+  auto take = [&](size_t bytes) { const size_t o = off; off += up(bytes); return o; };
+  const size_t o_tot = take((size_t)p.nb * 4 + (size_t)(p.max_big + 1) * 4);  // totals, then the tickets
+  const size_t o_state = take(16);
+  const size_t o_st = take((size_t)(p.nb + 1) * 4), o_cur = take((size_t)p.nb * 4);
+  const size_t o_ci = take((size_t)p.max_chunks * 12);
+  const size_t o_rc = take(((size_t)p.max_big << rs) * 4), o_co = take(((size_t)p.max_chunks << rs) * 4);
+  const size_t o_bin = take((size_t)p.n * 8), o_perm = take((size_t)p.n * 4), o_ptr = take((size_t)(p.rows + 1) * 8);
+  r.bytes = off;
+  if (ws == nullptr || ws_bytes < off || (reinterpret_cast<uintptr_t>(ws) & 15) != 0) return r;
+  char *base = static_cast<char *>(ws);
+  p.totals = reinterpret_cast<uint32_t *>(base + o_tot);
+  p.sync = p.totals + p.nb;
+  p.state = reinterpret_cast<int32_t *>(base + o_state);
+  p.starts = reinterpret_cast<uint32_t *>(base + o_st);
+  p.cursor = reinterpret_cast<uint32_t *>(base + o_cur);
+  p.chunk_info = reinterpret_cast<int32_t *>(base + o_ci);
+  p.row_cnt = reinterpret_cast<uint32_t *>(base + o_rc);
+  p.chunk_off = reinterpret_cast<uint32_t *>(base + o_co);
+  p.binned = reinterpret_cast<uint64_t *>(base + o_bin);
+  p.perm = reinterpret_cast<int32_t *>(base + o_perm);
+  p.ptr = reinterpret_cast<int64_t *>(base + o_ptr);
+  r.ok = true;
+  return r;
+}
+
+// Adds 1 to counter[bucket] for every lane with bucket >= 0 and returns the value before the lane's own
+// addition. Twice over, the lanes that share the bucket of the first lane still waiting go through one atomic
+// of their leader (with a heavy-tailed index nearly all lanes: the bucket of the hubs, which would otherwise
+// queue up on one LDS address); whoever is left adds on its own.
+__device__ __forceinline__ int32_t bin_take(int32_t *counter, int32_t bucket) {
+  int32_t before = 0;
+  bool waiting = bucket >= 0;
+#pragma unroll
+  for (int round = 0; round < 2; ++round) {
+    const uint64_t todo = __ballot(waiting);
+    if (todo == 0) break;
+    // head and first are the same for the whole wavefront: scalar registers, v_readlane instead of a shuffle
+    const int head = __builtin_ctzll((unsigned long long)todo);
+    const int32_t first = __builtin_amdgcn_readlane(bucket, head);
+    const bool with_head = waiting && bucket == first;
+    const uint64_t same = __ballot(with_head);
+    // lanes of `same` below this one (v_mbcnt): the head's is 0
+    const int32_t below = (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+    int32_t base = 0;
+    if (with_head && below == 0) base = atomicAdd(&counter[first], __popcll(same));
+    base = __builtin_amdgcn_readlane(base, head);
+    if (with_head) {
+      before = base + below;
+      waiting = false;
+    }
+  }
+  if (waiting) before = atomicAdd(&counter[bucket], 1);
+  return before;
+}
+
+// As bin_take, with the leader's round only where many lanes share its bucket (an index in order, a hub): elsewhere
+// every lane adds on its own, which costs fewer instructions.
+__device__ __forceinline__ uint32_t rs_take(uint32_t *counter, int32_t bucket) {
+  const int32_t first = __builtin_amdgcn_readfirstlane(bucket);
+  const uint64_t same = __ballot(bucket == first);
+  if (__popcll(same) >= 16) {
+    uint32_t base = 0;
+    const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+    if (bucket == first) {
+      if (first >= 0 && below == 0) base = atomicAdd(&counter[first], (uint32_t)__popcll(same));
+    } else if (bucket >= 0) {
+      base = atomicAdd(&counter[bucket], 1u);
+    }
+    const uint32_t lead = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);  // the first lane is the leader
+    return bucket == first ? lead + below : base;
+  }
+  return bucket >= 0 ? atomicAdd(&counter[bucket], 1u) : 0u;
+}
+// the same without the value before
+__device__ __forceinline__ void rs_count_one(uint32_t *counter, int32_t bucket) {
+  const int32_t first = __builtin_amdgcn_readfirstlane(bucket);
+  const uint64_t same = __ballot(bucket == first);
+  uint32_t add = 1;
+  if (__popcll(same) >= 16) {  // the first lane adds for all that share its bucket
+    add = (threadIdx.x & (kWave - 1)) == 0 ? (uint32_t)__popcll(same) : (bucket == first ? 0u : 1u);
+  }
+  if (bucket >= 0 && add != 0) atomicAdd(&counter[bucket], add);
+}
+
+// row of entry be of the flattened [B, E], -1 for an index outside [0, N)
+__device__ __forceinline__ int32_t rs_node(const RowSortArgs &p, int64_t be) {
+  if (p.flat) {
+    const int64_t idx = p.index[be];
+    return (uint64_t)idx < (uint64_t)p.N ? (int32_t)idx : -1;
+  }
+  uint32_t b = 0, e = (uint32_t)be;
+  if (p.B > 1) { b = (uint32_t)be / (uint32_t)p.E; e = (uint32_t)be - b * (uint32_t)p.E; }
+  const int64_t idx = p.index[(int64_t)b * p.sb + (int64_t)e * p.se];
+  return (idx >= 0 && idx < p.N) ? (int32_t)((int64_t)b * p.N + idx) : -1;
+}
+
+// exclusive prefix sums of s[0 .. n), in place; every lane owns `per` neighbouring values. Returns the total.
+template <int BLOCK> __device__ __forceinline__ uint32_t rs_scan_lds(uint32_t *s, int n, uint32_t *s_wave) {
+  const int per = (n + BLOCK - 1) / BLOCK;
+  const int i0 = threadIdx.x * per;
+  int32_t mine = 0;
+  for (int j = 0; j < per; ++j) mine += i0 + j < n ? (int32_t)s[i0 + j] : 0;
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int32_t incl = wave_inclusive_sum(mine);
+  if (lane == kWave - 1) s_wave[wave] = (uint32_t)incl;
+  __syncthreads();
+  uint32_t run = (uint32_t)(incl - mine), total = 0;
+#pragma unroll
+  for (int w = 0; w < BLOCK / kWave; ++w) {
+    const uint32_t x = s_wave[w];
+    run += w < wave ? x : 0u;
+    total += x;
+  }
+  for (int j = 0; j < per; ++j) {
+    if (i0 + j >= n) break;
+    const uint32_t h = s[i0 + j];
+    s[i0 + j] = run;
+    run += h;
+  }
+  __syncthreads();
+  return total;
+}
+
+static __global__ __launch_bounds__(kBlock) void rs_clear_kernel(uint32_t *p, int n) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
+static __global__ __launch_bounds__(kRsBlock) void rs_count_kernel(RowSortArgs p) {
+  __shared__ uint32_t s_hist[kRsMaxBuckets];
+  __shared__ uint32_t s_wave[3][kRsBlock / kWave];
+  __shared__ int s_desc, s_last;
+  for (int i = threadIdx.x; i < p.nb; i += kRsBlock) s_hist[i] = 0;
+  if (threadIdx.x == 0) s_desc = 0;
+  __syncthreads();
+  const int64_t per = (p.n + gridDim.x - 1) / gridDim.x;
+  const int64_t lo = (int64_t)blockIdx.x * per;
+  const int64_t hi = lo + per < p.n ? lo + per : p.n;
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  int32_t node[kRsCountPer], next[kRsCountPer];
+  auto load = [&](int64_t b0, int32_t *x) {
+#pragma unroll
+    for (int j = 0; j < kRsCountPer; ++j) {
+      const int64_t be = b0 + threadIdx.x + (int64_t)j * kRsBlock;
+      x[j] = be < hi ? rs_node(p, be) : -1;
+    }
+  };
+  bool descent = false;
+  if (lo < hi) load(lo, node);
+  for (int64_t b0 = lo; b0 < hi; b0 += (int64_t)kRsCountPer * kRsBlock) {
+    load(b0 + (int64_t)kRsCountPer * kRsBlock, next);  // past the end every lane gets -1 without a load
+    // The entry before a lane's entry is the neighbouring lane's; the first lane of a wavefront needs the entry before
+    // the wavefront's first one: lane j loads it for row j (one load instruction for all rows).
+    int32_t edge = -1;
+    if (lane < kRsCountPer) {
+      const int64_t be = b0 + (int64_t)(threadIdx.x - lane) + (int64_t)lane * kRsBlock;
+      if (be > 0 && be < hi) edge = rs_node(p, be - 1);
+    }
+#pragma unroll
+    for (int j = 0; j < kRsCountPer; ++j) {
+      const int32_t e0 = __builtin_amdgcn_readlane(edge, j);
+      const int32_t up = lane_up1(node[j]);  // by every lane: lane 0's value is what lane 1 reads
+      const int32_t prev = lane == 0 ? e0 : up;
+      const bool live = b0 + threadIdx.x + (int64_t)j * kRsBlock < hi;
+      descent = descent || (live && node[j] < prev) || (live && node[j] < 0);
+    }
+#pragma unroll
+    for (int j = 0; j < kRsCountPer; ++j) {
+      rs_count_one(s_hist, node[j] >= 0 ? node[j] >> p.rshift : -1);
+      node[j] = next[j];
+    }
+  }
+  if (__ballot(descent) != 0) s_desc = 1;
+  __syncthreads();
+  uint32_t sink = 0;
+  for (int i = threadIdx.x; i < p.nb; i += kRsBlock) {
+    const uint32_t h = s_hist[i];
+    if (h != 0) sink |= atomicAdd(&p.totals[i], h);
+  }
+  asm volatile("" ::"v"(sink) : "memory");  // the returns are in: this workgroup's share is in the totals
+  __syncthreads();
+  // the ticket counts the workgroups in its low half and those that saw a descent in its high half
+  if (threadIdx.x == 0) {
+    const uint32_t t = atomicAdd(p.sync, 1u + (s_desc ? 0x10000u : 0u));
+    s_last = (t & 0xFFFFu) == gridDim.x - 1 ? 1 : 0;
+    s_desc = (s_desc != 0 || (t >> 16) != 0) ? 1 : 0;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  // ---- the last workgroup: bucket starts, and the chunks of buckets above p.cap entries
+  const bool unsorted = s_desc != 0;
+  constexpr int PER = kRsMaxBuckets / kRsBlock;
+  const int pb = (p.nb + kRsBlock - 1) / kRsBlock;
+  uint32_t t[PER];
+  int32_t sum_t = 0, sum_c = 0, sum_b = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = threadIdx.x * pb + j;
+    t[j] = (j < pb && i < p.nb) ? atomicOr(&p.totals[i], 0u) : 0u;  // read where the additions were performed
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    sum_t += (int32_t)t[j];
+    if (t[j] > (uint32_t)p.cap) {
+      sum_c += (int32_t)((t[j] + p.cap - 1) / p.cap);
+      sum_b += 1;
+    }
+  }
+  const int32_t it = wave_inclusive_sum(sum_t), ic = wave_inclusive_sum(sum_c), ib = wave_inclusive_sum(sum_b);
+  if (lane == kWave - 1) {
+    s_wave[0][wave] = (uint32_t)it;
+    s_wave[1][wave] = (uint32_t)ic;
+    s_wave[2][wave] = (uint32_t)ib;
+  }
+  __syncthreads();
+  uint32_t run_t = (uint32_t)(it - sum_t), run_c = (uint32_t)(ic - sum_c), run_b = (uint32_t)(ib - sum_b);
+  uint32_t all_t = 0, all_c = 0, all_b = 0;
+#pragma unroll
+  for (int w = 0; w < kRsBlock / kWave; ++w) {
+    run_t += w < wave ? s_wave[0][w] : 0u;
+    run_c += w < wave ? s_wave[1][w] : 0u;
+    run_b += w < wave ? s_wave[2][w] : 0u;
+    all_t += s_wave[0][w];
+    all_c += s_wave[1][w];
+    all_b += s_wave[2][w];
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = threadIdx.x * pb + j;
+    if (j >= pb || i >= p.nb) break;
+    p.starts[i] = run_t;
+    p.cursor[i] = run_t;
+    run_t += t[j];
+    if (t[j] > (uint32_t)p.cap) {
+      const uint32_t m = (t[j] + p.cap - 1) / p.cap;
+      for (uint32_t c = 0; c < m; ++c) {
+        p.chunk_info[run_c + c] = i;
+        p.chunk_info[p.max_chunks + run_c + c] = (int32_t)run_c;
+        p.chunk_info[2 * p.max_chunks + run_c + c] = (int32_t)run_b;
+      }
+      run_c += m;
+      ++run_b;
+    }
+  }
+  if (threadIdx.x == 0) {
+    p.starts[p.nb] = all_t;
+    p.ptr[p.rows] = (int64_t)all_t;
+    p.state[0] = unsorted ? 1 : 0;
+    p.state[1] = unsorted ? (int32_t)all_c : 0;
+    p.state[2] = unsorted ? (int32_t)all_b : 0;
+  }
+}
+
+// row pointers and identity for an index in order and inside [0, N): the tile of entries at lo
+__device__ __forceinline__ void rs_identity(const RowSortArgs &p, int64_t lo, GapList &s_gaps) {
+  if (threadIdx.x == 0) s_gaps.n = 0;
+  __syncthreads();
+  for (int j = 0; j < kRsPer; ++j) {
+    const int64_t be = lo + threadIdx.x + (int64_t)j * kRsBlock;
+    const bool live = be < p.n;
+    int64_t top = -1, bot = 0;
+    if (live) {
+      p.perm[be] = (int32_t)be;
+      top = rs_node(p, be);
+      bot = be == 0 ? 0 : (int64_t)rs_node(p, be - 1) + 1;
+    }
+    gap_rows(p.ptr, bot, top, be, s_gaps);
+    gap_rows(p.ptr, top + 1, live && be == p.n - 1 ? p.rows : top, p.n, s_gaps);
+  }
+  __syncthreads();
+  gap_rows_finish(p.ptr, s_gaps);
+}
+
+// (eight wavefronts per SIMD, i.e. at most 64 vector registers: two workgroups per CU)
+static __global__ __launch_bounds__(kRsBlock) __attribute__((amdgpu_waves_per_eu(8, 8)))
+void rs_place_kernel(RowSortArgs p) {
+  extern __shared__ uint32_t s_rows[];
+  static_assert(kRsTile * 8 + 2048 + kRsMaxBuckets * 8 <= 160 * 1024, "a workgroup's LDS: 160 KB with counts and bases");
+  __shared__ uint64_t s_stage[kRsTile];
+  __shared__ uint32_t s_wave[kRsBlock / kWave];
+  __shared__ GapList s_gaps;
+  uint32_t *s_cnt = s_rows;  // [nb] counts, then the tile's exclusive prefix
+  uint32_t *s_base = s_cnt + p.nb;                        // [nb] first word of the tile's run in every bucket
+  const int64_t lo = (int64_t)blockIdx.x * kRsTile;
+  if (p.state[0] == 0) {
+    rs_identity(p, lo, s_gaps);
+    return;
+  }
+  // the row counts of large buckets, for the next launch
+  const int64_t n_cnt = (int64_t)p.state[2] << p.rshift;
+  for (int64_t i = (int64_t)blockIdx.x * kRsBlock + threadIdx.x; i < n_cnt; i += (int64_t)gridDim.x * kRsBlock) p.row_cnt[i] = 0;
+  for (int i = threadIdx.x; i < p.nb; i += kRsBlock) s_cnt[i] = 0;
+  int32_t node[kRsPer];
+  uint32_t rank[kRsPer];
+#pragma unroll
+  for (int j = 0; j < kRsPer; ++j) {
+    const int64_t be = lo + threadIdx.x + (int64_t)j * kRsBlock;
+    node[j] = be < p.n ? rs_node(p, be) : -1;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kRsPer; ++j)
+    rank[j] = rs_take(s_cnt, node[j] >= 0 ? node[j] >> p.rshift : -1);
+  __syncthreads();
+  for (int i = threadIdx.x; i < p.nb; i += kRsBlock) {
+    const uint32_t h = s_cnt[i];
+    if (h != 0) s_base[i] = atomicAdd(&p.cursor[i], h);
+  }
+  __syncthreads();
+  const int total = (int)rs_scan_lds<kRsBlock>(s_cnt, p.nb, s_wave);
+  const uint32_t mask = (1u << p.rshift) - 1;
+#pragma unroll
+  for (int j = 0; j < kRsPer; ++j) {
+    if (node[j] < 0) continue;
+    const uint32_t b = (uint32_t)node[j] >> p.rshift;
+    const uint32_t be = (uint32_t)(lo + threadIdx.x + (int64_t)j * kRsBlock);
+    s_stage[s_cnt[b] + rank[j]] = ((uint64_t)b << 45) | ((uint64_t)((uint32_t)node[j] & mask) << 32) | be;
+  }
+  __syncthreads();
+  for (int pos = threadIdx.x; pos < total; pos += kRsBlock) {
+    const uint64_t w = s_stage[pos];
+    const uint32_t b = (uint32_t)(w >> 45);
+    p.binned[s_base[b] + ((uint32_t)pos - s_cnt[b])] = w & (((uint64_t)1 << 45) - 1);
+  }
+}
+
+template <int BLOCK>
+static __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BLOCK == 512 ? 6 : 8)))
+void rs_sort_kernel(RowSortArgs p) {
+  constexpr int CAP = kRsSortPer * BLOCK, CAP_LOG = BLOCK == 512 ? 13 : 14;
+  extern __shared__ uint32_t s_rows[];
+  __shared__ uint32_t s_stage[CAP];
+  __shared__ uint32_t s_wave[BLOCK / kWave];
+  __shared__ int s_last;
+  static_assert(CAP * 4 + 1024 + (4 << kRsMaxShift) <= 160 * 1024, "a workgroup's LDS: 160 KB with the row counts");
+  uint32_t *s_hist = s_rows;  // [rows per bucket]
+  if (p.state[0] == 0) return;
+  const int R = 1 << p.rshift;
+  int bucket = (int)blockIdx.x, chunk = -1, big = 0, first = 0;
+  if (bucket >= p.nb) {
+    chunk = bucket - p.nb;
+    if (chunk >= p.state[1]) return;
+    bucket = p.chunk_info[chunk];
+    first = p.chunk_info[p.max_chunks + chunk];
+    big = p.chunk_info[2 * p.max_chunks + chunk];
+  }
+  const uint32_t b_lo = p.starts[bucket], b_hi = p.starts[bucket + 1];
+  uint32_t lo = b_lo, hi = b_hi;
+  if (chunk < 0) {
+    if (hi - lo > (uint32_t)CAP) return;
+  } else {
+    lo = b_lo + (uint32_t)(chunk - first) * CAP;
+    hi = lo + CAP < b_hi ? lo + CAP : b_hi;
+  }
+  for (int i = threadIdx.x; i < R; i += BLOCK) s_hist[i] = 0;
+  const int cnt = (int)(hi - lo);
+  uint64_t word[kRsSortPer];  // (row, entry), then (row << CAP_LOG | rank, entry)
+#pragma unroll
+  for (int j = 0; j < kRsSortPer; ++j) {
+    const int i = j * BLOCK + (int)threadIdx.x;
+    word[j] = i < cnt ? p.binned[lo + (uint32_t)i] : 0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kRsSortPer; ++j) {
+    const int i = j * BLOCK + (int)threadIdx.x;
+    const uint32_t r = (uint32_t)(word[j] >> 32);
+    const uint32_t rank = rs_take(s_hist, i < cnt ? (int32_t)r : -1);
+    word[j] = ((uint64_t)(r << CAP_LOG | rank) << 32) | (uint32_t)word[j];
+  }
+  __syncthreads();
+  const int64_t row0 = (int64_t)bucket << p.rshift;
+  const int n_rows = p.rows - row0 < R ? (int)(p.rows - row0) : R;
+  if (chunk < 0) {
+    rs_scan_lds<BLOCK>(s_hist, R, s_wave);
+    for (int i = threadIdx.x; i < n_rows; i += BLOCK) p.ptr[row0 + i] = (int64_t)(lo + s_hist[i]);
+#pragma unroll
+    for (int j = 0; j < kRsSortPer; ++j) {
+      const int i = j * BLOCK + (int)threadIdx.x;
+      const uint32_t rr = (uint32_t)(word[j] >> 32);
+      if (i < cnt) s_stage[s_hist[rr >> CAP_LOG] + (rr & (CAP - 1))] = (uint32_t)word[j];
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < cnt; i += BLOCK) p.perm[lo + (uint32_t)i] = (int32_t)s_stage[i];
+    return;
+  }
+  // a chunk of a large bucket: its counts to the bucket's; what they found there is the chunk's offset inside every row
+  uint32_t sink = 0;
+  for (int i = threadIdx.x; i < R; i += BLOCK) {
+    const uint32_t h = s_hist[i];
+    if (h == 0) continue;
+    const uint32_t before = atomicAdd(&p.row_cnt[((int64_t)big << p.rshift) + i], h);
+    p.chunk_off[((int64_t)chunk << p.rshift) + i] = before;
+    sink |= before;
+  }
+  asm volatile("" ::"v"(sink) : "memory");  // the returns are in: the counts are in memory
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t m = (b_hi - b_lo + CAP - 1) / CAP;
+    s_last = atomicAdd(&p.sync[1 + big], 1u) == m - 1 ? 1 : 0;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  for (int i = threadIdx.x; i < R; i += BLOCK) s_hist[i] = atomicOr(&p.row_cnt[((int64_t)big << p.rshift) + i], 0u);
+  __syncthreads();
+  rs_scan_lds<BLOCK>(s_hist, R, s_wave);
+  for (int i = threadIdx.x; i < n_rows; i += BLOCK) p.ptr[row0 + i] = (int64_t)(b_lo + s_hist[i]);
+}
+
+// the chunks of large buckets: sorted by row in LDS like a bucket, then every row's run to its place
+template <int BLOCK>
+static __global__ __launch_bounds__(BLOCK) void rs_place_chunks_kernel(RowSortArgs p) {
+  constexpr int CAP = kRsSortPer * BLOCK, CAP_LOG = BLOCK == 512 ? 13 : 14;
+  extern __shared__ uint32_t s_rows[];
+  __shared__ uint32_t s_stage[CAP];
+  __shared__ uint16_t s_srow[CAP];
+  __shared__ uint32_t s_wave[BLOCK / kWave];
+  static_assert(CAP * 6 + 1024 + (4 << kRsMaxShift) <= 160 * 1024, "a workgroup's LDS: 160 KB with the row counts");
+  const int R = 1 << p.rshift;
+  uint32_t *s_hist = s_rows;      // [rows per bucket] counts, then the chunk's exclusive prefix
+  const int n_chunks = p.state[1];
+  for (int chunk = (int)blockIdx.x; chunk < n_chunks; chunk += (int)gridDim.x) {
+    const int bucket = p.chunk_info[chunk];
+    const uint32_t b_lo = p.starts[bucket], b_hi = p.starts[bucket + 1];
+    const uint32_t lo = b_lo + (uint32_t)(chunk - p.chunk_info[p.max_chunks + chunk]) * CAP;
+    const uint32_t hi = lo + CAP < b_hi ? lo + CAP : b_hi;
+    const int cnt = (int)(hi - lo);
+    const int64_t row0 = (int64_t)bucket << p.rshift;
+    const uint32_t *off = p.chunk_off + ((int64_t)chunk << p.rshift);
+    for (int i = threadIdx.x; i < R; i += BLOCK) s_hist[i] = 0;
+    uint64_t word[kRsSortPer];
+#pragma unroll
+    for (int j = 0; j < kRsSortPer; ++j) {
+      const int i = j * BLOCK + (int)threadIdx.x;
+      word[j] = i < cnt ? p.binned[lo + (uint32_t)i] : 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kRsSortPer; ++j) {
+      const int i = j * BLOCK + (int)threadIdx.x;
+      const uint32_t r = (uint32_t)(word[j] >> 32);
+    const uint32_t rank = rs_take(s_hist, i < cnt ? (int32_t)r : -1);
+    word[j] = ((uint64_t)(r << CAP_LOG | rank) << 32) | (uint32_t)word[j];
+    }
+    __syncthreads();
+    rs_scan_lds<BLOCK>(s_hist, R, s_wave);
+#pragma unroll
+    for (int j = 0; j < kRsSortPer; ++j) {
+      const int i = j * BLOCK + (int)threadIdx.x;
+      const uint32_t rr = (uint32_t)(word[j] >> 32);
+      if (i < cnt) {
+        const uint32_t pos = s_hist[rr >> CAP_LOG] + (rr & (CAP - 1));
+        s_stage[pos] = (uint32_t)word[j];
+        s_srow[pos] = (uint16_t)(rr >> CAP_LOG);
+      }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < cnt; i += BLOCK) {
+      const uint32_t r = s_srow[i];
+      p.perm[(uint32_t)p.ptr[row0 + r] + off[r] + ((uint32_t)i - s_hist[r])] = (int32_t)s_stage[i];
+    }
+    __syncthreads();
+  }
+}
+
+// entries of every row, from the row pointers
+static __global__ __launch_bounds__(kBlock) void row_lengths_kernel(const int64_t *ptr, int32_t *len, int64_t rows) {
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < rows; i += (int64_t)gridDim.x * kBlock)
+    len[i] = (int32_t)(ptr[i + 1] - ptr[i]);
+}
+
+inline int launch_row_sort(const RowSortArgs &args, const int64_t *index, int64_t sb, int64_t se, hipStream_t stream) {
+  RowSortArgs p = args;
+  p.index = index;
+  p.sb = sb;
+  p.se = se;
+  p.flat = p.B == 1 && se == 1;
+  const int n_clear = p.nb + 1 + p.max_big;
+  hipLaunchKernelGGL(rs_clear_kernel, dim3((unsigned)((n_clear + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream, p.totals,
+                     n_clear);
+  int64_t groups = (p.n + kRsCountPer * kRsBlock - 1) / (kRsCountPer * kRsBlock);
+  if (groups > kRsCountGroups) groups = kRsCountGroups;
+  hipLaunchKernelGGL(rs_count_kernel, dim3((unsigned)groups), dim3(kRsBlock), 0, stream, p);
+  hipLaunchKernelGGL(rs_place_kernel, dim3((unsigned)((p.n + kRsTile - 1) / kRsTile)), dim3(kRsBlock), (size_t)p.nb * 8,
+                     stream, p);
+  const dim3 gs((unsigned)(p.nb + p.max_chunks)), gc((unsigned)(p.max_chunks < 1024 ? p.max_chunks : 1024));
+  const size_t lds = (size_t)4 << p.rshift;
+  if (p.cap == kRsSortPer * 512) {
+    hipLaunchKernelGGL(rs_sort_kernel<512>, gs, dim3(512), lds, stream, p);
+    if (p.max_chunks > 0) hipLaunchKernelGGL(rs_place_chunks_kernel<512>, gc, dim3(512), lds, stream, p);
+  } else {
+    hipLaunchKernelGGL(rs_sort_kernel<1024>, gs, dim3(1024), lds, stream, p);
+    if (p.max_chunks > 0) hipLaunchKernelGGL(rs_place_chunks_kernel<1024>, gc, dim3(1024), lds, stream, p);
+  }
+  return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
+}
+
+}  // namespace ts

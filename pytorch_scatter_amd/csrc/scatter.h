@@ -247,14 +247,6 @@ struct ScatterArgs {
   int skew_probe = 1;              // min/max: sample the index for skew (needs 256 bytes of workspace): 0 never, 2 at any size
   const int *skew_flag = nullptr;  // min/max kernels behind the probe: run only if (*skew_flag != 0) == (skew_want != 0)
   int skew_want = 0;
-  // A caller that can finish the scatter with the segmented reduction when the index turns out to be sorted
-  // (it launches that reduction afterwards, gated on the flag) sets sorted_route. The launcher then lets the
-  // count pass of the buckets check the whole index (in order, inside [0, N)), reports through *route_flag the
-  // device flag that reads 0 for such an index once the count pass has run, and launches nothing else that
-  // would handle the sorted case; *route_flag stays null when the buckets were not taken.
-  int sorted_route = 0;
-  const int **route_flag = nullptr;
-  int64_t *route_ptr = nullptr;  // [B][N + 1]: the row pointers of a sorted index, written by the place pass
 };
 
 // Inputs for which the min/max launcher samples the index (see index_skew_kernel): rows of 2-256 columns of
@@ -1925,35 +1917,22 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
         }
       }
     }
-    // Large inputs with rows of 64 bytes and more, given a workspace: unless the index is sorted (found out by
-    // the first pass), the entries are binned by bucket of output rows and summed in LDS (scatter_binned.h);
-    // the kernels launched below then return at once. A sorted index stays with them: they combine its runs
-    // (or, for a caller with sorted_route, is left to that caller's segmented reduction: then out is cleared
-    // only if the buckets are going to add into it).
+    // Up to four 4-byte values per entry, given a workspace: the values travel with their bucket of output rows
+    // (bin_plan_payload) unless a sample of the index says otherwise; then the kernels launched below take the call.
     BinPlan bp;
     bp.ok = false;
-    int lshift = -1;
-    if constexpr (BinSlotOk<T>::value) {
-      if (reduce == TS_SUM && n_src > 0 && a.bin_ws != nullptr && a.sk == 0 && a.K % VEC == 0) {
-        bp = bin_plan(a.B, a.E, a.K, a.N, (int)sizeof(T), a.bin_ws, a.bin_ws_bytes, a.bin_any_size != 0,
-                      (int)sizeof(typename BinSlot<T>::type), false, true);
-        lshift = bp.ok ? bin_lane_shift(bp.p, VEC) : -1;
-        if constexpr (sizeof(T) == 4) {
-          // up to eight 4-byte values per entry: the values travel in the binned words (bin_plan_payload)
-          if (!bp.ok && a.K <= kBinPayloadCols && a.lds_cache) {
-            bp = bin_plan_payload(a.B, a.E, a.K, a.N, (int)sizeof(T), a.bin_ws, a.bin_ws_bytes, a.bin_any_size != 0);
-            lshift = bp.ok ? 0 : -1;
-          }
-        }
-      }
+    if constexpr (sizeof(T) == 4) {
+      if (reduce == TS_SUM && n_src > 0 && a.bin_ws != nullptr && a.sk == 0 && a.K <= kBinPayloadCols && a.lds_cache)
+        bp = bin_plan_payload(a.B, a.E, a.K, a.N, (int)sizeof(T), a.bin_ws, a.bin_ws_bytes, a.bin_any_size != 0);
     }
+    const bool payload = bp.ok;
     // Single 4-byte values between the sizes of the table kernel and of the value buckets, given a workspace: tables
     // handed over in slabs (scatter_k1_sum.h), with the counts of scatter mean if the caller wants them.
     // TS_SCATTER_SLABS (tuning aid): 0 never, 2 at any size.
     if constexpr (__is_same(T, float) || __is_same(T, int32_t)) {
       const char *env = getenv("TS_SCATTER_SLABS");
       const int slab_mode = env ? atoi(env) : 1;
-      if (reduce == TS_SUM && lshift < 0 && n_src > 0 && slab_mode != 0 && a.bin_ws != nullptr && a.sk == 0 && a.se == 1 &&
+      if (reduce == TS_SUM && !payload && n_src > 0 && slab_mode != 0 && a.bin_ws != nullptr && a.sk == 0 && a.se == 1 &&
           a.lds_cache == 1 && a.src != nullptr && (reinterpret_cast<uintptr_t>(a.src) & 15) == 0 &&
           (reinterpret_cast<uintptr_t>(a.index) & 15) == 0) {
         const bool with_count = a.count_out != nullptr && a.count_done != nullptr;
@@ -1974,19 +1953,15 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
         }
       }
     }
-    const bool routed = lshift >= 0 && a.sorted_route && a.route_flag != nullptr && !a.out_given;
     // sums that go through the LDS table (scatter_add_lds_kernel; the sizes and crossovers are with its launch
     // below), and whether a sample of the index picks between it and the run kernel
     bool use_lds = false, sampled = false, three_way = false;
-    const bool payload = lshift >= 0 && bp.p.payload != 0;
     int tn = 1;
     if constexpr (__is_same(T, float) || __is_same(T, bf16_t) || __is_same(T, f16_t) || __is_same(T, double) ||
                   __is_same(T, int32_t) || __is_same(T, int64_t)) {
       if (reduce == TS_SUM && n_src > 0) {
         while ((int64_t)tn * 2 * a.K <= kLdsAcc && tn * 2 <= kLdsAccRows) tn *= 2;
-        // (behind the buckets only an index in order arrives here: that one has the table only if contended)
-        const bool by_size = sum_table_by_size(a.B, a.E, a.K, a.N, (int)sizeof(T)) &&
-                             (lshift < 0 || payload || n_edges >= 32 * a.B * a.N);
+        const bool by_size = sum_table_by_size(a.B, a.E, a.K, a.N, (int)sizeof(T));
         use_lds = a.lds_cache && a.sk == 0 && tn >= 64 && a.B * a.N < 0x7FFFFFFFll && (a.lds_cache == 2 || by_size);
         // single values through the buckets: the sample of the index gives one of three answers (sorted: the run
         // kernel; skewed: the table kernel; even: the buckets), which needs the table kernel and the sample
@@ -1994,7 +1969,7 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
         if (payload && !three_way) use_lds = false;
         // (a sample of the index: from 2^23 elements, where a sorted index does better through the run kernel;
         // below, the table is level with it and the launch that returns at once would cost 2-4 us)
-        sampled = use_lds && a.lds_cache != 2 && a.order_ws != nullptr && a.skip_flag == nullptr && lshift < 0 &&
+        sampled = use_lds && a.lds_cache != 2 && a.order_ws != nullptr && a.skip_flag == nullptr && !payload &&
                   a.run_reduce && n_edges >= 2 * kBinBlock && n_src >= ((int64_t)1 << 23);
       }
     }
@@ -2002,14 +1977,14 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
     // itself: it counts too, and the counts are cleared with out
     bool count_here = false;
     if constexpr (!(std::is_integral<T>::value && sizeof(T) < 4)) {
-      count_here = a.count_out != nullptr && a.count_done != nullptr && use_lds && !sampled && !three_way && lshift < 0 &&
+      count_here = a.count_out != nullptr && a.count_done != nullptr && use_lds && !sampled && !three_way && !payload &&
                    a.lds_cache != 2 && !a.bin_any_size;
     }
     if (count_here) {
       const int64_t n_clear = (a.out_given ? 0 : n_out) + a.B * a.N;
       hipLaunchKernelGGL(fill_out_count_kernel<T>, dim3(grid_for(n_clear)), dim3(kBlock), 0, stream, out,
                          a.out_given ? (int64_t)0 : n_out, a.count_out, a.B * a.N);
-    } else if (!a.out_given && !routed) {
+    } else if (!a.out_given) {
       if (sampled)
         hipLaunchKernelGGL(fill_sample_kernel<T>, dim3(g_out), dim3(kBlock), 0, stream, out, n_out, small_const<T>(0),
                            a, a.order_ws);
@@ -2019,20 +1994,15 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
     } else if (sampled) {
       hipLaunchKernelGGL(bin_sample_kernel, dim3(1), dim3(kBinBlock), 0, stream, a, a.order_ws);
     }
-    if constexpr (BinSlotOk<T>::value) {
-      if (lshift >= 0) {
-        ts_note_scatter_route(payload ? TS_ROUTE_SUM_VALUE_BUCKETS : routed ? TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED
-                                                                              : TS_ROUTE_SUM_BUCKETS_OR_RUNS);
-        if (a.count_out != nullptr && a.count_flag != nullptr && (payload || bp.p.rshift <= kBinCountShift)) {
+    if constexpr (sizeof(T) == 4) {
+      if (payload) {
+        ts_note_scatter_route(TS_ROUTE_SUM_VALUE_BUCKETS);
+        if (a.count_out != nullptr && a.count_flag != nullptr) {
           bp.p.count_out = a.count_out;
           *a.count_flag = bp.p.unsorted;
         }
-        launch_binned_add<T, VEC>(a, bp.p, lshift, stream, routed ? n_out : 0, three_way);
+        launch_binned_add<T>(a, bp.p, stream, three_way);
         a.skip_flag = bp.p.unsorted;
-        if (routed) {
-          *a.route_flag = bp.p.unsorted;
-          return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
-        }
       }
     }
     if (n_src > 0) {
@@ -2059,7 +2029,7 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
             if (three_way) t.skip_want = 2;  // (skip_flag is the buckets' flag: 2 = unsorted and skewed)
             const int64_t epb = per_cu_chunk_edges(a.lds_epb, n_edges, sum_table_min_chunk(a.K, (int)sizeof(T)),
                                                    131072 / a.K > 2048 ? 131072 / a.K : 2048);
-            if (lshift < 0) ts_note_scatter_route(sampled ? TS_ROUTE_SUM_TABLE_OR_RUNS : TS_ROUTE_SUM_TABLE);
+            if (!payload) ts_note_scatter_route(sampled ? TS_ROUTE_SUM_TABLE_OR_RUNS : TS_ROUTE_SUM_TABLE);
             if (count_here) {
               hipLaunchKernelGGL((scatter_add_lds_kernel<T, false, true>), dim3((unsigned)((n_edges + epb - 1) / epb)),
                                  dim3(kLdsAddBlock), 0, stream, t, tn - 1, epb);
@@ -2068,7 +2038,7 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
             }
             // behind value buckets that count as well: the table kernel, which takes a skewed index from them, counts too
             // (*count_done = 2 tells the caller, which then has no table of counts to launch for that verdict)
-            if (three_way && lshift >= 0 && bp.p.count_out != nullptr && a.count_done != nullptr) {
+            if (three_way && bp.p.count_out != nullptr && a.count_done != nullptr) {
               hipLaunchKernelGGL((scatter_add_lds_kernel<T, false, true>), dim3((unsigned)((n_edges + epb - 1) / epb)),
                                  dim3(kLdsAddBlock), 0, stream, t, tn - 1, epb);
               *a.count_done = 2;
@@ -2089,7 +2059,7 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
             // rows that cannot be written word by word: one column per lane and atomic
             const RunGrid g = run_grid(n_edges, a.K, 1, (int)sizeof(T));
             if (g.ok) {
-              if (lshift < 0 && !use_lds) ts_note_scatter_route(TS_ROUTE_SUM_RUNS);
+              if (!payload && !use_lds) ts_note_scatter_route(TS_ROUTE_SUM_RUNS);
               launch_add_run<T, 1, 1>(a, g, stream);
               return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
             }
@@ -2102,7 +2072,7 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
             const RunGrid g = run_grid(n_edges, a.K / (wide ? C : CN), wide ? C : CN, (wide ? C : CN) * (int)sizeof(T));
             if (g.ok) {
               constexpr int EWD = sizeof(T) < 4 ? 4 / (int)sizeof(T) : 1;  // a whole 32-bit word per atomic
-              if (lshift < 0 && !use_lds) ts_note_scatter_route(TS_ROUTE_SUM_RUNS);
+              if (!payload && !use_lds) ts_note_scatter_route(TS_ROUTE_SUM_RUNS);
               if (wide)
                 launch_add_run<T, C, EWD>(a, g, stream);
               else
@@ -2211,24 +2181,6 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
               launch_scatter_k1<T, false>(a, kp, stream);
             return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
           }
-        }
-      }
-      if ((a.lds_cache || a.bin_any_size) && a.sk == 0 && a.B * a.N < 0x7FFFFFFFll && a.bin_ws != nullptr &&
-          a.K % VEC == 0 && n_src > 0) {
-        // large inputs of wide rows with a workspace: entries binned by bucket of output rows, no table misses.
-        // Also for an index with few entries per output row (10 M entries onto 1 M rows, uniform / Zipf(1.2) /
-        // sorted index: K = 16 894 / 784 / 537 -> 565 / 452 / 357 us, K = 32 1618 / 1169 / 662 -> 757 / 645 / 614 us)
-        const BinPlan bp = bin_plan(a.B, a.E, a.K, a.N, (int)sizeof(T), a.bin_ws, a.bin_ws_bytes, a.bin_any_size != 0, 8,
-                                    true);
-        if (bp.ok && (bp.p.slices == 1 || bin_lane_shift(bp.p, VEC) >= 0)) {
-          ts_note_scatter_route(a.sorted_route && a.route_flag != nullptr ? TS_ROUTE_MINMAX_BUCKETS_OR_SEGMENTED
-                                                                          : TS_ROUTE_MINMAX_BUCKETS);
-          if (is_max)
-            launch_binned_keys<T, VEC, true>(a, bp.p, stream);
-          else
-            launch_binned_keys<T, VEC, false>(a, bp.p, stream);
-          if (a.sorted_route && a.route_flag != nullptr) *a.route_flag = bp.p.unsorted;
-          return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
         }
       }
       // one index per row, few entries per slot: combine runs of equal neighbouring indices in the

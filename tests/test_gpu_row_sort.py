@@ -1,0 +1,56 @@
+"""Scatter of wide rows through the sort of the index by row (csrc/row_sort.h) at the sizes where it can go wrong: tiles
+of 8192 entries, buckets at and above what one sorting workgroup holds (8192 entries, 16384 from 4 M entries on), buckets
+of one row and of 8192 rows, entries outside [0, N), an index in order. Sums of int32 are exact; min / max must give the
+first position of equal values. The expected results come from torch on the same device."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _index(kind, E, N, g):
+    index = torch.randint(0, N, (E,), generator=g, device=DEV)
+    if kind == "one row":
+        index.fill_(N // 2)
+    elif kind.startswith("hub"):  # exactly so many entries in one row, the others elsewhere
+        n = int(kind[3:])
+        index = torch.where(index == N // 3, (N // 3 + 1) % N, index)
+        index[torch.randperm(E, generator=g, device=DEV)[:n]] = N // 3
+    elif kind == "sorted":
+        index = index.sort()[0]
+    elif kind == "outside":
+        index[::3] += N
+        index[1::7] = -1 - index[1::7]
+    return index
+
+
+CASES = [("even", 8191, 300), ("even", 8192, 300), ("even", 8193, 300), ("one row", 8192, 5), ("one row", 8193, 5),
+         ("one row", 50001, 1), ("hub8191", 20000, 40), ("hub8192", 20000, 40), ("hub8193", 20000, 40),
+         ("hub30000", 60001, 100000), ("even", 30000, 600001), ("sorted", 30001, 7000), ("outside", 30001, 7000),
+         ("even", 1, 1), ("even", 4194303, 70001), ("even", 4194305, 70001), ("hub16384", 4194305, 2000003),
+         ("hub16385", 4194305, 2000003), ("hub1000000", 4194304, 1000)]
+
+
+@pytest.mark.parametrize("kind,E,N", CASES)
+def test_row_sort(kind, E, N, monkeypatch):
+    from pytorch_scatter_amd import capi
+    monkeypatch.setenv("TS_SCATTER_BINNED", "2")
+    g = torch.Generator(device=DEV).manual_seed(E + N)
+    K = 16 if E > 100000 or N > 1000000 else 32
+    index = _index(kind, E, N, g)
+    ok = (index >= 0) & (index < N)
+    src = torch.randint(-50, 51, (E, K), generator=g, device=DEV, dtype=torch.int32)
+    out = torch.full((N, K), 9, dtype=torch.int32, device=DEV)
+    capi.scatter_with_workspace(src, index, out, None, 1, E, K, N, 0, 1, 0, capi.SUM, 0)
+    want = torch.zeros((N, K), dtype=torch.int32, device=DEV).index_add_(0, index[ok], src[ok])
+    assert torch.equal(out, want)
+    arg = torch.empty((N, K), dtype=torch.int64, device=DEV)
+    capi.scatter_with_workspace(src, index, out, arg, 1, E, K, N, 0, 1, 0, capi.MAX, 0)
+    idx = index[ok].view(-1, 1).expand(-1, K)
+    top = torch.full((N, K), -1000, dtype=torch.int32, device=DEV).scatter_reduce_(0, idx, src[ok], "amax")
+    pos = torch.nonzero(ok).expand(-1, K)
+    first = torch.where(src[ok] == top.gather(0, idx), pos, E)
+    want_arg = torch.full((N, K), E, dtype=torch.int64, device=DEV).scatter_reduce_(0, idx, first, "amin")
+    assert torch.equal(out, torch.where(want_arg < E, top, 0))
+    assert torch.equal(arg, want_arg)
