@@ -429,8 +429,11 @@ int ts_group_std_backward_with_workspace(const void *src, const int64_t *index, 
  * ts_group_std_forward writes the group sums (total, element type), the entries per group (count, int32) and the
  * standard deviation (out) in one call: what ts_scatter(sum) + ts_scatter_count + ts_group_std leave. It needs that
  * workspace: TS_ERR_UNSUPPORTED when the route does not apply, TS_ERR_WORKSPACE when the workspace is too small.
+ * Where the buckets do not apply, wide rows of large inputs go through a sort of the entries by group instead:
+ * ts_group_std_workspace_bytes() is the scratch of whichever route serves the call, 0 when none does.
  * ts_group_logsumexp takes the same route by itself when its workspace has that size. */
 size_t ts_group_bins_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype);
+size_t ts_group_std_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype);
 /* The workspace with which every route of ts_group_softmax, ts_group_softmax_backward and ts_group_logsumexp is open
  * to a call of this shape: the three passes' part (ts_group_softmax_workspace_bytes), the buckets of groups where
  * they apply, and behind them the records of the one-pass tiles (which otherwise live in the three passes' part and

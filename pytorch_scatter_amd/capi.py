@@ -29,7 +29,7 @@ EXPORTS = (
     "ts_scatter", "ts_scatter_workspace_bytes", "ts_scatter_workspace_zero_bytes", "ts_scatter_with_workspace", "ts_scatter_count", "ts_scatter_count_workspace_bytes", "ts_scatter_count_with_workspace", "ts_scatter_sum_count_workspace_bytes", "ts_scatter_sum_count_with_workspace", "ts_divide_by_count", "ts_arg_backward",
     "ts_group_softmax_workspace_bytes", "ts_group_softmax", "ts_group_softmax_backward",
     "ts_group_logsumexp", "ts_group_logsumexp_backward",
-    "ts_group_std", "ts_group_std_backward", "ts_group_bins_workspace_bytes", "ts_group_workspace_bytes", "ts_group_std_forward",
+    "ts_group_std", "ts_group_std_backward", "ts_group_bins_workspace_bytes", "ts_group_std_workspace_bytes", "ts_group_workspace_bytes", "ts_group_std_forward",
     "ts_group_std_backward_with_workspace", "ts_group_logsumexp_backward_with_workspace",
     "ts_index_to_indptr", "ts_indptr_to_index_workspace_bytes", "ts_indptr_to_index",
     "ts_sort_index_workspace_bytes", "ts_sort_index",
@@ -63,6 +63,7 @@ def lib() -> ctypes.CDLL:
         _lib.ts_scatter_sum_count_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_sort_index_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_group_bins_workspace_bytes.restype = ctypes.c_size_t
+        _lib.ts_group_std_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_group_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_segment_csr_permuted_workspace_bytes.restype = ctypes.c_size_t
     return _lib
@@ -337,10 +338,10 @@ def group_std(src, index, total, count, out, B, E, K, N, sb, se, unbiased: bool 
 
 
 def group_std_forward(src, index, total, count, out, B, E, K, N, sb, se, unbiased: bool = True):
-    """Group sums, counts and standard deviation in one call through buckets of groups (ts_group_std_forward).
-    Returns the bytes of workspace used; raises where the route does not apply."""
+    """Group sums, counts and standard deviation in one call (ts_group_std_forward): through buckets of groups, or the
+    entries sorted by group. Returns the bytes of workspace used; raises where neither applies."""
     _dev(src, index, total, count, out)
-    nbytes = group_bins_workspace_bytes(B, E, K, N, out.dtype)
+    nbytes = int(lib().ts_group_std_workspace_bytes(_i(B), _i(E), _i(K), _i(N), DTYPE[out.dtype]))
     ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=out.device)
     with torch.cuda.device(out.device):
         _check(lib().ts_group_std_forward(_p(src), _p(index), _p(total), _p(count), _p(out), _i(B), _i(E), _i(K), _i(N),

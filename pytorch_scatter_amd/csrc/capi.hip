@@ -216,7 +216,23 @@ inline int rows_acc_bytes(int dtype, int reduce) {
   return kElemBytes[dtype] == 8 || (sum && is_float_dtype(dtype)) ? 8 : 4;
 }
 CsrPlan rows_csr_plan(int64_t rows, int64_t n, int64_t K, int dtype, bool al, int reduce) {
-  return csr_plan(rows, n, K, kElemBytes[dtype], al, false, reduce == TS_MIN || reduce == TS_MAX, false);
+  const bool minmax = reduce == TS_MIN || reduce == TS_MAX;
+  CsrPlan p = csr_plan(rows, n, K, kElemBytes[dtype], al, false, minmax, false);
+  if (getenv("TS_CSR_IPW")) return p;  // tuning aid
+  // Items per worker: about 1024 workgroups, 24 ... 72 items each, up to 144 where a worker takes single columns. A hub
+  // row is put together from the carries of all its tiles, so short tiles cost there what they gain elsewhere (970 k x
+  // 33 floats, a fifth of them in one row: sum 327 / 156 / 123 us at 24 / 72 / 144 items, max 279 / 183 / 135; even
+  // index, std of 1 M x 33: 274 / 274 / 278 us; 240 k x 256 floats, hub: sum 154 / 108 / 98 us).
+  const int64_t items = rows + n;
+  const int W = kCsrBlock / p.G;
+  const int most = p.vec == 1 ? 144 : (items >= ((int64_t)32 << 20) ? 64 : 72), least = minmax ? 40 : 24;
+  int64_t want = items / ((int64_t)W * 1024);
+  want = want > most ? most : (want < least ? least : want);
+  const int cap = kCsrMaxItems / W;
+  p.ipw = want > cap ? cap : (int)want;
+  p.BI = W * p.ipw;
+  p.nblk = (items + p.BI - 1) / p.BI;
+  return p;
 }
 inline int rows_meta_stride(const CsrPlan &p) { return p.ychunks > 4 ? p.ychunks : 4; }
 RowsRoute rows_route(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce) {
@@ -258,12 +274,10 @@ RowsRoute rows_route(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int 
   return r;
 }
 // perm / ptr as launch_row_sort leaves them; ws: RowsRoute::csr_bytes
-int run_rows_reduce(const void *src, const int32_t *perm, const int64_t *ptr, void *out, int64_t *arg_out, int64_t B,
-                    int64_t E, int64_t K, int64_t N, int dtype, int reduce, int out_given, void *ws, size_t ws_bytes,
-                    hipStream_t s) {
+int rows_reduce_args(CsrReduceArgs &a, const CsrPlan &p, const void *src, const int32_t *perm, const int64_t *ptr, void *out,
+                     int64_t *arg_out, int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce, int out_given,
+                     void *ws, size_t ws_bytes) {
   const int64_t n = B * E, rows = B * N;
-  const CsrPlan p = rows_csr_plan(rows, n, K, dtype, aligned16(src) && aligned16(out), reduce);
-  CsrReduceArgs a;
   size_t off_args = 0, off_meta = 0;
   a.meta_stride = rows_meta_stride(p);
   if (csr_ws_bytes(p, 1, K, rows_acc_bytes(dtype, reduce), reduce == TS_MIN || reduce == TS_MAX, &off_args, &off_meta,
@@ -297,7 +311,15 @@ int run_rows_reduce(const void *src, const int32_t *perm, const int64_t *ptr, vo
   a.status_reset = 0;
   a.status_nonce = 0;
   a.carry_spin = kCarrySpin;
-  return dispatch_csr_reduce(dtype, a, p, 1, reduce, s);
+  return TS_OK;
+}
+int run_rows_reduce(const void *src, const int32_t *perm, const int64_t *ptr, void *out, int64_t *arg_out, int64_t B,
+                    int64_t E, int64_t K, int64_t N, int dtype, int reduce, int out_given, void *ws, size_t ws_bytes,
+                    hipStream_t s) {
+  const CsrPlan p = rows_csr_plan(B * N, B * E, K, dtype, aligned16(src) && aligned16(out), reduce);
+  CsrReduceArgs a;
+  const int rc = rows_reduce_args(a, p, src, perm, ptr, out, arg_out, B, E, K, N, dtype, reduce, out_given, ws, ws_bytes);
+  return rc != TS_OK ? rc : dispatch_csr_reduce(dtype, a, p, 1, reduce, s);
 }
 
 int run_csr_gather(int dtype, const CsrGatherArgs &args, const CsrPlan &p, int64_t B, bool divide, hipStream_t s) {
@@ -1106,6 +1128,13 @@ size_t ts_group_bins_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N,
   return bins + group_tiles_plan(B, E, K, N, dtype, true, nullptr, 0, bins).bytes;
 }
 
+size_t ts_group_std_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype) {
+  const size_t bins = ts_group_bins_workspace_bytes(B, E, K, N, dtype);
+  if (bins > 0 || !valid_dtype(dtype) || !is_float_dtype(dtype) || !sizes_ok(B, N, E, K)) return bins;
+  const RowsRoute rr = rows_route(B, E, K, N, dtype, TS_SUM);
+  return rr.ok ? rr.sort_bytes + rr.csr_bytes : 0;
+}
+
 int ts_group_std_forward(const void *src, const int64_t *index, void *total, int32_t *count, void *out, int64_t B,
                          int64_t E, int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype,
                          int unbiased, void *workspace, size_t workspace_bytes, ts_stream_t stream) {
@@ -1115,7 +1144,32 @@ int ts_group_std_forward(const void *src, const int64_t *index, void *total, int
   if (!out || !total || !count || !src || !index) return TS_ERR_BAD_ARG;
   const bool al = aligned16(src);
   const GroupBinPlan plan = group_bins_plan(B, E, K, N, dtype, al, workspace, workspace_bytes);
-  if (plan.bytes == 0) return TS_ERR_UNSUPPORTED;
+  if (plan.bytes == 0) {
+    // rows that the buckets do not hold: the entries sorted by group, then two segmented reductions (sums; squared
+    // deviations from the means), the counts from the row pointers
+    const RowsRoute rr = rows_route(B, E, K, N, dtype, TS_SUM);
+    if (!rr.ok) return TS_ERR_UNSUPPORTED;
+    if (!workspace || workspace_bytes < rr.sort_bytes + rr.csr_bytes || !aligned16(workspace)) return TS_ERR_WORKSPACE;
+    RowSortPlan sp = row_sort_plan(B, E, N, workspace, rr.sort_bytes);
+    if (!sp.ok) return TS_ERR_WORKSPACE;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    void *const ws = static_cast<char *>(workspace) + rr.sort_bytes;
+    int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, s);
+    if (rc != TS_OK) return rc;
+    rc = run_rows_reduce(src, sp.p.perm, sp.p.ptr, total, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes, s);
+    if (rc != TS_OK) return rc;
+    hipLaunchKernelGGL(row_lengths_kernel, dim3(grid_for(B * N)), dim3(kBlock), 0, s, sp.p.ptr, count, B * N);
+    const CsrPlan p = rows_csr_plan(B * N, B * E, K, dtype, al && aligned16(total) && aligned16(out), TS_SUM);
+    CsrReduceArgs a;
+    rc = rows_reduce_args(a, p, src, sp.p.perm, sp.p.ptr, out, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes);
+    if (rc != TS_OK) return rc;
+    a.row_total = total;
+    a.unbiased = unbiased ? 1 : 0;
+    GroupArgs g = {};
+    g.rows = &a;
+    g.rows_plan = &p;
+    return dispatch_group_softmax(dtype, g, GS_STD_ROWS, p.vec, s);
+  }
   if (!plan.ok) return TS_ERR_WORKSPACE;
   GroupArgs g = {};
   g.src = src;

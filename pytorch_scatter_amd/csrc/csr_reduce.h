@@ -78,6 +78,9 @@ struct CsrReduceArgs {
   int any_order = 0;
   int64_t arg_E = 0;
   int meta_stride = 4;  // words of ws_meta per tile: at least one carry flag per column chunk
+  // kRowDeviation: the rows' sums in the element type [N, K], and whether the divisor is count - 1
+  const void *row_total = nullptr;
+  int unbiased = 0;
   unsigned long long *status;
   int status_reset;
   uint64_t status_nonce;  // never 0; the same for every slice of one call
@@ -120,10 +123,37 @@ template <typename A> __device__ __forceinline__ A carry_get(A *p) {
   return v;
 }
 
+// Internal reduction: standard deviation of a row from its sum (a.row_total). The squared deviations of the entries from
+// the row's mean are added like a sum; the row end divides by the count and takes the root.
+constexpr int kRowDeviation = 64;
+
+__device__ __forceinline__ float sqrt_acc(float v) { return sqrtf(v); }
+__device__ __forceinline__ double sqrt_acc(double v) { return sqrt(v); }
+// a value of the accumulate type as the element type would hold it
+template <typename T> __device__ __forceinline__ typename Acc<T>::type round_elem(typename Acc<T>::type v) {
+  return to_acc<T>(from_acc<T>(v));
+}
+// std: the group mean as the reference forms it (composite/std.py:27-31: sum / clamp(count, 1), in the
+// element type) and the divisor of the squared deviations (:36-38: count or clamp(count - 1, 1), plus 1e-6)
+template <typename T> __device__ __forceinline__ typename Acc<T>::type group_mean(T total, int32_t count) {
+  typedef typename Acc<T>::type F;
+  const F c = round_elem<T>((F)(count < 1 ? 1 : count));
+  return round_elem<T>(to_acc<T>(total) / c);
+}
+template <typename T> __device__ __forceinline__ typename Acc<T>::type group_divisor(int32_t count, int unbiased) {
+  typedef typename Acc<T>::type F;
+  F c = round_elem<T>((F)(count < 1 ? 1 : count));
+  if (unbiased) {
+    c = round_elem<T>(c - (F)1);
+    if (c < (F)1) c = (F)1;
+  }
+  return round_elem<T>(c + (F)1e-6);
+}
+
 // TIES: entries come in any order; among equal values the smaller position wins
 template <typename A, int REDUCE, bool TIES = false>
 __device__ __forceinline__ void reduce_step(A &acc, int32_t &arg, A v, int32_t e) {
-  if (REDUCE == TS_SUM || REDUCE == TS_MEAN) {
+  if (REDUCE == TS_SUM || REDUCE == TS_MEAN || REDUCE == kRowDeviation) {
     acc = acc + v;
   } else if (REDUCE == TS_MIN) {
     if (v < acc || (TIES && v == acc && e < arg)) { acc = v; arg = e; }
@@ -144,6 +174,7 @@ template <> struct ScatterAcc<int8_t> { typedef int32_t type; };
 template <> struct ScatterAcc<uint8_t> { typedef int32_t type; };
 template <typename T> struct CsrAcc<T, TS_SUM, 2> { typedef typename ScatterAcc<T>::type type; };
 template <typename T> struct CsrAcc<T, TS_MEAN, 2> { typedef typename ScatterAcc<T>::type type; };
+template <typename T> struct CsrAcc<T, kRowDeviation, 2> { typedef typename ScatterAcc<T>::type type; };
 template <typename T, typename A> struct MinMaxAcc { typedef A type; };
 template <typename T> struct MinMaxAcc<T, int16_t> { typedef int32_t type; };
 template <typename T> struct MinMaxAcc<T, int8_t> { typedef int32_t type; };
@@ -176,7 +207,11 @@ __device__ __forceinline__ void finalize_row_at(const CsrReduceArgs &a, T *op, i
 #pragma unroll
   for (int v = 0; v < VEC; ++v) {
     A x = acc[v];
-    if (REDUCE == TS_SUM || REDUCE == TS_MEAN) {
+    if constexpr (REDUCE == kRowDeviation) {
+      // (composite/std.py:33-39: the sum in the element type, divided, its root)
+      const F div = group_divisor<T>((int32_t)count, a.unbiased);
+      o.v[v] = from_acc<T>(sqrt_acc(round_elem<T>(round_elem<T>((F)x) / div)));
+    } else if (REDUCE == TS_SUM || REDUCE == TS_MEAN) {
       if (accumulate) x = (A)to_acc<T>(prev.v[v]) + x;
       T t = from_acc<T>((F)x);
       if (REDUCE == TS_MEAN && count > 1) t = div_elem<T>(t, count_as<T>(count));  // x / 1 == x
@@ -357,6 +392,27 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   int32_t rbeg = s_ptr[r];       // first edge of row r
   int32_t rend = row_end(r);
   int32_t rnext = row_end(r + 1);  // read one row ahead: a row end then never waits for LDS
+  // squared deviations: the mean of row r, and the sum of row r + 1 on its way
+  constexpr bool kDev = REDUCE == kRowDeviation;
+  typedef typename Acc<T>::type F;
+  F mean[kDev ? VEC : 1];
+  Vec<T, kDev ? VEC : 1> sum_next;
+  auto load_total = [&](int rr) {
+    if constexpr (kDev) {
+      int64_t row = i0 + rr;
+      row = row < a.N ? row : a.N - 1;  // (behind the last row: read, not used)
+      sum_next = load_vec<T, VEC>(static_cast<const T *>(a.row_total) + row * a.K + (col_ok ? col : 0));
+    }
+  };
+  auto next_mean = [&]() {
+    if constexpr (kDev) {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) mean[v] = group_mean<T>(sum_next.v[v], rend - rbeg);
+    }
+  };
+  load_total(r);
+  next_mean();
+  load_total(r + 1);
 
   auto flush = [&]() {
     if (r == ri0 && head_open) {
@@ -382,6 +438,8 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
     rbeg = rend;
     rend = rnext;
     rnext = row_end(r + 1);
+    next_mean();
+    load_total(r + 1);
   };
 
   const int64_t col_ld = col_ok ? col : 0;  // idle lanes re-read column 0
@@ -408,7 +466,14 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
         while (ce >= rend) flush();
         const int32_t ge = kTies && kArg ? s_perm[ce] : (int32_t)(j0 + ce);
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) reduce_step<A, REDUCE, kTies>(acc[v], arg[v], (A)to_acc<T>(x[u].v[v]), ge);
+        for (int v = 0; v < VEC; ++v) {
+          if constexpr (kDev) {
+            const F d = round_elem<T>(to_acc<T>(x[u].v[v]) - mean[v]);
+            acc[v] = acc[v] + (A)round_elem<T>(d * d);
+          } else {
+            reduce_step<A, REDUCE, kTies>(acc[v], arg[v], (A)to_acc<T>(x[u].v[v]), ge);
+          }
+        }
       }
     }
 #pragma unroll
@@ -937,6 +1002,17 @@ int launch_csr_reduce_v(const CsrReduceArgs &a, const CsrPlan &p, int64_t B, int
   case TS_MAX: return launch_csr_reduce_t<T, VEC, TS_MAX>(a, p, B, stream);
   default: return TS_ERR_UNSUPPORTED;
   }
+}
+
+// Standard deviation of every row, a.row_total holding the rows' sums. The second sweep over the entries is bound like
+// the first one by the gather of rows through perm; both together replace one atomic per element and the count's own
+// pass over the index (three passes of group_softmax.h). 1 M x 33 floats in 65 k groups: sums 53, count 43, deviations by
+// atomics 236 + 14 us before; 46, 5 (from the row pointers) and 51 us now.
+template <typename T, int VEC> int launch_csr_std_rows(const CsrReduceArgs &a, const CsrPlan &p, hipStream_t stream) {
+  if (!a.any_order || a.perm == nullptr || a.row_total == nullptr || !(a.lookback || p.nblk <= 1)) return TS_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL((csr_reduce_kernel<T, VEC, kRowDeviation, -1, 2>), dim3((unsigned)p.nblk, (unsigned)p.ychunks),
+                     dim3(kCsrBlock), ((size_t)p.BI + 8) * 4, stream, a);
+  return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
 }
 
 // One entry per element type, each defined in its own translation unit.

@@ -29,6 +29,7 @@
 
 #include <math.h>
 
+#include "csr_reduce.h"
 #include "scatter.h"
 
 namespace ts {
@@ -56,15 +57,9 @@ __device__ __forceinline__ float exp_acc(float v) { return expf(v); }
 __device__ __forceinline__ double exp_acc(double v) { return exp(v); }
 __device__ __forceinline__ float log_acc(float v) { return logf(v); }
 __device__ __forceinline__ double log_acc(double v) { return log(v); }
-__device__ __forceinline__ float sqrt_acc(float v) { return sqrtf(v); }
 __device__ __forceinline__ float max_acc(float a, float b) { return fmaxf(a, b); }
 __device__ __forceinline__ double max_acc(double a, double b) { return fmax(a, b); }
-__device__ __forceinline__ double sqrt_acc(double v) { return sqrt(v); }
 
-// a value of the accumulate type as the element type would hold it
-template <typename T> __device__ __forceinline__ typename Acc<T>::type round_elem(typename Acc<T>::type v) {
-  return to_acc<T>(from_acc<T>(v));
-}
 // key of "no entry has won": entries have to beat lowest() of the element type
 template <typename T> __device__ __forceinline__ typename OrdKey<typename Acc<T>::type>::bits group_empty_key() {
   return OrdKey<typename Acc<T>::type>::enc(to_acc<T>(ElemLim<T>::lowest()));
@@ -73,7 +68,8 @@ template <typename T> __device__ __forceinline__ typename OrdKey<typename Acc<T>
 enum {
   GS_SOFTMAX = 0, GS_LOG_SOFTMAX = 1, GS_SOFTMAX_BWD = 2, GS_LOG_SOFTMAX_BWD = 3, GS_LSE = 4, GS_LSE_BWD = 5,
   GS_STD = 6, GS_STD_BWD = 7,
-  GS_STD_BINS = 8, GS_LSE_BINS = 9  // std / logsumexp forward through buckets of groups (group_binned.h)
+  GS_STD_BINS = 8, GS_LSE_BINS = 9,  // std / logsumexp forward through buckets of groups (group_binned.h)
+  GS_STD_ROWS = 10  // std forward: the sweep of squared deviations over entries sorted by group (row_sort.h, csr_reduce.h)
 };
 
 struct BinArgs;
@@ -108,24 +104,9 @@ struct GroupArgs {
   const BinArgs *bins = nullptr;  // (host) plan of the buckets
   const FusedReduceArgs *tiles = nullptr;  // (host) std / logsumexp: plan of the one-pass tiles in front of the buckets
   int tiles_force = 0;                     //        ... which run whatever a sample of the index looks like
+  const CsrReduceArgs *rows = nullptr;  // (host) std over entries sorted by group: arguments and
+  const CsrPlan *rows_plan = nullptr;   //        plan of the segmented reduction
 };
-
-// std: the group mean as the reference forms it (composite/std.py:27-31: sum / clamp(count, 1), in the
-// element type) and the divisor of the squared deviations (:36-38: count or clamp(count - 1, 1), plus 1e-6)
-template <typename T> __device__ __forceinline__ typename Acc<T>::type group_mean(T total, int32_t count) {
-  typedef typename Acc<T>::type F;
-  const F c = round_elem<T>((F)(count < 1 ? 1 : count));
-  return round_elem<T>(to_acc<T>(total) / c);
-}
-template <typename T> __device__ __forceinline__ typename Acc<T>::type group_divisor(int32_t count, int unbiased) {
-  typedef typename Acc<T>::type F;
-  F c = round_elem<T>((F)(count < 1 ? 1 : count));
-  if (unbiased) {
-    c = round_elem<T>(c - (F)1);
-    if (c < (F)1) c = (F)1;
-  }
-  return round_elem<T>(c + (F)1e-6);
-}
 
 inline size_t group_align(size_t v) { return (v + 255) / 256 * 256; }
 // bytes of workspace: keys and sums, each [B, N, K] in 8 bytes at most, and behind them the word that tells
@@ -813,6 +794,7 @@ int launch_group_softmax_v(const GroupArgs &g, int mode, hipStream_t stream) {
   switch (mode) {
   case GS_STD: return launch_group_std_v<T, VEC>(g, false, stream);
   case GS_STD_BWD: return launch_group_std_v<T, VEC>(g, true, stream);
+  case GS_STD_ROWS: return launch_csr_std_rows<T, VEC>(*g.rows, *g.rows_plan, stream);
   case GS_STD_BINS: return launch_group_reduce<T, VEC, GS_STD>(g, stream);
   case GS_LSE_BINS: return launch_group_reduce<T, VEC, GS_LSE>(g, stream);
   case GS_LSE: return launch_group_lse_v<T, VEC>(g, false, stream);

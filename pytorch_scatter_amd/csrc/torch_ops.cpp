@@ -904,9 +904,9 @@ struct GroupStdFn : public torch::autograd::Function<GroupStdFn> {
     src = src.contiguous();
     const GroupLayout l = group_layout(src, index, dim);
     Tensor total, count, out;
-    const size_t bins_bytes = ts_group_bins_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src));
+    const size_t bins_bytes = ts_group_std_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src));
     if (bins_bytes > 0 && l.B * N * l.K > 0 && (reinterpret_cast<uintptr_t>(src.data_ptr()) & 15) == 0) {
-      // group sums, counts and result from one gather of src through buckets of groups
+      // group sums, counts and result in one call (buckets of groups, or the entries sorted by group)
       auto sizes = src.sizes().vec();
       sizes[dim] = N;
       total = at::empty(sizes, src.options());

@@ -54,3 +54,43 @@ def test_row_sort(kind, E, N, monkeypatch):
     want_arg = torch.full((N, K), E, dtype=torch.int64, device=DEV).scatter_reduce_(0, idx, first, "amin")
     assert torch.equal(out, torch.where(want_arg < E, top, 0))
     assert torch.equal(arg, want_arg)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind,B,E,K,N", [("even", 1, 3000, 33, 250), ("even", 2, 900, 130, 80), ("sorted", 1, 3001, 200, 7),
+                                          ("outside", 1, 20000, 64, 900), ("one row", 1, 30001, 32, 3),
+                                          ("hub500", 1, 2000, 513, 300), ("even", 1, 1, 64, 1), ("even", 1, 200, 64, 5000)])
+def test_std_rows(kind, B, E, K, N, dtype, monkeypatch):
+    """Standard deviation over entries sorted by group: every error against 64 bits within the roundings of the element
+    type: root, quotient, and the mean, whose rounding shifts all deviations of a group alike."""
+    from pytorch_scatter_amd import capi
+    if kind in ("one row", "hub500") and dtype in (torch.bfloat16, torch.float16):
+        pytest.skip("a sum of squares over hundreds of entries, rounded to 16 bits, is not meaningful")
+    monkeypatch.setenv("TS_SCATTER_BINNED", "2")
+    monkeypatch.setenv("TS_GROUP_BINS", "0")
+    g = torch.Generator(device=DEV).manual_seed(E + K)
+    index = _index(kind, E, N, g)
+    ok = (index >= 0) & (index < N)
+    src = (torch.randn((B, E, K), generator=g, device=DEV, dtype=torch.float64) * 3 + 1).to(dtype)
+    total, out = (torch.full((B, N, K), 7, dtype=dtype, device=DEV) for _ in range(2))
+    count = torch.full((B, N), -7, dtype=torch.int32, device=DEV)
+    capi.group_std_forward(src, index, total, count, out, B, E, K, N, 0, 1, True)
+    idx, x = index[ok], src[:, ok].double()
+    n = torch.bincount(idx, minlength=N)
+    assert torch.equal(count.long(), n.expand(B, N))
+    zero = torch.zeros((B, N, K), dtype=torch.float64, device=DEV)
+    sums, size = zero.index_add(1, idx, x), zero.index_add(1, idx, x.abs())
+    eps = torch.finfo(dtype).eps
+    assert bool(((total.double() - sums).abs() <= eps * sums.abs() + 1e-13 * size).all())
+    c = n.clamp(min=1).view(1, N, 1).double()
+    mean = sums / c
+    want = (zero.index_add(1, idx, (x - mean[:, idx]) ** 2) / ((c - 1).clamp(min=1) + 1e-6)).sqrt()
+    # roundings of the deviation and its square, of sum, quotient and root: 4 eps of the result; the mean is off by
+    # 2 eps of itself, times the root of n / (n - 1) <= 2 in the result
+    bound = 4 * eps * want + 4 * eps * mean.abs() + 1e-6 * eps
+    if dtype == torch.float64:  # n additions of squares on either side: n / 2 eps of the sum each, half that of its root
+        bound = bound + eps * c / 2 * want
+    if dtype == torch.float16:
+        bound = bound + 2.0 ** -12  # squares below 2^-14 are subnormal: 2^-25 apiece, 2^-12.5 under the root
+    bad = (out.double() - want).abs() > bound
+    assert not bool(bad.any()), float(((out.double() - want).abs() - bound).max())
