@@ -327,6 +327,14 @@ int ts_arg_backward(const void *grad_out, const int64_t *arg, void *grad_in,
                     int64_t B, int64_t N, int64_t E, int64_t K, int dtype,
                     ts_stream_t stream);
 
+/* The same for scatter min / max of wide rows under one index per row (index[b * index_stride_b + e * index_stride_e]):
+ * the entries are sorted by row first and every row of grad_in is then written once. The workspace query says 0, and the
+ * call TS_ERR_UNSUPPORTED, where ts_arg_backward is the faster one. */
+size_t ts_arg_backward_rows_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype);
+int ts_arg_backward_rows(const void *grad_out, const int64_t *arg, const int64_t *index, void *grad_in, int64_t B,
+                         int64_t N, int64_t E, int64_t K, int64_t index_stride_b, int64_t index_stride_e, int dtype,
+                         void *workspace, size_t workspace_bytes, ts_stream_t stream);
+
 /* ---------------------------------------------------------- group softmax
  * Softmax / log-softmax over the entries that share an index, one index per
  * row (index[b*sb + e*se] addresses all K columns of entry e):

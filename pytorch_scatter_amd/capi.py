@@ -27,6 +27,7 @@ EXPORTS = (
     "ts_segment_coo_workspace_bytes", "ts_segment_coo", "ts_gather_coo",
     "ts_segment_mean_coo_backward",
     "ts_scatter", "ts_scatter_workspace_bytes", "ts_scatter_workspace_zero_bytes", "ts_scatter_with_workspace", "ts_scatter_count", "ts_scatter_count_workspace_bytes", "ts_scatter_count_with_workspace", "ts_scatter_sum_count_workspace_bytes", "ts_scatter_sum_count_with_workspace", "ts_divide_by_count", "ts_arg_backward",
+    "ts_arg_backward_rows_workspace_bytes", "ts_arg_backward_rows",
     "ts_group_softmax_workspace_bytes", "ts_group_softmax", "ts_group_softmax_backward",
     "ts_group_logsumexp", "ts_group_logsumexp_backward",
     "ts_group_std", "ts_group_std_backward", "ts_group_bins_workspace_bytes", "ts_group_std_workspace_bytes", "ts_group_workspace_bytes", "ts_group_std_forward",
@@ -63,6 +64,7 @@ def lib() -> ctypes.CDLL:
         _lib.ts_scatter_sum_count_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_sort_index_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_group_bins_workspace_bytes.restype = ctypes.c_size_t
+        _lib.ts_arg_backward_rows_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_group_std_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_group_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_segment_csr_permuted_workspace_bytes.restype = ctypes.c_size_t

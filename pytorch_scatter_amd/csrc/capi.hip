@@ -926,6 +926,50 @@ int ts_arg_backward(const void *grad_out, const int64_t *arg, void *grad_in, int
   return dispatch_arg_backward(dtype, grad_out, arg, grad_in, B, N, E, K, static_cast<hipStream_t>(stream));
 }
 
+size_t ts_arg_backward_rows_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype) {
+  if (!valid_dtype(dtype) || !is_float_dtype(dtype) || !sizes_ok(B, N, E, K) || B * E == 0 || N == 0) return 0;
+  const int mode = env_int("TS_SCATTER_BINNED", 1);  // tuning aid: 0 never, 2 at any size
+  const int64_t row_bytes = K * kElemBytes[dtype];
+  if (mode == 0 || row_bytes < 64 || K >= (int64_t)1 << 20) return 0;
+  // As long as grad_in fits the 256 MB of the memory-side cache, the second pass over it is cheap (us of ts_arg_backward /
+  // this call, 64 floats, even index and a hub: 300 k entries, 3 a row 51 / 57 and 47 / 64; 1 M, 8 a row 110 / 101 and
+  // 72 / 108; 16 floats, 3 M, 3 a row 140 / 185). Beyond it pays wherever the elements of grad_out, 14 ps each in the
+  // scatter, outweigh the sort, 25 ps an entry and 30 us at the least (256 floats, 400 k, 15 a row 245 / 108 and 123 /
+  // 126; 64 floats, 2.3 M, 8 a row 466 / 236 and 226 / 200). Rows that fill no 16-byte vector do not gain (33 doubles,
+  // 2 M, 4 a row 458 / 480 and 223 / 348).
+  if (mode != 2 && (row_bytes < 256 || row_bytes % kVecBytes != 0 || B * E * row_bytes < 384000000 || B * N * K < ((int64_t)4 << 20) + 3 * B * E)) return 0;
+  return row_sort_plan(B, E, N, nullptr, 0).bytes;
+}
+
+int ts_arg_backward_rows(const void *grad_out, const int64_t *arg, const int64_t *index, void *grad_in, int64_t B, int64_t N,
+                         int64_t E, int64_t K, int64_t index_stride_b, int64_t index_stride_e, int dtype, void *workspace,
+                         size_t workspace_bytes, ts_stream_t stream) {
+  const size_t need = ts_arg_backward_rows_workspace_bytes(B, E, K, N, dtype);
+  if (need == 0) return TS_ERR_UNSUPPORTED;
+  if (!grad_out || !arg || !index || !grad_in) return TS_ERR_BAD_ARG;
+  if (!workspace || workspace_bytes < need || !aligned16(workspace)) return TS_ERR_WORKSPACE;
+  RowSortPlan sp = row_sort_plan(B, E, N, workspace, workspace_bytes);
+  if (!sp.ok) return TS_ERR_WORKSPACE;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, s);
+  if (rc != TS_OK) return rc;
+  RowSortArgs p = sp.p;
+  p.index = index;
+  p.sb = index_stride_b;
+  p.se = index_stride_e;
+  p.flat = B == 1 && index_stride_e == 1;
+  const int es = kElemBytes[dtype], full = kVecBytes / es;
+  const bool wide = K % full == 0 && aligned16(grad_out) && aligned16(arg) && aligned16(grad_in);
+  if (es == 2)
+    return wide ? launch_arg_rows<uint16_t, 8>(p, grad_out, arg, grad_in, K, s)
+                : launch_arg_rows<uint16_t, 1>(p, grad_out, arg, grad_in, K, s);
+  if (es == 4)
+    return wide ? launch_arg_rows<uint32_t, 4>(p, grad_out, arg, grad_in, K, s)
+                : launch_arg_rows<uint32_t, 1>(p, grad_out, arg, grad_in, K, s);
+  return wide ? launch_arg_rows<uint64_t, 2>(p, grad_out, arg, grad_in, K, s)
+              : launch_arg_rows<uint64_t, 1>(p, grad_out, arg, grad_in, K, s);
+}
+
 namespace {
 // std / logsumexp backward with a workspace of ts_group_softmax_workspace_bytes(): the values an entry needs of its group
 // are laid side by side first (one more launch over [B, N, K]) when there are at least as many entries as groups

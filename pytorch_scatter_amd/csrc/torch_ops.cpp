@@ -527,7 +527,9 @@ Tensor gather_coo_hip(Tensor src, Tensor index, OptTensor optional_out, OptTenso
 // the position that won it (csrc/scatter.cpp:184-196, segment_coo.cpp:132-144,
 // segment_csr.cpp:130-142 do this with a scatter_ into a buffer that has one
 // extra slot for the sentinel).
-Tensor arg_backward_hip(Tensor grad_out, const Tensor &arg_out, const std::vector<int64_t> &src_shape, int64_t dim) {
+// index (scatter): broadcast to src_shape; one index per row opens the route over entries sorted by row.
+Tensor arg_backward_hip(Tensor grad_out, const Tensor &arg_out, const std::vector<int64_t> &src_shape, int64_t dim,
+                        const Tensor &index = Tensor()) {
   c10::DeviceGuard guard(grad_out.device());
   grad_out = grad_out.contiguous();
   Tensor arg = arg_out.contiguous();
@@ -536,6 +538,19 @@ Tensor arg_backward_hip(Tensor grad_out, const Tensor &arg_out, const std::vecto
   const int64_t E = src_shape[dim];
   const int64_t K = prod(src_shape, dim + 1, static_cast<int64_t>(src_shape.size()));
   const int64_t N = grad_out.size(dim);
+  if (index.defined() && index.sizes() == at::IntArrayRef(src_shape)) {
+    auto sb = collapsed_stride(index, 0, dim), sk = collapsed_stride(index, dim + 1, index.dim());
+    const size_t bytes = sb.has_value() && sk.has_value() && sk.value() == 0
+                             ? ts_arg_backward_rows_workspace_bytes(B, E, K, N, dtype_code(grad_out)) : 0;
+    if (bytes > 0) {
+      Tensor ws = workspace(bytes, grad_out);
+      check_status(ts_arg_backward_rows(grad_out.data_ptr(), arg.data_ptr<int64_t>(), index.data_ptr<int64_t>(),
+                                        grad_in.data_ptr(), B, N, E, K, sb.value(), index.stride(dim), dtype_code(grad_out),
+                                        ws.data_ptr(), bytes, stream_of(grad_out)),
+                   "min/max backward");
+      return grad_in;
+    }
+  }
   check_status(ts_arg_backward(grad_out.data_ptr(), arg.data_ptr<int64_t>(), grad_in.data_ptr(), B, N, E, K,
                                dtype_code(grad_out), stream_of(grad_out)),
                "min/max backward");
@@ -648,11 +663,13 @@ template <int REDUCE> struct ScatterFn : public torch::autograd::Function<Scatte
     Variable arg_out = std::get<1>(result).value();
     ctx->save_for_backward({index, arg_out});
     ctx->mark_non_differentiable({arg_out});
+    ctx->set_materialize_grads(false);  // no zeros [.., N, ..] in the place of a gradient of the positions
     return {out, arg_out};
   }
 
   static variable_list backward(AutogradContext *ctx, variable_list grad_outs) {
     auto grad_out = grad_outs[0];
+    if (!grad_out.defined()) return variable_list(5);
     auto saved = ctx->get_saved_variables();
     const int64_t dim = ctx->saved_data["dim"].toInt();
     Variable grad_in;
@@ -664,7 +681,7 @@ template <int REDUCE> struct ScatterFn : public torch::autograd::Function<Scatte
     } else if (REDUCE == TS_MEAN) {
       grad_in = gather_grad_rows(grad_out, saved[0], dim, saved[1]);
     } else {
-      grad_in = arg_backward_hip(grad_out, saved[1], saved_shape(ctx), dim);
+      grad_in = arg_backward_hip(grad_out, saved[1], saved_shape(ctx), dim, saved[0]);
     }
     return {grad_in, Variable(), Variable(), Variable(), Variable()};
   }

@@ -94,3 +94,31 @@ def test_std_rows(kind, B, E, K, N, dtype, monkeypatch):
         bound = bound + 2.0 ** -12  # squares below 2^-14 are subnormal: 2^-25 apiece, 2^-12.5 under the root
     bad = (out.double() - want).abs() > bound
     assert not bool(bad.any()), float(((out.double() - want).abs() - bound).max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16])
+@pytest.mark.parametrize("kind,B,E,K,N", [("even", 1, 3000, 33, 250), ("even", 2, 900, 136, 80), ("sorted", 1, 3001, 200, 7),
+                                          ("outside", 1, 20000, 64, 900), ("outside", 2, 1001, 300, 50),
+                                          ("one row", 1, 9001, 64, 3), ("even", 1, 1, 64, 1), ("even", 1, 200, 520, 5000)])
+def test_arg_backward_rows(kind, B, E, K, N, dtype, monkeypatch):
+    """Backward of max over entries sorted by row: every element exactly, zeros for entries outside [0, N)."""
+    import ctypes
+    from pytorch_scatter_amd import capi
+    monkeypatch.setenv("TS_SCATTER_BINNED", "2")
+    g = torch.Generator(device=DEV).manual_seed(E + K)
+    index = _index(kind, E, N, g)
+    src = torch.randint(-9, 10, (B, E, K), generator=g, device=DEV).to(dtype)
+    out = torch.empty((B, N, K), dtype=dtype, device=DEV)
+    arg = torch.empty((B, N, K), dtype=torch.int64, device=DEV)
+    capi.scatter_with_workspace(src, index, out, arg, B, E, K, N, 0, 1, 0, capi.MAX, 0)
+    grad = torch.randn((B, N, K), generator=g, device=DEV).to(dtype)
+    want = torch.zeros((B, E + 1, K), dtype=dtype, device=DEV).scatter_(1, arg, grad)[:, :E]
+    got = torch.full((B, E, K), 7, dtype=dtype, device=DEV)
+    code, i = capi.DTYPE[dtype], ctypes.c_int64
+    nbytes = int(capi.lib().ts_arg_backward_rows_workspace_bytes(i(B), i(E), i(K), i(N), code))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    p = lambda x: ctypes.c_void_p(x.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    capi._check(capi.lib().ts_arg_backward_rows(p(grad), p(arg), p(index), p(got), i(B), i(N), i(E), i(K), i(0), i(1), code,
+                                                p(ws), ctypes.c_size_t(nbytes), stream))
+    assert torch.equal(got, want)
