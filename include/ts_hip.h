@@ -80,11 +80,16 @@ int64_t ts_hip_version(void);
  * untouched with out_given) and the call's tag is written into word 1. After
  * the stream has finished, word 1 == word 0 means that the latest call gave at
  * least one row up (ts_status_gave_up below); anything else: every row is
- * complete. Neither write has to happen before the other, and what an earlier
- * call left in word 1 never equals a later call's tag. Nothing in the library
- * reads the words back: a caller that cannot vouch for its row pointers must
- * (16 bytes, device to host). The torch operators do so after every segment
- * call when the environment variable TS_CHECK_STATUS is set to 1, and raise.
+ * complete. ts_scatter_with_workspace, ts_scatter_sum_count_with_workspace (at
+ * the end of what ts_scatter_workspace_bytes() reports for its sum) and
+ * ts_group_std_forward leave the same two words where they sort the entries by
+ * row and finish with the same reduction (TS_ROUTE_*_OR_SEGMENTED below).
+ * Neither write has to happen before the other, and what an earlier call left
+ * in word 1 never equals a later call's tag. Nothing in the library reads the
+ * words back: a caller that cannot vouch for its row pointers must (16 bytes,
+ * device to host). The torch operators do so after every segment, scatter and
+ * scatter_std call that has such words when the environment variable
+ * TS_CHECK_STATUS is set to 1, and raise.
  */
 #define TS_STATUS_BYTES 256
 /* words: a host copy of the two status words; 1 if the latest call gave a row up, else 0. Host arithmetic only:
@@ -438,7 +443,8 @@ int ts_group_std_backward_with_workspace(const void *src, const int64_t *index, 
  * standard deviation (out) in one call: what ts_scatter(sum) + ts_scatter_count + ts_group_std leave. It needs that
  * workspace: TS_ERR_UNSUPPORTED when the route does not apply, TS_ERR_WORKSPACE when the workspace is too small.
  * Where the buckets do not apply, wide rows of large inputs go through a sort of the entries by group instead:
- * ts_group_std_workspace_bytes() is the scratch of whichever route serves the call, 0 when none does.
+ * ts_group_std_workspace_bytes() is the scratch of whichever route serves the call, 0 when none does. It then ends in
+ * status words (TS_STATUS_BYTES, see ts_segment_csr), which the sort's reductions set and the buckets do not touch.
  * ts_group_logsumexp takes the same route by itself when its workspace has that size. */
 size_t ts_group_bins_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype);
 size_t ts_group_std_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype);

@@ -114,6 +114,14 @@ def _check_status(ws, nbytes, B, N, K):
             raise TsError(f"ts_hip: segment reduction left status word {word}: a row was given up")
 
 
+SORTED_ROWS = (6, 16)  # routes of enum ts_scatter_route whose workspace ends in status words: entries sorted by row
+
+
+def _check_scatter_status(ws, nbytes, B, N, K):
+    if lib().ts_scatter_last_route() in SORTED_ROWS:
+        _check_status(ws, nbytes, B, N, K)
+
+
 def scatter_last_route() -> str:
     """Name of the kernels the last scatter call of this thread launched (ts_scatter_last_route)."""
     L = lib()
@@ -218,6 +226,7 @@ def scatter_with_workspace(src, index, out, arg_out, B, E, K, N, sb, se, sk, red
         # min / max of single values: the word behind the key table is set when a bounded wait in the kernel ran out
         if int(ws[nzero - STATUS_BYTES:nzero - STATUS_BYTES + 8].view(torch.int64).item()) != 0:
             raise TsError("ts_hip: scatter min / max lost entries: a bounded wait inside the kernel ran out")
+    _check_scatter_status(ws, nbytes, B, N, K)
     return ws
 
 
@@ -249,6 +258,7 @@ def scatter_sum_count_with_workspace(src, index, out, count, B, E, K, N, sb, se,
         _check(L.ts_scatter_sum_count_with_workspace(_p(src), _p(index), _p(out), _p(count), _i(B), _i(E), _i(K), _i(N),
                                                      _i(sb), _i(se), DTYPE[out.dtype], 1 if out_given else 0,
                                                      _p(ws) if nbytes else None, ctypes.c_size_t(nbytes), _stream(out)))
+    _check_scatter_status(ws, L.ts_scatter_workspace_bytes(_i(B), _i(E), _i(K), _i(N), DTYPE[out.dtype], SUM), B, N, K)
     return nbytes
 
 
@@ -349,6 +359,8 @@ def group_std_forward(src, index, total, count, out, B, E, K, N, sb, se, unbiase
         _check(lib().ts_group_std_forward(_p(src), _p(index), _p(total), _p(count), _p(out), _i(B), _i(E), _i(K), _i(N),
                                           _i(sb), _i(se), DTYPE[out.dtype], int(unbiased), _p(ws),
                                           ctypes.c_size_t(nbytes), _stream(out)))
+    if group_bins_workspace_bytes(B, E, K, N, out.dtype) == 0:  # (the entries sorted by group)
+        _check_status(ws, nbytes, B, N, K)
     return nbytes
 
 

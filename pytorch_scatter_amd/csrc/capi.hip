@@ -206,10 +206,12 @@ int run_csr_reduce(const void *src, const int64_t *indptr, void *out, int64_t *a
 
 // ---- scatter of wide rows: the index is sorted by row (row_sort.h), then a segmented reduction over permuted rows.
 // No atomics on out, no table misses, whatever the index; an index found in order skips the sorting passes.
-// kRowsPlan: does a call take this route, and its workspace (row sort, then the carries of the reduction).
+// RowsRoute: does a call take this route, and its workspace: row sort, carries of the reduction, status words (the
+// last kStatusBytes: a row that crosses tiles is finished by a bounded wait, as in the segment operators).
 struct RowsRoute {
   bool ok;
   size_t sort_bytes, csr_bytes;
+  size_t total() const { return sort_bytes + csr_bytes + kStatusBytes; }
 };
 inline int rows_acc_bytes(int dtype, int reduce) {
   const bool sum = reduce == TS_SUM || reduce == TS_MEAN;
@@ -273,10 +275,11 @@ RowsRoute rows_route(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int 
   r.ok = true;
   return r;
 }
-// perm / ptr as launch_row_sort leaves them; ws: RowsRoute::csr_bytes
+// perm / ptr as launch_row_sort leaves them; ws: RowsRoute::csr_bytes and behind them the status words. status_nonce: one
+// for all reductions of a call; the first of them (status_reset) writes it into word 0.
 int rows_reduce_args(CsrReduceArgs &a, const CsrPlan &p, const void *src, const int32_t *perm, const int64_t *ptr, void *out,
                      int64_t *arg_out, int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce, int out_given,
-                     void *ws, size_t ws_bytes) {
+                     void *ws, size_t ws_bytes, uint64_t status_nonce, bool status_reset) {
   const int64_t n = B * E, rows = B * N;
   size_t off_args = 0, off_meta = 0;
   a.meta_stride = rows_meta_stride(p);
@@ -307,18 +310,19 @@ int rows_reduce_args(CsrReduceArgs &a, const CsrPlan &p, const void *src, const 
   a.perm_args = 0;
   a.any_order = 1;
   a.arg_E = E;
-  a.status = nullptr;
-  a.status_reset = 0;
-  a.status_nonce = 0;
-  a.carry_spin = kCarrySpin;
+  a.status = status_word(ws, ws_bytes + kStatusBytes);
+  a.status_reset = status_reset ? 1 : 0;
+  a.status_nonce = status_nonce;
+  a.carry_spin = env_int("TS_CSR_SPIN", kCarrySpin);  // test aid: -1 makes every look-back give up at once
   return TS_OK;
 }
 int run_rows_reduce(const void *src, const int32_t *perm, const int64_t *ptr, void *out, int64_t *arg_out, int64_t B,
                     int64_t E, int64_t K, int64_t N, int dtype, int reduce, int out_given, void *ws, size_t ws_bytes,
-                    hipStream_t s) {
+                    uint64_t status_nonce, hipStream_t s) {
   const CsrPlan p = rows_csr_plan(B * N, B * E, K, dtype, aligned16(src) && aligned16(out), reduce);
   CsrReduceArgs a;
-  const int rc = rows_reduce_args(a, p, src, perm, ptr, out, arg_out, B, E, K, N, dtype, reduce, out_given, ws, ws_bytes);
+  const int rc = rows_reduce_args(a, p, src, perm, ptr, out, arg_out, B, E, K, N, dtype, reduce, out_given, ws, ws_bytes,
+                                  status_nonce, true);
   return rc != TS_OK ? rc : dispatch_csr_reduce(dtype, a, p, 1, reduce, s);
 }
 
@@ -640,7 +644,7 @@ size_t ts_scatter_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, in
   const bool any_size = env_int("TS_SCATTER_BINNED", 1) == 2;
   const RowsRoute rr = reduce == TS_MEAN ? RowsRoute{false, 0, 0} : rows_route(B, E, K, N, dtype, reduce);
   if (reduce == TS_MIN || reduce == TS_MAX) {
-    if (rr.ok) return rr.sort_bytes + rr.csr_bytes;
+    if (rr.ok) return rr.total();
     if (kElemBytes[dtype] > 4) return 0;  // 64-bit elements do not use packed keys
     if (env_int("TS_SCATTER_LDS_K1", 1) && env_int("TS_SCATTER_LDS", 1)) {
       const size_t k1 = k1_plan(B, E, K, N, kElemBytes[dtype], nullptr, 0, env_int("TS_SCATTER_LDS", 1) == 2).bytes;
@@ -651,7 +655,7 @@ size_t ts_scatter_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, in
     return probe && skew_probe_shape(B, E, K, N, kElemBytes[dtype], probe == 2) ? 256 : 0;
   }
   if (reduce == TS_SUM && kAccBytes[dtype] >= 4) {  // table slots: int32 for int32, 8 bytes for the other types
-    if (rr.ok) return rr.sort_bytes + rr.csr_bytes;
+    if (rr.ok) return rr.total();
     if (env_int("TS_SCATTER_LDS", 1)) {
       // one 4-byte value per entry: (row in bucket, value) words, 8 bytes of scratch per entry
       const size_t payload = bin_plan_payload(B, E, K, N, kElemBytes[dtype], nullptr, 0, any_size).bytes;
@@ -696,6 +700,7 @@ int scatter_ws_impl(const void *src, const int64_t *index, void *out, int64_t *a
                     int *count_done = nullptr) {
   if (!valid_dtype(dtype) || !sizes_ok(B, N, E, K)) return TS_ERR_BAD_ARG;
   if (reduce != TS_SUM && reduce != TS_MUL && reduce != TS_MIN && reduce != TS_MAX) return TS_ERR_UNSUPPORTED;
+  ts_note_scatter_route(TS_ROUTE_NONE);
   if (B * N * K == 0) return TS_OK;
   if (!out || (B * E * K > 0 && (!src || !index))) return TS_ERR_BAD_ARG;
   if ((reduce == TS_MIN || reduce == TS_MAX) && !arg_out) return TS_ERR_BAD_ARG;
@@ -731,14 +736,14 @@ int scatter_ws_impl(const void *src, const int64_t *index, void *out, int64_t *a
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (a.bin_ws != nullptr && index_stride_k == 0 && B * E * K > 0 && aligned16(workspace)) {
     const RowsRoute rr = rows_route(B, E, K, N, dtype, reduce);
-    if (rr.ok && workspace_bytes >= rr.sort_bytes + rr.csr_bytes) {
+    if (rr.ok && workspace_bytes >= rr.total()) {
       RowSortPlan sp = row_sort_plan(B, E, N, workspace, rr.sort_bytes);
       if (!sp.ok) return TS_ERR_WORKSPACE;
       ts_note_scatter_route(reduce == TS_SUM ? TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED : TS_ROUTE_MINMAX_BUCKETS_OR_SEGMENTED);
       int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, s);
       if (rc != TS_OK) return rc;
       rc = run_rows_reduce(src, sp.p.perm, sp.p.ptr, out, arg_out, B, E, K, N, dtype, reduce, out_given,
-                           static_cast<char *>(workspace) + rr.sort_bytes, rr.csr_bytes, s);
+                           static_cast<char *>(workspace) + rr.sort_bytes, rr.csr_bytes, next_nonce(), s);
       if (rc != TS_OK || count_out == nullptr) return rc;
       hipLaunchKernelGGL(row_lengths_kernel, dim3(grid_for(B * N)), dim3(kBlock), 0, s, sp.p.ptr, count_out, B * N);
       if (count_done != nullptr) *count_done = 1;
@@ -1176,7 +1181,7 @@ size_t ts_group_std_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, 
   const size_t bins = ts_group_bins_workspace_bytes(B, E, K, N, dtype);
   if (bins > 0 || !valid_dtype(dtype) || !is_float_dtype(dtype) || !sizes_ok(B, N, E, K)) return bins;
   const RowsRoute rr = rows_route(B, E, K, N, dtype, TS_SUM);
-  return rr.ok ? rr.sort_bytes + rr.csr_bytes : 0;
+  return rr.ok ? rr.total() : 0;
 }
 
 int ts_group_std_forward(const void *src, const int64_t *index, void *total, int32_t *count, void *out, int64_t B,
@@ -1193,19 +1198,22 @@ int ts_group_std_forward(const void *src, const int64_t *index, void *total, int
     // deviations from the means), the counts from the row pointers
     const RowsRoute rr = rows_route(B, E, K, N, dtype, TS_SUM);
     if (!rr.ok) return TS_ERR_UNSUPPORTED;
-    if (!workspace || workspace_bytes < rr.sort_bytes + rr.csr_bytes || !aligned16(workspace)) return TS_ERR_WORKSPACE;
+    if (!workspace || workspace_bytes < rr.total() || !aligned16(workspace)) return TS_ERR_WORKSPACE;
     RowSortPlan sp = row_sort_plan(B, E, N, workspace, rr.sort_bytes);
     if (!sp.ok) return TS_ERR_WORKSPACE;
     hipStream_t s = static_cast<hipStream_t>(stream);
     void *const ws = static_cast<char *>(workspace) + rr.sort_bytes;
     int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, s);
     if (rc != TS_OK) return rc;
-    rc = run_rows_reduce(src, sp.p.perm, sp.p.ptr, total, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes, s);
+    const uint64_t status_nonce = next_nonce();
+    rc = run_rows_reduce(src, sp.p.perm, sp.p.ptr, total, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes,
+                         status_nonce, s);
     if (rc != TS_OK) return rc;
     hipLaunchKernelGGL(row_lengths_kernel, dim3(grid_for(B * N)), dim3(kBlock), 0, s, sp.p.ptr, count, B * N);
     const CsrPlan p = rows_csr_plan(B * N, B * E, K, dtype, al && aligned16(total) && aligned16(out), TS_SUM);
     CsrReduceArgs a;
-    rc = rows_reduce_args(a, p, src, sp.p.perm, sp.p.ptr, out, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes);
+    rc = rows_reduce_args(a, p, src, sp.p.perm, sp.p.ptr, out, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes,
+                          status_nonce, false);
     if (rc != TS_OK) return rc;
     a.row_total = total;
     a.unbiased = unbiased ? 1 : 0;

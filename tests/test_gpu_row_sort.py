@@ -122,3 +122,47 @@ def test_arg_backward_rows(kind, B, E, K, N, dtype, monkeypatch):
     capi._check(capi.lib().ts_arg_backward_rows(p(grad), p(arg), p(index), p(got), i(B), i(N), i(E), i(K), i(0), i(1), code,
                                                 p(ws), ctypes.c_size_t(nbytes), stream))
     assert torch.equal(got, want)
+
+
+def test_rows_that_were_given_up_are_reported(monkeypatch):
+    """The wait for the tiles before a row's last one is bounded. With the bound forced to "never wait" from the host
+    (TS_CSR_SPIN=-1; every kernel exits normally) the rows that cross tiles are given up: the status words say so and the
+    operators raise. Without the override the words stay clean and the values are right."""
+    import pytorch_scatter_amd as ts
+    from pytorch_scatter_amd import capi
+    monkeypatch.setenv("TS_SCATTER_BINNED", "2")
+    monkeypatch.setenv("TS_GROUP_BINS", "0")
+    E, N, K = 30001, 3, 64  # rows of thousands of entries
+    g = torch.Generator(device=DEV).manual_seed(1)
+    index = torch.randint(0, N, (E,), generator=g, device=DEV)
+    src = torch.randint(-50, 51, (E, K), generator=g, device=DEV).float()
+    sums = torch.zeros((N, K), device=DEV, dtype=torch.float64).index_add_(0, index, src.double()).float()  # exact
+    out, total = torch.empty((N, K), device=DEV), torch.empty((N, K), device=DEV)
+    arg = torch.empty((N, K), dtype=torch.long, device=DEV)
+    count = torch.empty(N, dtype=torch.int32, device=DEV)
+    i = capi._i
+    std_bytes = int(capi.lib().ts_group_std_workspace_bytes(i(1), i(E), i(K), i(N), 0))
+
+    def words(reduce):
+        monkeypatch.setattr(capi, "CHECK_STATUS", False)
+        ws = capi.scatter_with_workspace(src, index, out, arg if reduce == capi.MAX else None, 1, E, K, N, 0, 1, 0, reduce, 0)
+        nbytes = capi.lib().ts_scatter_workspace_bytes(i(1), i(E), i(K), i(N), 0, reduce)
+        monkeypatch.setattr(capi, "CHECK_STATUS", True)
+        return capi.status_word(ws, nbytes)
+
+    monkeypatch.setenv("TS_CSR_SPIN", "-1")
+    assert words(capi.SUM) == 1 and bool((out == 0).all())
+    assert words(capi.MAX) == 1 and bool((out == 0).all()) and bool((arg == E).all())
+    with pytest.raises(capi.TsError, match="given up"):
+        capi.group_std_forward(src, index, total, count, out, 1, E, K, N, 0, 1, True)
+    with pytest.raises(capi.TsError, match="given up"):
+        capi.scatter_sum_count_with_workspace(src, index, out, count, 1, E, K, N, 0, 1, False)
+    for op in (ts.scatter_sum, ts.scatter_mean, ts.scatter_max, ts.scatter_std):
+        with pytest.raises(RuntimeError, match="given up"):
+            op(src, index, dim=0, dim_size=N)
+    monkeypatch.delenv("TS_CSR_SPIN")
+    assert std_bytes >= capi.STATUS_BYTES
+    assert words(capi.SUM) == 0 and torch.equal(out, sums)
+    assert words(capi.MAX) == 0 and torch.equal(out.max(0)[0], src.max(0)[0])
+    for op in (ts.scatter_sum, ts.scatter_mean, ts.scatter_max, ts.scatter_std):
+        op(src, index, dim=0, dim_size=N)
