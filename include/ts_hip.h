@@ -441,7 +441,8 @@ int ts_group_std_backward_with_workspace(const void *src, const int64_t *index, 
  * (small inputs, rows held by more than 32 lanes, more groups than 16384 buckets hold).
  * ts_group_std_forward writes the group sums (total, element type), the entries per group (count, int32) and the
  * standard deviation (out) in one call: what ts_scatter(sum) + ts_scatter_count + ts_group_std leave. It needs that
- * workspace: TS_ERR_UNSUPPORTED when the route does not apply, TS_ERR_WORKSPACE when the workspace is too small.
+ * workspace: TS_ERR_UNSUPPORTED when the route does not apply (also for a src off a 16-byte border whose rows the buckets
+ * hold only with 16 bytes per lane), TS_ERR_WORKSPACE when the workspace is too small.
  * Where the buckets do not apply, wide rows of large inputs go through a sort of the entries by group instead:
  * ts_group_std_workspace_bytes() is the scratch of whichever route serves the call, 0 when none does. It then ends in
  * status words (TS_STATUS_BYTES, see ts_segment_csr), which the sort's reductions set and the buckets do not touch.

@@ -1194,6 +1194,8 @@ int ts_group_std_forward(const void *src, const int64_t *index, void *total, int
   const bool al = aligned16(src);
   const GroupBinPlan plan = group_bins_plan(B, E, K, N, dtype, al, workspace, workspace_bytes);
   if (plan.bytes == 0) {
+    // (an aligned src would have gone through the buckets, and the workspace is theirs: the three-call form has to serve it)
+    if (!al && group_bins_plan(B, E, K, N, dtype, true, nullptr, 0).bytes != 0) return TS_ERR_UNSUPPORTED;
     // rows that the buckets do not hold: the entries sorted by group, then two segmented reductions (sums; squared
     // deviations from the means), the counts from the row pointers
     const RowsRoute rr = rows_route(B, E, K, N, dtype, TS_SUM);

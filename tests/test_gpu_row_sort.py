@@ -166,3 +166,30 @@ def test_rows_that_were_given_up_are_reported(monkeypatch):
     assert words(capi.MAX) == 0 and torch.equal(out.max(0)[0], src.max(0)[0])
     for op in (ts.scatter_sum, ts.scatter_mean, ts.scatter_max, ts.scatter_std):
         op(src, index, dim=0, dim_size=N)
+
+
+@pytest.mark.parametrize("K,taken", [(64, False), (130, True)])
+def test_std_of_a_src_off_its_border(K, taken):
+    """ts_group_std_forward with the workspace that its query reports, src one element off a 16-byte border: rows that the
+    buckets then hold no longer (64 lanes) are refused as unsupported, not as a workspace too small; others are served."""
+    import ctypes
+    from pytorch_scatter_amd import capi
+    E, N = (1 << 22) // max(1, K // 16), 70_001
+    g = torch.Generator(device=DEV).manual_seed(K)
+    index = torch.randint(0, N, (E,), generator=g, device=DEV)
+    src = torch.randn(E * K + 1, generator=g, device=DEV)[1:].view(E, K)
+    assert src.data_ptr() % 16 == 4
+    total, out = torch.empty((N, K), device=DEV), torch.empty((N, K), device=DEV)
+    count = torch.empty(N, dtype=torch.int32, device=DEV)
+    i, p = capi._i, capi._p
+    nbytes = int(capi.lib().ts_group_std_workspace_bytes(i(1), i(E), i(K), i(N), 0))
+    assert nbytes > 0
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    rc = capi.lib().ts_group_std_forward(p(src), p(index), p(total), p(count), p(out), i(1), i(E), i(K), i(N), i(0), i(1), 0, 1,
+                                         p(ws), ctypes.c_size_t(nbytes), capi._stream(out))
+    assert rc == (0 if taken else 2)  # TS_OK, TS_ERR_UNSUPPORTED
+    import pytorch_scatter_amd as ts
+    got = ts.scatter_std(src, index, dim=0, dim_size=N)
+    want = ts.scatter_std(src.double(), index, dim=0, dim_size=N)
+    for x in [got] + ([out] if taken else []):
+        assert torch.allclose(x.double(), want, rtol=1e-5, atol=1e-6)
