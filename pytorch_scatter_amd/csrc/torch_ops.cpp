@@ -672,16 +672,19 @@ template <int REDUCE> struct ScatterFn : public torch::autograd::Function<Scatte
     ctx->save_for_backward({index, arg_out});
     ctx->mark_non_differentiable({arg_out});
     ctx->set_materialize_grads(false);  // no zeros [.., N, ..] in the place of a gradient of the positions
+    ctx->saved_data["src_dtype"] = static_cast<int64_t>(src.scalar_type());
     return {out, arg_out};
   }
 
   static variable_list backward(AutogradContext *ctx, variable_list grad_outs) {
     auto grad_out = grad_outs[0];
-    if (!grad_out.defined()) return variable_list(5);
     auto saved = ctx->get_saved_variables();
     const int64_t dim = ctx->saved_data["dim"].toInt();
     Variable grad_in;
-    if (REDUCE == TS_SUM) {
+    if (!grad_out.defined()) {  // (min / max: whoever used the values handed no gradient back) zeros, as everywhere else
+      const auto dtype = static_cast<at::ScalarType>(ctx->saved_data["src_dtype"].toInt());
+      grad_in = at::zeros(saved_shape(ctx), saved[1].options().dtype(dtype));
+    } else if (REDUCE == TS_SUM) {
       grad_in = gather_grad_rows(grad_out, saved[0], dim, std::nullopt);
     } else if (REDUCE == TS_MUL) {
       grad_in = at::gather(grad_out * saved[2], dim, saved[1], false).div_(saved[0]);

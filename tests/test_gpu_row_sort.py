@@ -193,3 +193,24 @@ def test_std_of_a_src_off_its_border(K, taken):
     want = ts.scatter_std(src.double(), index, dim=0, dim_size=N)
     for x in [got] + ([out] if taken else []):
         assert torch.allclose(x.double(), want, rtol=1e-5, atol=1e-6)
+
+
+class _NoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+@pytest.mark.parametrize("op", ["scatter_sum", "scatter_mean", "scatter_min", "scatter_max"])
+def test_no_gradient_from_above_is_zero(op):
+    """A function behind the call that hands no gradient back: the gradient of src is zeros, not missing."""
+    import pytorch_scatter_amd as ts
+    src = torch.randn((40, 3), dtype=torch.float64, device=DEV, requires_grad=True)
+    out = getattr(ts, op)(src, torch.arange(40, device=DEV) % 7, 0)
+    y = _NoGradient.apply(out[0] if isinstance(out, tuple) else out)
+    (grad,) = torch.autograd.grad(y.sum(), src)
+    assert grad.dtype == src.dtype and torch.equal(grad, torch.zeros_like(src))
