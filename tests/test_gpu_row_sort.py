@@ -2,6 +2,7 @@
 of 8192 entries, buckets at and above what one sorting workgroup holds (8192 entries, 16384 from 4 M entries on), buckets
 of one row and of 8192 rows, entries outside [0, N), an index in order. Sums of int32 are exact; min / max must give the
 first position of equal values. The expected results come from torch on the same device."""
+import numpy as np
 import pytest
 import torch
 
@@ -111,6 +112,12 @@ def test_arg_backward_rows(kind, B, E, K, N, dtype, monkeypatch):
     out = torch.empty((B, N, K), dtype=dtype, device=DEV)
     arg = torch.empty((B, N, K), dtype=torch.int64, device=DEV)
     capi.scatter_with_workspace(src, index, out, arg, B, E, K, N, 0, 1, 0, capi.MAX, 0)
+    ok = (index >= 0) & (index < N)
+    full, x = index[ok].view(1, -1, 1).expand(B, -1, K), src[:, ok].double()
+    top = torch.full((B, N, K), -100.0, dtype=torch.float64, device=DEV).scatter_reduce_(1, full, x, "amax")
+    first = torch.where(x == top.gather(1, full), torch.nonzero(ok).view(1, -1, 1).expand(B, -1, K), E)
+    want_arg = torch.full((B, N, K), E, device=DEV).scatter_reduce_(1, full, first, "amin")
+    assert torch.equal(arg, want_arg) and torch.equal(out.double(), torch.where(want_arg < E, top, 0.0))
     grad = torch.randn((B, N, K), generator=g, device=DEV).to(dtype)
     want = torch.zeros((B, E + 1, K), dtype=dtype, device=DEV).scatter_(1, arg, grad)[:, :E]
     got = torch.full((B, E, K), 7, dtype=dtype, device=DEV)
@@ -214,3 +221,147 @@ def test_no_gradient_from_above_is_zero(op):
     y = _NoGradient.apply(out[0] if isinstance(out, tuple) else out)
     (grad,) = torch.autograd.grad(y.sum(), src)
     assert grad.dtype == src.dtype and torch.equal(grad, torch.zeros_like(src))
+
+
+def _special_values(shape, dtype, rng):
+    """Small whole numbers (many ties) and, one in twenty, the values that trip a comparison: the limits of the type and, for
+    floating types, infinities, NaN and -0.0."""
+    x = torch.from_numpy(rng.integers(0 if dtype == torch.uint8 else -8, 9, size=shape)).to(dtype)
+    if dtype.is_floating_point:
+        info = torch.finfo(dtype)
+        extra = torch.tensor([info.min, info.max, float("inf"), -float("inf"), float("nan"), -0.0], dtype=dtype)
+    else:
+        info = torch.iinfo(dtype)
+        extra = torch.tensor([info.min, info.max, info.min + 1, info.max - 1], dtype=dtype)
+    pick = torch.from_numpy(rng.integers(0, len(extra), size=shape))
+    return torch.where(torch.from_numpy(rng.random(shape) < 0.05), extra[pick], x)
+
+
+def _index_layout(layout, B, E, N, kind, rng):
+    """[B, E] rows on the CPU; the device tensor that holds them and the strides of a batch and an entry in it."""
+    own = layout != "shared"
+    rows = rng.integers(0, N, size=(B if own else 1, E))
+    if kind == "hub":  # half of the entries in one row: more than 32 tiles of the reduction
+        rows = np.where(rng.random(rows.shape) < 0.5, N // 3, rows)
+    if kind == "sorted":
+        rows = np.sort(rows, axis=1)
+    rows = torch.from_numpy(rows)
+    if layout == "every second":
+        held = torch.full((rows.shape[0], 2 * E), -5, dtype=torch.long)
+        held[:, ::2] = rows
+        return rows.expand(B, E), held.to(DEV), 2 * E, 2
+    return rows.expand(B, E), rows.to(DEV), E if own else 0, 1
+
+
+LAYOUTS = [("even", "shared", 1, 3000, 250), ("hub", "shared", 1, 40001, 40), ("hub", "every second", 1, 9001, 300),
+           ("even", "own", 3, 3001, 90), ("sorted", "own", 3, 2500, 90), ("even", "every second", 2, 2500, 700)]
+
+
+@pytest.mark.parametrize("reduce", ["min", "max"])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.int64, torch.float32, torch.bfloat16, torch.int32, torch.uint8])
+@pytest.mark.parametrize("K", [64, 33, 520])
+@pytest.mark.parametrize("kind,layout,B,E,N", LAYOUTS)
+def test_minmax_rows(oracle, kind, layout, B, E, N, K, dtype, reduce, monkeypatch):
+    """Values and positions of min / max as the oracle has them, for every accumulator width (8-byte carries of values and
+    positions among them), 33 single columns, 520 columns in more than four column chunks, with and without an initial out."""
+    from pytorch_scatter_amd import capi
+    monkeypatch.setenv("TS_SCATTER_BINNED", "2")
+    if K * (torch.finfo(dtype) if dtype.is_floating_point else torch.iinfo(dtype)).bits < 512:
+        pytest.skip("rows under 64 bytes are not sorted")
+    if K == 520:
+        B, E = 1, min(E, 6000)
+    if kind == "hub" and K != 33:
+        E = min(E, 12001)
+    rng = np.random.default_rng(E + K)
+    rows, held, sb, se = _index_layout(layout, B, E, N, kind, rng)
+    src = _special_values((B, E, K), dtype, rng)
+    full = rows.unsqueeze(-1).expand(B, E, K)
+    for given in (False, True):
+        want = _special_values((B, N, K), dtype, rng) if given else None
+        out = want.to(DEV) if given else torch.empty((B, N, K), dtype=dtype, device=DEV)
+        arg = torch.empty((B, N, K), dtype=torch.long, device=DEV)
+        want, want_arg = oracle.scatter(src, full, 1, want, None if given else N, reduce)
+        capi.scatter_with_workspace(src.to(DEV), held, out, arg, B, E, K, N, sb, se, 0, capi.REDUCE[reduce], given)
+        assert capi.scatter_last_route().startswith("min/max: buckets or segmented")
+        assert torch.equal(arg.cpu(), want_arg), given
+        got = out.cpu()
+        same = (got == want) | ((got != got) & (want != want))
+        assert bool(same.all()), given
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind,layout,B,E,N", LAYOUTS[2:])
+def test_sum_and_std_layouts(kind, layout, B, E, N, dtype, monkeypatch):
+    """Sums (of whole numbers: exact) and standard deviations under an index of its own per batch and with strides."""
+    from pytorch_scatter_amd import capi
+    monkeypatch.setenv("TS_SCATTER_BINNED", "2")
+    monkeypatch.setenv("TS_GROUP_BINS", "0")
+    K = 40
+    rng = np.random.default_rng(E)
+    rows, held, sb, se = _index_layout(layout, B, E, N, kind, rng)
+    # (bf16: at most 4500 ones and zeros to a row, which a partial sum in more than 16 bits rounds once at the end)
+    src = torch.from_numpy(rng.integers(0, 2, size=(B, E, K)) if dtype == torch.bfloat16 else rng.integers(-9, 10, size=(B, E, K)))
+    want = torch.zeros((B, N, K), dtype=torch.long).scatter_add_(1, rows.unsqueeze(-1).expand(B, E, K), src)
+    for given in (False, True):
+        out = torch.full((B, N, K), 3, dtype=dtype, device=DEV)
+        capi.scatter_with_workspace(src.to(dtype).to(DEV), held, out, None, B, E, K, N, sb, se, 0, capi.SUM, given)
+        assert capi.scatter_last_route().startswith("sum: buckets or segmented")
+        assert torch.equal(out.cpu(), (want + (3 if given else 0)).to(dtype)), given
+    if dtype == torch.float32:
+        total, out = (torch.empty((B, N, K), device=DEV) for _ in range(2))
+        count = torch.empty((B, N), dtype=torch.int32, device=DEV)
+        capi.group_std_forward(src.to(dtype).to(DEV), held, total, count, out, B, E, K, N, sb, se, True)
+        n = torch.zeros((B, N), dtype=torch.long).scatter_add_(1, rows, torch.ones((B, E), dtype=torch.long))
+        assert torch.equal(count.cpu().long(), n) and torch.equal(total.cpu().long(), want)
+        full = rows.unsqueeze(-1).expand(B, E, K)
+        c = n.clamp(min=1).unsqueeze(-1).double()
+        dev = (src - (want / c).gather(1, full)) ** 2
+        exact = (torch.zeros((B, N, K), dtype=torch.double).scatter_add_(1, full, dev) / ((c - 1).clamp(min=1) + 1e-6)).sqrt()
+        # roundings as in test_std_rows; the mean is at most 9
+        assert bool(((out.cpu().double() - exact).abs() <= 2.0 ** -23 * (4 * exact + 36) + 1e-12).all())
+
+
+def test_more_than_1024_buckets(monkeypatch):
+    """From 12.6 M entries the buckets outnumber the lanes of the workgroup that turns their totals into starts; one of them is
+    a hub of many chunks."""
+    from pytorch_scatter_amd import capi
+    monkeypatch.setenv("TS_SCATTER_BINNED", "2")
+    E, N, K = 16_000_001, 1_500_007, 16
+    g = torch.Generator(device=DEV).manual_seed(3)
+    index = torch.randint(0, N, (E,), generator=g, device=DEV)
+    index[::9] = 77_777
+    src = torch.randint(-50, 51, (E, K), generator=g, device=DEV, dtype=torch.int32)
+    out = torch.full((N, K), 9, dtype=torch.int32, device=DEV)
+    capi.scatter_with_workspace(src, index, out, None, 1, E, K, N, 0, 1, 0, capi.SUM, 0)
+    want = torch.zeros((N, K), dtype=torch.int32, device=DEV).index_add_(0, index, src)
+    assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("op", ["scatter_max", "scatter_min"])
+@pytest.mark.parametrize("layout", ["expanded", "per batch", "every second", "full"])
+def test_arg_backward_through_autograd(op, layout, monkeypatch):
+    """Gradients of the operators through the rows in order (forced at this size); a full index keeps the other route."""
+    import pytorch_scatter_amd as ts
+    monkeypatch.setenv("TS_SCATTER_BINNED", "2")
+    B, E, N, K = 2, 3001, 70, 64
+    rng = np.random.default_rng(E)
+    rows, held, _, _ = _index_layout("every second" if layout == "every second" else "shared" if layout == "expanded" else "own",
+                                     B, E, N, "even", rng)
+    index = held[:, ::2] if layout == "every second" else held[0] if layout == "expanded" else held
+    if layout == "full":
+        index = index.unsqueeze(-1).expand(B, E, K).contiguous()
+    elif layout != "expanded":
+        index = index.unsqueeze(-1)
+    src = torch.from_numpy(rng.integers(-9, 10, size=(B, E, K))).double()
+    grad = torch.randn((B, N, K), dtype=torch.double)
+    full = rows.unsqueeze(-1).expand(B, E, K)
+    # the first position of the best value of every row, from the values alone
+    best = torch.zeros((B, N, K), dtype=torch.double).scatter_reduce_(1, full, src, "amax" if op == "scatter_max" else "amin", include_self=False)
+    at = torch.arange(E).view(1, E, 1).expand(B, E, K)
+    first = torch.full((B, N, K), E).scatter_reduce_(1, full, torch.where(src == best.gather(1, full), at, E), "amin")
+    want = torch.where(first.gather(1, full) == at, grad.gather(1, full), 0.0)
+    x = src.to(DEV).requires_grad_()
+    out, arg = getattr(ts, op)(x, index, dim=1, dim_size=N)
+    assert torch.equal(arg.cpu(), first) and torch.equal(out.detach().cpu(), best)
+    (got,) = torch.autograd.grad(out, x, grad.to(DEV))
+    assert torch.equal(got.cpu(), want)
