@@ -30,7 +30,8 @@ CASES = [("even", 8191, 300), ("even", 8192, 300), ("even", 8193, 300), ("one ro
          ("one row", 50001, 1), ("hub8191", 20000, 40), ("hub8192", 20000, 40), ("hub8193", 20000, 40),
          ("hub30000", 60001, 100000), ("even", 30000, 600001), ("sorted", 30001, 7000), ("outside", 30001, 7000),
          ("even", 1, 1), ("even", 4194303, 70001), ("even", 4194305, 70001), ("hub16384", 4194305, 2000003),
-         ("hub16385", 4194305, 2000003), ("hub1000000", 4194304, 1000)]
+         ("hub16385", 4194305, 2000003), ("hub1000000", 4194304, 1000),
+         ("hub200001", 600001, 8400007), ("even", 600001, 8400007)]
 
 
 @pytest.mark.parametrize("kind,E,N", CASES)
