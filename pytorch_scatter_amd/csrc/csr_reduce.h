@@ -115,6 +115,20 @@ template <typename A> __device__ __forceinline__ uint64_t carry_put(A *p, A v) {
   __builtin_memcpy(&bits, &v, sizeof(A));
   return (uint64_t)__hip_atomic_exchange(reinterpret_cast<U *>(p), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// a value of 4 bytes and its position as one word (half the atomics of a carry)
+template <typename A> __device__ __forceinline__ uint64_t carry_put_pair(uint64_t *p, A v, int32_t arg) {
+  uint32_t bits;
+  __builtin_memcpy(&bits, &v, 4);
+  return __hip_atomic_exchange(p, (uint64_t)(uint32_t)arg << 32 | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename A> __device__ __forceinline__ A carry_get_pair(uint64_t *p, int32_t &arg) {
+  const uint64_t w = __hip_atomic_fetch_or(p, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint32_t bits = (uint32_t)w;
+  arg = (int32_t)(w >> 32);
+  A v;
+  __builtin_memcpy(&v, &bits, 4);
+  return v;
+}
 template <typename A> __device__ __forceinline__ A carry_get(A *p) {
   typedef typename CarryBits<A>::type U;
   const U bits = __hip_atomic_fetch_or(reinterpret_cast<U *>(p), (U)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -344,9 +358,14 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   if constexpr (kThrough) {
     const int32_t *perm_b = a.perm + b * a.perm_batch_stride;
     const int32_t last_row = a.E > 0 ? (int32_t)(a.E - 1) : 0;
-    for (int t = tid; t < ne; t += kCsrBlock) {
-      const int32_t r = perm_b[j0 + t];
-      s_perm[t] = r < 0 ? 0 : (r > last_row ? last_row : r);  // a malformed perm must not read outside src
+    constexpr int PU = 4;  // loads on the way together
+    for (int t0 = tid; t0 < ne; t0 += PU * kCsrBlock) {
+      int32_t r[PU];
+#pragma unroll
+      for (int q = 0; q < PU; ++q) r[q] = perm_b[j0 + (t0 + q * kCsrBlock < ne ? t0 + q * kCsrBlock : ne - 1)];
+#pragma unroll
+      for (int q = 0; q < PU; ++q)  // a malformed perm must not read outside src
+        if (t0 + q * kCsrBlock < ne) s_perm[t0 + q * kCsrBlock] = r[q] < 0 ? 0 : (r[q] > last_row ? last_row : r[q]);
     }
     if (kArg && a.perm_args) arg_perm = perm_b;
   }
@@ -481,8 +500,16 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   }
   while (r < ri1) flush();
 
+  constexpr bool kCarryOk = sizeof(A) >= 4;  // carries move through 32- and 64-bit atomics
+  const bool lookback = kCarryOk && a.lookback != 0;
+  // A tile inside one row (most tiles of a hub): the workers' parts meet in registers, then the wavefronts' in LDS. (One after
+  // the other, as below, they took 30 of 300 us: max of 10 M x 32 floats in 7 rows. Not with single columns, few workers to
+  // a tile: a hub of 33 floats gained nothing, rows of fifteen entries lost, sum / max of 1 M entries 76 / 84 -> 86 / 94 us.)
+  constexpr bool kOneRow = kTies && VEC > 1;
+  const bool one_row = kOneRow && lookback && nr == 0 && ne > 0 && i0 < a.N;
+
   // edges of a row whose end lies beyond this worker
-  if (has_work && (i0 + r < a.N)) {
+  if (!one_row && has_work && (i0 + r < a.N)) {
     const int32_t rs = s_ptr[r];
     const int first = rs > je0 ? rs : je0;
     if (je1 > first) {
@@ -503,8 +530,6 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
       }
     }
   }
-  constexpr bool kCarryOk = sizeof(A) >= 4;  // carries move through 32- and 64-bit atomics
-  const bool lookback = kCarryOk && a.lookback != 0;
   // default: the tile leaves no open row; the worker that does overwrites this after the barrier
   if (!lookback && tid == 0 && blockIdx.y == 0) a.ws_meta[(b * a.nblk + blockIdx.x) * 4 + 2] = -1;
   __syncthreads();
@@ -534,14 +559,21 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   auto carry_pos = [&](int v) -> int64_t {
     return carry_transposed ? (int64_t)blockIdx.y * CW + (int64_t)v * G + lg : col + v;
   };
+  // scatter min / max of 4-byte accumulators: value and position side by side (the value slots of a tile hold 2 K of them)
+  constexpr bool kPair = kOneRow && kArg && sizeof(A) == 4;
+  uint64_t *pairs = static_cast<uint64_t *>(a.ws_vals);
   auto publish_carry = [&](uint64_t kind) {
     if constexpr (kCarryOk) {
     uint64_t sink = 0;
     if (col_ok) {
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {
-        sink |= carry_put<A>(ws_val_blk + a.K + carry_pos(v), acc[v]);
-        if (kArg) sink |= carry_put<int32_t>(ws_arg_blk + a.K + carry_pos(v), arg[v]);
+        if constexpr (kPair) {
+          sink |= carry_put_pair<A>(pairs + (b * a.nblk + blockIdx.x) * a.K + carry_pos(v), acc[v], arg[v]);
+        } else {
+          sink |= carry_put<A>(ws_val_blk + a.K + carry_pos(v), acc[v]);
+          if (kArg) sink |= carry_put<int32_t>(ws_arg_blk + a.K + carry_pos(v), arg[v]);
+        }
       }
     }
     asm volatile("" ::"v"(sink) : "memory");  // the returns are in: the carry is in memory
@@ -601,8 +633,12 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
 #pragma unroll
           for (int v = 0; v < VEC; ++v) {
             const int64_t cp = col_ok ? carry_pos(v) : (int64_t)v;
-            early[q][v] = carry_get<A>(vals_b + ((hi - q * stride) * 2 + 1) * a.K + cp);
-            if (kArg) early_arg[q][v] = carry_get<int32_t>(args_b + ((hi - q * stride) * 2 + 1) * a.K + cp);
+            if constexpr (kPair) {
+              early[q][v] = carry_get_pair<A>(pairs + (b * a.nblk + hi - q * stride) * a.K + cp, early_arg[q][v]);
+            } else {
+              early[q][v] = carry_get<A>(vals_b + ((hi - q * stride) * 2 + 1) * a.K + cp);
+              if (kArg) early_arg[q][v] = carry_get<int32_t>(args_b + ((hi - q * stride) * 2 + 1) * a.K + cp);
+            }
           }
         }
       }
@@ -645,6 +681,27 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
     }
   };
 
+  if constexpr (kOneRow) {
+    if (one_row) {
+      for (int step = G; step < kWave; step <<= 1) {
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) {
+          const A x = __shfl_xor(acc[v], step);
+          const int32_t xa = kArg ? __shfl_xor(arg[v], step) : 0;
+          reduce_step<A, REDUCE, true>(acc[v], arg[v], x, xa);
+        }
+      }
+      if ((tid & (kWave - 1)) < G) {
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) { my_head_val[v] = acc[v]; if (kArg) my_head_arg[v] = arg[v]; }
+      }
+      __syncthreads();
+      if (w != 0) return;
+      for (int ww = kWave / G; ww < W; ww += kWave / G) absorb_head(ww);
+      publish_carry(s_ptr[0] < 0 ? kCarryPass : kCarryTail);
+      return;
+    }
+  }
   if (s_tail_row[w] >= 0) {
     // this worker opened a row: gather the heads of the workers after it
     const int row = s_tail_row[w];
