@@ -218,16 +218,16 @@ inline int rows_acc_bytes(int dtype, int reduce) {
   return kElemBytes[dtype] == 8 || (sum && is_float_dtype(dtype)) ? 8 : 4;
 }
 CsrPlan rows_csr_plan(int64_t rows, int64_t n, int64_t K, int dtype, bool al, int reduce) {
-  const bool minmax = reduce == TS_MIN || reduce == TS_MAX;
-  CsrPlan p = csr_plan(rows, n, K, kElemBytes[dtype], al, false, minmax, false);
+  CsrPlan p = csr_plan(rows, n, K, kElemBytes[dtype], al, false, reduce == TS_MIN || reduce == TS_MAX, false);
   if (getenv("TS_CSR_IPW")) return p;  // tuning aid
-  // Items per worker: about 1024 workgroups, 24 ... 72 items each, up to 144 where a worker takes single columns. A hub
-  // row is put together from the carries of all its tiles, so short tiles cost there what they gain elsewhere (970 k x
-  // 33 floats, a fifth of them in one row: sum 327 / 156 / 123 us at 24 / 72 / 144 items, max 279 / 183 / 135; even
-  // index, std of 1 M x 33: 274 / 274 / 278 us; 240 k x 256 floats, hub: sum 154 / 108 / 98 us).
+  // Items per worker: about 1024 workgroups, 24 ... 72 items each, up to 192 where a worker takes single columns (144: the
+  // workgroups of 1 M entries just miss running all at once, sum / max of 1 M x 33 floats 59 / 67 against 50 / 62 us; 384:
+  // 59 / 77). A hub row is put together from the carries of all its tiles, so short tiles cost there what they gain
+  // elsewhere (1 M x 33 floats, a fifth of them in one row, sum / max: 24 items 90 / 116 us, 72 56 / 68, 192 50 / 64; 300 k x
+  // 32 floats, max: 24 items 38 us, 40 42, 64 50, even index 24 / 31 / 41).
   const int64_t items = rows + n;
   const int W = kCsrBlock / p.G;
-  const int most = p.vec == 1 ? 144 : (items >= ((int64_t)32 << 20) ? 64 : 72), least = minmax ? 40 : 24;
+  const int most = p.vec == 1 ? 192 : (items >= ((int64_t)32 << 20) ? 64 : 72), least = 24;
   int64_t want = items / ((int64_t)W * 1024);
   want = want > most ? most : (want < least ? least : want);
   const int cap = kCsrMaxItems / W;
@@ -275,9 +275,9 @@ RowsRoute rows_route(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int 
   r.ok = true;
   return r;
 }
-// perm / ptr as launch_row_sort leaves them; ws: RowsRoute::csr_bytes and behind them the status words. status_nonce: one
-// for all reductions of a call; the first of them (status_reset) writes it into word 0.
-int rows_reduce_args(CsrReduceArgs &a, const CsrPlan &p, const void *src, const int32_t *perm, const int64_t *ptr, void *out,
+// sorted: as launch_row_sort leaves it (without the identity); ws: RowsRoute::csr_bytes and behind them the status words.
+// status_nonce: one for all reductions of a call; the first of them (status_reset) writes it into word 0.
+int rows_reduce_args(CsrReduceArgs &a, const CsrPlan &p, const void *src, const RowSortArgs &sorted, void *out,
                      int64_t *arg_out, int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce, int out_given,
                      void *ws, size_t ws_bytes, uint64_t status_nonce, bool status_reset) {
   const int64_t n = B * E, rows = B * N;
@@ -287,7 +287,7 @@ int rows_reduce_args(CsrReduceArgs &a, const CsrPlan &p, const void *src, const 
                    a.meta_stride) > ws_bytes)
     return TS_ERR_WORKSPACE;
   a.src = src;
-  a.indptr = ptr;
+  a.indptr = sorted.ptr;
   a.out = out;
   a.arg_out = arg_out;
   a.count_out = nullptr;
@@ -305,7 +305,8 @@ int rows_reduce_args(CsrReduceArgs &a, const CsrPlan &p, const void *src, const 
   a.ws_meta = reinterpret_cast<int64_t *>(static_cast<char *>(ws) + off_meta);
   a.lookback = p.nblk > 1;
   a.nonce = next_nonce();
-  a.perm = perm;
+  a.perm = sorted.perm;
+  a.unsorted = sorted.state;
   a.perm_batch_stride = 0;
   a.perm_args = 0;
   a.any_order = 1;
@@ -316,12 +317,12 @@ int rows_reduce_args(CsrReduceArgs &a, const CsrPlan &p, const void *src, const 
   a.carry_spin = env_int("TS_CSR_SPIN", kCarrySpin);  // test aid: -1 makes every look-back give up at once
   return TS_OK;
 }
-int run_rows_reduce(const void *src, const int32_t *perm, const int64_t *ptr, void *out, int64_t *arg_out, int64_t B,
+int run_rows_reduce(const void *src, const RowSortArgs &sorted, void *out, int64_t *arg_out, int64_t B,
                     int64_t E, int64_t K, int64_t N, int dtype, int reduce, int out_given, void *ws, size_t ws_bytes,
                     uint64_t status_nonce, hipStream_t s) {
   const CsrPlan p = rows_csr_plan(B * N, B * E, K, dtype, aligned16(src) && aligned16(out), reduce);
   CsrReduceArgs a;
-  const int rc = rows_reduce_args(a, p, src, perm, ptr, out, arg_out, B, E, K, N, dtype, reduce, out_given, ws, ws_bytes,
+  const int rc = rows_reduce_args(a, p, src, sorted, out, arg_out, B, E, K, N, dtype, reduce, out_given, ws, ws_bytes,
                                   status_nonce, true);
   return rc != TS_OK ? rc : dispatch_csr_reduce(dtype, a, p, 1, reduce, s);
 }
@@ -740,9 +741,9 @@ int scatter_ws_impl(const void *src, const int64_t *index, void *out, int64_t *a
       RowSortPlan sp = row_sort_plan(B, E, N, workspace, rr.sort_bytes);
       if (!sp.ok) return TS_ERR_WORKSPACE;
       ts_note_scatter_route(reduce == TS_SUM ? TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED : TS_ROUTE_MINMAX_BUCKETS_OR_SEGMENTED);
-      int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, s);
+      int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, false, s);
       if (rc != TS_OK) return rc;
-      rc = run_rows_reduce(src, sp.p.perm, sp.p.ptr, out, arg_out, B, E, K, N, dtype, reduce, out_given,
+      rc = run_rows_reduce(src, sp.p, out, arg_out, B, E, K, N, dtype, reduce, out_given,
                            static_cast<char *>(workspace) + rr.sort_bytes, rr.csr_bytes, next_nonce(), s);
       if (rc != TS_OK || count_out == nullptr) return rc;
       hipLaunchKernelGGL(row_lengths_kernel, dim3(grid_for(B * N)), dim3(kBlock), 0, s, sp.p.ptr, count_out, B * N);
@@ -956,7 +957,7 @@ int ts_arg_backward_rows(const void *grad_out, const int64_t *arg, const int64_t
   RowSortPlan sp = row_sort_plan(B, E, N, workspace, workspace_bytes);
   if (!sp.ok) return TS_ERR_WORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, s);
+  const int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, true, s);
   if (rc != TS_OK) return rc;
   RowSortArgs p = sp.p;
   p.index = index;
@@ -1205,16 +1206,16 @@ int ts_group_std_forward(const void *src, const int64_t *index, void *total, int
     if (!sp.ok) return TS_ERR_WORKSPACE;
     hipStream_t s = static_cast<hipStream_t>(stream);
     void *const ws = static_cast<char *>(workspace) + rr.sort_bytes;
-    int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, s);
+    int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, false, s);
     if (rc != TS_OK) return rc;
     const uint64_t status_nonce = next_nonce();
-    rc = run_rows_reduce(src, sp.p.perm, sp.p.ptr, total, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes,
+    rc = run_rows_reduce(src, sp.p, total, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes,
                          status_nonce, s);
     if (rc != TS_OK) return rc;
     hipLaunchKernelGGL(row_lengths_kernel, dim3(grid_for(B * N)), dim3(kBlock), 0, s, sp.p.ptr, count, B * N);
     const CsrPlan p = rows_csr_plan(B * N, B * E, K, dtype, al && aligned16(total) && aligned16(out), TS_SUM);
     CsrReduceArgs a;
-    rc = rows_reduce_args(a, p, src, sp.p.perm, sp.p.ptr, out, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes,
+    rc = rows_reduce_args(a, p, src, sp.p, out, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes,
                           status_nonce, false);
     if (rc != TS_OK) return rc;
     a.row_total = total;

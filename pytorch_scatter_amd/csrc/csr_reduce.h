@@ -40,6 +40,7 @@ constexpr int kMaxBlockItems = 2048;  // rows + edges per workgroup tile
 constexpr int kCsrBlock = TS_CSR_BLOCK;  // lanes per workgroup of csr_reduce_kernel
 constexpr int kCsrMaxItems = kMaxBlockItems * kCsrBlock / 256;  // rows + edges per tile of csr_reduce_kernel
 constexpr int kSharedWalkMin = 32;  // tiles a row must have passed through before the workgroup shares the walk
+constexpr int kSharedWalkMinScatter = 8;  // ... of a scatter, whose heavy rows stand anywhere, also behind the last short one
 constexpr int kLoadsInFlight = TS_CSR_U;  // U: 16-byte loads per lane per batch (two batches in flight)
 
 struct CsrReduceArgs {
@@ -77,6 +78,7 @@ struct CsrReduceArgs {
   // arg_E: entries per batch, so that positions come out inside their batch. accumulate: combined with out.
   int any_order = 0;
   int64_t arg_E = 0;
+  const int32_t *unsorted = nullptr;  // reads 0: the index was in order, perm the identity (not read, it may be unwritten)
   int meta_stride = 4;  // words of ws_meta per tile: at least one carry flag per column chunk
   // kRowDeviation: the rows' sums in the element type [N, K], and whether the divisor is count - 1
   const void *row_total = nullptr;
@@ -199,6 +201,8 @@ template <typename T> struct CsrAcc<T, TS_MAX, 2> { typedef typename MinMaxAcc<T
 template <typename T, typename A, int REDUCE> __device__ __forceinline__ A csr_acc_init() {
   return (A)acc_init<typename Acc<T>::type, REDUCE>();
 }
+
+template <bool V> struct CsrTag { static constexpr bool value = V; };
 
 // Write one finished row slice. `count` is the full length of the row.
 // ACCUM: 0 = `out` is overwritten (known at compile time: the row-end code sits in divergent control flow,
@@ -355,11 +359,13 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   if (tid == 0) { s_ptr[nload] = INT32_MAX; s_ptr[nload + 1] = INT32_MAX; }  // rows past the last one never end
   int32_t *const s_perm = s_ptr + nload + 2;
   const int32_t *arg_perm = nullptr;  // set: positions leave the kernel in src's order
+  bool in_order = false;  // the same for every lane
+  if constexpr (kTies) in_order = a.unsorted != nullptr && *a.unsorted == 0;
   if constexpr (kThrough) {
     const int32_t *perm_b = a.perm + b * a.perm_batch_stride;
     const int32_t last_row = a.E > 0 ? (int32_t)(a.E - 1) : 0;
     constexpr int PU = 4;  // loads on the way together
-    for (int t0 = tid; t0 < ne; t0 += PU * kCsrBlock) {
+    for (int t0 = in_order ? ne : tid; t0 < ne; t0 += PU * kCsrBlock) {
       int32_t r[PU];
 #pragma unroll
       for (int q = 0; q < PU; ++q) r[q] = perm_b[j0 + (t0 + q * kCsrBlock < ne ? t0 + q * kCsrBlock : ne - 1)];
@@ -465,38 +471,51 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   const T *src_col = src_b + col_ld;
   // Software pipeline: the loads of batch i+1 are issued before batch i is
   // reduced, so a wavefront always has U to 2U 16-byte loads outstanding.
-  auto load_batch = [&](Vec<T, VEC> *x, int e) {
+  // Direct: rows in place; of a scatter whose index was in order, with positions that ascend (no ties to settle, nothing read
+  // from LDS for an entry: max of 2.3 M x 32 floats 94 -> 76 us)
+  auto sweep = [&](auto direct) __attribute__((always_inline)) {
+    constexpr bool kDirect = decltype(direct)::value;
+    auto load_batch = [&](Vec<T, VEC> *x, int e) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      int ee = e + u < je1 ? e + u : je1 - 1;
-      const int64_t srow = kThrough ? (int64_t)s_perm[ee] : j0 + ee;
-      x[u] = load_vec_stream<T, VEC>(src_col + srow * a.K);
-    }
-  };
-  Vec<T, VEC> x[U];
-  if (je0 < je1) load_batch(x, je0);
-  for (int e = je0; e < je1; e += U) {
-    Vec<T, VEC> y[U];
-    load_batch(y, e + U);  // unconditional (addresses are clamped): keeps the wait counts exact
+      for (int u = 0; u < U; ++u) {
+        int ee = e + u < je1 ? e + u : je1 - 1;
+        const int64_t srow = kDirect ? j0 + ee : (int64_t)s_perm[ee];
+        x[u] = load_vec_stream<T, VEC>(src_col + srow * a.K);
+      }
+    };
+    Vec<T, VEC> x[U];
+    if (je0 < je1) load_batch(x, je0);
+    for (int e = je0; e < je1; e += U) {
+      Vec<T, VEC> y[U];
+      load_batch(y, e + U);  // unconditional (addresses are clamped): keeps the wait counts exact
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int ce = e + u;
-      if (ce < je1) {
-        while (ce >= rend) flush();
-        const int32_t ge = kTies && kArg ? s_perm[ce] : (int32_t)(j0 + ce);
+      for (int u = 0; u < U; ++u) {
+        const int ce = e + u;
+        if (ce < je1) {
+          while (ce >= rend) flush();
+          const int32_t ge = kTies && kArg && !kDirect ? s_perm[ce] : (int32_t)(j0 + ce);
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) {
-          if constexpr (kDev) {
-            const F d = round_elem<T>(to_acc<T>(x[u].v[v]) - mean[v]);
-            acc[v] = acc[v] + (A)round_elem<T>(d * d);
-          } else {
-            reduce_step<A, REDUCE, kTies>(acc[v], arg[v], (A)to_acc<T>(x[u].v[v]), ge);
+          for (int v = 0; v < VEC; ++v) {
+            if constexpr (kDev) {
+              const F d = round_elem<T>(to_acc<T>(x[u].v[v]) - mean[v]);
+              acc[v] = acc[v] + (A)round_elem<T>(d * d);
+            } else {
+              reduce_step<A, REDUCE, kTies && !kDirect>(acc[v], arg[v], (A)to_acc<T>(x[u].v[v]), ge);
+            }
           }
         }
       }
-    }
 #pragma unroll
-    for (int u = 0; u < U; ++u) x[u] = y[u];
+      for (int u = 0; u < U; ++u) x[u] = y[u];
+    }
+  };
+  if constexpr (kTies) {
+    if (in_order)
+      sweep(CsrTag<true>());
+    else
+      sweep(CsrTag<false>());
+  } else {
+    sweep(CsrTag<!kThrough>());
   }
   while (r < ri1) flush();
 
@@ -504,7 +523,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   const bool lookback = kCarryOk && a.lookback != 0;
   // A tile inside one row (most tiles of a hub): the workers' parts meet in registers, then the wavefronts' in LDS. (One after
   // the other, as below, they took 30 of 300 us: max of 10 M x 32 floats in 7 rows. Not with single columns, few workers to
-  // a tile: a hub of 33 floats gained nothing, rows of fifteen entries lost, sum / max of 1 M entries 76 / 84 -> 86 / 94 us.)
+  // a tile: a hub of 33 floats gained nothing.)
   constexpr bool kOneRow = kTies && VEC > 1;
   const bool one_row = kOneRow && lookback && nr == 0 && ne > 0 && i0 < a.N;
 
@@ -539,7 +558,8 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   bool shared_walk = false;
   if (lookback && s_head_row[0] >= 0) {
     const int row0 = s_head_row[0];
-    shared_walk = (i0 + row0) + ((int64_t)s_ptr[row0] + j0) < ((int64_t)blockIdx.x - kSharedWalkMin) * a.BI;
+    constexpr int kWalkMin = kTies ? kSharedWalkMinScatter : kSharedWalkMin;
+    shared_walk = (i0 + row0) + ((int64_t)s_ptr[row0] + j0) < ((int64_t)blockIdx.x - kWalkMin) * a.BI;
   }
 
   // ---- combine partials of rows that cross worker boundaries, in edge order
@@ -591,11 +611,69 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
   // false: the wait for a carry ran out; the status word is set and the caller writes the row as empty
   auto walk_back = [&](int64_t first_tile, int64_t start, int64_t stride) -> bool {
     if constexpr (kCarryOk) {
+    if (first_tile < 0) first_tile = 0;
+    if constexpr (kTies) {
+      // Scatter (rows of 64 bytes and more: at least four lanes to a worker): every lane watches the flag of one tile, then
+      // the carries are read PF at a time. (Flags and carries PF at a time, as below: a hub of 1600 tiles in single columns
+      // was put together in 200 us.)
+      constexpr int PF = VEC == 1 ? 8 : (VEC <= 4 ? 4 : 2);
+      const uint64_t worker = G == kWave ? ~0ull : ((1ull << G) - 1) << (tid & (kWave - 1) & ~(G - 1));  // its lanes
+      const int64_t step = stride * (kPair ? 1 : 2) * a.K;
+      for (int64_t hi = start; hi >= first_tile; hi -= G * stride) {
+        const int64_t left = (hi - first_tile) / stride + 1;
+        const int n = left < G ? (int)left : G;  // tiles hi, hi - stride, ...
+        uint64_t *flag = carry_flags + (hi - (lg < n ? lg : 0) * stride) * a.meta_stride;
+        int spin = a.carry_spin;
+        while (spin >= 0) {
+          const uint64_t f = __hip_atomic_fetch_or(flag, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if ((__ballot((f >> 2) != a.nonce) & worker) == 0 || --spin <= 0) break;
+          __builtin_amdgcn_s_sleep(4);
+        }
+        if (spin <= 0) {
+          if (lg == 0 && a.status != nullptr)
+            __hip_atomic_exchange(a.status + 1, (unsigned long long)a.status_nonce, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+          return false;
+        }
+        asm volatile("" ::: "memory");
+        int64_t at = kPair ? hi * a.K : (hi * 2 + 1) * a.K;
+        for (int q0 = 0; q0 < n; q0 += PF) {
+          A early[PF][VEC];
+          int32_t early_arg[PF][VEC];
+#pragma unroll
+          for (int q = 0; q < PF; ++q) {
+            if (q0 + q < n) {
+#pragma unroll
+              for (int v = 0; v < VEC; ++v) {
+                const int64_t cp = at + (col_ok ? carry_pos(v) : (int64_t)v);
+                if constexpr (kPair) {
+                  early[q][v] = carry_get_pair<A>(pairs + cp, early_arg[q][v]);
+                } else {
+                  early[q][v] = carry_get<A>(static_cast<A *>(a.ws_vals) + cp);
+                  if (kArg) early_arg[q][v] = carry_get<int32_t>(a.ws_args + cp);
+                }
+              }
+              at -= step;
+            }
+          }
+#pragma unroll
+          for (int q = 0; q < PF; ++q) {
+            if (q0 + q < n) {
+#pragma unroll
+              for (int v = 0; v < VEC; ++v)
+                reduce_step<A, REDUCE, true>(acc[v], arg[v], early[q][v], kArg ? early_arg[q][v] : 0);
+            }
+          }
+        }
+        asm volatile("" ::: "memory");
+        if (lg < n) __hip_atomic_exchange(flag, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      return true;
+    }
     constexpr int PF = VEC <= 4 ? 4 : 2;
     A *vals_b = static_cast<A *>(a.ws_vals) + (b * a.nblk) * 2 * a.K;
     int32_t *args_b = kArg ? a.ws_args + (b * a.nblk) * 2 * a.K : nullptr;
     const int64_t c = col_ok ? col : 0;
-    if (first_tile < 0) first_tile = 0;
     for (int64_t hi = start; hi >= first_tile; hi -= PF * stride) {
       const int64_t left = (hi - first_tile) / stride + 1;
       const int n = left < PF ? (int)left : PF;  // tiles hi, hi - stride, ...

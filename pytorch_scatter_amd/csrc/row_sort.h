@@ -47,6 +47,7 @@ struct RowSortArgs {
   int64_t sb, se;        // element strides of the index over batches and entries
   int64_t B, E, N;
   int64_t n, rows;       // B * E entries, B * N rows
+  int identity;          // an index in order: write the identity to perm (a reader that looks at state[0] does without)
   int flat;              // one batch, unit stride: entry e is index[e] (no 64-bit multiplications per entry)
   int rshift, nb;        // rows per bucket (log2), buckets
   int cap;               // entries that one sorting workgroup takes
@@ -415,7 +416,7 @@ __device__ __forceinline__ void rs_identity(const RowSortArgs &p, int64_t lo, Ga
     const bool live = be < p.n;
     int64_t top = -1, bot = 0;
     if (live) {
-      p.perm[be] = (int32_t)be;
+      if (p.identity) p.perm[be] = (int32_t)be;
       top = rs_row(p, be, at[j]);
       bot = be == 0 ? 0 : (int64_t)rs_row(p, be - 1, before[j]) + 1;
     }
@@ -739,8 +740,10 @@ template <typename W> inline int launch_row_sort_words(const RowSortArgs &p, hip
   return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
 }
 
-inline int launch_row_sort(const RowSortArgs &args, const int64_t *index, int64_t sb, int64_t se, hipStream_t stream) {
+inline int launch_row_sort(const RowSortArgs &args, const int64_t *index, int64_t sb, int64_t se, bool identity,
+                           hipStream_t stream) {
   RowSortArgs p = args;
+  p.identity = identity ? 1 : 0;
   p.index = index;
   p.sb = sb;
   p.se = se;
