@@ -227,7 +227,11 @@ CsrPlan rows_csr_plan(int64_t rows, int64_t n, int64_t K, int dtype, bool al, in
   // 32 floats, max: 24 items 38 us, 40 42, 64 50, even index 24 / 31 / 41).
   const int64_t items = rows + n;
   const int W = kCsrBlock / p.G;
-  const int most = p.vec == 1 ? 192 : (items >= ((int64_t)32 << 20) ? 64 : 72), least = 24;
+  // (min / max of bytes, sixteen columns to a lane, and of rows of 16 lanes and more: 40 at least; 1 M x 64 bytes 153 us, 216 at
+  // 24, 600 k x 128 bf16 80 / 94)
+  const bool minmax = reduce == TS_MIN || reduce == TS_MAX;
+  const int most = p.vec == 1 ? 192 : (items >= ((int64_t)32 << 20) ? 64 : 72);
+  const int least = minmax && (kElemBytes[dtype] == 1 || p.G >= 16) ? 40 : 24;
   int64_t want = items / ((int64_t)W * 1024);
   want = want > most ? most : (want < least ? least : want);
   const int cap = kCsrMaxItems / W;
@@ -245,23 +249,48 @@ RowsRoute rows_route(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int 
   const bool minmax = reduce == TS_MIN || reduce == TS_MAX;
   if (!minmax && reduce != TS_SUM && reduce != TS_MEAN) return r;
   if (!minmax && kAccBytes[dtype] < 4) return r;
-  // From where the six launches of the sort and the reduction (31-37 us on the smallest inputs) cost less than the
-  // atomics of the other kernels (us without / with, 10 entries per row, even index, 32 columns; the skewed cases gain
-  // earlier, the host does not know them):
-  //   sums of 4 bytes    32 MB 35 / 43    48 MB 54 / 48     of 8 bytes  32 MB 32 / 42   48 MB 50 / 45
-  //   sums of 2 bytes    24 MB 45 / 53    32 MB 56 / 55     with 100 entries per row  4 MB 33 / 40   8 MB 45 / 41
-  //   min / max of 4 bytes  16 MB 32 / 54   24 MB 50 / 56   32 MB 56 / 57
-  //   min / max of 2 bytes  16 MB 62 / 73   24 MB 92 / 75   of 8 bytes  16 MB 44 / 44   24 MB 55 / 45
-  // (min / max without the sort fill and walk a table of 8-byte keys as large as out: from 256 MB of keys the sort
-  // wins at any size)
+  // From where the six launches of the sort and the reduction (31-37 us on the smallest inputs) cost less than the kernels
+  // without them. The host knows sizes only; a line lies where an even and a Zipf(1.2) index, each shuffled and in order,
+  // gain together (us of these four, without / with; measured from 0.1 to 10 M entries, 0.3 to 30000 a row):
+  //   sums, 4 bytes: 300 k x 64, 3 a row 81 95 41 60 / 54 64 52 59; 300 k x 32, 10 a row 45 57 27 52 / 40 53 37 44
+  //   fewer entries than rows (out is what moves): int64 1 M x 16 162 176 163 221 / 223 270 217 265, float 4.6 M x 16 534 402
+  //   527 363 / 595 565 512 501, bf16 600 k x 64 114 268 109 114 / 183 248 183 239
+  //   bf16, 1000 a row: 100 k x 64 26 24 17 17 / 40 47 35 37; doubles the same 31 27 16 17 / 39 48 34 37
+  //   rows of 64 bytes, 30000 entries a row: float 4.6 M x 16 144 143 114 133 / 181 181 109 109, double x 8 89 89 106 118 /
+  //   180 179 106 108
+  //   min / max, 4 bytes: 600 k x 16, 10 a row 73 97 47 63 / 55 105 45 90; 300 k x 32, 10 a row 62 87 42 94 / 47 77 40 64
+  //   1000 entries a row (a key table in LDS takes most): 600 k x 16 61 73 23 24 / 68 90 57 72, 300 k x 32 60 61 22 24 / 54 68
+  //   45 54, double 300 k x 8 63 59 27 29 / 52 69 45 57
+  //   30000 a row: 10 M x 16 269 298 157 160 / 379 370 220 217, 1 M x 32 61 62 39 43 / 91 95 68 70, bf16 300 k x 64 53 51 39 39
+  //   / 94 93 73 72
   const int es = kElemBytes[dtype];
-  const int64_t MB = 1000000;
-  // (sums of rows under 128 bytes, or with fewer than two entries per row, gain later: one entry per row, 16 / 32 / 128
-  // floats 96 MB 115 / 122, 106 / 80, 107 / 78)
-  int64_t min_bytes = minmax ? (rows * K * 8 >= 256 * MB ? MB : (es == 4 ? 28 * MB : es == 8 ? 16 * MB : 20 * MB))
-                             : (es >= 4 ? 40 * MB : (n >= 32 * rows ? 6 * MB : 32 * MB));
-  if (!minmax && row_bytes < 128) min_bytes *= 2;
-  if (!minmax && n < 2 * rows) min_bytes *= 2;
+  const int64_t MB = 1000000, kNever = INT64_MAX;
+  int64_t min_bytes;
+  if (minmax) {
+    // (without the sort they fill and walk a table of 8-byte keys as large as out: from 256 MB of keys the sort wins anyhow)
+    min_bytes = rows * K * 8 >= 256 * MB ? MB : (es == 4 ? 28 * MB : es == 8 ? 16 * MB : 20 * MB);
+    // rows that meet hundreds of entries: a key table in LDS takes most of them
+    if (n >= 512 * rows && es >= 4 && row_bytes <= 128) min_bytes = es == 8 ? 30 * MB : 70 * MB;
+    if (n >= 8192 * rows) {
+      const int64_t least = es == 8 ? (row_bytes < 128 ? 60 * MB : 0) : es == 4 ? (row_bytes < 128 ? kNever : 140 * MB)
+                                                                                : (row_bytes <= 128 ? 140 * MB : 30 * MB);
+      if (min_bytes < least) min_bytes = least;
+    }
+  } else {
+    min_bytes = es >= 4 ? 40 * MB : (n >= 32 * rows ? 6 * MB : 32 * MB);
+    if (row_bytes < 128) min_bytes *= 2;
+    if (n < 2 * rows) min_bytes *= 2;
+    // rows that the kernels without the sort add in whole words (the others element by element, which loses anywhere)
+    const bool words = es == 2 ? row_bytes % 4 == 0 : row_bytes % kVecBytes == 0;
+    if (reduce == TS_SUM && words) {  // (TS_MEAN: the deviation, whose other kernels cost more)
+      int64_t least = 0;
+      if (n < rows && row_bytes <= 512) least = row_bytes < 128 || (es == 8 && row_bytes <= 128) ? 320 * MB : 140 * MB;
+      if (es == 2 && n >= 512 * rows) least = 16 * MB;
+      if (es == 8 && n >= 64 * rows) least = 60 * MB;
+      if (es >= 4 && row_bytes == 64 && n >= 8192 * rows) least = kNever;
+      if (min_bytes < least) min_bytes = least;
+    }
+  }
   if (mode != 2 && n * row_bytes < min_bytes) return r;
   const RowSortPlan sp = row_sort_plan(B, E, N, nullptr, 0);
   if (sp.bytes == 0) return r;
@@ -938,12 +967,14 @@ size_t ts_arg_backward_rows_workspace_bytes(int64_t B, int64_t E, int64_t K, int
   const int64_t row_bytes = K * kElemBytes[dtype];
   if (mode == 0 || row_bytes < 64 || K >= (int64_t)1 << 20) return 0;
   // As long as grad_in fits the 256 MB of the memory-side cache, the second pass over it is cheap (us of ts_arg_backward /
-  // this call, 64 floats, even index and a hub: 300 k entries, 3 a row 51 / 57 and 47 / 64; 1 M, 8 a row 110 / 101 and
-  // 72 / 108; 16 floats, 3 M, 3 a row 140 / 185). Beyond it pays wherever the elements of grad_out, 14 ps each in the
-  // scatter, outweigh the sort, 25 ps an entry and 30 us at the least (256 floats, 400 k, 15 a row 245 / 108 and 123 /
-  // 126; 64 floats, 2.3 M, 8 a row 466 / 236 and 226 / 200). Rows that fill no 16-byte vector do not gain (33 doubles,
-  // 2 M, 4 a row 458 / 480 and 223 / 348).
-  if (mode != 2 && (row_bytes < 256 || row_bytes % kVecBytes != 0 || B * E * row_bytes < 384000000 || B * N * K < ((int64_t)4 << 20) + 3 * B * E)) return 0;
+  // this call, even index and a hub: 1 M x 64 floats, 10 a row 90 / 92 and 65 / 90). Beyond it the elements of grad_out, 14 ps
+  // each in the scatter, outweigh the sort (25 ps an entry and 30 us at the least) from B N K = 2.1 M + 1.8 B E on under an
+  // even index. Under a hub fewer of them win, so the line lies at about twice that: 2.3 M entries, 10 a row, 64 floats 414 /
+  // 196 and 188 / 168, 128 bf16 458 / 313 and 226 / 238; 30 a row, left to the scatter, 281 / 164 and 160 / 167, 368 / 225 and
+  // 176 / 236. Rows that fill no 16-byte vector do not gain (33 doubles, 2 M, 4 a row 458 / 480 and 223 / 348).
+  if (mode != 2 && (row_bytes < 256 || row_bytes % kVecBytes != 0 || B * E * row_bytes < 384000000 ||
+                    B * N * K < ((int64_t)4 << 20) + 3 * B * E))
+    return 0;
   return row_sort_plan(B, E, N, nullptr, 0).bytes;
 }
 
@@ -1181,7 +1212,7 @@ size_t ts_group_bins_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N,
 size_t ts_group_std_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype) {
   const size_t bins = ts_group_bins_workspace_bytes(B, E, K, N, dtype);
   if (bins > 0 || !valid_dtype(dtype) || !is_float_dtype(dtype) || !sizes_ok(B, N, E, K)) return bins;
-  const RowsRoute rr = rows_route(B, E, K, N, dtype, TS_SUM);
+  const RowsRoute rr = rows_route(B, E, K, N, dtype, TS_MEAN);
   return rr.ok ? rr.total() : 0;
 }
 
@@ -1199,7 +1230,7 @@ int ts_group_std_forward(const void *src, const int64_t *index, void *total, int
     if (!al && group_bins_plan(B, E, K, N, dtype, true, nullptr, 0).bytes != 0) return TS_ERR_UNSUPPORTED;
     // rows that the buckets do not hold: the entries sorted by group, then two segmented reductions (sums; squared
     // deviations from the means), the counts from the row pointers
-    const RowsRoute rr = rows_route(B, E, K, N, dtype, TS_SUM);
+    const RowsRoute rr = rows_route(B, E, K, N, dtype, TS_MEAN);
     if (!rr.ok) return TS_ERR_UNSUPPORTED;
     if (!workspace || workspace_bytes < rr.total() || !aligned16(workspace)) return TS_ERR_WORKSPACE;
     RowSortPlan sp = row_sort_plan(B, E, N, workspace, rr.sort_bytes);
