@@ -118,11 +118,14 @@ void maybe_check_status_words(const Tensor &ws, size_t ws_bytes, const char *wha
   TORCH_CHECK(!ts_status_gave_up(w), "torch_scatter (", what,
               "): a row that crosses tiles was given up and written as empty -- ", why);
 }
-// The same for a scatter, on the routes whose workspace ends in status words (entries sorted by row).
-void maybe_check_scatter_status(const Tensor &ws, size_t ws_bytes, const char *what) {
+// The same for a scatter, on the routes whose workspace ends in status words (entries sorted by row). The sizes are asked
+// for only when the words are to be read: the query costs a small call about a microsecond.
+void maybe_check_scatter_status(const Tensor &ws, int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce,
+                                const char *what) {
   const int route = ts_scatter_last_route();
-  if (route == TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED || route == TS_ROUTE_MINMAX_BUCKETS_OR_SEGMENTED)
-    maybe_check_status_words(ws, ws_bytes, what, "the bounded wait for the tiles before it ran out");
+  if ((route == TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED || route == TS_ROUTE_MINMAX_BUCKETS_OR_SEGMENTED) && status_checks_on())
+    maybe_check_status_words(ws, ts_scatter_workspace_bytes(B, E, K, N, dtype, reduce), what,
+                             "the bounded wait for the tiles before it ran out");
 }
 
 Tensor workspace(size_t bytes, const Tensor &like) {
@@ -264,7 +267,7 @@ std::tuple<Tensor, OptTensor> scatter_hip(Tensor src, Tensor index, int64_t dim,
                                                      optional_out.has_value() ? 1 : 0,
                                                      cs_bytes > 0 ? cws.data_ptr() : nullptr, cs_bytes, stream_of(src)),
                  "scatter (sum and count)");
-    maybe_check_scatter_status(cws, ts_scatter_workspace_bytes(B, E, K, N, dtype_code(src), TS_SUM), "scatter (sum and count)");
+    maybe_check_scatter_status(cws, B, E, K, N, dtype_code(src), TS_SUM, "scatter (sum and count)");
     *mean_count = count;
     return std::make_tuple(out, OptTensor());
   }
@@ -289,7 +292,7 @@ std::tuple<Tensor, OptTensor> scatter_hip(Tensor src, Tensor index, int64_t dim,
     if (lost) drop_kept_workspace(src, stream_of(src));
     TORCH_CHECK(!lost, "torch_scatter (scatter): a bounded wait inside the kernel ran out and entries were lost");
   }
-  if (ws_bytes > 0) maybe_check_scatter_status(ws, ws_bytes, "scatter");
+  if (ws_bytes > 0) maybe_check_scatter_status(ws, B, E, K, N, dtype_code(src), reduce, "scatter");
   return std::make_tuple(out, arg_out);
 }
 
@@ -945,7 +948,7 @@ struct GroupStdFn : public torch::autograd::Function<GroupStdFn> {
                                         count.data_ptr<int32_t>(), out.data_ptr(), l.B, l.E, l.K, N, l.sb, l.se,
                                         dtype_code(src), unbiased ? 1 : 0, ws.data_ptr(), bins_bytes, stream_of(src)),
                    "scatter_std");
-      if (ts_group_bins_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src)) == 0)
+      if (status_checks_on() && ts_group_bins_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src)) == 0)
         maybe_check_status_words(ws, bins_bytes, "scatter_std", "the bounded wait for the tiles before it ran out");
     } else {
       total = std::get<0>(scatter_hip(src, index, dim, std::nullopt, N, TS_SUM)).contiguous();
