@@ -211,11 +211,12 @@ int ts_scatter(const void *src, const int64_t *index, void *out,
                int64_t index_stride_k, int dtype, int reduce, int out_given,
                ts_stream_t stream);
 
-/* ts_scatter with an optional workspace (ts_scatter_workspace_bytes; 0 = no use for one). With it,
- * MIN / MAX of large inputs with rows of 64 bytes and more, and SUM of such rows under an index that
- * is not sorted, first bin the entries by bucket of output rows (8 bytes per entry) and reduce every
- * bucket in LDS: no atomics on the table in memory except one write-back per chunk. MIN / MAX of
- * other large inputs of 4-byte elements with few entries per output row ask for 256 bytes: one flag,
+/* ts_scatter with an optional workspace (ts_scatter_workspace_bytes; 0 = no use for one). With it, SUM, MIN and
+ * MAX of large inputs with rows of 64 bytes and more (SUM: elements of 16-bit floats or of 4 and 8 bytes; from about
+ * 6 ... 40 MB of src on, by element size and entries per row) sort the entries by row first (8 or 12 bytes of scratch
+ * per entry, 8 per row, and the carries) and reduce every row in one piece, without atomics on the table in memory; an
+ * index found in order is reduced in place. A row that crosses tiles of that reduction waits for them, and the wait is
+ * bounded: see the status words under ts_segment_csr. MIN / MAX of other large inputs of 4-byte elements with few entries per output row ask for 256 bytes: one flag,
  * written by a sample of the index, that picks the kernel for a skewed or an even index; so do SUMs
  * at the sizes that go through the accumulator table in LDS (from 2^23 elements on the sample keeps a
  * sorted index with the kernel that combines its runs: about twice as fast). SUM of up to four floats
@@ -258,8 +259,9 @@ enum ts_scatter_route {
   TS_ROUTE_SUM_RUNS = 2,                 /* runs of equal neighbouring indices combined in the wavefront, hot rows in LDS */
   TS_ROUTE_SUM_TABLE = 3,                /* accumulator table in LDS per workgroup */
   TS_ROUTE_SUM_TABLE_OR_RUNS = 4,        /* a sample of the index picks: table (unsorted) or runs (sorted) */
-  TS_ROUTE_SUM_BUCKETS_OR_RUNS = 5,      /* workspace: entries binned by bucket of output rows; a sorted-looking index: runs */
-  TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED = 6, /* workspace: buckets; an index found sorted: the segmented reduction */
+  TS_ROUTE_SUM_BUCKETS_OR_RUNS = 5,      /* (reserved: no call reports it any more) */
+  TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED = 6, /* workspace: entries sorted by row through buckets (an index found in order: as it
+                                            is), then the segmented reduction */
   TS_ROUTE_MUL_ATOMIC = 7,
   TS_ROUTE_MUL_TABLE = 8,
   TS_ROUTE_MINMAX_ATOMIC = 9,            /* packed 64-bit keys, one atomic max per element */
@@ -268,8 +270,8 @@ enum ts_scatter_route {
   TS_ROUTE_MINMAX_TABLE = 12,            /* key table in LDS per workgroup */
   TS_ROUTE_MINMAX_TABLE_K1 = 13,         /* the same for one value per entry */
   TS_ROUTE_MINMAX_K1_SLABS = 14,         /* workspace, one value per entry: tables handed over in slabs */
-  TS_ROUTE_MINMAX_BUCKETS = 15,          /* workspace: entries binned by bucket of output rows */
-  TS_ROUTE_MINMAX_BUCKETS_OR_SEGMENTED = 16, /* the same; an index found sorted: the segmented reduction */
+  TS_ROUTE_MINMAX_BUCKETS = 15,          /* (reserved: no call reports it any more) */
+  TS_ROUTE_MINMAX_BUCKETS_OR_SEGMENTED = 16, /* as TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED */
   TS_ROUTE_MINMAX_64BIT = 17,            /* 64-bit elements: value pass, then position pass */
   TS_ROUTE_SUM_VALUE_BUCKETS = 18,       /* workspace, one 4-byte value per entry: the values travel in the binned words;
                                             a sample of the index picks buckets (even), table (skewed) or runs (sorted) */

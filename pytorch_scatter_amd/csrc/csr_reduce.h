@@ -69,11 +69,6 @@ struct CsrReduceArgs {
   int64_t perm_batch_stride;
   int perm_args;      // min / max with perm: the kernel itself writes positions in src's order and applies
                       // scatter's rule for slots that never beat the initial value (no pass over arg_out after it)
-  // status words of the call (device memory, two 64-bit words, may be null): word 0 receives status_nonce from
-  // the first tile when status_reset is set ("the latest call"), word 1 receives status_nonce from a tile whose
-  // look-back ran out of polls ("the latest call that gave a row up"). The call gave a row up iff the two are
-  // equal afterwards: no write has to be ordered against another one, and a word left by an earlier call
-  // never matches.
   // rows of a scatter through perm in any order inside a row (row_sort.h): B and N flattened into one list of rows;
   // arg_E: entries per batch, so that positions come out inside their batch. accumulate: combined with out.
   int any_order = 0;
@@ -83,6 +78,11 @@ struct CsrReduceArgs {
   // kRowDeviation: the rows' sums in the element type [N, K], and whether the divisor is count - 1
   const void *row_total = nullptr;
   int unbiased = 0;
+  // status words of the call (device memory, two 64-bit words, may be null): word 0 receives status_nonce from
+  // the first tile when status_reset is set ("the latest call"), word 1 receives status_nonce from a tile whose
+  // look-back ran out of polls ("the latest call that gave a row up"). The call gave a row up iff the two are
+  // equal afterwards: no write has to be ordered against another one, and a word left by an earlier call
+  // never matches.
   unsigned long long *status;
   int status_reset;
   uint64_t status_nonce;  // never 0; the same for every slice of one call

@@ -20,7 +20,6 @@ namespace ts {
 constexpr int kBinBlock = 1024;
 constexpr int kBinMaxBuckets = 16384;  // LDS histogram of count / place (their LDS is sized for 8192 or 16384 buckets)
 constexpr int kBinSmallCap = 8192;
-constexpr int kBinChunk = 8192;       // entries per chunk of a bucket in reduce (fewer for inputs under 4 M entries)
 constexpr int kBinPlaceChunk = 10240;  // most entries per workgroup in place: one batch of 10 per lane
 constexpr int kCombPos = 64;          // combining kernel: keys per step of a bucket of many chunks,
 constexpr int kCombFew = 32;          // many: more than this
@@ -43,9 +42,9 @@ struct BinArgs {
   int32_t *chunk_start;    // [nb + 1]
   int32_t *wg_bucket;      // [max_wgs] bucket of a reducing workgroup, -1: none
   uint64_t *binned;        // [B * E] (row in bucket << 32) | entry number
-  int32_t *slab_start;     // min / max: [nb + 1] first slab of a bucket that is reduced in more than one chunk
-  uint64_t *slabs;         // min / max: [slab][K << rshift] the tables of those chunks
-  int32_t *comb_list;      // min / max: buckets that the combining kernel finishes (not exactly one chunk): those of
+  int32_t *slab_start;     // group statistics: [nb + 1] first slab of a bucket that is reduced in more than one chunk
+  uint64_t *slabs;         // ...: what those chunks leave
+  int32_t *comb_list;      // ...: buckets that the combining kernel finishes (not exactly one chunk): those of
                            //            up to kCombFew chunks from the front, those of more from slot nb - 1 down
   int32_t *comb_count;     //            how many of either
 
