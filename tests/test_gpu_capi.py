@@ -658,17 +658,17 @@ def test_scatter_minmax_lds_cached_variant(capi, oracle, shape, reduce, dtype, m
 @pytest.mark.parametrize("shape,reduce,dtype", list(product(
     [(1, 60000, 32, 300), (2, 40000, 16, 700), (1, 50000, 128, 90), (1, 30000, 24, 5000), (1, 20000, 64, 100000),
      (3, 9000, 512, 5), (1, 70000, 17, 40),
-     (2, 30000, 64, 40000),   # 625 buckets over two batch rows: the place pass that sorts its tile in LDS
-     (1, 8000, 1024, 50), (2, 5000, 768, 33)],   # rows wider than a table row: reduced in slices of columns
+     (2, 30000, 64, 40000),   # two batch rows
+     (1, 8000, 1024, 50), (2, 5000, 768, 33)],   # rows of several column chunks
     ["min", "max"], [torch.float32, torch.bfloat16, torch.int32, torch.int8]))
-    + [((1, 20000, 64, 600000), "max", torch.float32), ((1, 20000, 64, 600000), "min", torch.int32),  # 4688 buckets
-       ((1, 20000, 128, 540000), "max", torch.float32),  # 8438 buckets
-       # too many buckets of whole rows (16 875): four slices of 128 columns, 4219 buckets
+    + [((1, 20000, 64, 600000), "max", torch.float32), ((1, 20000, 64, 600000), "min", torch.int32),
+       ((1, 20000, 128, 540000), "max", torch.float32),
+       # rows of several column chunks
        ((1, 20000, 512, 270000), "max", torch.float32), ((1, 20000, 512, 270000), "min", torch.bfloat16)])
 def test_scatter_minmax_binned_variant(capi, oracle, shape, reduce, dtype, monkeypatch):
-    """min / max with a workspace: entries binned by bucket of output rows and reduced in LDS (forced on at
-    these sizes), skewed index with heavy ties, with and without previous content in out. Rows under 64 bytes
-    (int8 at K < 64, ...) keep the path without workspace."""
+    """min / max with a workspace: entries sorted by row, then a segmented reduction (forced on at these sizes),
+    skewed index with heavy ties, with and without previous content in out. Rows under 64 bytes (int8 at K < 64,
+    ...) keep the path without workspace."""
     monkeypatch.setenv("TS_SCATTER_BINNED", "2")
     B, E, K, N = shape
     rng = np.random.default_rng(E + K)
@@ -760,21 +760,18 @@ def test_scatter_minmax_skew_probe(capi, oracle, shape, kind, reduce, dtype, mon
 @pytest.mark.parametrize("shape,kind,dtype", list(product(
     [(1, 60000, 32, 300), (2, 40000, 16, 700), (1, 50000, 128, 90), (1, 20000, 64, 100000), (3, 9000, 256, 5),
      (1, 30000, 24, 500), (2, 30000, 64, 40000),
-     (1, 8000, 1024, 50), (2, 5000, 96, 330)],   # reduced in slices of columns (96: no power of two of lanes)
+     (1, 8000, 1024, 50), (2, 5000, 96, 330)],   # several column chunks; 96: no power of two of lanes
     ["zipf", "sorted", "one descent"],
     [torch.float32, torch.float64, torch.bfloat16, torch.float16, torch.int32, torch.int64, torch.int16]))
-    + [((1, 20000, 64, 600000), "zipf", torch.float32), ((1, 20000, 64, 600000), "one descent", torch.int32),  # 4688 buckets
-       ((1, 20000, 128, 540000), "zipf", torch.int32),  # 8438 buckets
-       ((1, 20000, 512, 270000), "zipf", torch.float32)])  # four slices of 128 columns, 4219 buckets
+    + [((1, 20000, 64, 600000), "zipf", torch.float32), ((1, 20000, 64, 600000), "one descent", torch.int32),
+       ((1, 20000, 128, 540000), "zipf", torch.int32),
+       ((1, 20000, 512, 270000), "zipf", torch.float32)])  # several column chunks
 def test_scatter_sum_binned_variant(capi, oracle, shape, kind, dtype, monkeypatch):
-    """Sum with a workspace (forced on at these sizes): a sample of the index (or, with the sample switched
-    off as in the "one descent" cases, the count pass) finds out whether the index is sorted;
-    if not, the entries are binned by bucket of output rows and added in LDS (double slots for floating
-    types), else the usual kernels run. Exact for integers (int16 and K = 24 keep the path without
-    workspace), within tolerance of the exact sum for floats, with and without previous content in out."""
+    """Sum with a workspace (forced on at these sizes): the count pass of the sort by row finds out whether the index
+    is in order (one descent is enough that it is not); the segmented reduction then adds in 64 bits for floating
+    types. Exact for integers (int16 keeps the path without workspace), within tolerance of the exact sum for floats,
+    with and without previous content in out."""
     monkeypatch.setenv("TS_SCATTER_BINNED", "2")
-    if kind == "one descent":
-        monkeypatch.setenv("TS_BIN_NO_SAMPLE", "1")
     B, E, K, N = shape
     rng = np.random.default_rng(E + K + len(kind))
     p = np.arange(1, N + 1, dtype=np.float64) ** -1.2
@@ -821,9 +818,9 @@ SORTED_KINDS = ["sorted", "sorted gaps", "one descent", "beyond N", "negative fi
     [(1, 60000, 32, 300), (2, 40000, 16, 700), (1, 20000, 64, 100000), (1, 8000, 1024, 50), (3, 9000, 512, 5)],
     ["sum", "min", "max"], SORTED_KINDS, [torch.float32, torch.bfloat16, torch.int32])))
 def test_scatter_sorted_index_with_workspace(capi, oracle, shape, reduce, kind, dtype, monkeypatch):
-    """With a workspace, the count pass of the buckets (forced on at these sizes) checks the whole index; one that
-    is in order and inside [0, N) is finished by the segmented reduction (row pointers from the index, one pass
-    over src, no atomics), anything else by the buckets. Both must give scatter's result: values that never beat
+    """With a workspace, the count pass of the sort by row (forced on at these sizes) checks the whole index; one that
+    is in order and inside [0, N) is reduced in place (row pointers from the index, one pass over src, no atomics),
+    anything else is sorted first. Both must give scatter's result: values that never beat
     the initial value of the element type (-inf, lowest()) leave 0 with position E, empty rows too; a single
     descent, an index beyond N at the end or a negative one in front sends the call down the other path."""
     monkeypatch.setenv("TS_SCATTER_BINNED", "2")
@@ -887,8 +884,8 @@ def test_scatter_sorted_index_with_workspace(capi, oracle, shape, reduce, kind, 
 @pytest.mark.parametrize("reduce,dtype", product(["sum", "max"], [torch.float32, torch.float64, torch.int32]))
 def test_scatter_sorted_index_per_batch_rows(capi, oracle, reduce, dtype, monkeypatch):
     """A batched index [B, E] whose rows are sorted one by one (different rows per batch, stride E): in order as a
-    whole for the count pass of the buckets, row pointers per batch for the segmented reduction. The second batch
-    row of the last case has one descent: the whole call then goes through the buckets."""
+    whole for the count pass of the sort by row. The second batch row of the last case has one descent: the whole
+    call is then sorted."""
     monkeypatch.setenv("TS_SCATTER_BINNED", "2")
     B, E, K, N = 3, 30000, 32, 900
     rng = np.random.default_rng(K + len(reduce))
@@ -904,8 +901,6 @@ def test_scatter_sorted_index_per_batch_rows(capi, oracle, reduce, dtype, monkey
             src = random_values(rng, (B, E, K), dtype, ties=True)
         out = torch.full((B, N, K), 9, dtype=dtype, device=DEV)
         arg = torch.empty((B, N, K), dtype=torch.long, device=DEV) if reduce == "max" else None
-        if dtype == torch.float64 and reduce == "max":
-            continue  # 64-bit elements keep the two-pass kernels (no packed keys, no workspace)
         capi.scatter_with_workspace(src.to(DEV), index2.to(DEV), out, arg, B, E, K, N, E, 1, 0, capi.REDUCE[reduce], 0)
         torch.cuda.synchronize()
         want, want_arg = oracle.scatter(src, index, 1, None, N, reduce)
@@ -925,8 +920,8 @@ def test_scatter_sorted_index_per_batch_rows(capi, oracle, reduce, dtype, monkey
 def test_scatter_with_workspace_agrees_with_plain_scatter_on_random_shapes(capi, seed, monkeypatch):
     """Forty random calls per seed (1-3 batches, 4-1024 columns, 1 - 1.2 M output rows, seven element types, uniform /
     Zipf / sorted / sorted with entries outside [0, N) / one descent / three distinct values, with and without a
-    given out), buckets forced on: min / max with a workspace (buckets, column slices, slabs, the segmented
-    reduction for a sorted index) give the bits of the call without workspace; floating sums stay within
+    given out), the sort by row forced on: min / max with a workspace give the bits of the call without workspace;
+    floating sums stay within
     4 * min(n, 128) half-ulp roundings of the exact sum."""
     monkeypatch.setenv("TS_SCATTER_BINNED", "2")
     rng = np.random.default_rng(seed)

@@ -366,3 +366,40 @@ def test_arg_backward_through_autograd(op, layout, monkeypatch):
     assert torch.equal(arg.cpu(), first) and torch.equal(out.detach().cpu(), best)
     (got,) = torch.autograd.grad(out, x, grad.to(DEV))
     assert torch.equal(got.cpu(), want)
+
+
+def test_rows_under_graph_replay(monkeypatch):
+    """A captured launch keeps its tag and its workspace: the readers of carries clear their flags, the totals of the sort are
+    cleared by the call. Replays with another index each time (hubs over many tiles, one row, in order), eager calls in
+    between, each against the eager result."""
+    import pytorch_scatter_amd as ts
+    monkeypatch.setenv("TS_SCATTER_BINNED", "2")
+    monkeypatch.setenv("TS_GROUP_BINS", "0")
+    E, N = 30001, 400
+    g = torch.Generator(device=DEV).manual_seed(5)
+    index = torch.randint(0, N, (E,), generator=g, device=DEV)
+    wide, odd = (torch.zeros((E, K), device=DEV) for K in (32, 33))
+
+    def step():
+        return (ts.scatter_sum(wide, index, 0, dim_size=N), *ts.scatter_max(wide, index, 0, dim_size=N),
+                ts.scatter_sum(odd, index, 0, dim_size=N), *ts.scatter_min(odd, index, 0, dim_size=N),
+                ts.scatter_std(odd, index, 0, dim_size=N))
+
+    for _ in range(2):
+        step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for kind in ("hub20000", "one row", "even", "sorted", "hub9000", "hub20000"):
+        index.copy_(_index(kind, E, N, g))
+        for x in (wide, odd):
+            x.copy_(torch.randint(-50, 51, x.shape, generator=g, device=DEV))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in out]
+        for a, b in zip(got[:-1], step()[:-1]):
+            assert torch.equal(a, b), kind
+        assert torch.allclose(got[-1], step()[-1], rtol=1e-6, atol=0), kind  # sums of squares: another order of additions
+        want = torch.zeros((N, 32), dtype=torch.float64, device=DEV).index_add_(0, index, wide.double())
+        assert torch.equal(got[0].double(), want), kind
