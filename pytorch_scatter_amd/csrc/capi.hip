@@ -249,7 +249,7 @@ RowsRoute rows_route(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int 
   const bool minmax = reduce == TS_MIN || reduce == TS_MAX;
   if (!minmax && reduce != TS_SUM && reduce != TS_MEAN) return r;
   if (!minmax && kAccBytes[dtype] < 4) return r;
-  // From where the six launches of the sort and the reduction (31-37 us on the smallest inputs) cost less than the kernels
+  // From where the launches of the sort and the reduction (six when measured, now five) (31-37 us on the smallest inputs) cost less than the kernels
   // without them. The host knows sizes only; a line lies where an even and a Zipf(1.2) index, each shuffled and in order,
   // gain together (us of these four, without / with; measured from 0.1 to 10 M entries, 0.3 to 30000 a row):
   //   sums, 4 bytes: 300 k x 64, 3 a row 81 95 41 60 / 54 64 52 59; 300 k x 32, 10 a row 45 57 27 52 / 40 53 37 44
@@ -770,7 +770,7 @@ int scatter_ws_impl(const void *src, const int64_t *index, void *out, int64_t *a
       RowSortPlan sp = row_sort_plan(B, E, N, workspace, rr.sort_bytes);
       if (!sp.ok) return TS_ERR_WORKSPACE;
       ts_note_scatter_route(reduce == TS_SUM ? TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED : TS_ROUTE_MINMAX_BUCKETS_OR_SEGMENTED);
-      int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, false, s);
+      int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, false, next_nonce(), s);
       if (rc != TS_OK) return rc;
       rc = run_rows_reduce(src, sp.p, out, arg_out, B, E, K, N, dtype, reduce, out_given,
                            static_cast<char *>(workspace) + rr.sort_bytes, rr.csr_bytes, next_nonce(), s);
@@ -975,7 +975,7 @@ size_t ts_arg_backward_rows_workspace_bytes(int64_t B, int64_t E, int64_t K, int
   if (mode != 2 && (row_bytes < 256 || row_bytes % kVecBytes != 0 || B * E * row_bytes < 384000000 ||
                     B * N * K < ((int64_t)4 << 20) + 3 * B * E))
     return 0;
-  return row_sort_plan(B, E, N, nullptr, 0).bytes;
+  return row_sort_plan(B, E, N, nullptr, 0, true).bytes;
 }
 
 int ts_arg_backward_rows(const void *grad_out, const int64_t *arg, const int64_t *index, void *grad_in, int64_t B, int64_t N,
@@ -985,10 +985,10 @@ int ts_arg_backward_rows(const void *grad_out, const int64_t *arg, const int64_t
   if (need == 0) return TS_ERR_UNSUPPORTED;
   if (!grad_out || !arg || !index || !grad_in) return TS_ERR_BAD_ARG;
   if (!workspace || workspace_bytes < need || !aligned16(workspace)) return TS_ERR_WORKSPACE;
-  RowSortPlan sp = row_sort_plan(B, E, N, workspace, workspace_bytes);
+  RowSortPlan sp = row_sort_plan(B, E, N, workspace, workspace_bytes, true);
   if (!sp.ok) return TS_ERR_WORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, true, s);
+  const int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, true, next_nonce(), s);
   if (rc != TS_OK) return rc;
   RowSortArgs p = sp.p;
   p.index = index;
@@ -1237,7 +1237,7 @@ int ts_group_std_forward(const void *src, const int64_t *index, void *total, int
     if (!sp.ok) return TS_ERR_WORKSPACE;
     hipStream_t s = static_cast<hipStream_t>(stream);
     void *const ws = static_cast<char *>(workspace) + rr.sort_bytes;
-    int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, false, s);
+    int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, false, next_nonce(), s);
     if (rc != TS_OK) return rc;
     const uint64_t status_nonce = next_nonce();
     rc = run_rows_reduce(src, sp.p, total, nullptr, B, E, K, N, dtype, TS_SUM, 0, ws, rr.csr_bytes,

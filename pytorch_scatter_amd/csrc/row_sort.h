@@ -1,46 +1,40 @@
 // An index in any order -> the entries in order of their rows: perm (entry numbers) and row pointers, the input of
 // the segmented reductions (csr_reduce.h with rows through perm). Two levels: entries are binned by bucket of R
-// consecutive rows, then every bucket is sorted by row in LDS.
-//   count : at most 256 workgroups with equal shares of the index, each a histogram over the buckets in LDS that it adds
-//           to the bucket totals; also: is the index in order and inside [0, N)? The workgroup that arrives last turns
-//           the totals into bucket starts (a launch of its own for that took 10-15 us of a single CU's latencies).
-//   place : a workgroup per tile: the tile sorted by bucket in LDS, one atomic per bucket that occurs reserves the
-//           tile's run, (row in bucket, entry) words leave in runs. An index found in order gets its row pointers and
-//           the identity from this launch instead, and the passes behind it return at once. Words of 32 bits where both
-//           fit (10 M entries onto 100 k rows: 24 + 6 bits), else of 64: place and sort move 8 or 12 bytes an entry less.
-//   sort  : a workgroup per bucket of up to 8192 or 16384 entries: counting sort by row in LDS, row pointers and perm out. A
-//           bucket with more entries (hubs, few rows) is taken in chunks: each goes back in order of its rows, the row
+// consecutive rows inside tiles of up to 8192 entries, then every bucket is sorted by row in LDS.
+//   place : a workgroup per tile: the tile's entries sorted by bucket in LDS leave as 32-bit words in one piece, with the
+//           offset of every bucket among them. Also: does the index descend or leave [0, N) in this tile? If no tile says
+//           so the row pointers that the tiles wrote on the way stand, and the passes behind return at once.
+//   sort  : a workgroup per bucket of up to 8192 or 16384 entries collects its runs from all tiles. What lies before the
+//           bucket is the sum of its offsets over the tiles, so nothing has to be counted in front, nothing is cleared,
+//           and nothing meets in memory. Counting sort by row in LDS, row pointers and perm out.
+//   chunk : a bucket with more entries (hubs, few rows) is taken in chunks: each is left in order of its rows, the row
 //           counts meet in memory, the chunk that arrives last turns them into row pointers,
 //   place chunks : ... and the chunks' entries then go from there to their places, each behind the row's entries of the
 //           chunks that were counted before.
 // Entries of a row come in no particular order (a reader that needs the first of equal values compares positions).
 // Entries outside [0, N) are left out.
-// What it costs: 16 bytes of index, 4 or 8 written and read per entry for the words, 4 for perm; what bounds the passes is the
-// chain of each workgroup (load, rank, reserve, store), so every lane has all its loads on the way before it needs one. us for
-// clear / count / place / sort / place chunks: 2.3 M entries onto 268 k rows 5 / 16 / 15 / 9 / 5, 10 M even onto 100 k rows
-// 5 / 26 / 50 / 26 / 5, 10 M under a Zipf(1.2) index onto 100 k rows 5 / 26 / 46 / 36 / 18 (two thirds of them in one bucket;
-// with loads one after the other, words of 64 bits and the chunks ranked a second time 5 / 53 / 59 / 44 / 47, the scatter sum
-// of 32 floats 432 us against 358 now and 367 with the tables below). In front of a segmented reduction this replaced tables of
-// output rows in LDS per bucket (one LDS atomic per element, bank conflicts, slabs or atomics to put chunks together):
-// 2.3 M x 128 bf16, sum 660 -> 205 us; 10 M x 64 floats onto 1 M rows, sum / max 965 / 946 -> 719 / 843 us.
+// What it costs: 8 bytes of index, 4 written and read per entry for the words, 4 for perm. What bounds it: place the loads
+// (10 M entries: 120 MB in 27 us), sort the instructions, about 35 an entry (with the prefix over a workgroup's wavefronts
+// as a loop over their sums, a third more: 69 us at 10 M). us of place / sort / chunk / place chunks, the last two at least
+// 4.6 each for launches that return at once: 1 M entries onto 66 k rows 7 / 10 / 5 / 5, 2.3 M onto 268 k 10 / 13 / 5 / 5,
+// 5 M 16 / 24 / 5 / 5, 10 M onto 333 k 27 / 51 / 5 / 5, 10 M onto 100 k, a fifth of them in one row, 29 / 47 / 30 / 14.
+// With a pass over the index that counted into the buckets first and place sending every run to its bucket (clear / count /
+// place / sort / place chunks): 1 M 5 / 10 / 9 / 8 / 4, 2.3 M 5 / 16 / 16 / 9 / 5, 10 M even 5 / 26 / 50 / 26 / 5. Scatter sums
+// and maxima of 0.3 to 10 M entries, rows of 64 to 256 bytes: 0.94 of the time in the geometric mean.
 #pragma once
 
 #include "device_utils.h"
 
 namespace ts {
 
-constexpr int kRsBlock = 1024;        // count, place
-constexpr int kRsPer = 8;             // entries per lane of place
-constexpr int kRsTile = kRsPer * kRsBlock;
-// entries that one sorting workgroup holds in LDS (in registers before: 16 per lane): 512 lanes below kRsLarge entries
-// (more, shorter workgroups: 2.3 M entries 10.7 against 16.8 us), 1024 above, where fewer buckets save more in count
-// and place (10 M entries onto 1 M rows: 138 against 147 us for the three passes)
+constexpr int kRsBlock = 1024;        // place
+constexpr int kRsLocal = 13;          // bits of an entry's place in its tile: tiles of up to 8192 entries
+// entries that one sorting workgroup holds in registers: 16 per lane, 512 lanes below kRsLarge entries (more, shorter
+// workgroups), 1024 above, where fewer buckets leave longer runs in the tiles
 constexpr int kRsSortPer = 16;
 constexpr int64_t kRsLarge = (int64_t)1 << 22;
-constexpr int kRsMaxBuckets = 4096;   // histogram of count and place
-constexpr int kRsMaxShift = 13;       // rows per bucket (log2): histogram of the sorting workgroup
-constexpr int kRsCountPer = 8;
-constexpr int kRsCountGroups = 256;   // (512: twice the additions to the totals)
+constexpr int kRsMaxBuckets = 4096;   // counters of place
+constexpr int kRsMaxShift = 13;       // rows per bucket (log2): counters of the sorting workgroup
 
 struct RowSortArgs {
   const int64_t *index;
@@ -50,20 +44,27 @@ struct RowSortArgs {
   int identity;          // an index in order: write the identity to perm (a reader that looks at state[0] does without)
   int flat;              // one batch, unit stride: entry e is index[e] (no 64-bit multiplications per entry)
   int rshift, nb;        // rows per bucket (log2), buckets
+  int per;               // entries per lane of place: a tile holds per * kRsBlock
+  int tiles;
+  int pitch;             // 16-bit words from one tile's offsets to the next: nb + 1, rounded up
   int cap;               // entries that one sorting workgroup takes
   int max_big;           // buckets above that: at most this many ...
   int max_chunks;        // ... in at most this many chunks
-  uint32_t *totals;      // [nb] entries per bucket, cleared by the call
-  uint32_t *sync;        // [0] ticket of the count pass, [1 ...] of every large bucket: cleared with totals
-  int32_t *state;        // [0] 0: the index is in order, 1: it is not; [1] chunks of large buckets; [2] large buckets
-  uint32_t *starts;      // [nb + 1]
-  uint32_t *cursor;      // [nb]
-  int32_t *chunk_info;   // [3][max_chunks]: bucket, first chunk of the bucket, number of the large bucket
+  uint32_t nonce;        // tag of the call, never 0
+  int32_t *state;        // [0] 0: the index is in order, 1: it is not; [1] chunks of large buckets; [2] large buckets;
+                         // [3] the nonce of the latest call that met an index that is not in order
+  uint16_t *off;         // [tiles][pitch] first entry of every bucket among the tile's words; [nb]: how many there are
+  int log;               // a tile's words lie at tile << log
+  uint32_t *words;       // [tiles << log] a tile's entries by bucket: row in the bucket << kRsLocal | place in the tile
+  uint32_t *big;         // [max_big][4] large buckets: bucket, first place in perm, entries, first chunk
+  uint32_t *arrived;     // [max_big] chunks that have added their counts
+  int32_t *chunk_big;    // [max_chunks] the chunk's large bucket
   uint32_t *row_cnt;     // [max_big << rshift]
   uint32_t *chunk_off;   // [max_chunks << rshift] offset of a chunk's entries inside every row
-  int eshift;            // words of the binned entries: (row in bucket << eshift) | entry; below 32: words of 32 bits
-  void *binned;          // [n] words of 32 or 64 bits
+  uint32_t *by_row;      // [n] entries of chunks, each chunk in order of its rows,
+  uint16_t *by_row_row;  // [n] and their rows in the bucket
   int32_t *perm;         // [n] out
+  int32_t *perm_row;     // [n] out, may be null: the row of every entry of perm
   int64_t *ptr;          // [rows + 1] out
 };
 
@@ -73,7 +74,8 @@ struct RowSortPlan {
   size_t bytes;
 };
 
-inline RowSortPlan row_sort_plan(int64_t B, int64_t E, int64_t N, void *ws, size_t ws_bytes) {
+// with_rows: perm_row as well
+inline RowSortPlan row_sort_plan(int64_t B, int64_t E, int64_t N, void *ws, size_t ws_bytes, bool with_rows = false) {
   RowSortPlan r;
   r.ok = false;
   r.bytes = 0;
@@ -85,8 +87,8 @@ inline RowSortPlan row_sort_plan(int64_t B, int64_t E, int64_t N, void *ws, size
   p.n = B * E;
   p.rows = B * N;
   if (p.n > 0x7FFFF000ll || p.rows >= 0x7FFFF000ll) return r;
-  // Buckets: about 1024 (the tiles of place then write runs of 8 entries, 64 bytes), fewer for small inputs, more so
-  // that a bucket of average size stays below the capacity of a sorting workgroup.
+  // Buckets: about 1024 (a tile of place then leaves runs of 8 entries), fewer for small inputs, more so that a bucket
+  // of average size stays below the capacity of a sorting workgroup.
   p.cap = kRsSortPer * (p.n < kRsLarge ? 512 : 1024);
   int64_t want = p.n / (p.cap / 4);
   if (want > 1024) want = 1024;
@@ -101,33 +103,40 @@ inline RowSortPlan row_sort_plan(int64_t B, int64_t E, int64_t N, void *ws, size
   }
   p.rshift = rs;
   p.nb = (int)buckets(rs);
-  p.eshift = 1;
-  while (((int64_t)1 << p.eshift) < p.n) ++p.eshift;
-  if (p.eshift + rs > 32) p.eshift = 32;
+  // tiles: up to 8192 entries, fewer where all tiles then run at once (two workgroups per CU)
+  const int64_t per = (p.n + 512 * kRsBlock - 1) / (512 * kRsBlock);
+  p.per = per > 8 ? 8 : (int)per;
+  p.log = 10;
+  while (1 << (p.log - 10) < p.per) ++p.log;
+  const int64_t tile = (int64_t)p.per * kRsBlock;
+  p.tiles = (int)((p.n + tile - 1) / tile);
+  p.pitch = (p.nb + 2) & ~1;
   p.max_big = (int)(p.n / p.cap);
   p.max_chunks = 2 * p.max_big;
   auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
   size_t off = 0;
   auto take = [&](size_t bytes) { const size_t o = off; off += up(bytes); return o; };
-  const size_t o_tot = take((size_t)p.nb * 4 + (size_t)(p.max_big + 1) * 4);  // totals, then the tickets
-  const size_t o_state = take(16);
-  const size_t o_st = take((size_t)(p.nb + 1) * 4), o_cur = take((size_t)p.nb * 4);
-  const size_t o_ci = take((size_t)p.max_chunks * 12);
+  const size_t big_n = p.max_big > 0 ? (size_t)p.n : 0;
+  const size_t o_state = take(16), o_off = take((size_t)p.tiles * p.pitch * 2), o_words = take(((size_t)p.tiles << p.log) * 4);
+  const size_t o_big = take((size_t)p.max_big * 16), o_arr = take((size_t)p.max_big * 4), o_cb = take((size_t)p.max_chunks * 4);
   const size_t o_rc = take(((size_t)p.max_big << rs) * 4), o_co = take(((size_t)p.max_chunks << rs) * 4);
-  const size_t o_bin = take((size_t)p.n * (p.eshift < 32 ? 4 : 8)), o_perm = take((size_t)p.n * 4), o_ptr = take((size_t)(p.rows + 1) * 8);
+  const size_t o_br = take(big_n * 4), o_brr = take(big_n * 2);
+  const size_t o_perm = take((size_t)p.n * 4), o_prow = take(with_rows ? (size_t)p.n * 4 : 0), o_ptr = take((size_t)(p.rows + 1) * 8);
   r.bytes = off;
   if (ws == nullptr || ws_bytes < off || (reinterpret_cast<uintptr_t>(ws) & 15) != 0) return r;
   char *base = static_cast<char *>(ws);
-  p.totals = reinterpret_cast<uint32_t *>(base + o_tot);
-  p.sync = p.totals + p.nb;
   p.state = reinterpret_cast<int32_t *>(base + o_state);
-  p.starts = reinterpret_cast<uint32_t *>(base + o_st);
-  p.cursor = reinterpret_cast<uint32_t *>(base + o_cur);
-  p.chunk_info = reinterpret_cast<int32_t *>(base + o_ci);
+  p.off = reinterpret_cast<uint16_t *>(base + o_off);
+  p.words = reinterpret_cast<uint32_t *>(base + o_words);
+  p.big = reinterpret_cast<uint32_t *>(base + o_big);
+  p.arrived = reinterpret_cast<uint32_t *>(base + o_arr);
+  p.chunk_big = reinterpret_cast<int32_t *>(base + o_cb);
   p.row_cnt = reinterpret_cast<uint32_t *>(base + o_rc);
   p.chunk_off = reinterpret_cast<uint32_t *>(base + o_co);
-  p.binned = base + o_bin;
+  p.by_row = reinterpret_cast<uint32_t *>(base + o_br);
+  p.by_row_row = reinterpret_cast<uint16_t *>(base + o_brr);
   p.perm = reinterpret_cast<int32_t *>(base + o_perm);
+  p.perm_row = with_rows ? reinterpret_cast<int32_t *>(base + o_prow) : nullptr;
   p.ptr = reinterpret_cast<int64_t *>(base + o_ptr);
   r.ok = true;
   return r;
@@ -182,28 +191,6 @@ __device__ __forceinline__ uint32_t rs_take(uint32_t *counter, int32_t bucket, i
   hot = __builtin_amdgcn_readfirstlane(bucket);
   return bucket >= 0 ? atomicAdd(&counter[bucket], 1u) : 0u;
 }
-// Counts without the value before. A wavefront keeps the bucket that many of its lanes met last (a hub, an index in order) and
-// that bucket's count in scalar registers; everybody else adds in LDS, where lanes with one address queue up.
-struct RsHot {
-  int32_t bucket;
-  uint32_t count;
-};
-__device__ __forceinline__ void rs_count_flush(uint32_t *counter, const RsHot &hot) {
-  if (hot.count != 0 && hot.bucket >= 0 && (threadIdx.x & (kWave - 1)) == 0) atomicAdd(&counter[hot.bucket], hot.count);
-}
-__device__ __forceinline__ void rs_count_one(uint32_t *counter, int32_t bucket, RsHot &hot) {
-  const uint32_t c = (uint32_t)__popcll(__ballot(bucket == hot.bucket));
-  if (c >= 6) {
-    hot.count += c;
-    if (bucket >= 0 && bucket != hot.bucket) atomicAdd(&counter[bucket], 1u);
-  } else {
-    rs_count_flush(counter, hot);
-    hot.bucket = __builtin_amdgcn_readfirstlane(bucket);
-    hot.count = 0;
-    if (bucket >= 0) atomicAdd(&counter[bucket], 1u);
-  }
-}
-
 // Index of entry be of the flattened [B, E], and the row it means: -1 for an index outside [0, N). FLAT: RowSortArgs::flat at
 // compile time (-1: not). Apart, so that a lane has all its loads on the way before it needs the first: a load behind a
 // condition is waited for on the spot (8 loads one after the other: count and place of 10 M entries 33 and 58 us, so 26 and 51).
@@ -222,6 +209,16 @@ template <int FLAT = -1> __device__ __forceinline__ int32_t rs_node(const RowSor
   return rs_row<FLAT>(p, be, rs_load<FLAT>(p, be));
 }
 
+// s_wave: a number per wavefront. Their sum over the wavefronts before this one, and over all of them: a scan in every wavefront
+// (a loop over the numbers takes three instructions for each, a third of what the sorting workgroups executed).
+template <int BLOCK> __device__ __forceinline__ uint32_t rs_waves_before(const uint32_t *s_wave, uint32_t &total) {
+  constexpr int W = BLOCK / kWave;
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const int32_t incl = wave_inclusive_sum(lane < W ? (int32_t)s_wave[lane] : 0);
+  total = (uint32_t)__builtin_amdgcn_readlane(incl, W - 1);
+  return wave > 0 ? (uint32_t)__builtin_amdgcn_readlane(incl, wave - 1) : 0u;
+}
+
 // exclusive prefix sums of s[0 .. n), in place; every lane owns `per` neighbouring values. Returns the total.
 template <int BLOCK> __device__ __forceinline__ uint32_t rs_scan_lds(uint32_t *s, int n, uint32_t *s_wave) {
   const int per = (n + BLOCK - 1) / BLOCK;
@@ -232,13 +229,7 @@ template <int BLOCK> __device__ __forceinline__ uint32_t rs_scan_lds(uint32_t *s
   const int32_t incl = wave_inclusive_sum(mine);
   if (lane == kWave - 1) s_wave[wave] = (uint32_t)incl;
   __syncthreads();
-  uint32_t run = (uint32_t)(incl - mine), total = 0;
-#pragma unroll
-  for (int w = 0; w < BLOCK / kWave; ++w) {
-    const uint32_t x = s_wave[w];
-    run += w < wave ? x : 0u;
-    total += x;
-  }
+  uint32_t total, run = (uint32_t)(incl - mine) + rs_waves_before<BLOCK>(s_wave, total);
   for (int j = 0; j < per; ++j) {
     if (i0 + j >= n) break;
     const uint32_t h = s[i0 + j];
@@ -249,177 +240,89 @@ template <int BLOCK> __device__ __forceinline__ uint32_t rs_scan_lds(uint32_t *s
   return total;
 }
 
-static __global__ __launch_bounds__(kBlock) void rs_clear_kernel(uint32_t *p, int n) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
-template <int FLAT> static __global__ __launch_bounds__(kRsBlock) void rs_count_kernel(RowSortArgs p) {
-  __shared__ uint32_t s_hist[kRsMaxBuckets];
-  __shared__ uint32_t s_wave[3][kRsBlock / kWave];
-  __shared__ int s_desc, s_last;
-  for (int i = threadIdx.x; i < p.nb; i += kRsBlock) s_hist[i] = 0;
-  if (threadIdx.x == 0) s_desc = 0;
-  __syncthreads();
-  const int64_t per = (p.n + gridDim.x - 1) / gridDim.x;
-  const int64_t lo = (int64_t)blockIdx.x * per;
-  const int64_t hi = lo + per < p.n ? lo + per : p.n;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  int32_t node[kRsCountPer];
-  int64_t next[kRsCountPer];
-  auto load = [&](int64_t b0) {  // (past the end: the last entry again)
+// A tile of entries by bucket. A tile whose rows do not descend writes the row pointers that its entries mark as well: they
+// stand if no tile has seen a descent, else the sorting passes write all of them again.
+template <int FLAT, int PER>
+static __global__ __launch_bounds__(kRsBlock) __attribute__((amdgpu_waves_per_eu(8, 8)))
+void rs_place_kernel(RowSortArgs p) {
+  constexpr int TILE = PER * kRsBlock;
+  static_assert(TILE <= 1 << kRsLocal, "a place in the tile has kRsLocal bits");
+  extern __shared__ uint32_t s_cnt[];  // [nb] counts, then the tile's exclusive prefix
+  __shared__ uint32_t s_stage[TILE];
+  __shared__ uint32_t s_wave[kRsBlock / kWave];
+  __shared__ GapList s_gaps;
+  __shared__ int s_desc;
+  const int64_t lo = (int64_t)blockIdx.x * TILE;
+  const int lane = threadIdx.x & (kWave - 1);
+  int32_t node[PER];
+  uint32_t rank[PER];
+  int64_t idx[PER];
+  const uint32_t left = (uint32_t)(p.n - lo < TILE ? p.n - lo : TILE);
 #pragma unroll
-    for (int j = 0; j < kRsCountPer; ++j) {
-      const int64_t be = b0 + threadIdx.x + (int64_t)j * kRsBlock;
-      next[j] = rs_load<FLAT>(p, be < hi ? be : hi - 1);
-    }
-  };
+  for (int j = 0; j < PER; ++j) {  // (past the end: the last entry again)
+    const uint32_t i = threadIdx.x + j * kRsBlock < left ? threadIdx.x + j * kRsBlock : left - 1;
+    idx[j] = FLAT ? (p.index + lo)[i] : rs_load<FLAT>(p, lo + i);
+  }
+  // The entry before a lane's entry is the neighbouring lane's; the first lane of a wavefront needs the entry before the
+  // wavefront's first one: lane j loads it for row j (one load instruction for all rows).
+  int32_t edge = -1;
+  if (lane < PER) {
+    const int64_t be = lo + (int64_t)(threadIdx.x - lane) + (int64_t)lane * kRsBlock;
+    if (be > 0 && be < p.n) edge = rs_node<FLAT>(p, be - 1);
+  }
+  for (int i = threadIdx.x; i < p.nb; i += kRsBlock) s_cnt[i] = 0;
+  if (threadIdx.x == 0) {
+    s_desc = 0;
+    s_gaps.n = 0;
+    if (blockIdx.x == 0) p.state[1] = p.state[2] = 0;
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const uint32_t i = threadIdx.x + j * kRsBlock;
+    node[j] = i < left ? rs_row<FLAT>(p, lo + i, idx[j]) : -1;
+  }
+  __syncthreads();
   bool descent = false;
-  RsHot hot = {-1, 0};
-  if (lo < hi) load(lo);
-  for (int64_t b0 = lo; b0 < hi; b0 += (int64_t)kRsCountPer * kRsBlock) {
-#pragma unroll
-    for (int j = 0; j < kRsCountPer; ++j) {
-      const int64_t be = b0 + threadIdx.x + (int64_t)j * kRsBlock;
-      node[j] = be < hi ? rs_row<FLAT>(p, be, next[j]) : -1;
-    }
-    if (b0 + (int64_t)kRsCountPer * kRsBlock < hi) load(b0 + (int64_t)kRsCountPer * kRsBlock);
-    // The entry before a lane's entry is the neighbouring lane's; the first lane of a wavefront needs the entry before
-    // the wavefront's first one: lane j loads it for row j (one load instruction for all rows).
-    int32_t edge = -1;
-    if (lane < kRsCountPer) {
-      const int64_t be = b0 + (int64_t)(threadIdx.x - lane) + (int64_t)lane * kRsBlock;
-      if (be > 0 && be < hi) edge = rs_node<FLAT>(p, be - 1);
-    }
-#pragma unroll
-    for (int j = 0; j < kRsCountPer; ++j) {
-      const int32_t e0 = __builtin_amdgcn_readlane(edge, j);
-      const int32_t up = lane_up1(node[j]);  // by every lane: lane 0's value is what lane 1 reads
-      const int32_t prev = lane == 0 ? e0 : up;
-      const bool live = b0 + threadIdx.x + (int64_t)j * kRsBlock < hi;
-      descent = descent || (live && node[j] < prev) || (live && node[j] < 0);
-    }
-#pragma unroll
-    for (int j = 0; j < kRsCountPer; ++j) rs_count_one(s_hist, node[j] >> p.rshift, hot);  // (-1 stays -1)
-  }
-  rs_count_flush(s_hist, hot);
-  if (__ballot(descent) != 0) s_desc = 1;
-  __syncthreads();
-  constexpr int PER = kRsMaxBuckets / kRsBlock;
-  uint32_t back[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int i = threadIdx.x + k * kRsBlock;
-    const uint32_t h = i < p.nb ? s_hist[i] : 0;
-    back[k] = h != 0 ? atomicAdd(&p.totals[i], h) : 0;
-  }
-  uint32_t sink = 0;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) sink |= back[k];
-  asm volatile("" ::"v"(sink) : "memory");  // the returns are in: this workgroup's share is in the totals
-  __syncthreads();
-  // the ticket counts the workgroups in its low half and those that saw a descent in its high half
-  if (threadIdx.x == 0) {
-    const uint32_t t = atomicAdd(p.sync, 1u + (s_desc ? 0x10000u : 0u));
-    s_last = (t & 0xFFFFu) == gridDim.x - 1 ? 1 : 0;
-    s_desc = (s_desc != 0 || (t >> 16) != 0) ? 1 : 0;
-  }
-  __syncthreads();
-  if (!s_last) return;
-  // ---- the last workgroup: bucket starts, and the chunks of buckets above p.cap entries
-  const bool unsorted = s_desc != 0;
-  const int pb = (p.nb + kRsBlock - 1) / kRsBlock;
-  uint32_t t[PER];
-  int32_t sum_t = 0, sum_c = 0, sum_b = 0;
+  int32_t hot = -1;
+  auto before = [&](int j) {
+    const int32_t e0 = __builtin_amdgcn_readlane(edge, j);
+    const int32_t up = lane_up1(node[j]);  // by every lane: lane 0's value is what lane 1 reads
+    return lane == 0 ? e0 : up;
+  };
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int i = threadIdx.x * pb + j;
-    t[j] = (j < pb && i < p.nb) ? atomicOr(&p.totals[i], 0u) : 0u;  // read where the additions were performed
+    const int32_t prev = before(j);
+    descent = descent || (threadIdx.x + j * kRsBlock < left && (node[j] < prev || node[j] < 0));
+    rank[j] = rs_take(s_cnt, node[j] >> p.rshift, hot);  // (-1 stays -1)
   }
+  if (__ballot(descent) != 0 && lane == 0) s_desc = 1;
+  __syncthreads();
+  const bool in_order = s_desc == 0;
+  if (!in_order && threadIdx.x == 0) p.state[3] = (int32_t)p.nonce;
+  const int total = (int)rs_scan_lds<kRsBlock>(s_cnt, p.nb, s_wave);
+  uint16_t *off = p.off + (size_t)blockIdx.x * p.pitch;
+  for (int i = threadIdx.x; i <= p.nb; i += kRsBlock) off[i] = (uint16_t)(i < p.nb ? s_cnt[i] : (uint32_t)total);
+  const uint32_t mask = (1u << p.rshift) - 1;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    sum_t += (int32_t)t[j];
-    if (t[j] > (uint32_t)p.cap) {
-      sum_c += (int32_t)((t[j] + p.cap - 1) / p.cap);
-      sum_b += 1;
-    }
-  }
-  const int32_t it = wave_inclusive_sum(sum_t), ic = wave_inclusive_sum(sum_c), ib = wave_inclusive_sum(sum_b);
-  if (lane == kWave - 1) {
-    s_wave[0][wave] = (uint32_t)it;
-    s_wave[1][wave] = (uint32_t)ic;
-    s_wave[2][wave] = (uint32_t)ib;
+    if (node[j] < 0) continue;
+    const uint32_t at = threadIdx.x + (uint32_t)(j * kRsBlock);
+    s_stage[s_cnt[(uint32_t)node[j] >> p.rshift] + rank[j]] = ((uint32_t)node[j] & mask) << kRsLocal | at;
   }
   __syncthreads();
-  uint32_t run_t = (uint32_t)(it - sum_t), run_c = (uint32_t)(ic - sum_c), run_b = (uint32_t)(ib - sum_b);
-  uint32_t all_t = 0, all_c = 0, all_b = 0;
-#pragma unroll
-  for (int w = 0; w < kRsBlock / kWave; ++w) {
-    run_t += w < wave ? s_wave[0][w] : 0u;
-    run_c += w < wave ? s_wave[1][w] : 0u;
-    run_b += w < wave ? s_wave[2][w] : 0u;
-    all_t += s_wave[0][w];
-    all_c += s_wave[1][w];
-    all_b += s_wave[2][w];
-  }
+  uint32_t *words = p.words + ((size_t)blockIdx.x << p.log);
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int i = threadIdx.x * pb + j;
-    if (j >= pb || i >= p.nb) break;
-    p.starts[i] = run_t;
-    p.cursor[i] = run_t;
-    run_t += t[j];
-    if (t[j] > (uint32_t)p.cap) {
-      s_hist[run_b] = run_c << 12 | (uint32_t)i;  // (chunks < 2^18, buckets <= 2^12)
-      run_c += (t[j] + p.cap - 1) / p.cap;
-      ++run_b;
-    }
+    const int pos = (int)threadIdx.x + j * kRsBlock;
+    if (pos < total) words[pos] = s_stage[pos];
   }
-  if (unsorted && all_c != 0) {
-    // who is chunk c: the last large bucket whose first chunk is not behind it (one lane that lists the chunks of its bucket
-    // is what the launch then waits for: 10 M entries, 409 chunks in one bucket, 13 us)
-    __syncthreads();
-    for (uint32_t c = threadIdx.x; c < all_c; c += kRsBlock) {
-      uint32_t b = 0, n = all_b;
-      while (n > 1) {
-        const uint32_t half = n / 2;
-        if ((s_hist[b + half] >> 12) <= c) { b += half; n -= half; } else { n = half; }
-      }
-      p.chunk_info[c] = (int32_t)(s_hist[b] & 0xFFFu);
-      p.chunk_info[p.max_chunks + c] = (int32_t)(s_hist[b] >> 12);
-      p.chunk_info[2 * p.max_chunks + c] = (int32_t)b;
-    }
-  }
-  if (threadIdx.x == 0) {
-    p.starts[p.nb] = all_t;
-    p.ptr[p.rows] = (int64_t)all_t;
-    p.state[0] = unsorted ? 1 : 0;
-    p.state[1] = unsorted ? (int32_t)all_c : 0;
-    p.state[2] = unsorted ? (int32_t)all_b : 0;
-  }
-}
-
-// row pointers and identity for an index in order and inside [0, N): the tile of entries at lo
-__device__ __forceinline__ void rs_identity(const RowSortArgs &p, int64_t lo, GapList &s_gaps) {
-  if (threadIdx.x == 0) s_gaps.n = 0;
-  __syncthreads();
-  int64_t at[kRsPer], before[kRsPer];
+  if (!in_order) return;
 #pragma unroll
-  for (int j = 0; j < kRsPer; ++j) {
-    const int64_t be = lo + threadIdx.x + (int64_t)j * kRsBlock, c = be < p.n ? be : p.n - 1;
-    at[j] = rs_load(p, c);
-    before[j] = rs_load(p, c > 0 ? c - 1 : 0);
-  }
-#pragma unroll
-  for (int j = 0; j < kRsPer; ++j) {
+  for (int j = 0; j < PER; ++j) {
     const int64_t be = lo + threadIdx.x + (int64_t)j * kRsBlock;
     const bool live = be < p.n;
-    int64_t top = -1, bot = 0;
-    if (live) {
-      if (p.identity) p.perm[be] = (int32_t)be;
-      top = rs_row(p, be, at[j]);
-      bot = be == 0 ? 0 : (int64_t)rs_row(p, be - 1, before[j]) + 1;
-    }
+    const int32_t prev = before(j);
+    const int64_t top = live ? (int64_t)node[j] : -1, bot = live ? (be == 0 ? 0 : (int64_t)prev + 1) : 0;
     gap_rows(p.ptr, bot, top, be, s_gaps);
     gap_rows(p.ptr, top + 1, live && be == p.n - 1 ? p.rows : top, p.n, s_gaps);
   }
@@ -427,236 +330,313 @@ __device__ __forceinline__ void rs_identity(const RowSortArgs &p, int64_t lo, Ga
   gap_rows_finish(p.ptr, s_gaps);
 }
 
-// (eight wavefronts per SIMD, i.e. at most 64 vector registers: two workgroups per CU)
-template <int FLAT, typename W>
-static __global__ __launch_bounds__(kRsBlock) __attribute__((amdgpu_waves_per_eu(8, 8)))
-void rs_place_kernel(RowSortArgs p) {
-  extern __shared__ uint32_t s_rows[];
-  static_assert(kRsTile * 8 + 2048 + kRsMaxBuckets * 8 <= 160 * 1024, "a workgroup's LDS: 160 KB with counts and bases");
-  __shared__ uint64_t s_stage[kRsTile];
-  __shared__ uint32_t s_wave[kRsBlock / kWave];
-  __shared__ GapList s_gaps;
-  uint32_t *s_cnt = s_rows;  // [nb] counts, then the tile's exclusive prefix
-  uint32_t *s_base = s_cnt + p.nb;  // [nb] first word of the tile's run in every bucket, less the run's place in the tile
-  const int64_t lo = (int64_t)blockIdx.x * kRsTile;
-  if (p.state[0] == 0) {
-    rs_identity(p, lo, s_gaps);
-    return;
-  }
-  // the row counts of large buckets, for the next launch
-  const int64_t n_cnt = (int64_t)p.state[2] << p.rshift;
-  for (int64_t i = (int64_t)blockIdx.x * kRsBlock + threadIdx.x; i < n_cnt; i += (int64_t)gridDim.x * kRsBlock) p.row_cnt[i] = 0;
-  for (int i = threadIdx.x; i < p.nb; i += kRsBlock) s_cnt[i] = 0;
-  int32_t node[kRsPer];
-  uint32_t rank[kRsPer];
-  {
-    int64_t idx[kRsPer];
-#pragma unroll
-    for (int j = 0; j < kRsPer; ++j) {
-      const int64_t be = lo + threadIdx.x + (int64_t)j * kRsBlock;
-      idx[j] = rs_load<FLAT>(p, be < p.n ? be : p.n - 1);
-    }
-#pragma unroll
-    for (int j = 0; j < kRsPer; ++j) {
-      const int64_t be = lo + threadIdx.x + (int64_t)j * kRsBlock;
-      node[j] = be < p.n ? rs_row<FLAT>(p, be, idx[j]) : -1;
-    }
-  }
-  __syncthreads();
-  int32_t hot = -1;
-#pragma unroll
-  for (int j = 0; j < kRsPer; ++j)
-    rank[j] = rs_take(s_cnt, node[j] >> p.rshift, hot);  // (-1 stays -1)
-  __syncthreads();
-  constexpr int PER = kRsMaxBuckets / kRsBlock;
-  uint32_t first[PER];  // of buckets threadIdx.x + k * kRsBlock
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int i = threadIdx.x + k * kRsBlock;
-    const uint32_t h = i < p.nb ? s_cnt[i] : 0;
-    first[k] = h != 0 ? atomicAdd(&p.cursor[i], h) : 0;
-  }
-  __syncthreads();
-  const int total = (int)rs_scan_lds<kRsBlock>(s_cnt, p.nb, s_wave);
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int i = threadIdx.x + k * kRsBlock;
-    if (i < p.nb) s_base[i] = first[k] - s_cnt[i];
-  }
-  const uint32_t mask = (1u << p.rshift) - 1;
-  constexpr int BITS = sizeof(W) == 4 ? 32 : 45;  // of a word (13 for the row in its bucket), above them its bucket
-#pragma unroll
-  for (int j = 0; j < kRsPer; ++j) {
-    if (node[j] < 0) continue;
-    const uint32_t b = (uint32_t)node[j] >> p.rshift;
-    const uint32_t be = (uint32_t)(lo + threadIdx.x + (int64_t)j * kRsBlock);
-    s_stage[s_cnt[b] + rank[j]] = (uint64_t)b << BITS | (W)((uint32_t)node[j] & mask) << (sizeof(W) == 4 ? p.eshift : 32) | be;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j0 = 0; j0 < kRsPer; j0 += 4) {
-    uint64_t w[4];
-    uint32_t to[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int pos = (int)threadIdx.x + (j0 + j) * kRsBlock;
-      w[j] = s_stage[pos];
-      w[j] = pos < total ? w[j] : 0;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) to[j] = s_base[(uint32_t)(w[j] >> BITS)] + threadIdx.x + (uint32_t)((j0 + j) * kRsBlock);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if ((int)threadIdx.x + (j0 + j) * kRsBlock < total) static_cast<W *>(p.binned)[to[j]] = (W)(w[j] & (((uint64_t)1 << BITS) - 1));
+// Where the entries of a bucket lie: in every tile a run of its words. Places of the bucket are numbered through all tiles.
+template <int BLOCK> struct RsRuns {
+  uint32_t start[BLOCK];                      // of a round of BLOCK tiles, the runs that are not empty: word - place
+  uint32_t bits[kRsSortPer * BLOCK / 32];     // places at which a run begins,
+  uint32_t pre[kRsSortPer * BLOCK / 32];      // their number before every 32 places
+  uint32_t wave[3][BLOCK / kWave];
+  uint32_t first;                             // number of the first run that holds one of the places asked for
+};
+
+// the offsets of bucket `bucket` in tile t: first word, number of words
+__device__ __forceinline__ void rs_run_of(const RowSortArgs &p, int bucket, int t, uint32_t &a, uint32_t &c) {
+  a = c = 0;
+  if (t < p.tiles) {
+    uint32_t two;  // (one load, whatever its alignment: every tile's offsets lie in a line of their own)
+    __builtin_memcpy(&two, p.off + (size_t)t * p.pitch + bucket, 4);
+    a = two & 0xFFFFu;
+    c = (two >> 16) - a;
   }
 }
 
-template <int BLOCK, typename W>
-static __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BLOCK == 512 ? 6 : 8)))
-void rs_sort_kernel(RowSortArgs p) {
-  constexpr int CAP = kRsSortPer * BLOCK, CAP_LOG = BLOCK == 512 ? 13 : 14;
-  extern __shared__ uint32_t s_rows[];
-  __shared__ uint32_t s_stage[CAP];
-  __shared__ uint32_t s_wave[BLOCK / kWave];
-  __shared__ int s_last;
-  static_assert(CAP * 4 + 1024 + (4 << kRsMaxShift) <= 160 * 1024, "a workgroup's LDS: 160 KB with the row counts");
-  uint32_t *s_hist = s_rows;  // [rows per bucket]
-  if (p.state[0] == 0) return;
-  const int R = 1 << p.rshift;
-  // (the chunks come first: each takes as long as the largest bucket)
-  int bucket = (int)blockIdx.x - p.max_chunks, chunk = -1, big = 0, first = 0;
-  if (bucket < 0) {
-    chunk = (int)blockIdx.x;
-    if (chunk >= p.state[1]) return;
-    bucket = p.chunk_info[chunk];
-    first = p.chunk_info[p.max_chunks + chunk];
-    big = p.chunk_info[2 * p.max_chunks + chunk];
+// at[j]: the word at place skip + j * BLOCK + threadIdx.x of the bucket, for places below skip + cnt (else 0). a0, c0:
+// rs_run_of of tile threadIdx.x. A place finds its run by counting the run starts before it (a search over the runs'
+// starts takes nine dependent LDS reads an entry).
+template <int BLOCK>
+__device__ __forceinline__ void rs_places(const RowSortArgs &p, int bucket, uint32_t skip, int cnt, uint32_t a0, uint32_t c0,
+                                          RsRuns<BLOCK> &s, uint32_t (&at)[kRsSortPer]) {
+  constexpr int WORDS = kRsSortPer * BLOCK / 32;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+#pragma unroll
+  for (int j = 0; j < kRsSortPer; ++j) at[j] = 0;
+  uint32_t done = 0;  // entries of the bucket in the tiles before the round's
+  for (int t0 = 0; t0 < p.tiles && done < skip + (uint32_t)cnt; t0 += BLOCK) {
+    uint32_t a = a0, c = c0;
+    if (t0 > 0) rs_run_of(p, bucket, t0 + tid, a, c);
+    const uint32_t incl = (uint32_t)wave_inclusive_sum((int32_t)c);
+    const uint64_t some = __ballot(c > 0);
+    uint32_t ord = __builtin_amdgcn_mbcnt_hi((uint32_t)(some >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)some, 0u));
+    if (lane == kWave - 1) {
+      s.wave[0][wave] = incl;
+      s.wave[1][wave] = (uint32_t)__popcll(some);
+    }
+    if (tid < WORDS) s.bits[tid] = 0;
+    __syncthreads();
+    uint32_t total, runs;
+    const uint32_t before = incl - c + rs_waves_before<BLOCK>(s.wave[0], total);
+    ord += rs_waves_before<BLOCK>(s.wave[1], runs);
+    if (done + total > skip) {  // (the same for the workgroup)
+      const int32_t from = (int32_t)(done + before - skip);  // the run's first place among those asked for
+      const int32_t head = from > 0 ? from : 0, end = from + (int32_t)c < cnt ? from + (int32_t)c : cnt;
+      if (c > 0 && head < end) {
+        s.start[ord] = ((uint32_t)(t0 + tid) << p.log) + a - (uint32_t)from;
+        atomicOr(&s.bits[head >> 5], 1u << (head & 31));
+        if (from <= 0 || before == 0) s.first = ord;
+      }
+      __syncthreads();
+      const uint32_t pc = tid < WORDS ? (uint32_t)__popc(s.bits[tid]) : 0u;
+      const uint32_t pi = (uint32_t)wave_inclusive_sum((int32_t)pc);
+      if (lane == kWave - 1) s.wave[2][wave] = pi;
+      __syncthreads();
+      const uint32_t pb = pi - pc + s.first + rs_waves_before<BLOCK>(s.wave[2], runs);
+      if (tid < WORDS) s.pre[tid] = pb;
+      __syncthreads();
+      const int lo = (int32_t)(done - skip) > 0 ? (int32_t)(done - skip) : 0;
+      const int hi = (int32_t)(done + total - skip) < cnt ? (int32_t)(done + total - skip) : cnt;
+      const uint32_t upto = 0xFFFFFFFFu >> (31 - (tid & 31));
+#pragma unroll
+      for (int j = 0; j < kRsSortPer; ++j) {
+        const int i = j * BLOCK + tid, w = j * (BLOCK / 32) + (tid >> 5);
+        const uint32_t run = s.pre[w] + (uint32_t)__popc(s.bits[w] & upto) - 1;
+        if (i >= lo && i < hi) at[j] = s.start[run] + (uint32_t)i;
+        if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();
+    done += total;
   }
-  const uint32_t b_lo = p.starts[bucket], b_hi = p.starts[bucket + 1];
-  uint32_t lo = b_lo, hi = b_hi;
-  if (chunk < 0) {
-    if (hi - lo > (uint32_t)CAP) return;
-  } else {
-    lo = b_lo + (uint32_t)(chunk - first) * CAP;
-    hi = lo + CAP < b_hi ? lo + CAP : b_hi;
-  }
-  for (int i = threadIdx.x; i < R; i += BLOCK) s_hist[i] = 0;
-  const int cnt = (int)(hi - lo);
-  const int shift = sizeof(W) == 4 ? p.eshift : 32;
-  const W *words = static_cast<const W *>(p.binned);
-  W word[kRsSortPer];
-  uint32_t row_rank[kRsSortPer];  // row << CAP_LOG | rank in the row
+}
+
+// The words at[] on the way together, then the rank of every entry in its row: entry[j] and row << CAP_LOG | rank.
+template <int BLOCK, int CAP_LOG>
+__device__ __forceinline__ void rs_rank(const RowSortArgs &p, const uint32_t (&at)[kRsSortPer], int cnt, uint32_t *s_hist,
+                                        uint32_t (&entry)[kRsSortPer], uint32_t (&row_rank)[kRsSortPer]) {
+  const uint32_t tile = (uint32_t)(p.per * kRsBlock);
 #pragma unroll
   for (int j = 0; j < kRsSortPer; ++j) {
-    const int i = j * BLOCK + (int)threadIdx.x;
-    word[j] = words[i < cnt ? lo + (uint32_t)i : 0];
+    entry[j] = p.words[at[j]];
+    if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // (the addresses of all 16 at once take 32 registers)
   }
-  __syncthreads();
   int32_t hot = -1;
 #pragma unroll
   for (int j = 0; j < kRsSortPer; ++j) {
-    if (j * BLOCK >= cnt) break;  // (the same for the workgroup)
-    const int i = j * BLOCK + (int)threadIdx.x;
-    const uint32_t r = (uint32_t)(word[j] >> shift);
-    row_rank[j] = r << CAP_LOG | rs_take(s_hist, i < cnt ? (int32_t)r : -1, hot);
+    const uint32_t r = entry[j] >> kRsLocal;
+    row_rank[j] = r << CAP_LOG;
+    if (j * BLOCK < cnt)  // (the same for the workgroup)
+      row_rank[j] |= rs_take(s_hist, j * BLOCK + (int)threadIdx.x < cnt ? (int32_t)r : -1, hot);
+    // (from kRsLarge entries on a tile fills its 1 << kRsLocal words)
+    if (BLOCK == 1024)
+      entry[j] = (at[j] & ~((1u << kRsLocal) - 1)) | (entry[j] & ((1u << kRsLocal) - 1));
+    else
+      entry[j] = __umul24(at[j] >> p.log, tile) + (entry[j] & ((1u << kRsLocal) - 1));
+    if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);
   }
-  const uint32_t entry_mask = sizeof(W) == 4 ? (1u << p.eshift) - 1 : ~0u;
+}
+
+// row0 + the row in the bucket of every entry, in the order of s_hist, to out: through the stage, for stores in whole lines
+template <int BLOCK, int CAP_LOG, typename U>
+__device__ __forceinline__ void rs_store_rows(const uint32_t (&row_rank)[kRsSortPer], int cnt, const uint32_t *s_hist,
+                                              uint32_t *s_stage, int32_t row0, U *out) {
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kRsSortPer; ++j) {
+    const uint32_t rr = row_rank[j];
+    if (j * BLOCK + (int)threadIdx.x < cnt)
+      s_stage[s_hist[rr >> CAP_LOG] + (rr & ((1u << CAP_LOG) - 1))] = (uint32_t)row0 + (rr >> CAP_LOG);
+    if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+  }
+  __syncthreads();
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < (uint32_t)cnt; i += BLOCK) out[i] = (U)s_stage[i];
+}
+
+template <int BLOCK>
+static __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BLOCK == 512 ? 6 : 8)))
+void rs_sort_kernel(RowSortArgs p) {
+  constexpr int CAP = kRsSortPer * BLOCK, CAP_LOG = BLOCK == 512 ? 13 : 14;
+  extern __shared__ uint32_t s_hist[];  // [rows per bucket]
+  __shared__ uint32_t s_stage[CAP];
+  __shared__ RsRuns<BLOCK> s_runs;
+  __shared__ uint32_t s_wave[BLOCK / kWave];
+  static_assert(CAP * 4 + sizeof(RsRuns<BLOCK>) + 256 + (4 << kRsMaxShift) <= 160 * 1024, "a workgroup's LDS: 160 KB");
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const bool unsorted = p.state[3] == (int32_t)p.nonce;
+  if (blockIdx.x == 0 && tid == 0) p.state[0] = unsorted ? 1 : 0;
+  if (!unsorted) {
+    if (p.identity) {
+      for (int64_t i = (int64_t)blockIdx.x * BLOCK + tid; i < p.n; i += (int64_t)gridDim.x * BLOCK) {
+        p.perm[i] = (int32_t)i;
+        if (p.perm_row != nullptr) p.perm_row[i] = rs_node(p, i);
+      }
+    }
+    return;
+  }
+  // neighbouring buckets, whose runs share lines, on one of the eight dies (workgroups go to them in turn)
+  const int per_die = (p.nb + 7) / 8, bucket = (int)(blockIdx.x & 7) * per_die + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_die || bucket >= p.nb) return;
+  // The bucket's first place in perm is the number of entries in buckets before it: the sum of its offsets in all tiles.
+  uint32_t a0, c0, base = 0, cnt_u = 0;
+  rs_run_of(p, bucket, tid, a0, c0);
+  {
+    uint32_t a = a0, c = c0;
+    for (int t = tid + BLOCK; t < p.tiles; t += BLOCK) {
+      uint32_t at, ct;
+      rs_run_of(p, bucket, t, at, ct);
+      a += at;
+      c += ct;
+    }
+    const int32_t ia = wave_inclusive_sum((int32_t)a), ic = wave_inclusive_sum((int32_t)c);
+    if (lane == kWave - 1) {
+      s_runs.wave[0][wave] = (uint32_t)ia;
+      s_runs.wave[1][wave] = (uint32_t)ic;
+    }
+    const int R = 1 << p.rshift;
+    for (int i = tid; i < R; i += BLOCK) s_hist[i] = 0;
+    __syncthreads();
+#pragma unroll 4
+    for (int w = 0; w < BLOCK / kWave; ++w) {
+      base += s_runs.wave[0][w];
+      cnt_u += s_runs.wave[1][w];
+    }
+    __syncthreads();
+  }
+  if (bucket == p.nb - 1 && tid == 0) p.ptr[p.rows] = (int64_t)base + cnt_u;
+  const int R = 1 << p.rshift;
+  if (cnt_u > (uint32_t)CAP) {
+    // for the passes behind: the bucket's chunks, its counters cleared
+    const uint32_t m = (cnt_u + CAP - 1) / CAP;
+    if (tid == 0) {
+      const uint32_t first = (uint32_t)atomicAdd(&p.state[1], (int32_t)m), big = (uint32_t)atomicAdd(&p.state[2], 1);
+      s_runs.wave[0][0] = first;
+      s_runs.wave[1][0] = big;
+      uint32_t *rec = p.big + 4 * (size_t)big;
+      rec[0] = (uint32_t)bucket;
+      rec[1] = base;
+      rec[2] = cnt_u;
+      rec[3] = first;
+      p.arrived[big] = 0;
+    }
+    __syncthreads();
+    const uint32_t first = s_runs.wave[0][0], big = s_runs.wave[1][0];
+    for (uint32_t c = tid; c < m; c += BLOCK) p.chunk_big[first + c] = (int32_t)big;
+    for (int i = tid; i < R; i += BLOCK) p.row_cnt[((int64_t)big << p.rshift) + i] = 0;
+    return;
+  }
+  const int cnt = (int)cnt_u;
+  uint32_t at[kRsSortPer], entry[kRsSortPer], row_rank[kRsSortPer];
+  rs_places<BLOCK>(p, bucket, 0, cnt, a0, c0, s_runs, at);
+  rs_rank<BLOCK, CAP_LOG>(p, at, cnt, s_hist, entry, row_rank);
   __syncthreads();
   const int64_t row0 = (int64_t)bucket << p.rshift;
   const int n_rows = p.rows - row0 < R ? (int)(p.rows - row0) : R;
-  if (chunk < 0) {
-    rs_scan_lds<BLOCK>(s_hist, R, s_wave);
-    for (int i = threadIdx.x; i < n_rows; i += BLOCK) p.ptr[row0 + i] = (int64_t)(lo + s_hist[i]);
+  rs_scan_lds<BLOCK>(s_hist, R, s_wave);
+  for (int i = tid; i < n_rows; i += BLOCK) p.ptr[row0 + i] = (int64_t)(base + s_hist[i]);
 #pragma unroll
-    for (int j = 0; j < kRsSortPer; ++j) {
-      const int i = j * BLOCK + (int)threadIdx.x;
-      const uint32_t rr = row_rank[j];
-      if (i < cnt) s_stage[s_hist[rr >> CAP_LOG] + (rr & (CAP - 1))] = (uint32_t)word[j] & entry_mask;
-    }
-    __syncthreads();
-#pragma unroll 8
-    for (int i = threadIdx.x; i < cnt; i += BLOCK) p.perm[lo + (uint32_t)i] = (int32_t)s_stage[i];
-    return;
+  for (int j = 0; j < kRsSortPer; ++j) {
+    const uint32_t rr = row_rank[j];
+    if (j * BLOCK + tid < cnt) s_stage[s_hist[rr >> CAP_LOG] + (rr & (CAP - 1))] = entry[j];
+    if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);
   }
-  // A chunk of a large bucket: its counts to the bucket's; what they found there is the chunk's offset inside every row. The
-  // chunk's words go back in order of their rows; of 64 bits as [cnt] entries of 32 and behind them [cnt] rows of 16 bits.
+  __syncthreads();
+  int32_t *perm = p.perm + base;
+#pragma unroll 4
+  for (uint32_t i = tid; i < (uint32_t)cnt; i += BLOCK) perm[i] = (int32_t)s_stage[i];
+  if (p.perm_row != nullptr)
+    rs_store_rows<BLOCK, CAP_LOG>(row_rank, cnt, s_hist, s_stage, (int32_t)row0, p.perm_row + base);
+}
+
+// The chunks of large buckets. A chunk's row counts go to the bucket's; what they found there is the chunk's offset inside
+// every row. Its entries are left in order of their rows.
+template <int BLOCK>
+static __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BLOCK == 512 ? 6 : 8)))
+void rs_chunk_kernel(RowSortArgs p) {
+  constexpr int CAP = kRsSortPer * BLOCK, CAP_LOG = BLOCK == 512 ? 13 : 14;
+  extern __shared__ uint32_t s_hist[];  // [rows per bucket]
+  __shared__ uint32_t s_stage[CAP];
+  __shared__ RsRuns<BLOCK> s_runs;
+  __shared__ uint32_t s_wave[BLOCK / kWave];
+  __shared__ int s_last;
+  const int tid = threadIdx.x, chunk = (int)blockIdx.x;
+  if (p.state[0] == 0 || chunk >= p.state[1]) return;
+  const int big = p.chunk_big[chunk];
+  const uint32_t *rec = p.big + 4 * (size_t)big;
+  const int bucket = (int)rec[0];
+  const uint32_t base = rec[1], total = rec[2], skip = (uint32_t)(chunk - (int)rec[3]) * CAP;
+  const int cnt = total - skip < (uint32_t)CAP ? (int)(total - skip) : CAP;
+  const int R = 1 << p.rshift;
+  for (int i = tid; i < R; i += BLOCK) s_hist[i] = 0;
+  uint32_t a0, c0;
+  rs_run_of(p, bucket, tid, a0, c0);
+  uint32_t at[kRsSortPer], entry[kRsSortPer], row_rank[kRsSortPer];
+  rs_places<BLOCK>(p, bucket, skip, cnt, a0, c0, s_runs, at);
+  rs_rank<BLOCK, CAP_LOG>(p, at, cnt, s_hist, entry, row_rank);
+  __syncthreads();
+  const int64_t row0 = (int64_t)bucket << p.rshift;
+  const int n_rows = p.rows - row0 < R ? (int)(p.rows - row0) : R;
   rs_scan_lds<BLOCK>(s_hist, R, s_wave);
   uint32_t sink = 0;
-  for (int i = threadIdx.x; i < R; i += BLOCK) {
-    const uint32_t at = s_hist[i], h = (i + 1 < R ? s_hist[i + 1] : (uint32_t)cnt) - at;
+  for (int i = tid; i < R; i += BLOCK) {
+    const uint32_t from = s_hist[i], h = (i + 1 < R ? s_hist[i + 1] : (uint32_t)cnt) - from;
     if (h == 0) continue;
     const uint32_t before = atomicAdd(&p.row_cnt[((int64_t)big << p.rshift) + i], h);
-    p.chunk_off[((int64_t)chunk << p.rshift) + i] = before - at;
+    p.chunk_off[((int64_t)chunk << p.rshift) + i] = before - from;
     sink |= before;
   }
 #pragma unroll
   for (int j = 0; j < kRsSortPer; ++j) {
-    const int i = j * BLOCK + (int)threadIdx.x;
     const uint32_t rr = row_rank[j];
-    if (i < cnt) s_stage[s_hist[rr >> CAP_LOG] + (rr & (CAP - 1))] = (uint32_t)word[j];
+    if (j * BLOCK + tid < cnt) s_stage[s_hist[rr >> CAP_LOG] + (rr & (CAP - 1))] = entry[j];
+    if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);
   }
-  __syncthreads();
-  uint32_t *entries = reinterpret_cast<uint32_t *>(static_cast<W *>(p.binned) + lo);
-  for (int i = threadIdx.x; i < cnt; i += BLOCK) entries[i] = s_stage[i];
   asm volatile("" ::"v"(sink) : "memory");  // the returns are in: the counts are in memory
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const uint32_t m = (b_hi - b_lo + CAP - 1) / CAP;
-    s_last = atomicAdd(&p.sync[1 + big], 1u) == m - 1 ? 1 : 0;
+  if (tid == 0) {
+    const uint32_t m = (total + CAP - 1) / CAP;
+    s_last = atomicAdd(&p.arrived[big], 1u) == m - 1 ? 1 : 0;
   }
-  if constexpr (sizeof(W) == 8) {
-    uint16_t *s_srow = reinterpret_cast<uint16_t *>(s_stage);
-#pragma unroll
-    for (int j = 0; j < kRsSortPer; ++j) {
-      const uint32_t rr = row_rank[j];
-      if (j * BLOCK + (int)threadIdx.x < cnt) s_srow[s_hist[rr >> CAP_LOG] + (rr & (CAP - 1))] = (uint16_t)(rr >> CAP_LOG);
-    }
-    __syncthreads();
-    uint16_t *rows = reinterpret_cast<uint16_t *>(entries + cnt);
-    for (int i = threadIdx.x; i < cnt; i += BLOCK) rows[i] = s_srow[i];
-  } else {
-    __syncthreads();
-  }
+#pragma unroll 8
+  for (int i = tid; i < cnt; i += BLOCK) p.by_row[base + skip + (uint32_t)i] = s_stage[i];
+  rs_store_rows<BLOCK, CAP_LOG>(row_rank, cnt, s_hist, s_stage, 0, p.by_row_row + base + skip);
+  __syncthreads();
   if (!s_last) return;
-  for (int i = threadIdx.x; i < R; i += BLOCK) s_hist[i] = atomicOr(&p.row_cnt[((int64_t)big << p.rshift) + i], 0u);
+  // the chunk that arrives last: the bucket's row pointers
+  for (int i = tid; i < R; i += BLOCK) s_hist[i] = atomicOr(&p.row_cnt[((int64_t)big << p.rshift) + i], 0u);
   __syncthreads();
   rs_scan_lds<BLOCK>(s_hist, R, s_wave);
-  for (int i = threadIdx.x; i < n_rows; i += BLOCK) p.ptr[row0 + i] = (int64_t)(b_lo + s_hist[i]);
+  for (int i = tid; i < n_rows; i += BLOCK) p.ptr[row0 + i] = (int64_t)(base + s_hist[i]);
 }
 
 // the chunks of large buckets, each in order of its rows: every entry to its place among its row's
 constexpr int kRsPiece = 8;  // entries per lane; a chunk is 4 or 8 pieces
-template <typename W> static __global__ __launch_bounds__(kBlock) void rs_place_chunks_kernel(RowSortArgs p) {
+static __global__ __launch_bounds__(kBlock) void rs_place_chunks_kernel(RowSortArgs p) {
+  if (p.state[0] == 0) return;
   const int pieces = p.cap / (kRsPiece * kBlock), n = p.state[1] * pieces;
   for (int q = (int)blockIdx.x; q < n; q += (int)gridDim.x) {
     const int chunk = q / pieces, i0 = (q - chunk * pieces) * (kRsPiece * kBlock) + (int)threadIdx.x;
-    const int bucket = p.chunk_info[chunk];
-    const uint32_t lo = p.starts[bucket] + (uint32_t)(chunk - p.chunk_info[p.max_chunks + chunk]) * (uint32_t)p.cap;
-    const uint32_t left = p.starts[bucket + 1] - lo;
+    const uint32_t *rec = p.big + 4 * (size_t)p.chunk_big[chunk];
+    const uint32_t skip = (uint32_t)(chunk - (int)rec[3]) * (uint32_t)p.cap, left = rec[2] - skip;
     const int cnt = left < (uint32_t)p.cap ? (int)left : p.cap;
-    const int64_t *ptr = p.ptr + ((int64_t)bucket << p.rshift);
+    const int64_t row0 = (int64_t)rec[0] << p.rshift;
+    const int64_t *ptr = p.ptr + row0;
     const uint32_t *off = p.chunk_off + ((int64_t)chunk << p.rshift);
-    const uint32_t *entries = reinterpret_cast<const uint32_t *>(static_cast<const W *>(p.binned) + lo);
-    const uint16_t *rows = reinterpret_cast<const uint16_t *>(entries + cnt);  // (words of 64 bits)
-    uint32_t e[kRsPiece], r[kRsPiece];
+    const uint32_t *entries = p.by_row + rec[1] + skip;
+    const uint16_t *rows = p.by_row_row + rec[1] + skip;
+    uint32_t e[kRsPiece], r[kRsPiece], to[kRsPiece];
 #pragma unroll
     for (int j = 0; j < kRsPiece; ++j) {  // (past the end: the last entry again)
       const int i = i0 + j * kBlock < cnt ? i0 + j * kBlock : cnt - 1;
       e[j] = entries[i];
-      if constexpr (sizeof(W) == 8) r[j] = rows[i];
-    }
-    if constexpr (sizeof(W) == 4) {
-#pragma unroll
-      for (int j = 0; j < kRsPiece; ++j) {
-        r[j] = e[j] >> p.eshift;
-        e[j] &= (1u << p.eshift) - 1;
-      }
+      r[j] = rows[i];
     }
 #pragma unroll
-    for (int j = 0; j < kRsPiece; ++j) r[j] = (uint32_t)ptr[r[j]] + off[r[j]] + (uint32_t)(i0 + j * kBlock);
+    for (int j = 0; j < kRsPiece; ++j) to[j] = (uint32_t)ptr[r[j]] + off[r[j]] + (uint32_t)(i0 + j * kBlock);
 #pragma unroll
-    for (int j = 0; j < kRsPiece; ++j)
-      if (i0 + j * kBlock < cnt) p.perm[r[j]] = (int32_t)e[j];
+    for (int j = 0; j < kRsPiece; ++j) {
+      if (i0 + j * kBlock >= cnt) continue;
+      p.perm[to[j]] = (int32_t)e[j];
+      if (p.perm_row != nullptr) p.perm_row[to[j]] = (int32_t)row0 + (int32_t)r[j];
+    }
   }
 }
 
@@ -669,7 +649,8 @@ static __global__ __launch_bounds__(kBlock) void row_lengths_kernel(const int64_
 // Backward of scatter min / max over entries sorted by row: grad_in[e, k] = grad[row, k] where arg[row, k] == e, else 0.
 // Every row of grad_in is written once, in one piece, and the entries of a row read its gradient and positions from the
 // vector L1. (A fill of grad_in and a scatter of single elements into it writes the buffer twice: 2.3 M x 64 floats onto
-// 282 k rows 368 us, of which the scatter 260; now 220 with 55 for the sort, 3.7 TB/s in rows of 256 bytes in no order.) U: bits of an element. A workgroup takes 4 positions per worker.
+// 282 k rows 368 us, of which the scatter 260; this kernel 210 and the sort 33, 3.9 TB/s in rows of 256 bytes in no order.)
+// U: bits of an element. A workgroup takes 4 positions per worker.
 template <typename U, int VEC>
 static __global__ __launch_bounds__(kBlock) void rs_arg_rows_kernel(RowSortArgs p, const U *__restrict__ grad,
                                                                     const int64_t *__restrict__ arg,
@@ -684,7 +665,7 @@ static __global__ __launch_bounds__(kBlock) void rs_arg_rows_kernel(RowSortArgs 
 #pragma unroll
   for (int q = 0; q < Q; ++q) e[q] = base + (int64_t)q * W < n ? p.perm[base + (int64_t)q * W] : -1;
 #pragma unroll
-  for (int q = 0; q < Q; ++q) row[q] = e[q] >= 0 ? rs_node(p, e[q]) : 0;
+  for (int q = 0; q < Q; ++q) row[q] = e[q] >= 0 ? p.perm_row[base + (int64_t)q * W] : 0;
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     if (e[q] < 0) continue;
@@ -721,43 +702,48 @@ inline int launch_arg_rows(const RowSortArgs &p, const void *grad, const int64_t
   return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
 }
 
-template <typename W> inline int launch_row_sort_words(const RowSortArgs &p, hipStream_t stream) {
-  const dim3 gt((unsigned)((p.n + kRsTile - 1) / kRsTile));
-  if (p.flat)
-    hipLaunchKernelGGL((rs_place_kernel<1, W>), gt, dim3(kRsBlock), (size_t)p.nb * 8, stream, p);
-  else
-    hipLaunchKernelGGL((rs_place_kernel<0, W>), gt, dim3(kRsBlock), (size_t)p.nb * 8, stream, p);
-  const dim3 gs((unsigned)(p.nb + p.max_chunks));
-  const size_t lds = (size_t)4 << p.rshift;
-  if (p.cap == kRsSortPer * 512)
-    hipLaunchKernelGGL((rs_sort_kernel<512, W>), gs, dim3(512), lds, stream, p);
-  else
-    hipLaunchKernelGGL((rs_sort_kernel<1024, W>), gs, dim3(1024), lds, stream, p);
-  if (p.max_chunks > 0) {
-    const int64_t pieces = (int64_t)p.max_chunks * (p.cap / (kRsPiece * kBlock));
-    hipLaunchKernelGGL(rs_place_chunks_kernel<W>, dim3((unsigned)(pieces < 2048 ? pieces : 2048)), dim3(kBlock), 0, stream, p);
+template <int FLAT> inline void launch_rs_place(const RowSortArgs &p, hipStream_t stream) {
+  const dim3 grid((unsigned)p.tiles);
+  const size_t lds = (size_t)p.nb * 4;
+  switch (p.per) {
+  case 1: hipLaunchKernelGGL((rs_place_kernel<FLAT, 1>), grid, dim3(kRsBlock), lds, stream, p); break;
+  case 2: hipLaunchKernelGGL((rs_place_kernel<FLAT, 2>), grid, dim3(kRsBlock), lds, stream, p); break;
+  case 3: hipLaunchKernelGGL((rs_place_kernel<FLAT, 3>), grid, dim3(kRsBlock), lds, stream, p); break;
+  case 4: hipLaunchKernelGGL((rs_place_kernel<FLAT, 4>), grid, dim3(kRsBlock), lds, stream, p); break;
+  case 5: hipLaunchKernelGGL((rs_place_kernel<FLAT, 5>), grid, dim3(kRsBlock), lds, stream, p); break;
+  case 6: hipLaunchKernelGGL((rs_place_kernel<FLAT, 6>), grid, dim3(kRsBlock), lds, stream, p); break;
+  case 7: hipLaunchKernelGGL((rs_place_kernel<FLAT, 7>), grid, dim3(kRsBlock), lds, stream, p); break;
+  default: hipLaunchKernelGGL((rs_place_kernel<FLAT, 8>), grid, dim3(kRsBlock), lds, stream, p); break;
   }
-  return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
+}
+template <int BLOCK> inline void launch_rs_sort(const RowSortArgs &p, hipStream_t stream) {
+  const size_t lds = (size_t)4 << p.rshift;
+  hipLaunchKernelGGL(rs_sort_kernel<BLOCK>, dim3((unsigned)((p.nb + 7) / 8 * 8)), dim3(BLOCK), lds, stream, p);
+  if (p.max_chunks == 0) return;
+  hipLaunchKernelGGL(rs_chunk_kernel<BLOCK>, dim3((unsigned)p.max_chunks), dim3(BLOCK), lds, stream, p);
+  const int64_t pieces = (int64_t)p.max_chunks * (p.cap / (kRsPiece * kBlock));
+  hipLaunchKernelGGL(rs_place_chunks_kernel, dim3((unsigned)(pieces < 2048 ? pieces : 2048)), dim3(kBlock), 0, stream, p);
 }
 
+// nonce: tag of the call (any value; a repeated one only costs an index in order its short way)
 inline int launch_row_sort(const RowSortArgs &args, const int64_t *index, int64_t sb, int64_t se, bool identity,
-                           hipStream_t stream) {
+                           uint64_t nonce, hipStream_t stream) {
   RowSortArgs p = args;
   p.identity = identity ? 1 : 0;
   p.index = index;
   p.sb = sb;
   p.se = se;
   p.flat = p.B == 1 && se == 1;
-  const int n_clear = p.nb + 1 + p.max_big;
-  hipLaunchKernelGGL(rs_clear_kernel, dim3((unsigned)((n_clear + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream, p.totals,
-                     n_clear);
-  int64_t groups = (p.n + kRsCountPer * kRsBlock - 1) / (kRsCountPer * kRsBlock);
-  if (groups > kRsCountGroups) groups = kRsCountGroups;
+  p.nonce = (uint32_t)nonce | 1u;
   if (p.flat)
-    hipLaunchKernelGGL(rs_count_kernel<1>, dim3((unsigned)groups), dim3(kRsBlock), 0, stream, p);
+    launch_rs_place<1>(p, stream);
   else
-    hipLaunchKernelGGL(rs_count_kernel<0>, dim3((unsigned)groups), dim3(kRsBlock), 0, stream, p);
-  return p.eshift < 32 ? launch_row_sort_words<uint32_t>(p, stream) : launch_row_sort_words<uint64_t>(p, stream);
+    launch_rs_place<0>(p, stream);
+  if (p.cap == kRsSortPer * 512)
+    launch_rs_sort<512>(p, stream);
+  else
+    launch_rs_sort<1024>(p, stream);
+  return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
 }
 
 }  // namespace ts

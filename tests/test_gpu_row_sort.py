@@ -1,5 +1,5 @@
 """Scatter of wide rows through the sort of the index by row (csrc/row_sort.h) at the sizes where it can go wrong: tiles
-of 8192 entries, buckets at and above what one sorting workgroup holds (8192 entries, 16384 from 4 M entries on), buckets
+of 1024 to 8192 entries, buckets at and above what one sorting workgroup holds (8192 entries, 16384 from 4 M entries on), buckets
 of one row and of 8192 rows, entries outside [0, N), an index in order. Sums of int32 are exact; min / max must give the
 first position of equal values. The expected results come from torch on the same device."""
 import numpy as np
@@ -20,6 +20,9 @@ def _index(kind, E, N, g):
         index[torch.randperm(E, generator=g, device=DEV)[:n]] = N // 3
     elif kind == "sorted":
         index = index.sort()[0]
+    elif kind == "pieces":  # in order but for pieces of 5000 entries: a bucket's entries in one or two tiles
+        index = index.sort()[0]
+        index = index[(torch.arange(E, device=DEV) // 5000 + torch.rand(E, generator=g, device=DEV, dtype=torch.float64)).argsort()]
     elif kind == "outside":
         index[::3] += N
         index[1::7] = -1 - index[1::7]
@@ -31,7 +34,10 @@ CASES = [("even", 8191, 300), ("even", 8192, 300), ("even", 8193, 300), ("one ro
          ("hub30000", 60001, 100000), ("even", 30000, 600001), ("sorted", 30001, 7000), ("outside", 30001, 7000),
          ("even", 1, 1), ("even", 4194303, 70001), ("even", 4194305, 70001), ("hub16384", 4194305, 2000003),
          ("hub16385", 4194305, 2000003), ("hub1000000", 4194304, 1000),
-         ("hub200001", 600001, 8400007), ("even", 600001, 8400007)]
+         ("hub200001", 600001, 8400007), ("even", 600001, 8400007),
+         # a lane more in place from 524288 entries on; more than 1024 tiles: the runs of a bucket in two rounds
+         ("even", 524288, 5000), ("even", 524289, 5000), ("pieces", 60001, 3000), ("pieces", 8500001, 400000),
+         ("hub40000", 8500001, 40000), ("outside", 8388609, 40000)]
 
 
 @pytest.mark.parametrize("kind,E,N", CASES)
