@@ -379,6 +379,34 @@ int ts_group_softmax_backward(const void *result, const void *grad_out,
                               int dtype, int log_space, void *workspace,
                               size_t workspace_bytes, ts_stream_t stream);
 
+/*
+ * The same with the entries sorted by group first, for an index in any order:
+ * src is read once and the result written once, and the backward pass takes the
+ * order of the forward pass. order: ts_group_order_bytes() bytes of device
+ * memory, written by the forward call; hand it, unchanged and with the same
+ * index, sizes and dtype, to the backward call. 0 bytes: this form does not
+ * take the call (TS_ERR_UNSUPPORTED; small inputs, which ts_group_softmax does
+ * faster). workspace: ts_group_order_workspace_bytes() bytes of scratch (the
+ * backward call needs less). Both 16-byte aligned. Group sums are held in
+ * double. result and grad_out: what the forward call returned and its gradient.
+ */
+size_t ts_group_order_bytes(int64_t B, int64_t E, int64_t K, int64_t N,
+                            int dtype);
+size_t ts_group_order_workspace_bytes(int64_t B, int64_t E, int64_t K,
+                                      int64_t N, int dtype, int backward);
+int ts_group_softmax_ordered(const void *src, const int64_t *index, void *out,
+                             int64_t B, int64_t E, int64_t K, int64_t N,
+                             int64_t index_stride_b, int64_t index_stride_e,
+                             int dtype, int log_space, double eps, void *order,
+                             size_t order_bytes, void *workspace,
+                             size_t workspace_bytes, ts_stream_t stream);
+int ts_group_softmax_ordered_backward(
+    const void *result, const void *grad_out, const int64_t *index,
+    void *grad_in, int64_t B, int64_t E, int64_t K, int64_t N,
+    int64_t index_stride_b, int64_t index_stride_e, int dtype, int log_space,
+    const void *order, size_t order_bytes, void *workspace,
+    size_t workspace_bytes, ts_stream_t stream);
+
 /* logsumexp over the entries that share an index, one index per row:
  *   out[b, n, k] = log(sum_group exp(src - m) + eps) + m,  m = group max starting from -inf;
  *   NaN entries drop out; NaN and -inf results (empty groups) become 0, +inf the largest finite value.

@@ -1119,6 +1119,142 @@ int run_group_softmax(const void *src, const void *grad, const int64_t *index, v
 }
 }  // namespace
 
+namespace {
+// Softmax over entries sorted by group (row_sort.h, the ordered tiles of group_fused.h). Where the tiles for an index in
+// order apply they come first, behind a sample of the index, and what follows returns at once if they took the call: an
+// index in order costs what it did without the sort (and the sort of one that is not, 14 us for the launches in front).
+// Where the line lies (us without / with, groups of 30; even, Zipf(1.2) hub, both in no order, then both in order):
+//   forward, from 8 MB: 100 k x 8 floats 45 48 23 23 / 35 66 28 44, 300 k x 8 56 89 45 76 / 43 75 32 46, 100 k x 32 47 70 44 68 /
+//   40 78 33 54. Up to 128 entries a group: with 1000 the tables in LDS hold every group, 300 k x 8 62 82 52 70 / 61 75 49 48,
+//   but 300 k x 4 60 95 48 77 / 53 71 40 42 against 100 k x 32 52 53 33 34 / 57 79 49 56 and, in order, 3 M x 32 430 550 / 471 1314.
+//   backward, from 16 to 128 MB, up to 64 entries a group and 64 bytes a row: 1 M x 8 88 118 57 57 / 62 92 48 74, 3 M x 8 244 455
+//   80 157 / 159 239 81 152; beyond, two arrays of gathered rows leave the 256 MB of the memory-side cache: 10 M x 8 817 875 / 883
+//   1178. 1 M x 32 205 323 / 173 293, but in order, where no tiles come first, 139 228 / 131 234 and 3 M x 64 784 793 / 1068 1989.
+// TS_GROUP_ORDER (tuning aid): 0 never, 2 at any size; 3: at any size, and never the tiles for an index in order.
+bool group_order_rule(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, bool backward) {
+  if (!valid_dtype(dtype) || !is_float_dtype(dtype) || !sizes_ok(B, N, E, K) || B * E * K == 0 || N == 0) return false;
+  const int mode = env_int("TS_GROUP_ORDER", 1);
+  const int64_t row_bytes = K * kElemBytes[dtype], bytes = B * E * row_bytes;
+  if (mode == 0 || K >= (int64_t)1 << 20 || row_bytes % kVecBytes != 0) return false;
+  if (backward && row_bytes > 64) return false;
+  if (mode >= 2) return true;
+  if (backward) return E <= 64 * N && bytes >= ((int64_t)16 << 20) && bytes <= ((int64_t)128 << 20);
+  return E <= 128 * N && bytes >= ((int64_t)8 << 20);
+}
+// plan of the tiles for an index in order, their records at ws; false: they do not apply
+bool group_order_tiles(GroupArgs &g, int dtype, int mode, void *ws, size_t ws_bytes, int *flag, FusedArgs &f) {
+  if (env_int("TS_GROUP_FUSED", 1) == 0 || env_int("TS_GROUP_ORDER", 1) == 3) return false;
+  const bool backward = mode == GS_SOFTMAX_BWD || mode == GS_LOG_SOFTMAX_BWD;
+  if (!group_fused_plan(g, mode, kElemBytes[dtype], ws, ws_bytes, backward, f)) return false;
+  f.flag = flag;
+  return true;
+}
+size_t group_order_records(int64_t B, int64_t E, int64_t K, int dtype, bool backward) {
+  const size_t ordered = group_fused_ordered_plan(B * E, K, kElemBytes[dtype], backward, nullptr).bytes;
+  const size_t tiles = group_fused_scratch_bytes(B, E, K, kElemBytes[dtype]);
+  return ordered > tiles ? ordered : tiles;  // (one after the other)
+}
+// sorted: the order, made by a forward call and read by a backward call
+int run_group_ordered(const void *src, const void *grad, const int64_t *index, void *out, int64_t B, int64_t E, int64_t K,
+                      int64_t N, int64_t sb, int64_t se, int dtype, int mode, double eps, const RowSortArgs &sorted,
+                      void *records, size_t records_bytes, hipStream_t stream) {
+  const bool backward = mode == GS_SOFTMAX_BWD || mode == GS_LOG_SOFTMAX_BWD;
+  if (!aligned16(src) || !aligned16(out) || (grad != nullptr && !aligned16(grad))) return TS_ERR_UNSUPPORTED;
+  const int vec = kVecBytes / kElemBytes[dtype];
+  FusedOrderedPlan p = group_fused_ordered_plan(B * E, K, kElemBytes[dtype], backward, records);
+  if (p.bytes == 0) return TS_ERR_UNSUPPORTED;
+  GroupArgs g = {};
+  g.src = src;
+  g.grad = grad;
+  g.index = index;
+  g.out = out;
+  g.B = B;
+  g.E = E;
+  g.K = K;
+  g.N = N;
+  g.sb = sb;
+  g.se = se;
+  g.eps = eps;
+  // Does the forward call try the tiles for an index in order? The backward call then follows its verdict.
+  FusedArgs tiles;
+  int *const flag = sorted.state + 4;
+  const int fwd_mode = mode == GS_SOFTMAX_BWD ? GS_SOFTMAX : mode == GS_LOG_SOFTMAX_BWD ? GS_LOG_SOFTMAX : mode;
+  const bool tried = group_order_tiles(g, dtype, fwd_mode, records, records_bytes, flag, tiles);
+  if (tried) {
+    if (backward && !group_order_tiles(g, dtype, mode, records, records_bytes, flag, tiles)) return TS_ERR_UNSUPPORTED;
+    g.in_order = &tiles;
+    g.in_order_sample = backward ? 0 : 1;
+    const int rc = dispatch_group_softmax(dtype, g, mode, vec, stream);
+    if (rc != TS_OK) return rc;
+    g.in_order = nullptr;
+  }
+  if (!backward) {
+    const int rc = launch_row_sort(sorted, index, sb, se, false, next_nonce(), stream, tried ? flag : nullptr);
+    if (rc != TS_OK) return rc;
+  }
+  p.f.gate = tried ? flag : nullptr;
+  p.f.state = sorted.state;
+  p.f.n_sorted = sorted.ptr + B * N;
+  p.f.perm = sorted.perm;
+  p.f.group = sorted.perm_row;
+  p.f.ptr = sorted.ptr;
+  p.f.index = index;
+  p.f.sb = sb;
+  p.f.se = se;
+  p.f.E0 = E;
+  p.f.N0 = N;
+  g.B = 1;
+  g.E = B * E;
+  g.N = B * N;
+  g.ordered = &p.f;
+  return dispatch_group_softmax(dtype, g, mode, vec, stream);
+}
+}  // namespace
+
+size_t ts_group_order_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype) {
+  return group_order_rule(B, E, K, N, dtype, false) ? row_sort_plan(B, E, N, nullptr, 0, true).kept_bytes : 0;
+}
+
+size_t ts_group_order_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int backward) {
+  if (ts_group_order_bytes(B, E, K, N, dtype) == 0) return 0;
+  if (backward && !group_order_rule(B, E, K, N, dtype, true)) return 0;
+  const RowSortPlan sp = row_sort_plan(B, E, N, nullptr, 0, true);
+  return group_order_records(B, E, K, dtype, backward != 0) + (backward ? 0 : sp.bytes - sp.kept_bytes);
+}
+
+int ts_group_softmax_ordered(const void *src, const int64_t *index, void *out, int64_t B, int64_t E, int64_t K, int64_t N,
+                             int64_t index_stride_b, int64_t index_stride_e, int dtype, int log_space, double eps,
+                             void *order, size_t order_bytes, void *workspace, size_t workspace_bytes, ts_stream_t stream) {
+  const size_t need = ts_group_order_bytes(B, E, K, N, dtype);
+  if (need == 0) return TS_ERR_UNSUPPORTED;
+  if (!src || !index || !out) return TS_ERR_BAD_ARG;
+  if (!order || order_bytes < need || !aligned16(order) || !workspace || !aligned16(workspace) ||
+      workspace_bytes < ts_group_order_workspace_bytes(B, E, K, N, dtype, 0))
+    return TS_ERR_WORKSPACE;
+  const size_t records = group_order_records(B, E, K, dtype, false);
+  const RowSortPlan sp = row_sort_plan(B, E, N, static_cast<char *>(workspace) + records, workspace_bytes - records, true, order);
+  if (!sp.ok) return TS_ERR_WORKSPACE;
+  return run_group_ordered(src, nullptr, index, out, B, E, K, N, index_stride_b, index_stride_e, dtype,
+                           log_space ? GS_LOG_SOFTMAX : GS_SOFTMAX, eps, sp.p, workspace, records,
+                           static_cast<hipStream_t>(stream));
+}
+
+int ts_group_softmax_ordered_backward(const void *result, const void *grad_out, const int64_t *index, void *grad_in, int64_t B,
+                                      int64_t E, int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e,
+                                      int dtype, int log_space, const void *order, size_t order_bytes, void *workspace,
+                                      size_t workspace_bytes, ts_stream_t stream) {
+  const size_t need = ts_group_order_bytes(B, E, K, N, dtype), scratch = ts_group_order_workspace_bytes(B, E, K, N, dtype, 1);
+  if (need == 0 || scratch == 0) return TS_ERR_UNSUPPORTED;
+  if (!result || !grad_out || !index || !grad_in) return TS_ERR_BAD_ARG;
+  if (!order || order_bytes < need || !aligned16(order) || !workspace || !aligned16(workspace) || workspace_bytes < scratch)
+    return TS_ERR_WORKSPACE;
+  const RowSortPlan sp = row_sort_plan(B, E, N, nullptr, 0, true, const_cast<void *>(order));
+  if (!sp.ok) return TS_ERR_WORKSPACE;
+  return run_group_ordered(result, grad_out, index, grad_in, B, E, K, N, index_stride_b, index_stride_e, dtype,
+                           log_space ? GS_LOG_SOFTMAX_BWD : GS_SOFTMAX_BWD, 0.0, sp.p, workspace, scratch,
+                           static_cast<hipStream_t>(stream));
+}
+
 size_t ts_group_softmax_workspace_bytes(int64_t B, int64_t N, int64_t K, int dtype) {
   if (!valid_dtype(dtype) || B < 0 || N < 0 || K < 0) return 0;
   return group_workspace_bytes(B, N, K, kElemBytes[dtype]);

@@ -73,6 +73,7 @@ enum {
 };
 
 struct BinArgs;
+struct FusedArgs;
 struct FusedReduceArgs;
 
 struct GroupArgs {
@@ -104,6 +105,9 @@ struct GroupArgs {
   const BinArgs *bins = nullptr;  // (host) plan of the buckets
   const FusedReduceArgs *tiles = nullptr;  // (host) std / logsumexp: plan of the one-pass tiles in front of the buckets
   int tiles_force = 0;                     //        ... which run whatever a sample of the index looks like
+  const FusedArgs *ordered = nullptr;  // (host) softmax over entries sorted by group: plan of the tiles; or
+  const FusedArgs *in_order = nullptr;  // (host) the tiles for an index in order alone, and whether a sample of it comes first
+  int in_order_sample = 0;
   const CsrReduceArgs *rows = nullptr;  // (host) std over entries sorted by group: arguments and
   const CsrPlan *rows_plan = nullptr;   //        plan of the segmented reduction
 };
@@ -682,6 +686,11 @@ int launch_group_softmax_m(const GroupArgs &g_in, hipStream_t stream) {
   GroupArgs g = g_in;
   const int64_t n_edges = g.B * g.E;
   if (g.B * g.N >= 0x7FFFFFFFll) return TS_ERR_UNSUPPORTED;
+  if (g.in_order != nullptr) return launch_group_fused<T, VEC, MODE>(g, *g.in_order, false, stream, g.in_order_sample != 0);
+  if (g.ordered != nullptr) {
+    if constexpr (VEC * sizeof(T) == kVecBytes) return launch_group_fused_ordered<T, VEC, MODE>(g, *g.ordered, stream);
+    return TS_ERR_UNSUPPORTED;
+  }
   const RunGrid rg = run_grid(n_edges, g.K / VEC, VEC, VEC * (int)sizeof(T));
   if (!rg.ok) return TS_ERR_UNSUPPORTED;
   // An index that looks sorted goes through the one-pass kernels first; the three passes below then run only

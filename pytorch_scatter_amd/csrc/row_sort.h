@@ -41,7 +41,8 @@ struct RowSortArgs {
   int64_t sb, se;        // element strides of the index over batches and entries
   int64_t B, E, N;
   int64_t n, rows;       // B * E entries, B * N rows
-  int identity;          // an index in order: write the identity to perm (a reader that looks at state[0] does without)
+  int identity;          // an index in order: write the identity to perm (a reader that looks at state[0] does without);
+                         // perm_row is written whenever there is one
   int flat;              // one batch, unit stride: entry e is index[e] (no 64-bit multiplications per entry)
   int rshift, nb;        // rows per bucket (log2), buckets
   int per;               // entries per lane of place: a tile holds per * kRsBlock
@@ -51,8 +52,9 @@ struct RowSortArgs {
   int max_big;           // buckets above that: at most this many ...
   int max_chunks;        // ... in at most this many chunks
   uint32_t nonce;        // tag of the call, never 0
+  const int *gate;       // reads 0: every pass returns at once (null: they run)
   int32_t *state;        // [0] 0: the index is in order, 1: it is not; [1] chunks of large buckets; [2] large buckets;
-                         // [3] the nonce of the latest call that met an index that is not in order
+                         // [3] the nonce of the latest call that met an index that is not in order; [4] the caller's
   uint16_t *off;         // [tiles][pitch] first entry of every bucket among the tile's words; [nb]: how many there are
   int log;               // a tile's words lie at tile << log
   uint32_t *words;       // [tiles << log] a tile's entries by bucket: row in the bucket << kRsLocal | place in the tile
@@ -71,14 +73,17 @@ struct RowSortArgs {
 struct RowSortPlan {
   bool ok;
   RowSortArgs p;
-  size_t bytes;
+  size_t bytes;       // results and scratch
+  size_t kept_bytes;  // the results (state, perm, perm_row, ptr) alone, which come first
 };
 
-// with_rows: perm_row as well
-inline RowSortPlan row_sort_plan(int64_t B, int64_t E, int64_t N, void *ws, size_t ws_bytes, bool with_rows = false) {
+// with_rows: perm_row as well. kept: the results lie there and the scratch alone at ws (bytes - kept_bytes); with ws null
+// the plan describes the results of an earlier call.
+inline RowSortPlan row_sort_plan(int64_t B, int64_t E, int64_t N, void *ws, size_t ws_bytes, bool with_rows = false,
+                                 void *kept = nullptr) {
   RowSortPlan r;
   r.ok = false;
-  r.bytes = 0;
+  r.bytes = r.kept_bytes = 0;
   RowSortArgs &p = r.p;
   if (B < 1 || E < 1 || N < 1 || B > 0x7FFFFFFFll / E || B > 0x7FFFFFFFll / N) return r;
   p.B = B;
@@ -117,15 +122,20 @@ inline RowSortPlan row_sort_plan(int64_t B, int64_t E, int64_t N, void *ws, size
   size_t off = 0;
   auto take = [&](size_t bytes) { const size_t o = off; off += up(bytes); return o; };
   const size_t big_n = p.max_big > 0 ? (size_t)p.n : 0;
-  const size_t o_state = take(16), o_off = take((size_t)p.tiles * p.pitch * 2), o_words = take(((size_t)p.tiles << p.log) * 4);
+  const size_t o_state = take(32);
+  const size_t o_perm = take((size_t)p.n * 4), o_prow = take(with_rows ? (size_t)p.n * 4 : 0), o_ptr = take((size_t)(p.rows + 1) * 8);
+  r.kept_bytes = off;
+  const size_t o_off = take((size_t)p.tiles * p.pitch * 2), o_words = take(((size_t)p.tiles << p.log) * 4);
   const size_t o_big = take((size_t)p.max_big * 16), o_arr = take((size_t)p.max_big * 4), o_cb = take((size_t)p.max_chunks * 4);
   const size_t o_rc = take(((size_t)p.max_big << rs) * 4), o_co = take(((size_t)p.max_chunks << rs) * 4);
   const size_t o_br = take(big_n * 4), o_brr = take(big_n * 2);
-  const size_t o_perm = take((size_t)p.n * 4), o_prow = take(with_rows ? (size_t)p.n * 4 : 0), o_ptr = take((size_t)(p.rows + 1) * 8);
   r.bytes = off;
-  if (ws == nullptr || ws_bytes < off || (reinterpret_cast<uintptr_t>(ws) & 15) != 0) return r;
-  char *base = static_cast<char *>(ws);
-  p.state = reinterpret_cast<int32_t *>(base + o_state);
+  if (ws == nullptr && kept == nullptr) return r;
+  if (ws != nullptr && (ws_bytes < (kept != nullptr ? off - r.kept_bytes : off) || (reinterpret_cast<uintptr_t>(ws) & 15) != 0)) return r;
+  if ((reinterpret_cast<uintptr_t>(kept) & 15) != 0) return r;
+  char *results = static_cast<char *>(kept != nullptr ? kept : ws);
+  char *base = kept == nullptr ? results : static_cast<char *>(ws) - r.kept_bytes;
+  p.state = reinterpret_cast<int32_t *>(results + o_state);
   p.off = reinterpret_cast<uint16_t *>(base + o_off);
   p.words = reinterpret_cast<uint32_t *>(base + o_words);
   p.big = reinterpret_cast<uint32_t *>(base + o_big);
@@ -135,9 +145,9 @@ inline RowSortPlan row_sort_plan(int64_t B, int64_t E, int64_t N, void *ws, size
   p.chunk_off = reinterpret_cast<uint32_t *>(base + o_co);
   p.by_row = reinterpret_cast<uint32_t *>(base + o_br);
   p.by_row_row = reinterpret_cast<uint16_t *>(base + o_brr);
-  p.perm = reinterpret_cast<int32_t *>(base + o_perm);
-  p.perm_row = with_rows ? reinterpret_cast<int32_t *>(base + o_prow) : nullptr;
-  p.ptr = reinterpret_cast<int64_t *>(base + o_ptr);
+  p.perm = reinterpret_cast<int32_t *>(results + o_perm);
+  p.perm_row = with_rows ? reinterpret_cast<int32_t *>(results + o_prow) : nullptr;
+  p.ptr = reinterpret_cast<int64_t *>(results + o_ptr);
   r.ok = true;
   return r;
 }
@@ -240,8 +250,8 @@ template <int BLOCK> __device__ __forceinline__ uint32_t rs_scan_lds(uint32_t *s
   return total;
 }
 
-// A tile of entries by bucket. A tile whose rows do not descend writes the row pointers that its entries mark as well: they
-// stand if no tile has seen a descent, else the sorting passes write all of them again.
+// A tile of entries by bucket. A tile whose rows do not descend writes the row pointers that its entries mark and perm_row
+// as well: they stand if no tile has seen a descent, else the sorting passes write all of them again.
 template <int FLAT, int PER>
 static __global__ __launch_bounds__(kRsBlock) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void rs_place_kernel(RowSortArgs p) {
@@ -253,6 +263,7 @@ void rs_place_kernel(RowSortArgs p) {
   __shared__ GapList s_gaps;
   __shared__ int s_desc;
   const int64_t lo = (int64_t)blockIdx.x * TILE;
+  if (p.gate != nullptr && *p.gate == 0) return;
   const int lane = threadIdx.x & (kWave - 1);
   int32_t node[PER];
   uint32_t rank[PER];
@@ -323,8 +334,9 @@ void rs_place_kernel(RowSortArgs p) {
     const bool live = be < p.n;
     const int32_t prev = before(j);
     const int64_t top = live ? (int64_t)node[j] : -1, bot = live ? (be == 0 ? 0 : (int64_t)prev + 1) : 0;
+    if (live && p.perm_row != nullptr) p.perm_row[be] = node[j];
     gap_rows(p.ptr, bot, top, be, s_gaps);
-    gap_rows(p.ptr, top + 1, live && be == p.n - 1 ? p.rows : top, p.n, s_gaps);
+    if (lo + TILE >= p.n) gap_rows(p.ptr, top + 1, live && be == p.n - 1 ? p.rows : top, p.n, s_gaps);
   }
   __syncthreads();
   gap_rows_finish(p.ptr, s_gaps);
@@ -461,15 +473,12 @@ void rs_sort_kernel(RowSortArgs p) {
   __shared__ uint32_t s_wave[BLOCK / kWave];
   static_assert(CAP * 4 + sizeof(RsRuns<BLOCK>) + 256 + (4 << kRsMaxShift) <= 160 * 1024, "a workgroup's LDS: 160 KB");
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  if (p.gate != nullptr && *p.gate == 0) return;
   const bool unsorted = p.state[3] == (int32_t)p.nonce;
   if (blockIdx.x == 0 && tid == 0) p.state[0] = unsorted ? 1 : 0;
   if (!unsorted) {
-    if (p.identity) {
-      for (int64_t i = (int64_t)blockIdx.x * BLOCK + tid; i < p.n; i += (int64_t)gridDim.x * BLOCK) {
-        p.perm[i] = (int32_t)i;
-        if (p.perm_row != nullptr) p.perm_row[i] = rs_node(p, i);
-      }
-    }
+    if (p.identity)
+      for (int64_t i = (int64_t)blockIdx.x * BLOCK + tid; i < p.n; i += (int64_t)gridDim.x * BLOCK) p.perm[i] = (int32_t)i;
     return;
   }
   // neighbouring buckets, whose runs share lines, on one of the eight dies (workgroups go to them in turn)
@@ -558,6 +567,7 @@ void rs_chunk_kernel(RowSortArgs p) {
   __shared__ uint32_t s_wave[BLOCK / kWave];
   __shared__ int s_last;
   const int tid = threadIdx.x, chunk = (int)blockIdx.x;
+  if (p.gate != nullptr && *p.gate == 0) return;
   if (p.state[0] == 0 || chunk >= p.state[1]) return;
   const int big = p.chunk_big[chunk];
   const uint32_t *rec = p.big + 4 * (size_t)big;
@@ -610,7 +620,7 @@ void rs_chunk_kernel(RowSortArgs p) {
 // the chunks of large buckets, each in order of its rows: every entry to its place among its row's
 constexpr int kRsPiece = 8;  // entries per lane; a chunk is 4 or 8 pieces
 static __global__ __launch_bounds__(kBlock) void rs_place_chunks_kernel(RowSortArgs p) {
-  if (p.state[0] == 0) return;
+  if ((p.gate != nullptr && *p.gate == 0) || p.state[0] == 0) return;
   const int pieces = p.cap / (kRsPiece * kBlock), n = p.state[1] * pieces;
   for (int q = (int)blockIdx.x; q < n; q += (int)gridDim.x) {
     const int chunk = q / pieces, i0 = (q - chunk * pieces) * (kRsPiece * kBlock) + (int)threadIdx.x;
@@ -727,8 +737,9 @@ template <int BLOCK> inline void launch_rs_sort(const RowSortArgs &p, hipStream_
 
 // nonce: tag of the call (any value; a repeated one only costs an index in order its short way)
 inline int launch_row_sort(const RowSortArgs &args, const int64_t *index, int64_t sb, int64_t se, bool identity,
-                           uint64_t nonce, hipStream_t stream) {
+                           uint64_t nonce, hipStream_t stream, const int *gate = nullptr) {
   RowSortArgs p = args;
+  p.gate = gate;
   p.identity = identity ? 1 : 0;
   p.index = index;
   p.sb = sb;

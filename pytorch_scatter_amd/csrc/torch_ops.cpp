@@ -128,6 +128,8 @@ void maybe_check_scatter_status(const Tensor &ws, int64_t B, int64_t E, int64_t 
                              "the bounded wait for the tiles before it ran out");
 }
 
+bool on_16_bytes(const Tensor &t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+
 Tensor workspace(size_t bytes, const Tensor &like) {
   return at::empty({static_cast<int64_t>(bytes > 0 ? bytes : 1)}, like.options().dtype(at::kByte));
 }
@@ -848,23 +850,36 @@ struct GroupSoftmaxFn : public torch::autograd::Function<GroupSoftmaxFn> {
     c10::DeviceGuard guard(src.device());
     src = src.contiguous();
     const GroupLayout l = group_layout(src, index, dim);
-    Tensor out = at::empty_like(src);
-    // the workspace that opens every route: three passes, buckets of groups, one-pass tiles
-    Tensor ws = workspace(ts_group_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src)), src);
-    check_status(ts_group_softmax(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(), l.B, l.E, l.K, N, l.sb,
-                                  l.se, dtype_code(src), log_space ? 1 : 0, eps, ws.data_ptr(),
-                                  static_cast<size_t>(ws.numel()), stream_of(src)),
-                 "scatter_softmax");
+    Tensor out = at::empty_like(src), order;
+    const size_t order_bytes = on_16_bytes(src) ? ts_group_order_bytes(l.B, l.E, l.K, N, dtype_code(src)) : 0;
+    if (order_bytes > 0) {
+      // the entries sorted by group; the backward pass takes the order of this call
+      order = workspace(order_bytes, src);
+      const size_t ws_bytes = ts_group_order_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src), 0);
+      Tensor ws = workspace(ws_bytes, src);
+      check_status(ts_group_softmax_ordered(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(), l.B, l.E, l.K, N,
+                                            l.sb, l.se, dtype_code(src), log_space ? 1 : 0, eps, order.data_ptr(),
+                                            order_bytes, ws.data_ptr(), ws_bytes, stream_of(src)),
+                   "scatter_softmax");
+      if (!src.requires_grad() || ts_group_order_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src), 1) == 0) order = Tensor();
+    } else {
+      // the workspace that opens every other route: three passes, buckets of groups, one-pass tiles
+      Tensor ws = workspace(ts_group_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src)), src);
+      check_status(ts_group_softmax(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(), l.B, l.E, l.K, N, l.sb,
+                                    l.se, dtype_code(src), log_space ? 1 : 0, eps, ws.data_ptr(),
+                                    static_cast<size_t>(ws.numel()), stream_of(src)),
+                   "scatter_softmax");
+    }
     ctx->saved_data["dim"] = dim;
     ctx->saved_data["N"] = N;
     ctx->saved_data["log"] = log_space;
-    ctx->save_for_backward({out, index});
+    ctx->save_for_backward({out, index, order});
     return {out};
   }
 
   static variable_list backward(AutogradContext *ctx, variable_list grad_outs) {
     auto saved = ctx->get_saved_variables();
-    Tensor out = saved[0], index = saved[1];
+    Tensor out = saved[0], index = saved[1], order = saved[2];
     Tensor grad_out = grad_outs[0].contiguous();
     c10::DeviceGuard guard(out.device());
     const int64_t dim = ctx->saved_data["dim"].toInt();
@@ -872,6 +887,17 @@ struct GroupSoftmaxFn : public torch::autograd::Function<GroupSoftmaxFn> {
     const bool log_space = ctx->saved_data["log"].toBool();
     const GroupLayout l = group_layout(out, index, dim);
     Tensor grad_in = at::empty_like(out);
+    if (order.defined() && on_16_bytes(out) && on_16_bytes(grad_out)) {
+      const size_t ws_bytes = ts_group_order_workspace_bytes(l.B, l.E, l.K, N, dtype_code(out), 1);
+      Tensor ws = workspace(ws_bytes, out);
+      check_status(ts_group_softmax_ordered_backward(out.data_ptr(), grad_out.data_ptr(), index.data_ptr<int64_t>(),
+                                                     grad_in.data_ptr(), l.B, l.E, l.K, N, l.sb, l.se, dtype_code(out),
+                                                     log_space ? 1 : 0, order.data_ptr(),
+                                                     static_cast<size_t>(order.numel()), ws.data_ptr(), ws_bytes,
+                                                     stream_of(out)),
+                   "scatter_softmax backward");
+      return {grad_in, Variable(), Variable(), Variable(), Variable(), Variable()};
+    }
     Tensor ws = workspace(ts_group_workspace_bytes(l.B, l.E, l.K, N, dtype_code(out)), out);
     check_status(ts_group_softmax_backward(out.data_ptr(), grad_out.data_ptr(), index.data_ptr<int64_t>(),
                                            grad_in.data_ptr(), l.B, l.E, l.K, N, l.sb, l.se, dtype_code(out),
