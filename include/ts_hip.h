@@ -297,6 +297,16 @@ int ts_scatter_count(const int64_t *index, int32_t *count, int64_t B, int64_t E,
                      int64_t N, int64_t index_stride_b, int64_t index_stride_e,
                      ts_stream_t stream);
 
+/* Sum, mean (reduce TS_MEAN: divided by the entries per row), min or max of a small input with one index per row, in one
+ * launch: float types (min / max: of up to 32 bits), up to 8192 entries a batch and 2^18 values; ts_scatter_small_applies()
+ * says whether a call fits (else TS_ERR_UNSUPPORTED). out is written whole; with out_given its content takes part, as in
+ * ts_scatter. count (sum, mean): [B, N] in the element type, the divisor of the mean (at least 1), or null. arg_out (min,
+ * max): [B, N, K], as ts_scatter leaves it. */
+int ts_scatter_small_applies(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce);
+int ts_scatter_small(const void *src, const int64_t *index, void *out, void *count, int64_t *arg_out, int64_t B, int64_t E,
+                     int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype, int reduce, int out_given,
+                     ts_stream_t stream);
+
 /* The same count with scratch memory (ts_scatter_count_workspace_bytes; 0 = no use for it): from 2 M entries on an
  * unsorted index is binned by bucket of output rows (8 bytes per entry) and counted in LDS, as
  * ts_scatter_with_workspace does for the sum of one value per entry. Same result. */

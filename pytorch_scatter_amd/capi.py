@@ -28,6 +28,7 @@ EXPORTS = (
     "ts_segment_mean_coo_backward",
     "ts_scatter", "ts_scatter_workspace_bytes", "ts_scatter_workspace_zero_bytes", "ts_scatter_with_workspace", "ts_scatter_count", "ts_scatter_count_workspace_bytes", "ts_scatter_count_with_workspace", "ts_scatter_sum_count_workspace_bytes", "ts_scatter_sum_count_with_workspace", "ts_divide_by_count", "ts_arg_backward",
     "ts_arg_backward_rows_workspace_bytes", "ts_arg_backward_rows",
+    "ts_scatter_small_applies", "ts_scatter_small",
     "ts_group_softmax_workspace_bytes", "ts_group_softmax", "ts_group_softmax_backward",
     "ts_group_order_bytes", "ts_group_order_workspace_bytes", "ts_group_softmax_ordered", "ts_group_softmax_ordered_backward",
     "ts_group_logsumexp", "ts_group_logsumexp_backward",
@@ -263,6 +264,18 @@ def scatter_sum_count_with_workspace(src, index, out, count, B, E, K, N, sb, se,
                                                      _p(ws) if nbytes else None, ctypes.c_size_t(nbytes), _stream(out)))
     _check_scatter_status(ws, L.ts_scatter_workspace_bytes(_i(B), _i(E), _i(K), _i(N), DTYPE[out.dtype], SUM), B, N, K)
     return nbytes
+
+
+def scatter_small_applies(B, E, K, N, dtype, reduce: int) -> bool:
+    return bool(lib().ts_scatter_small_applies(_i(B), _i(E), _i(K), _i(N), DTYPE[dtype], reduce))
+
+
+def scatter_small(src, index, out, count, arg, B, E, K, N, sb, se, reduce: int, out_given: bool):
+    """Scatter of a small input in one launch (ts_scatter_small); count: None or [B, N] in the element type."""
+    _dev(src, index, out)
+    with torch.cuda.device(out.device):
+        _check(lib().ts_scatter_small(_p(src), _p(index), _p(out), _p(count), _p(arg), _i(B), _i(E), _i(K), _i(N), _i(sb),
+                                      _i(se), DTYPE[out.dtype], reduce, 1 if out_given else 0, _stream(out)))
 
 
 def divide_by_count(out, count, B, N, K):

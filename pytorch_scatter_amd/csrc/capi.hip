@@ -16,6 +16,7 @@
 #include "group_softmax.h"
 #include "index_format.h"
 #include "row_sort.h"
+#include "scatter_small.h"
 
 using namespace ts;
 
@@ -795,6 +796,60 @@ int ts_scatter_with_workspace(const void *src, const int64_t *index, void *out, 
                               size_t workspace_bytes, ts_stream_t stream) {
   return scatter_ws_impl(src, index, out, arg_out, B, E, K, N, index_stride_b, index_stride_e, index_stride_k, dtype, reduce,
                          out_given, workspace, workspace_bytes, stream, nullptr, nullptr);
+}
+
+}  // extern "C"
+namespace {
+// TS_SCATTER_SMALL (tuning aid): 0 never, 2 at any size that the kernel holds
+SmallPlan scatter_small_plan(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce, bool aligned) {
+  const int mode = env_int("TS_SCATTER_SMALL", 1);
+  if (mode == 0 || !valid_dtype(dtype) || !is_float_dtype(dtype) || !sizes_ok(B, N, E, K) ||
+      (reduce != TS_SUM && reduce != TS_MEAN && reduce != TS_MIN && reduce != TS_MAX))
+    return small_plan(0, 0, 0, 0, 4, 1, TS_SUM, false);
+  const int es = kElemBytes[dtype], full = kVecBytes / es;
+  return small_plan(B, E, K, N, es, K % full == 0 && aligned ? full : 1, reduce, mode == 2);
+}
+template <typename T> int run_scatter_small(const SmallArgs &a, const SmallPlan &p, bool aligned, int reduce, hipStream_t s) {
+  constexpr int kFull = kVecBytes / (int)sizeof(T);
+  if (reduce == TS_MEAN) reduce = TS_SUM;
+  return a.K % kFull == 0 && aligned ? launch_scatter_small<T, kFull>(a, p, reduce, s) : launch_scatter_small<T, 1>(a, p, reduce, s);
+}
+}  // namespace
+extern "C" {
+
+int ts_scatter_small_applies(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce) {
+  if (E > kSmallPer * kSmallBlock) return 0;  // (most calls end here: nothing is read from the environment)
+  return scatter_small_plan(B, E, K, N, dtype, reduce, true).ok && scatter_small_plan(B, E, K, N, dtype, reduce, false).ok ? 1 : 0;
+}
+
+int ts_scatter_small(const void *src, const int64_t *index, void *out, void *count, int64_t *arg_out, int64_t B, int64_t E,
+                     int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype, int reduce, int out_given,
+                     ts_stream_t stream) {
+  if (!ts_scatter_small_applies(B, E, K, N, dtype, reduce)) return TS_ERR_UNSUPPORTED;
+  if (!src || !index || !out || ((reduce == TS_MIN || reduce == TS_MAX) && !arg_out)) return TS_ERR_BAD_ARG;
+  const bool al = aligned16(src);
+  const SmallPlan p = scatter_small_plan(B, E, K, N, dtype, reduce, al);
+  SmallArgs a = {};
+  a.src = src;
+  a.index = index;
+  a.out = out;
+  a.count = count;
+  a.arg_out = arg_out;
+  a.sb = index_stride_b;
+  a.se = index_stride_e;
+  a.B = B;
+  a.E = E;
+  a.K = K;
+  a.N = N;
+  a.mean = reduce == TS_MEAN ? 1 : 0;
+  a.out_given = out_given ? 1 : 0;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (dtype) {
+  case TS_F32: return run_scatter_small<float>(a, p, al, reduce, s);
+  case TS_F64: return run_scatter_small<double>(a, p, al, reduce, s);
+  case TS_F16: return run_scatter_small<f16_t>(a, p, al, reduce, s);
+  default: return run_scatter_small<bf16_t>(a, p, al, reduce, s);
+  }
 }
 
 size_t ts_scatter_count_workspace_bytes(int64_t B, int64_t E, int64_t N) {

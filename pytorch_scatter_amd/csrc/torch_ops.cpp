@@ -192,8 +192,15 @@ BatchedIndex batched_index(const Tensor &idx) {
 // mean_count (sum only): if the call is a sum under one index per row, the entries of every output row are counted
 // in the same call (ts_scatter_sum_count_with_workspace) and the int32 counts [B * N]
 // are left here; else it stays undefined
+// small_mean (sum only): a small call divides by the count in the launch that adds; *divided then reads true and, with
+// counted, *small_count holds the divisor in the element type [B * N]
+struct SmallMean {
+  bool counted = false, divided = false;
+  Tensor count;
+};
 std::tuple<Tensor, OptTensor> scatter_hip(Tensor src, Tensor index, int64_t dim, OptTensor optional_out,
-                                          OptInt dim_size, int reduce, Tensor *mean_count = nullptr) {
+                                          OptInt dim_size, int reduce, Tensor *mean_count = nullptr,
+                                          SmallMean *small_mean = nullptr) {
   check_device(src, "src");
   check_device(index, "index");
   if (optional_out.has_value()) check_device(optional_out.value(), "out");
@@ -259,6 +266,19 @@ std::tuple<Tensor, OptTensor> scatter_hip(Tensor src, Tensor index, int64_t dim,
     sb = E * K;
     se = K;
     sk = 1;
+  }
+  const int small_reduce = small_mean != nullptr ? TS_MEAN : reduce;
+  if (sk.value() == 0 && (mean_count == nullptr || small_mean != nullptr) &&
+      ts_scatter_small_applies(B, E, K, N, dtype_code(src), small_reduce)) {
+    const bool mean = small_mean != nullptr;
+    if (mean && small_mean->counted) small_mean->count = at::empty({B * N}, src.options());
+    check_status(ts_scatter_small(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(),
+                                  mean && small_mean->counted ? small_mean->count.data_ptr() : nullptr,
+                                  minmax ? arg_out.value().data_ptr<int64_t>() : nullptr, B, E, K, N, sb.value(), se,
+                                  dtype_code(src), small_reduce, optional_out.has_value() ? 1 : 0, stream_of(src)),
+                 "scatter");
+    if (mean) small_mean->divided = true;
+    return std::make_tuple(out, arg_out);
   }
   if (mean_count != nullptr && reduce == TS_SUM && sk.value() == 0 && B * N < 0x7FFFFFFFll) {
     const size_t cs_bytes = ts_scatter_sum_count_workspace_bytes(B, E, K, N, dtype_code(src));
@@ -611,8 +631,13 @@ template <int REDUCE> struct ScatterFn : public torch::autograd::Function<Scatte
     Variable old_index = index;
     index = broadcast(index, src, dim);
     Tensor fused_count;  // mean of single values: counted together with the sum
+    // mean with one index per row (a 1-D index along dim 0, or an index shaped like src's leading dims)
+    bool per_row = REDUCE == TS_MEAN && old_index.dim() == dim + 1 && src.numel() > 0 && old_index.size(dim) == src.size(dim);
+    for (int64_t i = 0; per_row && i < dim; i++) per_row = old_index.size(i) == src.size(i);
+    SmallMean small;
+    small.counted = per_row && src.requires_grad();  // for the backward pass
     auto result = scatter_hip(src, index, dim, optional_out, dim_size, REDUCE == TS_MEAN ? TS_SUM : REDUCE,
-                              REDUCE == TS_MEAN ? &fused_count : nullptr);
+                              REDUCE == TS_MEAN ? &fused_count : nullptr, per_row ? &small : nullptr);
     Variable out = std::get<0>(result);
     if (optional_out.has_value()) ctx->mark_dirty({optional_out.value()});
     if (REDUCE == TS_SUM) {
@@ -624,12 +649,17 @@ template <int REDUCE> struct ScatterFn : public torch::autograd::Function<Scatte
       return {out};
     }
     if (REDUCE == TS_MEAN) {
-      // count over the index as given (csrc/scatter.cpp:131-141). One index per row (a 1-D index along
-      // dim 0, or an index shaped like src's leading dims): the entries are counted straight from the
-      // index (no tensor of ones; exact int32 counts) and one kernel clamps, casts and divides.
-      bool per_row = old_index.dim() == dim + 1 && src.numel() > 0 && out.numel() > 0 && old_index.size(dim) == src.size(dim);
-      for (int64_t i = 0; per_row && i < dim; i++) per_row = old_index.size(i) == src.size(i);
-      if (per_row) {
+      if (small.divided) {
+        if (small.counted) {
+          auto count_sizes = out.sizes().vec();
+          count_sizes.resize(dim + 1);
+          ctx->save_for_backward({index, broadcast(small.count.view(count_sizes), out, dim)});
+        }
+        return {out};
+      }
+      // count over the index as given (csrc/scatter.cpp:131-141). One index per row: the entries are counted straight
+      // from the index (no tensor of ones; exact int32 counts) and one kernel clamps, casts and divides.
+      if (per_row && out.numel() > 0) {
         const int64_t B = prod(src.sizes(), 0, dim), E = src.size(dim), N = out.size(dim);
         const int64_t K = prod(src.sizes(), dim + 1, src.dim());
         const BatchedIndex bi = batched_index(old_index);
