@@ -888,7 +888,7 @@ int ts_scatter_count_with_workspace(const int64_t *index, int32_t *count, int64_
     a.precheck = 1;
     a.lds_cache = env_int("TS_SCATTER_LDS", 1);
     a.lds_epb = env_int("TS_SCATTER_EPB", 0);
-    bool binned = false, three_way = false;
+    bool binned = false, three_way = false, table_launched = false;
     // A large count under an unsorted index, given scratch: the entries are binned by bucket of output rows like a sum
     // of one value per entry (bin_plan_payload; the "value" of an entry is 1) instead of one device atomic per entry
     // that misses the table. A sample of the index decides; the kernels below then run only for an index that looks sorted.
@@ -900,7 +900,14 @@ int ts_scatter_count_with_workspace(const int64_t *index, int32_t *count, int64_
         // kernel below), even (the buckets); without the table kernel or the sample only the first and the last
         three_way = a.lds_cache == 1 && sum_table_by_size(B, E, 1, N, 4) && B * E >= 2 * kBinBlock &&
                     !getenv("TS_BIN_NO_SAMPLE");
-        launch_binned_add<int32_t>(a, bp.p, s, three_way);
+        TableCall table;
+        if (three_way && value_tiles_take(bp.p, B * E)) {
+          table.tn_mask = kLdsAccRows - 1;
+          table.epb = per_cu_chunk_edges(a.lds_epb, B * E, sum_table_min_chunk(1, 4), 131072);
+          table.grid = (unsigned)((B * E + table.epb - 1) / table.epb);
+        }
+        launch_binned_add<int32_t>(a, bp.p, s, three_way, false, table);
+        table_launched = table.grid != 0;
         a.skip_flag = bp.p.unsorted;
         binned = true;
       }
@@ -910,7 +917,7 @@ int ts_scatter_count_with_workspace(const int64_t *index, int32_t *count, int64_
     const bool contended = a.lds_cache == 2 || (a.lds_cache == 1 && sum_table_by_size(B, E, 1, N, 4));
     if (binned) {
       // behind the buckets: the table kernel for a skewed index (flag 2), the run kernel for a sorted one (flag 0)
-      if (three_way) {
+      if (three_way && !table_launched) {
         ScatterArgs t = a;
         t.skip_want = 2;
         const int64_t epb = per_cu_chunk_edges(a.lds_epb, B * E, sum_table_min_chunk(1, 4), 131072);

@@ -1451,14 +1451,9 @@ template <typename L> __device__ __forceinline__ void lds_slot_mul(L *slot, L v)
 // through scatter_atomic_kernel); here a row's entries meet in LDS and memory sees one factor per row and workgroup.
 // COUNT = true (sums): the entries of every output row are counted as well, into the zeroed int32 array a.count_out
 // (scatter mean), in a table of their own beside the sums; the lane that holds an entry's first column counts it.
-template <typename T, bool MUL = false, bool COUNT = false>
-__global__ __launch_bounds__(kLdsAddBlock) void scatter_add_lds_kernel(ScatterArgs a, int tn_mask, int64_t epb) {
+template <typename T, bool MUL, bool COUNT>
+__device__ __forceinline__ void scatter_add_lds_body(const ScatterArgs &a, int tn_mask, int64_t epb) {
   constexpr int U = 4;
-  if (a.skip_flag != nullptr && a.skip_want >= 0) {
-    if (*a.skip_flag != a.skip_want) return;
-  } else if (a.skip_flag != nullptr && (*a.skip_flag != 0) != (a.skip_inverse != 0)) {
-    return;
-  }
   // double slots for the floating types: ds_add_f32 loses its rate when many lanes meet on one address (a hub, or a
   // sorted index whose neighbouring entries share a row), ds_add_f64 does not (Zipf(1.2) index, K = 8: 391 -> 263 us;
   // sorted: 476 -> 177 us). Integers keep their own width (their sums wrap, which a double cannot follow).
@@ -1560,6 +1555,15 @@ __global__ __launch_bounds__(kLdsAddBlock) void scatter_add_lds_kernel(ScatterAr
     const int row = i / K;
     table_add_out<T>(out + (int64_t)s_tags[row] * a.K + (i - row * K), from_acc<T>((typename Acc<T>::type)v), out, out_end);
   }
+}
+template <typename T, bool MUL = false, bool COUNT = false>
+__global__ __launch_bounds__(kLdsAddBlock) void scatter_add_lds_kernel(ScatterArgs a, int tn_mask, int64_t epb) {
+  if (a.skip_flag != nullptr && a.skip_want >= 0) {
+    if (*a.skip_flag != a.skip_want) return;
+  } else if (a.skip_flag != nullptr && (*a.skip_flag != 0) != (a.skip_inverse != 0)) {
+    return;
+  }
+  scatter_add_lds_body<T, MUL, COUNT>(a, tn_mask, epb);
 }
 
 template <typename T, bool IS_MAX>
@@ -1788,6 +1792,15 @@ __global__ __launch_bounds__(kBlock) void fill_sample_kernel(T *p, int64_t n, T 
     if (threadIdx.x == 0) *flag = s_desc * 64 >= kBinBlock ? 1 : 0;
   }
 }
+// The same for the sample with three answers (bin_sample_skew), which the first workgroup takes while the others fill: 3 M
+// entries of three floats, 5.9 us in place of 2.5 and 5.4.
+template <typename T>
+__global__ __launch_bounds__(kBinBlock) void fill_skew_sample_kernel(T *p, int64_t n, T value, ScatterArgs a, int *flag, int quarters,
+                                                                     unsigned long long *totals, int nb) {
+  if (blockIdx.x == 0) return bin_sample_skew(a, flag, quarters, totals, nb);
+  const int64_t step = (int64_t)(gridDim.x - 1) * kBinBlock;
+  for (int64_t i = (int64_t)(blockIdx.x - 1) * kBinBlock + threadIdx.x; i < n; i += step) p[i] = value;
+}
 // out[out == init] = 0 (csrc/cuda/scatter_cuda.cu:126-127)
 template <typename T>
 __global__ __launch_bounds__(kBlock) void mask_init_kernel(T *p, int64_t n, T init) {
@@ -1980,6 +1993,7 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
       count_here = a.count_out != nullptr && a.count_done != nullptr && use_lds && !sampled && !three_way && !payload &&
                    a.lds_cache != 2 && !a.bin_any_size;
     }
+    const bool fill_samples = payload && three_way && !a.out_given;
     if (count_here) {
       const int64_t n_clear = (a.out_given ? 0 : n_out) + a.B * a.N;
       hipLaunchKernelGGL(fill_out_count_kernel<T>, dim3(grid_for(n_clear)), dim3(kBlock), 0, stream, out,
@@ -1988,12 +2002,19 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
       if (sampled)
         hipLaunchKernelGGL(fill_sample_kernel<T>, dim3(g_out), dim3(kBlock), 0, stream, out, n_out, small_const<T>(0),
                            a, a.order_ws);
+      else if (fill_samples)
+        hipLaunchKernelGGL(fill_skew_sample_kernel<T>, dim3(1 + (g_out + 3) / 4), dim3(kBinBlock), 0, stream, out, n_out,
+                           small_const<T>(0), a, bp.p.unsorted, bin_skew_quarters(bp.p), bp.p.totals, bp.p.nb);
       else
         hipLaunchKernelGGL(fill_kernel<T>, dim3(g_out), dim3(kBlock), 0, stream, out, n_out,
                            small_const<T>(reduce == TS_MUL ? 1 : 0));
     } else if (sampled) {
       hipLaunchKernelGGL(bin_sample_kernel, dim3(1), dim3(kBinBlock), 0, stream, a, a.order_ws);
     }
+    const int64_t table_epb = per_cu_chunk_edges(a.lds_epb, n_edges, sum_table_min_chunk(a.K, (int)sizeof(T)),
+                                                 131072 / a.K > 2048 ? 131072 / a.K : 2048);
+    const unsigned table_grid = (unsigned)((n_edges + table_epb - 1) / table_epb);
+    bool table_launched = false;
     if constexpr (sizeof(T) == 4) {
       if (payload) {
         ts_note_scatter_route(TS_ROUTE_SUM_VALUE_BUCKETS);
@@ -2001,7 +2022,15 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
           bp.p.count_out = a.count_out;
           *a.count_flag = bp.p.unsorted;
         }
-        launch_binned_add<T>(a, bp.p, stream, three_way);
+        TableCall table;
+        if (three_way && value_tiles_take(bp.p, n_edges) && (bp.p.count_out == nullptr || a.count_done != nullptr)) {
+          table.tn_mask = tn - 1;
+          table.epb = table_epb;
+          table.grid = table_grid;
+          table_launched = true;
+          if (bp.p.count_out != nullptr) *a.count_done = 2;
+        }
+        launch_binned_add<T>(a, bp.p, stream, three_way, fill_samples, table);
         a.skip_flag = bp.p.unsorted;
       }
     }
@@ -2014,7 +2043,7 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
                       __is_same(T, int32_t) || __is_same(T, int64_t)) {
           // many entries per output slot: reduce in LDS first (see scatter_add_lds_kernel)
           // (sizes: sum_table_by_size)
-          if (use_lds) {
+          if (use_lds && !table_launched) {
             // The table is for an index in no particular order. One that is sorted does better through the run
             // kernel below (9 M entries of the graph of C3, sorted: K = 8 343 against 156 us, K = 4 152 / 96,
             // K = 1 60 / 44; shuffled: 448 / 463), so with a word of scratch a sample of the index decides on the
@@ -2027,24 +2056,22 @@ int launch_scatter_v(const ScatterArgs &args, int reduce, hipStream_t stream) {
               a.skip_flag = a.order_ws;
             }
             if (three_way) t.skip_want = 2;  // (skip_flag is the buckets' flag: 2 = unsorted and skewed)
-            const int64_t epb = per_cu_chunk_edges(a.lds_epb, n_edges, sum_table_min_chunk(a.K, (int)sizeof(T)),
-                                                   131072 / a.K > 2048 ? 131072 / a.K : 2048);
             if (!payload) ts_note_scatter_route(sampled ? TS_ROUTE_SUM_TABLE_OR_RUNS : TS_ROUTE_SUM_TABLE);
             if (count_here) {
-              hipLaunchKernelGGL((scatter_add_lds_kernel<T, false, true>), dim3((unsigned)((n_edges + epb - 1) / epb)),
-                                 dim3(kLdsAddBlock), 0, stream, t, tn - 1, epb);
+              hipLaunchKernelGGL((scatter_add_lds_kernel<T, false, true>), dim3(table_grid),
+                                 dim3(kLdsAddBlock), 0, stream, t, tn - 1, table_epb);
               *a.count_done = 1;
               return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
             }
             // behind value buckets that count as well: the table kernel, which takes a skewed index from them, counts too
             // (*count_done = 2 tells the caller, which then has no table of counts to launch for that verdict)
             if (three_way && bp.p.count_out != nullptr && a.count_done != nullptr) {
-              hipLaunchKernelGGL((scatter_add_lds_kernel<T, false, true>), dim3((unsigned)((n_edges + epb - 1) / epb)),
-                                 dim3(kLdsAddBlock), 0, stream, t, tn - 1, epb);
+              hipLaunchKernelGGL((scatter_add_lds_kernel<T, false, true>), dim3(table_grid),
+                                 dim3(kLdsAddBlock), 0, stream, t, tn - 1, table_epb);
               *a.count_done = 2;
             } else {
-              hipLaunchKernelGGL(scatter_add_lds_kernel<T>, dim3((unsigned)((n_edges + epb - 1) / epb)),
-                                 dim3(kLdsAddBlock), 0, stream, t, tn - 1, epb);
+              hipLaunchKernelGGL(scatter_add_lds_kernel<T>, dim3(table_grid),
+                                 dim3(kLdsAddBlock), 0, stream, t, tn - 1, table_epb);
             }
             if (!sampled && !three_way) return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
           }

@@ -29,6 +29,17 @@ constexpr int kBinPlaceBlock = 1024;   // (measured slower: 256 lanes x 4 batche
 // record of K + 1 32-bit words (the values, then the row in the bucket)
 constexpr int kBinPayloadCols = 4;
 
+// Slot type of the table: floating types accumulate in double. ds_add_f64 and the integer adds keep their rate
+// when many lanes meet on one address (a hub row); ds_add_f32 does not (measured: 10 M entries of a Zipf(1.2)
+// index, K = 32: 2.2 ms with fp32 slots, 0.44 ms with int32 or double slots).
+template <typename T> struct BinSlot { typedef double type; };
+template <> struct BinSlot<int32_t> { typedef int32_t type; };
+template <> struct BinSlot<int64_t> { typedef int64_t type; };
+
+}  // namespace ts
+#include "value_tiles.h"
+namespace ts {
+
 struct BinArgs {
   int rshift;              // log2 of the rows per bucket
   int chunk;               // entries per reducing workgroup
@@ -62,6 +73,7 @@ struct BinArgs {
   int sort_tile = 6144;    // entries per workgroup of the place pass that sorts its tile in LDS (records: fewer)
   int32_t *count_out = nullptr;  // sums: the adding pass also counts the entries of every output row into this
                            // [B * N] array (the divisor of a mean, from the same words)
+  ValueTiles tiles;        // sums of up to 8 M entries: the passes of value_tiles.h in place of these
 };
 
 struct BinPlan {
@@ -88,9 +100,11 @@ inline BinPlan bin_plan_payload(int64_t B, int64_t E, int64_t K, int64_t N, int 
   // from 2 M entries: an even index gains from there on (74 against 106 us; 2.3 M entries of a graph in random order
   // 85 against 125 us); a skewed one, which the sample hands to the table kernel, pays about 15 us for the launches
   // that return at once (2.3 M entries: 51 against 36 us)
-  // (several values per entry: the place pass grows with them, the atomics they replace do not -- three values from
-  // 3 M entries, four from 4 M: 2.2 M / 3 M entries of four floats 121 / 149 us against 115 / 155 us)
-  if (!any_size && n_edges < (K <= 2 ? (int64_t)1 << 21 : K == 3 ? (int64_t)3 << 20 : (int64_t)1 << 22)) return r;
+  // (several values per entry: the launches in front cost the more of an index in order, which takes the table below these
+  // sizes, the more values it has -- 3 M entries of three floats even 178 -> 50, in order 63 to 75 -> 70 to 80 us; 2 M 118 -> 38,
+  // in order 25 to 47 -> 47 to 55; 3 M of four floats even 157 -> 71, in order 37 to 55 -> 42 to 59: three values from 2.6 M
+  // entries, four from 4 M)
+  if (!any_size && n_edges < (K <= 2 ? (int64_t)1 << 21 : K == 3 ? (int64_t)5 << 19 : (int64_t)1 << 22)) return r;
   // chunk: entries per reducing workgroup, about 1024 workgroups, 2048 ... 65536 entries
   int64_t chunk = (n_edges / 1024 + 1023) & ~(int64_t)1023;
   if (chunk < 2048) chunk = 2048;
@@ -132,7 +146,11 @@ inline BinPlan bin_plan_payload(int64_t B, int64_t E, int64_t K, int64_t N, int 
   auto take = [&](size_t bytes) { const size_t o = off; off += up(bytes); return o; };
   const size_t o_tot = take((size_t)nb * 8), o_cur = take((size_t)nb * 8), o_st = take((size_t)(nb + 1) * 8);
   const size_t o_cs = take((size_t)(nb + 1) * 4), o_wb = take((size_t)p.max_wgs * 4);
-  const size_t o_bin = take(K > 1 ? (size_t)n_edges * 4 * (size_t)(K + 1) : (size_t)n_edges * 8), o_flag = take(256);
+  size_t tiles_bytes = 0;
+  value_tiles_plan(B, E, K, N, nullptr, 0, &tiles_bytes);
+  size_t bin_bytes = K > 1 ? (size_t)n_edges * 4 * (size_t)(K + 1) : (size_t)n_edges * 8;
+  if (bin_bytes < tiles_bytes) bin_bytes = tiles_bytes;
+  const size_t o_bin = take(bin_bytes), o_flag = take(256);
   r.bytes = off;
   if (ws == nullptr || ws_bytes < off || (reinterpret_cast<uintptr_t>(ws) & 15) != 0) return r;
   char *base = static_cast<char *>(ws);
@@ -143,12 +161,18 @@ inline BinPlan bin_plan_payload(int64_t B, int64_t E, int64_t K, int64_t N, int 
   p.wg_bucket = reinterpret_cast<int32_t *>(base + o_wb);
   p.binned = reinterpret_cast<uint64_t *>(base + o_bin);
   p.unsorted = reinterpret_cast<int *>(base + o_flag);
+  p.tiles = value_tiles_plan(B, E, K, N, base + o_bin, bin_bytes, &tiles_bytes);
   p.slab_start = nullptr;
   p.comb_list = nullptr;
   p.comb_count = nullptr;
   p.slabs = nullptr;
   r.ok = true;
   return r;
+}
+
+// Do the passes of value_tiles.h take the call? They also launch the table of hot rows that follows a sample with three answers.
+inline bool value_tiles_take(const BinArgs &p, int64_t n_edges) {
+  return p.tiles.ok && n_edges >= 2 * kBinBlock && !getenv("TS_BIN_NO_SAMPLE") && !getenv("TS_BIN_NO_TILES");  // tuning aids
 }
 
 // node (b * N + index) of entry be, -1 for an index outside [0, N)
@@ -242,8 +266,7 @@ static __global__ __launch_bounds__(kBinBlock) void bin_sample_kernel(ScatterArg
 // launches that return included; the buckets' time does not depend on where the hot rows lie.)
 // (quarters: the bar in quarters of the sample. Several values per entry: one half, since the buckets' time grows with
 // the values per entry and the table's does not.)
-static __global__ __launch_bounds__(kBinBlock) void bin_sample_skew_kernel(ScatterArgs a, int *flag, int quarters,
-                                                                           unsigned long long *totals, int nb) {
+__device__ __forceinline__ void bin_sample_skew(const ScatterArgs &a, int *flag, int quarters, unsigned long long *totals, int nb) {
   constexpr int kSlots = 2048;
   __shared__ int s_set[kSlots];
   __shared__ int s_desc, s_dup;
@@ -271,6 +294,11 @@ static __global__ __launch_bounds__(kBinBlock) void bin_sample_skew_kernel(Scatt
   __syncthreads();
   if (threadIdx.x == 0) *flag = s_desc * 64 < kBinBlock ? 0 : (s_dup * 4 >= quarters * kBinBlock ? 2 : 1);
 }
+static __global__ __launch_bounds__(kBinBlock) void bin_sample_skew_kernel(ScatterArgs a, int *flag, int quarters,
+                                                                           unsigned long long *totals, int nb) {
+  bin_sample_skew(a, flag, quarters, totals, nb);
+}
+inline int bin_skew_quarters(const BinArgs &p) { return p.planes > 1 ? 2 : 3; }
 
 // Count pass: entries per bucket (and, for callers that ask, whether the index is in order and inside [0, N)).
 // At most two workgroups per CU, each with an equal share of the entries, which it walks in batches of four
@@ -632,13 +660,6 @@ static __global__ __launch_bounds__(kBlock) void bin_clear_kernel(unsigned long 
 
 // ---- sum: the same buckets with a table of accumulators (fp32 for 16-bit floats). Every entry is one LDS
 // atomic add; the table goes to `out` with one atomic per touched element and chunk.
-// Slot type of the table: floating types accumulate in double. ds_add_f64 and the integer adds keep their rate
-// when many lanes meet on one address (a hub row); ds_add_f32 does not (measured: 10 M entries of a Zipf(1.2)
-// index, K = 32: 2.2 ms with fp32 slots, 0.44 ms with int32 or double slots).
-template <typename T> struct BinSlot { typedef double type; };
-template <> struct BinSlot<int32_t> { typedef int32_t type; };
-template <> struct BinSlot<int64_t> { typedef int64_t type; };
-
 // Sum of one 4-byte value per entry from (row in bucket, value) words: see bin_plan_payload. A workgroup streams
 // its chunk of a bucket with 16-byte loads (two words per lane, four loads in flight), adds into the bucket's table
 // in LDS (double slots for floats: ds_add_f64 keeps its rate when many lanes meet on one address, a hub row) and
@@ -801,17 +822,23 @@ inline void launch_bin_count(const ScatterArgs &a, const BinArgs &p, hipStream_t
 // three_way: the caller has the table kernel behind this launch for a skewed index (flag value 2, see
 // bin_sample_skew_kernel); needs the sample (enough entries), else the answer stays 0 / 1
 template <typename T>
-void launch_binned_add(const ScatterArgs &a, const BinArgs &plan, hipStream_t stream, bool three_way = false) {
+void launch_binned_add(const ScatterArgs &a, const BinArgs &plan, hipStream_t stream, bool three_way = false, bool have_sample = false,
+                       const TableCall &table = TableCall()) {
   BinArgs p = plan;
   p.sampled = a.B * a.E >= 2 * kBinBlock && !getenv("TS_BIN_NO_SAMPLE");  // env: tuning aid (sorted = no descent at all)
-  if (p.sampled && three_way)
-    hipLaunchKernelGGL(bin_sample_skew_kernel, dim3(1), dim3(kBinBlock), 0, stream, a, p.unsorted, p.planes > 1 ? 2 : 3,
+  if (have_sample) {
+  } else if (p.sampled && three_way)
+    hipLaunchKernelGGL(bin_sample_skew_kernel, dim3(1), dim3(kBinBlock), 0, stream, a, p.unsorted, bin_skew_quarters(p),
                        p.totals, p.nb);
   else if (p.sampled)
     hipLaunchKernelGGL(bin_sample_kernel, dim3(1), dim3(kBinBlock), 0, stream, a, p.unsorted, p.totals, p.nb);
   else  // (the sample kernels clear the buckets' counts on the way)
     hipLaunchKernelGGL(bin_clear_kernel, dim3((p.nb + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, p.totals, p.nb,
                        p.unsorted);
+  if (value_tiles_take(p, a.B * a.E)) {
+    launch_value_tiles<T>(a, p.tiles, p.unsorted, p.count_out, table, stream);
+    return;
+  }
   launch_bin_count(a, p, stream);
   hipLaunchKernelGGL(bin_scan_kernel, dim3(1), dim3(kBinBlock), 0, stream, p);
   if (p.payload && p.planes > 1)
