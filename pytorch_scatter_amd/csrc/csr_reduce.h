@@ -149,6 +149,7 @@ __device__ __forceinline__ double sqrt_acc(double v) { return sqrt(v); }
 template <typename T> __device__ __forceinline__ typename Acc<T>::type round_elem(typename Acc<T>::type v) {
   return to_acc<T>(from_acc<T>(v));
 }
+template <> __device__ __forceinline__ float round_elem<bf16_t>(float v) { return (float)(__bf16)v; }  // (any NaN stays one)
 // std: the group mean as the reference forms it (composite/std.py:27-31: sum / clamp(count, 1), in the
 // element type) and the divisor of the squared deviations (:36-38: count or clamp(count - 1, 1), plus 1e-6)
 template <typename T> __device__ __forceinline__ typename Acc<T>::type group_mean(T total, int32_t count) {
