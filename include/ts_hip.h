@@ -397,8 +397,10 @@ int ts_group_softmax_backward(const void *result, const void *grad_out,
  * memory, written by the forward call; hand it, unchanged and with the same
  * index, sizes and dtype, to the backward call. 0 bytes: this form does not
  * take the call (TS_ERR_UNSUPPORTED; small inputs, which ts_group_softmax does
- * faster). workspace: ts_group_order_workspace_bytes() bytes of scratch (the
- * backward call needs less). Both 16-byte aligned. Group sums are held in
+ * faster, or rows that are not whole 16-byte units: ts_group_rows_order_bytes()
+ * below). workspace: ts_group_order_workspace_bytes() bytes of scratch (the
+ * backward call needs less). Both 16-byte aligned; so is everything else where
+ * the backward call returns TS_ERR_UNSUPPORTED otherwise. Group sums are held in
  * double. result and grad_out: what the forward call returned and its gradient.
  */
 size_t ts_group_order_bytes(int64_t B, int64_t E, int64_t K, int64_t N,
@@ -417,6 +419,26 @@ int ts_group_softmax_ordered_backward(
     int64_t index_stride_b, int64_t index_stride_e, int dtype, int log_space,
     const void *order, size_t order_bytes, void *workspace,
     size_t workspace_bytes, ts_stream_t stream);
+
+/*
+ * The same order for every group statistic, for rows of any width and alignment. op: 0 softmax and log-softmax (which
+ * ts_group_softmax_ordered and its backward take with these sizes as well), 1 logsumexp, 2 standard deviation. 0 bytes: the
+ * order does not pay for this call (TS_ERR_UNSUPPORTED). The backward call is handed the order of the forward call, with the
+ * same index, sizes and dtype, and needs the records' part of the workspace alone.
+ * ts_group_reduce_ordered: logsumexp (std_dev 0; eps) or the deviation (std_dev 1; unbiased) of every group into out
+ * [B, N, K], std also the group sums (total, element type) and the entries per group (count). All three fully written.
+ */
+size_t ts_group_rows_order_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int op);
+size_t ts_group_rows_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int op, int backward);
+int ts_group_reduce_ordered(const void *src, const int64_t *index, void *out, void *total, int32_t *count, int64_t B,
+                            int64_t E, int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype,
+                            int std_dev, int unbiased, double eps, void *order, size_t order_bytes, void *workspace,
+                            size_t workspace_bytes, ts_stream_t stream);
+int ts_group_reduce_ordered_backward(const void *src, const int64_t *index, const void *out, const void *total,
+                                     const int32_t *count, const void *grad_out, void *grad_in, int64_t B, int64_t E,
+                                     int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype,
+                                     int std_dev, int unbiased, const void *order, size_t order_bytes, void *workspace,
+                                     size_t workspace_bytes, ts_stream_t stream);
 
 /* logsumexp over the entries that share an index, one index per row:
  *   out[b, n, k] = log(sum_group exp(src - m) + eps) + m,  m = group max starting from -inf;

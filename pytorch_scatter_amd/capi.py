@@ -31,6 +31,7 @@ EXPORTS = (
     "ts_scatter_small_applies", "ts_scatter_small",
     "ts_group_softmax_workspace_bytes", "ts_group_softmax", "ts_group_softmax_backward",
     "ts_group_order_bytes", "ts_group_order_workspace_bytes", "ts_group_softmax_ordered", "ts_group_softmax_ordered_backward",
+    "ts_group_rows_order_bytes", "ts_group_rows_workspace_bytes", "ts_group_reduce_ordered", "ts_group_reduce_ordered_backward",
     "ts_group_logsumexp", "ts_group_logsumexp_backward",
     "ts_group_std", "ts_group_std_backward", "ts_group_bins_workspace_bytes", "ts_group_std_workspace_bytes", "ts_group_workspace_bytes", "ts_group_std_forward",
     "ts_group_std_backward_with_workspace", "ts_group_logsumexp_backward_with_workspace",
@@ -61,6 +62,8 @@ def lib() -> ctypes.CDLL:
         _lib.ts_group_softmax_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_group_order_bytes.restype = ctypes.c_size_t
         _lib.ts_group_order_workspace_bytes.restype = ctypes.c_size_t
+        _lib.ts_group_rows_order_bytes.restype = ctypes.c_size_t
+        _lib.ts_group_rows_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_indptr_to_index_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_scatter_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_scatter_workspace_zero_bytes.restype = ctypes.c_size_t
@@ -330,7 +333,7 @@ def group_softmax_ordered(src, index, out, B, E, K, N, sb, se, log_space: bool, 
     """Softmax with the entries sorted by group first (ts_group_softmax_ordered). Returns the order, for the backward call."""
     _dev(src, index, out)
     sizes = (_i(B), _i(E), _i(K), _i(N), DTYPE[out.dtype])
-    order_bytes, nbytes = int(lib().ts_group_order_bytes(*sizes)), int(lib().ts_group_order_workspace_bytes(*sizes, 0))
+    order_bytes, nbytes = int(lib().ts_group_rows_order_bytes(*sizes, 0)), int(lib().ts_group_rows_workspace_bytes(*sizes, 0, 0))
     order, ws = (torch.empty(max(n, 1), dtype=torch.uint8, device=out.device) for n in (order_bytes, nbytes))
     with torch.cuda.device(out.device):
         _check(lib().ts_group_softmax_ordered(_p(src), _p(index), _p(out), *sizes[:4], _i(sb), _i(se), sizes[4],
@@ -342,13 +345,40 @@ def group_softmax_ordered(src, index, out, B, E, K, N, sb, se, log_space: bool, 
 def group_softmax_ordered_backward(result, grad_out, index, grad_in, B, E, K, N, sb, se, log_space: bool, order):
     _dev(result, grad_out, index, grad_in, order)
     sizes = (_i(B), _i(E), _i(K), _i(N), DTYPE[grad_in.dtype])
-    nbytes = int(lib().ts_group_order_workspace_bytes(*sizes, 1))
+    nbytes = int(lib().ts_group_rows_workspace_bytes(*sizes, 0, 1))
     ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=grad_in.device)
     with torch.cuda.device(grad_in.device):
         _check(lib().ts_group_softmax_ordered_backward(_p(result), _p(grad_out), _p(index), _p(grad_in), *sizes[:4], _i(sb),
                                                        _i(se), sizes[4], 1 if log_space else 0, _p(order),
                                                        ctypes.c_size_t(order.numel()), _p(ws), ctypes.c_size_t(nbytes),
                                                        _stream(grad_in)))
+
+
+def group_reduce_ordered(src, index, out, total, count, B, E, K, N, sb, se, unbiased: bool = True, eps: float = 1e-12):
+    """logsumexp (total None) or standard deviation over entries sorted by group first (ts_group_reduce_ordered). Returns the
+    order, for the backward call."""
+    _dev(*(t for t in (src, index, out, total, count) if t is not None))
+    sizes, op = (_i(B), _i(E), _i(K), _i(N), DTYPE[out.dtype]), 1 if total is None else 2
+    order_bytes, nbytes = int(lib().ts_group_rows_order_bytes(*sizes, op)), int(lib().ts_group_rows_workspace_bytes(*sizes, op, 0))
+    order, ws = (torch.empty(max(n, 1), dtype=torch.uint8, device=out.device) for n in (order_bytes, nbytes))
+    with torch.cuda.device(out.device):
+        _check(lib().ts_group_reduce_ordered(_p(src), _p(index), _p(out), _p(total), _p(count), *sizes[:4], _i(sb), _i(se),
+                                             sizes[4], op - 1, int(unbiased), ctypes.c_double(eps), _p(order),
+                                             ctypes.c_size_t(order_bytes), _p(ws), ctypes.c_size_t(nbytes), _stream(out)))
+    return order
+
+
+def group_reduce_ordered_backward(src, index, out, total, count, grad_out, grad_in, B, E, K, N, sb, se, order,
+                                  unbiased: bool = True):
+    _dev(*(t for t in (src, index, out, total, count, grad_out, grad_in, order) if t is not None))
+    sizes, op = (_i(B), _i(E), _i(K), _i(N), DTYPE[out.dtype]), 1 if total is None else 2
+    nbytes = int(lib().ts_group_rows_workspace_bytes(*sizes, op, 1))
+    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=grad_in.device)
+    with torch.cuda.device(grad_in.device):
+        _check(lib().ts_group_reduce_ordered_backward(_p(src), _p(index), _p(out), _p(total), _p(count), _p(grad_out),
+                                                      _p(grad_in), *sizes[:4], _i(sb), _i(se), sizes[4], op - 1, int(unbiased),
+                                                      _p(order), ctypes.c_size_t(order.numel()), _p(ws),
+                                                      ctypes.c_size_t(nbytes), _stream(grad_in)))
 
 
 def group_logsumexp(src, index, out, B, E, K, N, sb, se, eps: float = 1e-12, bins: bool = True):

@@ -14,6 +14,7 @@
 #include "scatter.h"
 #include "elementwise.h"
 #include "group_softmax.h"
+#include "group_rows.h"
 #include "index_format.h"
 #include "row_sort.h"
 #include "scatter_small.h"
@@ -76,6 +77,16 @@ int dispatch_group_softmax(int dtype, const GroupArgs &g, int mode, int vec, hip
   case TS_F64: return launch_group_softmax<double>(g, mode, vec, s);
   case TS_F16: return launch_group_softmax<f16_t>(g, mode, vec, s);
   case TS_BF16: return launch_group_softmax<bf16_t>(g, mode, vec, s);
+  default: return TS_ERR_UNSUPPORTED;
+  }
+}
+
+int dispatch_group_rows(int dtype, const GroupArgs &g, const GroupRowsArgs &f, int mode, hipStream_t s) {
+  switch (dtype) {
+  case TS_F32: return launch_group_rows<float>(g, f, mode, s);
+  case TS_F64: return launch_group_rows<double>(g, f, mode, s);
+  case TS_F16: return launch_group_rows<f16_t>(g, f, mode, s);
+  case TS_BF16: return launch_group_rows<bf16_t>(g, f, mode, s);
   default: return TS_ERR_UNSUPPORTED;
   }
 }
@@ -1190,7 +1201,7 @@ int run_group_softmax(const void *src, const void *grad, const int64_t *index, v
 }  // namespace
 
 namespace {
-// Softmax over entries sorted by group (row_sort.h, the ordered tiles of group_fused.h). Where the tiles for an index in
+// Softmax over entries sorted by group (row_sort.h, group_rows.h, the ordered tiles of group_fused.h). Where the tiles for an index in
 // order apply they come first, behind a sample of the index, and what follows returns at once if they took the call: an
 // index in order costs what it did without the sort (and the sort of one that is not, 14 us for the launches in front).
 // Where the line lies (us without / with, groups of 30; even, Zipf(1.2) hub, both in no order, then both in order):
@@ -1200,23 +1211,50 @@ namespace {
 //   78 / 49 71 39 44, 100 k x 32 65 69 32 34 / 50 70 43 46, 100 k x 64 92 99 56 56 / 62 79 55 54; groups of 60, 50 k x 64 59 64 32 34 /
 //   43 70 36 46. With 1000 the tables in LDS hold every group, 300 k x 8 62 82 52 70 / 61 75 49 48, but 300 k x 4 60 95 48 77 / 53 71 40
 //   42 against 100 k x 32 52 53 33 34 / 57 79 49 56 and, in order, 3 M x 32 430 550 / 471 1314.
-//   backward, from 16 to 128 MB, up to 64 entries a group and 64 bytes a row: 600 k x 8 58 68 44 44 / 39 61 33 48, 1 M x 8 83 115 54 53 /
-//   58 88 33 69, 500 k x 16 71 63 52 53 / 39 61 34 77, 2 M x 8 168 294 56 115 / 107 161 54 110 (a hub in order below 64 MB loses what the
-//   launches that return at once cost); beyond, two arrays of gathered rows leave the 256 MB of the memory-side cache: 10 M x 8 817 875 /
-//   883 1178. 1 M x 32 205 323 / 173 293, but in order, where no tiles come first, 139 228 / 131 234 and 3 M x 64 784 793 / 1068 1989.
 // TS_GROUP_ORDER (tuning aid): 0 never, 2 at any size; 3: at any size, and never the tiles for an index in order.
-bool group_order_rule(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, bool backward) {
+bool group_order_rule(int64_t B, int64_t E, int64_t K, int64_t N, int dtype) {
   if (!valid_dtype(dtype) || !is_float_dtype(dtype) || !sizes_ok(B, N, E, K) || B * E * K == 0 || N == 0) return false;
   const int mode = env_int("TS_GROUP_ORDER", 1);
   const int64_t row_bytes = K * kElemBytes[dtype], bytes = B * E * row_bytes;
   if (mode == 0 || K >= (int64_t)1 << 20 || row_bytes % kVecBytes != 0) return false;
-  if (backward && row_bytes > 64) return false;
-  if (group_fused_ordered_plan(B * E, K, kElemBytes[dtype], backward, nullptr).bytes == 0) return false;  // (too many column slices)
   if (mode >= 2) return true;
-  if (backward) return E <= 64 * N && bytes >= ((int64_t)16 << 20) && bytes <= ((int64_t)128 << 20);
   const int64_t least = (int64_t)(row_bytes <= 128 ? 8 : 10) << 20;
   const int64_t most = bytes >= (int64_t)16 << 20 || row_bytes <= 64 ? 128 : row_bytes <= 128 ? 64 : 32;
   return bytes >= least && E <= most * N;
+}
+// What else goes over the sorted entries (group_rows.h). op: 0 softmax, 1 logsumexp, 2 std. The passes that it replaces add and
+// compare in memory, element by element unless rows are whole 16-byte units, so rows that are not, and 16-bit elements, gain from
+// smaller inputs on. us without / with the sort, forward and backward (f: forward alone), entries x columns:
+//   softmax    1.7 M x 199 bf16, 4 a group 7719 / 2561; 580 k x 98 floats, 39 a group 1321 / 589; f 1.3 M x 1 bf16, 30 a group 177 / 48;
+//              f 29 k x 64 bf16 46 / 30; 18 k x 146 floats, 260 a group 252 / 81. Left: f 950 k x 1 floats in order 30 / 53; 5.4 M x 1
+//              floats under a hub, 280 a group 412 / 612; 4.8 M x 128 floats in order, 147 a group (2.3 GB) 3886 / 5101
+//   logsumexp  606 k x 256 floats 1793 / 685, f 348 k x 32 floats 128 / 63, f 8.1 M x 3 f16 359 / 247. Left: 3.3 M x 1 floats, 46 a
+//              group 159 / 207; f 4.8 M x 256 bf16 in order (2.3 GB) 2342 / 3118
+//   std        f 2.65 M x 64 floats, 207 a group 897 / 476; 484 k x 128 floats under a hub 518 / 320. Left: f 580 k x 256 floats in
+//              order 253 / 402; 5.1 M x 100 floats in order (2 GB) 2295 / 3334; 1.7 M x 100 floats, 297 a group 865 / 1198 (pieces that
+//              are not lines); 19 M x 4 floats under a hub, 359 a group 1204 / 1868
+// 440 drawn calls of all sizes, those that stay among them: 0.86 of the time in the geometric mean.
+bool group_rows_rule(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int op) {
+  if (!valid_dtype(dtype) || !is_float_dtype(dtype) || !sizes_ok(B, N, E, K) || B * E * K == 0 || N == 0) return false;
+  if (op < 0 || op > 2 || K >= (int64_t)1 << 20) return false;
+  const int mode = env_int("TS_GROUP_ORDER", 1);
+  if (mode == 0) return false;
+  if (mode >= 2) return true;
+  const int es = kElemBytes[dtype];
+  const int64_t row_bytes = K * es, bytes = B * E * row_bytes, MB = (int64_t)1 << 20;
+  if (op == 0) {
+    if (group_order_rule(B, E, K, N, dtype)) return true;
+    if (E > 128 * N && (bytes > 1024 * MB || row_bytes < 32)) return false;
+    if (row_bytes >= 128) return bytes >= (es == 2 ? MB : 8 * MB);
+    return bytes >= (es == 2 ? 2 * MB : 8 * MB) && E <= (K <= 2 ? 32 : 512) * N;
+  }
+  if (op == 1 && es == 2 && bytes > 1024 * MB) return false;
+  if (op == 2) {
+    if (row_bytes > 512 || bytes > 1024 * MB || E > (row_bytes < 64 ? 128 : 4096) * N) return false;
+    if (row_bytes > 256 && row_bytes % 128 != 0 && bytes > 256 * MB) return false;
+  }
+  if (K == 1) return bytes >= 4 * MB && E <= 16 * N;
+  return bytes >= (row_bytes >= 128 ? 4 * MB : 8 * MB);
 }
 // plan of the tiles for an index in order, their records at ws; false: they do not apply
 bool group_order_tiles(GroupArgs &g, int dtype, int mode, void *ws, size_t ws_bytes, int *flag, FusedArgs &f) {
@@ -1226,110 +1264,234 @@ bool group_order_tiles(GroupArgs &g, int dtype, int mode, void *ws, size_t ws_by
   f.flag = flag;
   return true;
 }
-size_t group_order_records(int64_t B, int64_t E, int64_t K, int dtype, bool backward) {
-  const size_t ordered = group_fused_ordered_plan(B * E, K, kElemBytes[dtype], backward, nullptr).bytes;
-  const size_t tiles = group_fused_scratch_bytes(B, E, K, kElemBytes[dtype]);
-  return ordered > tiles ? ordered : tiles;  // (one after the other)
+// 16-bit rows of whole 16-byte units: the forward pass of softmax takes the tiles of group_fused.h over the sorted entries,
+// whose lanes hold eight elements (128 columns of bf16 in groups of 20, 2.6 M entries: 884 us, 1059 with the rows in registers;
+// 64 columns in groups of 5, 5.1 M entries: 873 / 938), and whose tiles are longer where groups are (128 floats in groups of 117,
+// 1.3 M entries: 611 / 766). Other rows the other way round: 128 floats, groups of 6, 1.3 M entries, forward and backward 1537 / 842.
+bool group_rows_in_tiles(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int mode) {
+  return (mode == GS_SOFTMAX || mode == GS_LOG_SOFTMAX) && (kElemBytes[dtype] == 2 || E > 64 * N) &&
+         group_order_rule(B, E, K, N, dtype) && group_fused_ordered_plan(B * E, K, kElemBytes[dtype], nullptr).bytes > 0;
 }
-// sorted: the order, made by a forward call and read by a backward call
-int run_group_ordered(const void *src, const void *grad, const int64_t *index, void *out, int64_t B, int64_t E, int64_t K,
-                      int64_t N, int64_t sb, int64_t se, int dtype, int mode, double eps, const RowSortArgs &sorted,
-                      void *records, size_t records_bytes, hipStream_t stream) {
-  const bool backward = mode == GS_SOFTMAX_BWD || mode == GS_LOG_SOFTMAX_BWD;
-  if (!aligned16(src) || !aligned16(out) || (grad != nullptr && !aligned16(grad))) return TS_ERR_UNSUPPORTED;
-  const int vec = kVecBytes / kElemBytes[dtype];
-  FusedOrderedPlan p = group_fused_ordered_plan(B * E, K, kElemBytes[dtype], backward, records);
+size_t group_rows_records(int64_t B, int64_t E, int64_t K, int64_t N, int dtype) {
+  size_t most = group_rows_plan(B * E, B * N, K, kElemBytes[dtype], nullptr).bytes;  // (one after the other)
+  auto with = [&](size_t bytes) { most = bytes > most ? bytes : most; };
+  with(group_fused_scratch_bytes(B, E, K, kElemBytes[dtype]));
+  with(group_reduce_fused_plan(B, E, K, N, kElemBytes[dtype], true, nullptr, 0, false).bytes);
+  if (group_rows_in_tiles(B, E, K, N, dtype, GS_SOFTMAX)) with(group_fused_ordered_plan(B * E, K, kElemBytes[dtype], nullptr).bytes);
+  return most;
+}
+// sorted: the order, made by a forward call and read by a backward call. g: the call's own arrays, for one list of entries and
+// groups still to be described. sorted.state[4] reads 0 if the tiles for an index in order took the forward call: then there is
+// no order.
+int run_group_rows(GroupArgs g, int64_t B, int64_t E, int64_t K, int64_t N, int64_t sb, int64_t se, int dtype, int mode,
+                   const RowSortArgs &sorted, void *records, size_t records_bytes, hipStream_t stream) {
+  const bool softmax = mode == GS_SOFTMAX || mode == GS_LOG_SOFTMAX || mode == GS_SOFTMAX_BWD || mode == GS_LOG_SOFTMAX_BWD;
+  const bool backward = mode == GS_SOFTMAX_BWD || mode == GS_LOG_SOFTMAX_BWD || mode == GS_STD_BWD || mode == GS_LSE_BWD;
+  const int es = kElemBytes[dtype];
+  GroupRowsPlan p = group_rows_plan(B * E, B * N, K, es, records);
   if (p.bytes == 0) return TS_ERR_UNSUPPORTED;
-  GroupArgs g = {};
-  g.src = src;
-  g.grad = grad;
-  g.index = index;
-  g.out = out;
   g.B = B;
   g.E = E;
   g.K = K;
   g.N = N;
   g.sb = sb;
   g.se = se;
-  g.eps = eps;
-  // Does the forward call try the tiles for an index in order? The backward call then follows its verdict.
-  FusedArgs tiles;
+  bool tried = false;  // the tiles for an index in order, in front
   int *const flag = sorted.state + 4;
-  const int fwd_mode = mode == GS_SOFTMAX_BWD ? GS_SOFTMAX : mode == GS_LOG_SOFTMAX_BWD ? GS_LOG_SOFTMAX : mode;
-  const bool tried = group_order_tiles(g, dtype, fwd_mode, records, records_bytes, flag, tiles);
-  if (tried) {
-    if (backward && !group_order_tiles(g, dtype, mode, records, records_bytes, flag, tiles)) return TS_ERR_UNSUPPORTED;
-    g.in_order = &tiles;
-    g.in_order_sample = backward ? 0 : 1;
-    const int rc = dispatch_group_softmax(dtype, g, mode, vec, stream);
-    if (rc != TS_OK) return rc;
-    g.in_order = nullptr;
+  const bool al = aligned16(g.src) && aligned16(g.out) && (g.grad == nullptr || aligned16(g.grad));
+  if (softmax && K * es <= 64) {  // (rows that the tiles of either direction hold)
+    FusedArgs tiles;
+    GroupArgs any = g;  // (do the sizes allow them?)
+    any.src = any.grad = any.out = nullptr;
+    const int fwd_mode = mode == GS_SOFTMAX_BWD ? GS_SOFTMAX : mode == GS_LOG_SOFTMAX_BWD ? GS_LOG_SOFTMAX : mode;
+    tried = group_order_tiles(any, dtype, fwd_mode, records, records_bytes, flag, tiles);
+    if (tried && backward && !al) return TS_ERR_UNSUPPORTED;  // (they may hold the only way to the result)
+    tried = tried && al;
+    if (tried) {
+      if (!group_order_tiles(g, dtype, mode, records, records_bytes, flag, tiles)) return TS_ERR_UNSUPPORTED;
+      g.in_order = &tiles;
+      g.in_order_sample = backward ? 0 : 1;
+      const int full = kVecBytes / es;
+      const int rc = dispatch_group_softmax(dtype, g, mode, K % full == 0 ? full : 1, stream);
+      if (rc != TS_OK) return rc;
+      g.in_order = nullptr;
+    }
+  } else if ((mode == GS_LSE || mode == GS_STD) && K * es <= kFusedRowBytes && env_int("TS_GROUP_FUSED", 1) != 0 &&
+             env_int("TS_GROUP_ORDER", 1) != 3) {
+    // (wider rows: the tiles in front are behind; 64 floats in groups of 91, in order, 8.4 M entries, std forward and backward
+    // 2581 us with them, 2217 without; 32 floats in groups of 9, logsumexp forward: 257 / 559)
+    FusedReducePlan tiles = group_reduce_fused_plan(B, E, K, N, es, aligned16(g.src), records, records_bytes, false);
+    tried = tiles.ok;
+    if (tried) {
+      tiles.f.flag = flag;
+      g.tiles = &tiles.f;
+      const int rc = dispatch_group_softmax(dtype, g, mode == GS_STD ? GS_STD_BINS : GS_LSE_BINS,
+                                            group_bins_vec(K, dtype, aligned16(g.src)), stream);
+      if (rc != TS_OK) return rc;
+      g.tiles = nullptr;
+    }
   }
   if (!backward) {
-    const int rc = launch_row_sort(sorted, index, sb, se, false, next_nonce(), stream, tried ? flag : nullptr);
+    const int rc = launch_row_sort(sorted, g.index, sb, se, false, next_nonce(), stream, tried ? flag : nullptr);
     if (rc != TS_OK) return rc;
+  }
+  g.B = 1;
+  g.E = B * E;
+  g.N = B * N;
+  if (al && group_rows_in_tiles(B, E, K, N, dtype, mode)) {
+    FusedOrderedPlan o = group_fused_ordered_plan(B * E, K, es, records);
+    o.f.gate = tried ? flag : nullptr;
+    o.f.state = sorted.state;
+    o.f.n_sorted = sorted.ptr + B * N;
+    o.f.perm = sorted.perm;
+    o.f.group = sorted.perm_row;
+    o.f.ptr = sorted.ptr;
+    o.f.index = g.index;
+    o.f.sb = sb;
+    o.f.se = se;
+    o.f.E0 = E;
+    o.f.N0 = N;
+    g.ordered = &o.f;
+    return dispatch_group_softmax(dtype, g, mode, kVecBytes / es, stream);
   }
   p.f.gate = tried ? flag : nullptr;
   p.f.state = sorted.state;
-  p.f.n_sorted = sorted.ptr + B * N;
+  p.f.ptr = sorted.ptr;
   p.f.perm = sorted.perm;
   p.f.group = sorted.perm_row;
-  p.f.ptr = sorted.ptr;
-  p.f.index = index;
+  p.f.index = g.index;
   p.f.sb = sb;
   p.f.se = se;
   p.f.E0 = E;
   p.f.N0 = N;
-  g.B = 1;
-  g.E = B * E;
-  g.N = B * N;
-  g.ordered = &p.f;
-  return dispatch_group_softmax(dtype, g, mode, vec, stream);
+  if (!aligned16(g.out)) p.f.stream = 0;
+  return dispatch_group_rows(dtype, g, p.f, mode, stream);
+}
+// (sizes that the rule and the plans take)
+bool group_rows_ok(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int op) {
+  return group_rows_rule(B, E, K, N, dtype, op) && row_sort_plan(B, E, N, nullptr, 0, true).bytes > 0 &&
+         group_rows_plan(B * E, B * N, K, kElemBytes[dtype], nullptr).bytes > 0;
+}
+// the order of a backward call, as the forward call left it
+int group_rows_saved(const void *order, size_t order_bytes, void *workspace, size_t workspace_bytes, int64_t B, int64_t E,
+                     int64_t K, int64_t N, int dtype, int op, RowSortPlan &sp) {
+  if (!group_rows_ok(B, E, K, N, dtype, op)) return TS_ERR_UNSUPPORTED;
+  sp = row_sort_plan(B, E, N, nullptr, 0, true, const_cast<void *>(order));
+  if (!order || order_bytes < sp.kept_bytes || !aligned16(order) || !workspace || !aligned16(workspace) ||
+      workspace_bytes < group_rows_records(B, E, K, N, dtype) || !sp.ok)
+    return TS_ERR_WORKSPACE;
+  return TS_OK;
+}
+int group_rows_made(void *order, size_t order_bytes, void *workspace, size_t workspace_bytes, int64_t B, int64_t E, int64_t K,
+                    int64_t N, int dtype, int op, RowSortPlan &sp) {
+  if (!group_rows_ok(B, E, K, N, dtype, op)) return TS_ERR_UNSUPPORTED;
+  const size_t records = group_rows_records(B, E, K, N, dtype);
+  if (!order || !aligned16(order) || !workspace || !aligned16(workspace) || workspace_bytes < records) return TS_ERR_WORKSPACE;
+  sp = row_sort_plan(B, E, N, static_cast<char *>(workspace) + records, workspace_bytes - records, true, order);
+  return sp.ok && order_bytes >= sp.kept_bytes ? TS_OK : TS_ERR_WORKSPACE;
 }
 }  // namespace
 
 size_t ts_group_order_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype) {
-  return group_order_rule(B, E, K, N, dtype, false) ? row_sort_plan(B, E, N, nullptr, 0, true).kept_bytes : 0;
+  // (a slice of the tiles that this form used to take held 16-byte units of 128 bytes)
+  if (!group_order_rule(B, E, K, N, dtype) || (K * kElemBytes[dtype] + 127) / 128 > 65535) return 0;
+  return ts_group_rows_order_bytes(B, E, K, N, dtype, 0);
 }
 
 size_t ts_group_order_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int backward) {
   if (ts_group_order_bytes(B, E, K, N, dtype) == 0) return 0;
-  if (backward && !group_order_rule(B, E, K, N, dtype, true)) return 0;
+  return ts_group_rows_workspace_bytes(B, E, K, N, dtype, 0, backward);
+}
+
+size_t ts_group_rows_order_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int op) {
+  return group_rows_ok(B, E, K, N, dtype, op) ? row_sort_plan(B, E, N, nullptr, 0, true).kept_bytes : 0;
+}
+
+size_t ts_group_rows_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int op, int backward) {
+  if (!group_rows_ok(B, E, K, N, dtype, op)) return 0;
   const RowSortPlan sp = row_sort_plan(B, E, N, nullptr, 0, true);
-  return group_order_records(B, E, K, dtype, backward != 0) + (backward ? 0 : sp.bytes - sp.kept_bytes);
+  return group_rows_records(B, E, K, N, dtype) + (backward ? 0 : sp.bytes - sp.kept_bytes);
 }
 
 int ts_group_softmax_ordered(const void *src, const int64_t *index, void *out, int64_t B, int64_t E, int64_t K, int64_t N,
                              int64_t index_stride_b, int64_t index_stride_e, int dtype, int log_space, double eps,
                              void *order, size_t order_bytes, void *workspace, size_t workspace_bytes, ts_stream_t stream) {
-  const size_t need = ts_group_order_bytes(B, E, K, N, dtype);
-  if (need == 0) return TS_ERR_UNSUPPORTED;
+  RowSortPlan sp;
+  if (!group_rows_ok(B, E, K, N, dtype, 0)) return TS_ERR_UNSUPPORTED;
   if (!src || !index || !out) return TS_ERR_BAD_ARG;
-  if (!order || order_bytes < need || !aligned16(order) || !workspace || !aligned16(workspace) ||
-      workspace_bytes < ts_group_order_workspace_bytes(B, E, K, N, dtype, 0))
-    return TS_ERR_WORKSPACE;
-  const size_t records = group_order_records(B, E, K, dtype, false);
-  const RowSortPlan sp = row_sort_plan(B, E, N, static_cast<char *>(workspace) + records, workspace_bytes - records, true, order);
-  if (!sp.ok) return TS_ERR_WORKSPACE;
-  return run_group_ordered(src, nullptr, index, out, B, E, K, N, index_stride_b, index_stride_e, dtype,
-                           log_space ? GS_LOG_SOFTMAX : GS_SOFTMAX, eps, sp.p, workspace, records,
-                           static_cast<hipStream_t>(stream));
+  const int rc = group_rows_made(order, order_bytes, workspace, workspace_bytes, B, E, K, N, dtype, 0, sp);
+  if (rc != TS_OK) return rc;
+  GroupArgs g = {};
+  g.src = src;
+  g.index = index;
+  g.out = out;
+  g.eps = eps;
+  return run_group_rows(g, B, E, K, N, index_stride_b, index_stride_e, dtype, log_space ? GS_LOG_SOFTMAX : GS_SOFTMAX, sp.p,
+                        workspace, group_rows_records(B, E, K, N, dtype), static_cast<hipStream_t>(stream));
 }
 
 int ts_group_softmax_ordered_backward(const void *result, const void *grad_out, const int64_t *index, void *grad_in, int64_t B,
                                       int64_t E, int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e,
                                       int dtype, int log_space, const void *order, size_t order_bytes, void *workspace,
                                       size_t workspace_bytes, ts_stream_t stream) {
-  const size_t need = ts_group_order_bytes(B, E, K, N, dtype), scratch = ts_group_order_workspace_bytes(B, E, K, N, dtype, 1);
-  if (need == 0 || scratch == 0) return TS_ERR_UNSUPPORTED;
+  RowSortPlan sp;
+  if (!group_rows_ok(B, E, K, N, dtype, 0)) return TS_ERR_UNSUPPORTED;
   if (!result || !grad_out || !index || !grad_in) return TS_ERR_BAD_ARG;
-  if (!order || order_bytes < need || !aligned16(order) || !workspace || !aligned16(workspace) || workspace_bytes < scratch)
-    return TS_ERR_WORKSPACE;
-  const RowSortPlan sp = row_sort_plan(B, E, N, nullptr, 0, true, const_cast<void *>(order));
-  if (!sp.ok) return TS_ERR_WORKSPACE;
-  return run_group_ordered(result, grad_out, index, grad_in, B, E, K, N, index_stride_b, index_stride_e, dtype,
-                           log_space ? GS_LOG_SOFTMAX_BWD : GS_SOFTMAX_BWD, 0.0, sp.p, workspace, scratch,
-                           static_cast<hipStream_t>(stream));
+  const int rc = group_rows_saved(order, order_bytes, workspace, workspace_bytes, B, E, K, N, dtype, 0, sp);
+  if (rc != TS_OK) return rc;
+  GroupArgs g = {};
+  g.src = result;
+  g.grad = grad_out;
+  g.index = index;
+  g.out = grad_in;
+  return run_group_rows(g, B, E, K, N, index_stride_b, index_stride_e, dtype, log_space ? GS_LOG_SOFTMAX_BWD : GS_SOFTMAX_BWD,
+                        sp.p, workspace, group_rows_records(B, E, K, N, dtype), static_cast<hipStream_t>(stream));
+}
+
+int ts_group_reduce_ordered(const void *src, const int64_t *index, void *out, void *total, int32_t *count, int64_t B, int64_t E,
+                            int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype, int std_dev,
+                            int unbiased, double eps, void *order, size_t order_bytes, void *workspace, size_t workspace_bytes,
+                            ts_stream_t stream) {
+  RowSortPlan sp;
+  const int op = std_dev ? 2 : 1;
+  if (!group_rows_ok(B, E, K, N, dtype, op)) return TS_ERR_UNSUPPORTED;
+  if (!src || !index || !out || (std_dev && (!total || !count))) return TS_ERR_BAD_ARG;
+  const int rc = group_rows_made(order, order_bytes, workspace, workspace_bytes, B, E, K, N, dtype, op, sp);
+  if (rc != TS_OK) return rc;
+  GroupArgs g = {};
+  g.src = src;
+  g.index = index;
+  g.out = out;
+  g.total_w = total;
+  g.count_w = count;
+  g.unbiased = unbiased ? 1 : 0;
+  g.eps = eps;
+  return run_group_rows(g, B, E, K, N, index_stride_b, index_stride_e, dtype, std_dev ? GS_STD : GS_LSE, sp.p, workspace,
+                        group_rows_records(B, E, K, N, dtype), static_cast<hipStream_t>(stream));
+}
+
+int ts_group_reduce_ordered_backward(const void *src, const int64_t *index, const void *out, const void *total,
+                                     const int32_t *count, const void *grad_out, void *grad_in, int64_t B, int64_t E, int64_t K,
+                                     int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype, int std_dev,
+                                     int unbiased, const void *order, size_t order_bytes, void *workspace,
+                                     size_t workspace_bytes, ts_stream_t stream) {
+  RowSortPlan sp;
+  const int op = std_dev ? 2 : 1;
+  if (!group_rows_ok(B, E, K, N, dtype, op)) return TS_ERR_UNSUPPORTED;
+  if (!src || !index || !out || !grad_out || !grad_in || (std_dev && (!total || !count))) return TS_ERR_BAD_ARG;
+  const int rc = group_rows_saved(order, order_bytes, workspace, workspace_bytes, B, E, K, N, dtype, op, sp);
+  if (rc != TS_OK) return rc;
+  GroupArgs g = {};
+  g.src = src;
+  g.index = index;
+  g.out = grad_in;
+  g.node_out = out;
+  g.node_grad = grad_out;
+  g.total = total;
+  g.count = count;
+  g.unbiased = unbiased ? 1 : 0;
+  return run_group_rows(g, B, E, K, N, index_stride_b, index_stride_e, dtype, std_dev ? GS_STD_BWD : GS_LSE_BWD, sp.p, workspace,
+                        group_rows_records(B, E, K, N, dtype), static_cast<hipStream_t>(stream));
 }
 
 size_t ts_group_softmax_workspace_bytes(int64_t B, int64_t N, int64_t K, int dtype) {

@@ -179,12 +179,7 @@ __device__ __forceinline__ void group_bin_emit(const GroupArgs &g, int64_t i, in
     static_cast<KB *>(g.gmax)[slot] = (KB)s.a;
     static_cast<F *>(g.gsum)[slot] = (F)s.b;
   } else {
-    const F m = OrdKey<F>::dec((KB)s.a);
-    const F l = round_elem<T>(log_acc(round_elem<T>(round_elem<T>((F)s.b) + (F)g.eps)));
-    F o = round_elem<T>(l + m);
-    if (o != o || o == -INFINITY) o = (F)0;
-    if (o == INFINITY) o = to_acc<T>(ElemLim<T>::max());
-    out[i] = from_acc<T>(o);
+    out[i] = group_lse_of<T>(OrdKey<F>::dec((KB)s.a), (F)s.b, (F)g.eps);
   }
 }
 

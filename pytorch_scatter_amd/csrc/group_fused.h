@@ -11,16 +11,14 @@
 // caller's three-pass kernels, gated on that flag, then overwrite the result. No atomics on data: the result
 // does not depend on scheduling.
 //
-// ORDERED: an index in any order whose entries were sorted by group first (row_sort.h). The same tiles over the sorted
+// ORDERED (forward): an index in any order whose entries were sorted by group first (row_sort.h); the rows that group_rows.h, which
+// holds them in registers, does not do better (16-bit elements, groups of 65 to 128 entries). The same tiles over the sorted
 // entries: the rows of a tile are gathered through perm and the results go back the same way, so src is still read once
-// and out written once, the backward pass takes the order of the forward pass, and no launch depends on a verdict. A tile
-// takes the groups that begin in its window of three quarters of what it holds; the row pointers tell which groups are
-// too long for that, and only those leave partials, put together once per group by a launch of their own. Rows wider than
-// a tile holds are taken in column slices. Sums are held in double. What bounds it: the chain of a tile (row pointers, perm,
-// rows, four passes over LDS) at four workgroups per CU; 2.3 M x 8 floats 95 us for 296 MB of half-used 64-byte pieces,
-// 1 M x 64 floats 174 us for 512 MB (2.9 TB/s). us of the whole forward pass, without the order / with it, even index in
-// no order: 1 M x 8 floats in groups of 30 114 / 75, 3 M x 8 258 / 147, 1 M x 32 225 / 133, 3 M x 64 1705 / 550; backward
-// 3 M x 8 244 / 159 (no sort there).
+// and out written once, and no launch depends on a verdict. A tile takes the groups that begin in its window of three quarters
+// of what it holds; the row pointers tell which groups are too long for that, and only those leave partials, put together once
+// per group by a launch of their own. Rows wider than a tile holds are taken in column slices. Sums are held in double. What
+// bounds it: the chain of a tile (row pointers, perm, rows, four passes over LDS) at four workgroups per CU; 1 M x 64 floats
+// 174 us for 512 MB (2.9 TB/s).
 //
 //   forward   m = run maximum (entries beat lowest(), NaN never wins, no winner: 0), e = exp(src - m),
 //             s = sum e;  softmax e / s,  log-softmax (src - m) - log(s + eps)
@@ -289,6 +287,7 @@ __global__ __launch_bounds__(kBlock, 4) void group_fused_kernel(GroupArgs g, Fus
   typedef typename OrdKey<F>::bits KB;
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
   constexpr bool kBackward = MODE == GS_SOFTMAX_BWD || MODE == GS_LOG_SOFTMAX_BWD;
+  static_assert(!ORDERED || !kBackward, "the backward pass over sorted entries: group_rows.h");
   constexpr int W = kBlock / kWave;
   // [tile of src][backward: tile of grad][run starts: te + 2 16-bit words, bit 15: index outside [0, N)]
   extern __shared__ u4 s_dyn[];
@@ -333,7 +332,7 @@ __global__ __launch_bounds__(kBlock, 4) void group_fused_kernel(GroupArgs g, Fus
   constexpr int kPer = 16 / (int)sizeof(T);
   const uint32_t inv = ORDERED ? (blockIdx.y == gridDim.y - 1 ? f.inv_last : f.inv_units) : 0;
   // ORDERED, not flat: a lane's unit q of a tile is unit tid + q * kBlock, of the row at place[q]
-  constexpr int Q = kBackward ? kFusedVecs / 2 : kFusedVecs;
+  constexpr int Q = kFusedVecs;
   int32_t place[ORDERED ? Q : 1];
   auto unit_at = [&](int q) {
     const int v = tid + q * kBlock, u = v < nvec ? v : nvec - 1;
@@ -351,10 +350,10 @@ __global__ __launch_bounds__(kBlock, 4) void group_fused_kernel(GroupArgs g, Fus
       if (v < nstage && vv < nvec) stage[q] = __builtin_nontemporal_load((second ? p1 : p0) + vv);
     }
   } else if constexpr (ORDERED) {
-    const T *p0 = static_cast<const T *>(g.src), *p1 = kBackward ? static_cast<const T *>(g.grad) : p0;
+    const T *p0 = static_cast<const T *>(g.src);
     static_assert(!ORDERED || CV * sizeof(T) == 16, "rows of whole 16-byte units");
     // No load behind a condition of its own (past the end: the last unit again), else the lane waits for each load of perm on
-    // the spot (1 M x 64 floats in groups of three: 255 us, 174 like this; 2.3 M x 8 floats 111 / 95, backward 124 / 113).
+    // the spot (1 M x 64 floats in groups of three: 255 us, 174 like this; 2.3 M x 8 floats 111 / 95).
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       const int v = tid + q * kBlock;
@@ -365,10 +364,7 @@ __global__ __launch_bounds__(kBlock, 4) void group_fused_kernel(GroupArgs g, Fus
       for (int q = 0; q < Q; ++q) place[q] = f.perm[place[q]];
     }
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      stage[q] = *reinterpret_cast<const u4 *>(p0 + unit_at(q));
-      if (kBackward) stage[q + kFusedVecs - Q] = *reinterpret_cast<const u4 *>(p1 + unit_at(q));
-    }
+    for (int q = 0; q < Q; ++q) stage[q] = *reinterpret_cast<const u4 *>(p0 + unit_at(q));
   }
 
   // ---- runs: a lane looks at epl neighbouring entries
@@ -384,7 +380,6 @@ __global__ __launch_bounds__(kBlock, 4) void group_fused_kernel(GroupArgs g, Fus
         const int v = tid + q * kBlock;
         if (v >= nvec) continue;
         s_dyn[v] = stage[q];
-        if (kBackward) s_dyn[f.tile_vecs + v] = stage[q + kFusedVecs - Q];
       }
       return;
     }
@@ -618,7 +613,7 @@ __global__ __launch_bounds__(kBlock, 4) void group_fused_kernel(GroupArgs g, Fus
     // Backward: the tiles of y and g in LDS, one pass over the runs that sums and finishes in place.
     auto run_bwd = [&](int r, int c0, int first, int step) {
       const int lo = s_start[r] & 0x7FFF, hi = s_start[r + 1] & 0x7FFF;
-      const bool valid = ORDERED || (s_start[r] >> 15) == 0;
+      const bool valid = (s_start[r] >> 15) == 0;
       const bool frag_in = r == 0 && enters, frag_out = r == nruns - 1 && leaves;
       S s[CV];
 #pragma unroll
@@ -655,11 +650,7 @@ __global__ __launch_bounds__(kBlock, 4) void group_fused_kernel(GroupArgs g, Fus
     for_runs(run_bwd, true);
     __syncthreads();
     // the finished runs leave the tile: whole 16-byte units, single elements at the two ends
-    if (!flat) {
-#pragma unroll
-      for (int q = 0; q < Q; ++q)
-        if (tid + q * kBlock < nvec) store_unit(q, s_dyn[tid + q * kBlock]);
-    } else if (w_hi > w_lo) {
+    if (w_hi > w_lo) {
       const int v_lo = (el_lo + kPer - 1) / kPer, v_hi = el_hi / kPer;
       if (v_lo >= v_hi) {
         for (int i = el_lo + tid; i < el_hi; i += kBlock) out_t[i] = s_src[i];
@@ -716,9 +707,7 @@ __global__ __launch_bounds__(kFusedFragBlock) void group_fused_fragment_kernel(G
       const KB *key = static_cast<const KB *>(f.ckey) + (first * 2 + 1) * KR + k_first;
       const S *sum = static_cast<const S *>(f.csum) + (first * 2 + 1) * KR + k_first;
       for (int k = lane; k < K; k += kWave) {
-        F m = (F)0;
-        if constexpr (!kBackward) m = key[k] == group_empty_key<T>() ? (F)0 : OrdKey<F>::dec(key[k]);
-        s_fin[(wave * K + k) * 2] = m;
+        s_fin[(wave * K + k) * 2] = key[k] == group_empty_key<T>() ? (F)0 : OrdKey<F>::dec(key[k]);
         s_fin[(wave * K + k) * 2 + 1] = (F)sum[k];
       }
     }
@@ -815,7 +804,7 @@ __global__ __launch_bounds__(kFusedFragBlock) void group_fused_fragment_kernel(G
       for (int v0 = lo * units + tid; v0 < hi * units; v0 += U * kFusedFragBlock) {
         int64_t at[U];
         int k[U];
-        Vec<T, C> x[U], gr[U];
+        Vec<T, C> x[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {  // (past the end: the last unit again)
           const int v = v0 + u * kFusedFragBlock < hi * units ? v0 + u * kFusedFragBlock : hi * units - 1;
@@ -831,14 +820,13 @@ __global__ __launch_bounds__(kFusedFragBlock) void group_fused_fragment_kernel(G
         for (int u = 0; u < U; ++u) {
           at[u] = at[u] * KR + k_first + k[u];
           x[u] = load_vec<T, C>(src_t + at[u]);
-          if (kBackward) gr[u] = load_vec<T, C>(grad_t + at[u]);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           if (v0 + u * kFusedFragBlock >= hi * units) continue;
 #pragma unroll
           for (int c = 0; c < C; ++c)
-            x[u].v[c] = from_acc<T>(finish(to_acc<T>(x[u].v[c]), kBackward ? to_acc<T>(gr[u].v[c]) : (F)0, k[u] + c));
+            x[u].v[c] = from_acc<T>(finish(to_acc<T>(x[u].v[c]), (F)0, k[u] + c));
           store_vec<T, C>(out_t + at[u], x[u]);
         }
       }
@@ -871,11 +859,10 @@ int launch_group_fused(const GroupArgs &g, const FusedArgs &f, bool force, hipSt
 // all tiles that it crosses (every tile for itself is quadratic in their number: 10 M entries x 32 floats, a fifth of them in
 // one group, 7 ms). Bound by the longest group's chain: 10 M x 8 floats, 2 M in one group, 54 us with every partial waited
 // for on the spot, 28 with eight on the way. At least 4.8 us, with or without such a group.
-template <typename T, int MODE>
+template <typename T>
 __global__ __launch_bounds__(kBlock) void group_fused_combine_kernel(GroupArgs g, FusedArgs f) {
   typedef typename Acc<T>::type F;
   typedef typename OrdKey<F>::bits KB;
-  constexpr bool kBackward = MODE == GS_SOFTMAX_BWD || MODE == GS_LOG_SOFTMAX_BWD;
   __shared__ KB s_key[kBlock];
   __shared__ double s_sum[kBlock];
   if (f.gate != nullptr && *f.gate == 0) return;
@@ -890,7 +877,7 @@ __global__ __launch_bounds__(kBlock) void group_fused_combine_kernel(GroupArgs g
   double *csum = static_cast<double *>(f.csum) + k_first;
   for (int k0 = 0; k0 < K; k0 += G) {
     const int k = k0 + lg < K ? k0 + lg : K - 1;
-    KB key = kBackward ? (KB)0 : group_empty_key<T>();
+    KB key = group_empty_key<T>();
     double sum = 0.0;
     constexpr int U = 8;  // partials on the way together
     for (int64_t i0 = t + j; i0 <= last; i0 += U * parts) {
@@ -900,59 +887,53 @@ __global__ __launch_bounds__(kBlock) void group_fused_combine_kernel(GroupArgs g
       for (int u = 0; u < U; ++u) {  // (past the end: the last tile's again)
         const int64_t i = i0 + u * parts < last ? i0 + u * parts : last;
         const int64_t p = (i * 2 + (i == t ? 1 : 0)) * KR + k;
-        if (!kBackward) ku[u] = ckey[p];
+        ku[u] = ckey[p];
         su[u] = csum[p];
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (i0 + u * parts > last) continue;
-        if constexpr (kBackward)
-          sum += su[u];
-        else
-          fused_absorb<T>(key, sum, ku[u], su[u]);
+        fused_absorb<T>(key, sum, ku[u], su[u]);
       }
     }
-    if constexpr (!kBackward) s_key[threadIdx.x] = key;
+    s_key[threadIdx.x] = key;
     s_sum[threadIdx.x] = sum;
     __syncthreads();
     for (int half = parts / 2; half >= 1; half >>= 1) {
       if (j < half) {
         const int o = threadIdx.x + half * G;
-        if constexpr (kBackward)
-          s_sum[threadIdx.x] += s_sum[o];
-        else
-          fused_absorb<T>(s_key[threadIdx.x], s_sum[threadIdx.x], s_key[o], s_sum[o]);
+        fused_absorb<T>(s_key[threadIdx.x], s_sum[threadIdx.x], s_key[o], s_sum[o]);
       }
       __syncthreads();
     }
     if (j == 0 && k0 + lg < K) {
       const int64_t p = (t * 2 + 1) * KR + k;
-      if constexpr (!kBackward) ckey[p] = s_key[threadIdx.x];
+      ckey[p] = s_key[threadIdx.x];
       csum[p] = s_sum[threadIdx.x];
     }
     __syncthreads();
   }
 }
 
-// Tiles over entries that were sorted by group. K columns in slices of at most 128 bytes (backward, with two tiles: 64).
+// Tiles over entries that were sorted by group. K columns in slices of at most 128 bytes.
 // bytes: of the tiles' records; ws null: only that.
 struct FusedOrderedPlan {
   size_t bytes;
   FusedArgs f;
 };
-inline FusedOrderedPlan group_fused_ordered_plan(int64_t n, int64_t K, int elem_bytes, bool backward, void *ws) {
+inline FusedOrderedPlan group_fused_ordered_plan(int64_t n, int64_t K, int elem_bytes, void *ws) {
   FusedOrderedPlan r;
   r.bytes = 0;
   FusedArgs &f = r.f;
   const int vec = 16 / elem_bytes;
   if (K % vec != 0) return r;
-  const int64_t most = (backward ? 64 : 128) / elem_bytes;
+  const int64_t most = 128 / elem_bytes;
   int64_t slices = (K + most - 1) / most, kc = (K + slices - 1) / slices;
   kc = (kc + vec - 1) / vec * vec;
   slices = (K + kc - 1) / kc;
   if (slices > 65535) return r;
   const int64_t row = kc * elem_bytes;
-  int64_t te = (backward ? 16384 : 32768) / row;
+  int64_t te = 32768 / row;
   if (const char *env = getenv("TS_GROUP_TILE")) te = te < atoi(env) ? te : atoi(env);  // tuning aid
   int epl = 1;
   while (epl * 2 * kBlock <= te && epl * 2 <= kFusedPer) epl *= 2;
@@ -982,12 +963,11 @@ inline FusedOrderedPlan group_fused_ordered_plan(int64_t n, int64_t K, int elem_
   return r;
 }
 template <typename T, int CV, int MODE> int launch_group_fused_ordered(const GroupArgs &g, const FusedArgs &f, hipStream_t stream) {
-  constexpr bool kBackward = MODE == GS_SOFTMAX_BWD || MODE == GS_LOG_SOFTMAX_BWD;
   typedef typename Acc<T>::type F;
-  const size_t lds = (size_t)f.tile_vecs * 16 * (kBackward ? 2 : 1) + ((size_t)f.te + 2) * 2;
+  const size_t lds = (size_t)f.tile_vecs * 16 + ((size_t)f.te + 2) * 2;
   const dim3 grid((unsigned)f.nt, (unsigned)f.slices);
   hipLaunchKernelGGL((group_fused_kernel<T, CV, MODE, true>), grid, dim3(kBlock), lds, stream, g, f);
-  hipLaunchKernelGGL((group_fused_combine_kernel<T, MODE>), grid, dim3(kBlock), 0, stream, g, f);
+  hipLaunchKernelGGL((group_fused_combine_kernel<T>), grid, dim3(kBlock), 0, stream, g, f);
   hipLaunchKernelGGL((group_fused_fragment_kernel<T, MODE, true>), grid, dim3(kFusedFragBlock),
                      (size_t)f.kcols * 4 * sizeof(F), stream, g, f);
   return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;

@@ -614,6 +614,15 @@ __global__ __launch_bounds__(kBlock) void group_finish_kernel(GroupArgs g) {
 // logsumexp: result per group, log(sum + eps) + max with the reference's clean-up
 // (composite/logsumexp.py:51-54: NaN and -inf -> 0, +inf -> largest finite value)
 template <typename T>
+__device__ __forceinline__ T group_lse_of(typename Acc<T>::type top, typename Acc<T>::type sum, typename Acc<T>::type eps) {
+  typedef typename Acc<T>::type F;
+  const F l = round_elem<T>(log_acc(round_elem<T>(round_elem<T>(sum) + eps)));
+  F o = round_elem<T>(l + top);
+  if (o != o || o == -INFINITY) o = (F)0;
+  if (o == INFINITY) o = to_acc<T>(ElemLim<T>::max());
+  return from_acc<T>(o);
+}
+template <typename T>
 __global__ __launch_bounds__(kBlock) void group_lse_finish_kernel(GroupArgs g) {
   typedef typename Acc<T>::type F;
   typedef typename OrdKey<F>::bits KB;
@@ -624,12 +633,7 @@ __global__ __launch_bounds__(kBlock) void group_lse_finish_kernel(GroupArgs g) {
   const F eps = (F)g.eps;
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
     const int64_t node = i / g.K, w = node * g.gs + (i - node * g.K);
-    const F m = OrdKey<F>::dec(gmax[w]);
-    const F l = round_elem<T>(log_acc(round_elem<T>(round_elem<T>(gsum[w]) + eps)));
-    F o = round_elem<T>(l + m);
-    if (o != o || o == -INFINITY) o = (F)0;
-    if (o == INFINITY) o = to_acc<T>(ElemLim<T>::max());
-    out[i] = from_acc<T>(o);
+    out[i] = group_lse_of<T>(OrdKey<F>::dec(gmax[w]), gsum[w], eps);
   }
 }
 
@@ -676,7 +680,7 @@ template <typename T, int VEC, int MODE>
 int launch_group_reduce(const GroupArgs &g, hipStream_t stream) {
   if (g.tiles == nullptr) return launch_group_bins<T, VEC, MODE>(g, stream);
   const int rc = launch_group_reduce_fused<T, VEC, MODE>(g, *g.tiles, g.tiles_force != 0, stream);
-  if (rc != TS_OK) return rc;
+  if (rc != TS_OK || g.bins == nullptr) return rc;
   return launch_group_bins<T, VEC, MODE>(g, stream, g.tiles->flag);
 }
 
@@ -688,7 +692,8 @@ int launch_group_softmax_m(const GroupArgs &g_in, hipStream_t stream) {
   if (g.B * g.N >= 0x7FFFFFFFll) return TS_ERR_UNSUPPORTED;
   if (g.in_order != nullptr) return launch_group_fused<T, VEC, MODE>(g, *g.in_order, false, stream, g.in_order_sample != 0);
   if (g.ordered != nullptr) {
-    if constexpr (VEC * sizeof(T) == kVecBytes) return launch_group_fused_ordered<T, VEC, MODE>(g, *g.ordered, stream);
+    if constexpr (kForward && VEC * sizeof(T) == kVecBytes)
+      return launch_group_fused_ordered<T, VEC, MODE>(g, *g.ordered, stream);
     return TS_ERR_UNSUPPORTED;
   }
   const RunGrid rg = run_grid(n_edges, g.K / VEC, VEC, VEC * (int)sizeof(T));

@@ -56,7 +56,8 @@ struct RowSortArgs {
   uint32_t nonce;        // tag of the call, never 0
   const int *gate;       // reads 0: every pass returns at once (null: they run)
   int32_t *state;        // [0] 0: the index is in order, 1: it is not; [1] chunks of large buckets; [2] large buckets;
-                         // [3] the nonce of the latest call that met an index that is not in order; [4] the caller's
+                         // [3] the nonce of the latest call that met an index that is not in order; [4] 1 if these
+                         // passes ran (the caller's word for a gate)
   uint16_t *off;         // [tiles][pitch] first entry of every bucket among the tile's words; [nb]: how many there are
   int log;               // a tile's words lie at tile << log
   uint32_t *words;       // [tiles << log] a tile's entries by bucket: row in the bucket << kRsLocal | place in the tile
@@ -296,7 +297,10 @@ void rs_place_kernel(RowSortArgs p) {
   if (threadIdx.x == 0) {
     s_desc = 0;
     s_gaps.n = 0;
-    if (blockIdx.x == 0) p.state[1] = p.state[2] = 0;
+    if (blockIdx.x == 0) {
+      p.state[1] = p.state[2] = 0;
+      p.state[4] = 1;
+    }
   }
 #pragma unroll
   for (int j = 0; j < PER; ++j) {

@@ -883,17 +883,17 @@ struct GroupSoftmaxFn : public torch::autograd::Function<GroupSoftmaxFn> {
     src = src.contiguous();
     const GroupLayout l = group_layout(src, index, dim);
     Tensor out = at::empty_like(src), order;
-    const size_t order_bytes = on_16_bytes(src) ? ts_group_order_bytes(l.B, l.E, l.K, N, dtype_code(src)) : 0;
+    const size_t order_bytes = on_16_bytes(src) ? ts_group_rows_order_bytes(l.B, l.E, l.K, N, dtype_code(src), 0) : 0;
     if (order_bytes > 0) {
       // the entries sorted by group; the backward pass takes the order of this call
       order = workspace(order_bytes, src);
-      const size_t ws_bytes = ts_group_order_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src), 0);
+      const size_t ws_bytes = ts_group_rows_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src), 0, 0);
       Tensor ws = workspace(ws_bytes, src);
       check_status(ts_group_softmax_ordered(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(), l.B, l.E, l.K, N,
                                             l.sb, l.se, dtype_code(src), log_space ? 1 : 0, eps, order.data_ptr(),
                                             order_bytes, ws.data_ptr(), ws_bytes, stream_of(src)),
                    "scatter_softmax");
-      if (!train || ts_group_order_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src), 1) == 0) order = Tensor();
+      if (!train) order = Tensor();
     } else {
       // the workspace that opens every other route: three passes, buckets of groups, one-pass tiles
       Tensor ws = workspace(ts_group_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src)), src);
@@ -920,7 +920,7 @@ struct GroupSoftmaxFn : public torch::autograd::Function<GroupSoftmaxFn> {
     const GroupLayout l = group_layout(out, index, dim);
     Tensor grad_in = at::empty_like(out);
     if (order.defined() && on_16_bytes(order) && on_16_bytes(out) && on_16_bytes(grad_out)) {  // (hooks may have moved what was saved)
-      const size_t ws_bytes = ts_group_order_workspace_bytes(l.B, l.E, l.K, N, dtype_code(out), 1);
+      const size_t ws_bytes = ts_group_rows_workspace_bytes(l.B, l.E, l.K, N, dtype_code(out), 0, 1);
       Tensor ws = workspace(ws_bytes, out);
       check_status(ts_group_softmax_ordered_backward(out.data_ptr(), grad_out.data_ptr(), index.data_ptr<int64_t>(),
                                                      grad_in.data_ptr(), l.B, l.E, l.K, N, l.sb, l.se, dtype_code(out),
@@ -947,31 +947,55 @@ struct GroupLogSumExpFn : public torch::autograd::Function<GroupLogSumExpFn> {
     check_device(src, "src");
     check_device(index, "index");
     c10::DeviceGuard guard(src.device());
+    const bool train = src.requires_grad();  // (a copy, made with gradients off, would say no)
     src = src.contiguous();
     const GroupLayout l = group_layout(src, index, dim);
     auto sizes = src.sizes().vec();
     sizes[dim] = N;
     Tensor out = at::empty(sizes, src.options());
-    // the larger workspace of the route through buckets of groups, where that route applies
-    const size_t ws_bytes = ts_group_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src));
-    Tensor ws = workspace(ws_bytes, src);
-    check_status(ts_group_logsumexp(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(), l.B, l.E, l.K, N, l.sb,
-                                    l.se, dtype_code(src), eps, ws.data_ptr(), static_cast<size_t>(ws.numel()),
-                                    stream_of(src)),
-                 "scatter_logsumexp");
+    Tensor order;
+    const size_t order_bytes = ts_group_rows_order_bytes(l.B, l.E, l.K, N, dtype_code(src), 1);
+    if (order_bytes > 0) {
+      order = workspace(order_bytes, src);
+      const size_t ws_bytes = ts_group_rows_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src), 1, 0);
+      Tensor ws = workspace(ws_bytes, src);
+      check_status(ts_group_reduce_ordered(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(), nullptr, nullptr, l.B,
+                                           l.E, l.K, N, l.sb, l.se, dtype_code(src), 0, 0, eps, order.data_ptr(), order_bytes,
+                                           ws.data_ptr(), ws_bytes, stream_of(src)),
+                   "scatter_logsumexp");
+      if (!train) order = Tensor();
+    } else {
+      // the larger workspace of the route through buckets of groups, where that route applies
+      const size_t ws_bytes = ts_group_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src));
+      Tensor ws = workspace(ws_bytes, src);
+      check_status(ts_group_logsumexp(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(), l.B, l.E, l.K, N, l.sb,
+                                      l.se, dtype_code(src), eps, ws.data_ptr(), static_cast<size_t>(ws.numel()),
+                                      stream_of(src)),
+                   "scatter_logsumexp");
+    }
     ctx->saved_data["dim"] = dim;
-    ctx->save_for_backward({src, index, out});
+    ctx->save_for_backward({src, index, out, order});
     return {out};
   }
 
   static variable_list backward(AutogradContext *ctx, variable_list grad_outs) {
     auto saved = ctx->get_saved_variables();
-    Tensor src = saved[0], index = saved[1], out = saved[2];
+    Tensor src = saved[0], index = saved[1], out = saved[2], order = saved[3];
     Tensor grad_out = grad_outs[0].contiguous();
     c10::DeviceGuard guard(src.device());
     const int64_t dim = ctx->saved_data["dim"].toInt();
     const GroupLayout l = group_layout(src, index, dim);
     Tensor grad_in = at::empty_like(src);
+    if (order.defined() && on_16_bytes(order)) {  // (hooks may have moved what was saved)
+      const size_t ws_bytes = ts_group_rows_workspace_bytes(l.B, l.E, l.K, out.size(dim), dtype_code(src), 1, 1);
+      Tensor ws = workspace(ws_bytes, src);
+      check_status(ts_group_reduce_ordered_backward(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(), nullptr, nullptr,
+                                                    grad_out.data_ptr(), grad_in.data_ptr(), l.B, l.E, l.K, out.size(dim), l.sb,
+                                                    l.se, dtype_code(src), 0, 0, order.data_ptr(),
+                                                    static_cast<size_t>(order.numel()), ws.data_ptr(), ws_bytes, stream_of(src)),
+                   "scatter_logsumexp backward");
+      return {grad_in, Variable(), Variable(), Variable(), Variable()};
+    }
     Tensor ws = workspace(ts_group_softmax_workspace_bytes(l.B, out.size(dim), l.K, dtype_code(src)), src);
     check_status(ts_group_logsumexp_backward_with_workspace(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(),
                                                             grad_out.data_ptr(), grad_in.data_ptr(), l.B, l.E, l.K,
@@ -990,11 +1014,28 @@ struct GroupStdFn : public torch::autograd::Function<GroupStdFn> {
     check_device(src, "src");
     check_device(index, "index");
     c10::DeviceGuard guard(src.device());
+    const bool train = src.requires_grad();
     src = src.contiguous();
     const GroupLayout l = group_layout(src, index, dim);
-    Tensor total, count, out;
+    Tensor total, count, out, order;
+    const size_t order_bytes = ts_group_rows_order_bytes(l.B, l.E, l.K, N, dtype_code(src), 2);
     const size_t bins_bytes = ts_group_std_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src));
-    if (bins_bytes > 0 && l.B * N * l.K > 0 && (reinterpret_cast<uintptr_t>(src.data_ptr()) & 15) == 0) {
+    if (order_bytes > 0) {
+      auto sizes = src.sizes().vec();
+      sizes[dim] = N;
+      total = at::empty(sizes, src.options());
+      count = at::empty({l.B * N}, src.options().dtype(at::kInt));
+      out = at::empty_like(total);
+      order = workspace(order_bytes, src);
+      const size_t ws_bytes = ts_group_rows_workspace_bytes(l.B, l.E, l.K, N, dtype_code(src), 2, 0);
+      Tensor ws = workspace(ws_bytes, src);
+      check_status(ts_group_reduce_ordered(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(), total.data_ptr(),
+                                           count.data_ptr<int32_t>(), l.B, l.E, l.K, N, l.sb, l.se, dtype_code(src), 1,
+                                           unbiased ? 1 : 0, 0.0, order.data_ptr(), order_bytes, ws.data_ptr(), ws_bytes,
+                                           stream_of(src)),
+                   "scatter_std");
+      if (!train) order = Tensor();
+    } else if (bins_bytes > 0 && l.B * N * l.K > 0 && (reinterpret_cast<uintptr_t>(src.data_ptr()) & 15) == 0) {
       // group sums, counts and result in one call (buckets of groups, or the entries sorted by group)
       auto sizes = src.sizes().vec();
       sizes[dim] = N;
@@ -1023,19 +1064,30 @@ struct GroupStdFn : public torch::autograd::Function<GroupStdFn> {
     }
     ctx->saved_data["dim"] = dim;
     ctx->saved_data["unbiased"] = unbiased;
-    ctx->save_for_backward({src, index, total, count, out});
+    ctx->save_for_backward({src, index, total, count, out, order});
     return {out};
   }
 
   static variable_list backward(AutogradContext *ctx, variable_list grad_outs) {
     auto saved = ctx->get_saved_variables();
-    Tensor src = saved[0], index = saved[1], total = saved[2], count = saved[3], out = saved[4];
+    Tensor src = saved[0], index = saved[1], total = saved[2], count = saved[3], out = saved[4], order = saved[5];
     Tensor grad_out = grad_outs[0].contiguous();
     c10::DeviceGuard guard(src.device());
     const int64_t dim = ctx->saved_data["dim"].toInt();
     const bool unbiased = ctx->saved_data["unbiased"].toBool();
     const GroupLayout l = group_layout(src, index, dim);
     Tensor grad_in = at::empty_like(src);
+    if (order.defined() && on_16_bytes(order)) {
+      const size_t ws_bytes = ts_group_rows_workspace_bytes(l.B, l.E, l.K, out.size(dim), dtype_code(src), 2, 1);
+      Tensor ws = workspace(ws_bytes, src);
+      check_status(ts_group_reduce_ordered_backward(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(), total.data_ptr(),
+                                                    count.data_ptr<int32_t>(), grad_out.data_ptr(), grad_in.data_ptr(), l.B, l.E,
+                                                    l.K, out.size(dim), l.sb, l.se, dtype_code(src), 1, unbiased ? 1 : 0,
+                                                    order.data_ptr(), static_cast<size_t>(order.numel()), ws.data_ptr(), ws_bytes,
+                                                    stream_of(src)),
+                   "scatter_std backward");
+      return {grad_in, Variable(), Variable(), Variable(), Variable()};
+    }
     Tensor ws = workspace(ts_group_softmax_workspace_bytes(l.B, out.size(dim), l.K, dtype_code(src)), src);
     check_status(ts_group_std_backward_with_workspace(src.data_ptr(), index.data_ptr<int64_t>(), total.data_ptr(),
                                                       count.data_ptr<int32_t>(), out.data_ptr(), grad_out.data_ptr(),
