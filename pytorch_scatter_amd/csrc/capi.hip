@@ -257,7 +257,7 @@ RowsRoute rows_route(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int 
   RowsRoute r = {false, 0, 0};
   const int mode = env_int("TS_SCATTER_BINNED", 1);  // tuning aid: 0 never, 2 at any size
   const int64_t row_bytes = K * kElemBytes[dtype], n = B * E, rows = B * N;
-  if (mode == 0 || B < 1 || E < 1 || N < 1 || row_bytes < 64 || !env_int("TS_CSR_LOOKBACK", 1)) return r;
+  if (mode == 0 || B < 1 || E < 1 || N < 1 || row_bytes < 64 || row_bytes > 0xFFFFFFFFll || !env_int("TS_CSR_LOOKBACK", 1)) return r;
   const bool minmax = reduce == TS_MIN || reduce == TS_MAX;
   if (!minmax && reduce != TS_SUM && reduce != TS_MEAN) return r;
   if (!minmax && kAccBytes[dtype] < 4) return r;

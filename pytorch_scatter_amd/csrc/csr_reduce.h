@@ -149,7 +149,10 @@ __device__ __forceinline__ double sqrt_acc(double v) { return sqrt(v); }
 template <typename T> __device__ __forceinline__ typename Acc<T>::type round_elem(typename Acc<T>::type v) {
   return to_acc<T>(from_acc<T>(v));
 }
-template <> __device__ __forceinline__ float round_elem<bf16_t>(float v) { return (float)(__bf16)v; }  // (any NaN stays one)
+template <> __device__ __forceinline__ float round_elem<bf16_t>(float v) {
+  asm("" : "+v"(v));  // see float_to_bf16
+  return (float)(__bf16)v;  // (any NaN stays one)
+}
 // std: the group mean as the reference forms it (composite/std.py:27-31: sum / clamp(count, 1), in the
 // element type) and the divisor of the squared deviations (:36-38: count or clamp(count - 1, 1), plus 1e-6)
 template <typename T> __device__ __forceinline__ typename Acc<T>::type group_mean(T total, int32_t count) {
@@ -470,6 +473,7 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
 
   const int64_t col_ld = col_ok ? col : 0;  // idle lanes re-read column 0
   const T *src_col = src_b + col_ld;
+  const uint32_t row_bytes = (uint32_t)a.K * (uint32_t)sizeof(T);  // (scatter: the host sees that they fit)
   // Software pipeline: the loads of batch i+1 are issued before batch i is
   // reduced, so a wavefront always has U to 2U 16-byte loads outstanding.
   // Direct: rows in place; of a scatter whose index was in order, with positions that ascend (no ties to settle, nothing read
@@ -480,15 +484,18 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         int ee = e + u < je1 ? e + u : je1 - 1;
-        const int64_t srow = kDirect ? j0 + ee : (int64_t)s_perm[ee];
-        x[u] = load_vec_stream<T, VEC>(src_col + srow * a.K);
+        if constexpr (kTies) {
+          // (entries and bytes of a row in 32 bits: one multiplication and addition instead of three and four instructions)
+          const uint32_t srow = kDirect ? (uint32_t)j0 + (uint32_t)ee : (uint32_t)s_perm[ee];
+          x[u] = load_vec_stream<T, VEC>(reinterpret_cast<const T *>(reinterpret_cast<const char *>(src_col) +
+                                                                     (uint64_t)srow * row_bytes));
+        } else {
+          const int64_t srow = kDirect ? j0 + ee : (int64_t)s_perm[ee];
+          x[u] = load_vec_stream<T, VEC>(src_col + srow * a.K);
+        }
       }
     };
-    Vec<T, VEC> x[U];
-    if (je0 < je1) load_batch(x, je0);
-    for (int e = je0; e < je1; e += U) {
-      Vec<T, VEC> y[U];
-      load_batch(y, e + U);  // unconditional (addresses are clamped): keeps the wait counts exact
+    auto reduce_batch = [&](const Vec<T, VEC> *x, int e) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int ce = e + u;
@@ -506,8 +513,26 @@ __global__ __launch_bounds__(kCsrBlock, (csr_reduce_min_blocks<T, VEC, REDUCE, P
           }
         }
       }
+    };
+    Vec<T, VEC> x[U];
+    if (je0 < je1) load_batch(x, je0);
+    if constexpr (kThrough && !kArg) {
+      Vec<T, VEC> y[U];
+      // two batches in turn: a copy from one to the other waits for its loads at the end of every round and takes 4 U instructions
+      for (int e = je0; e < je1; e += 2 * U) {
+        load_batch(y, e + U);
+        reduce_batch(x, e);
+        load_batch(x, e + 2 * U);
+        reduce_batch(y, e + U);
+      }
+    } else {
+      for (int e = je0; e < je1; e += U) {
+        Vec<T, VEC> y[U];
+        load_batch(y, e + U);  // unconditional (addresses are clamped): keeps the wait counts exact
+        reduce_batch(x, e);
 #pragma unroll
-      for (int u = 0; u < U; ++u) x[u] = y[u];
+        for (int u = 0; u < U; ++u) x[u] = y[u];
+      }
     }
   };
   if constexpr (kTies) {
