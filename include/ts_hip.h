@@ -249,6 +249,22 @@ int ts_scatter_with_workspace(const void *src, const int64_t *index, void *out,
                               int dtype, int reduce, int out_given, void *workspace,
                               size_t workspace_bytes, ts_stream_t stream);
 
+/* The same for wide rows of floating types whose entries are sorted by row (ts_scatter_last_route() names the route), with the
+ * order left in `order` for the backward call: ts_scatter_order_bytes() bytes of device memory (0: the order is not made for
+ * this call, TS_ERR_UNSUPPORTED), 16-byte aligned, as is the workspace of ts_scatter_order_workspace_bytes() bytes, whose last
+ * TS_STATUS_BYTES are status words. reduce: TS_SUM, TS_MIN, TS_MAX; count (may be null): entries per row.
+ * The backward call gives every entry its row's gradient (mean: divided by the row's entries) where arg is null, else (min,
+ * max) to the entry at its position alone; entries outside [0, N) get zeros. Same index, sizes and dtype as the forward call. */
+size_t ts_scatter_order_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce);
+size_t ts_scatter_order_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce);
+int ts_scatter_ordered(const void *src, const int64_t *index, void *out, int64_t *arg_out, int32_t *count, int64_t B,
+                       int64_t E, int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype, int reduce,
+                       int out_given, void *order, size_t order_bytes, void *workspace, size_t workspace_bytes,
+                       ts_stream_t stream);
+int ts_scatter_ordered_backward(const void *grad_out, const int64_t *arg, const int64_t *index, void *grad_in, int64_t B,
+                                int64_t E, int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype,
+                                int mean, const void *order, size_t order_bytes, ts_stream_t stream);
+
 /* Which kernels the last ts_scatter / ts_scatter_with_workspace / ts_scatter_small call of the calling thread launched: a host-side
  * note for tests and tools (no device call, no synchronisation). Where two kernels are launched and a flag
  * written on the device picks the one that does the work (a sample or a full check of the index), the name says

@@ -29,6 +29,7 @@ EXPORTS = (
     "ts_scatter", "ts_scatter_workspace_bytes", "ts_scatter_workspace_zero_bytes", "ts_scatter_with_workspace", "ts_scatter_count", "ts_scatter_count_workspace_bytes", "ts_scatter_count_with_workspace", "ts_scatter_sum_count_workspace_bytes", "ts_scatter_sum_count_with_workspace", "ts_divide_by_count", "ts_arg_backward",
     "ts_arg_backward_rows_workspace_bytes", "ts_arg_backward_rows",
     "ts_scatter_small_applies", "ts_scatter_small",
+    "ts_scatter_order_bytes", "ts_scatter_order_workspace_bytes", "ts_scatter_ordered", "ts_scatter_ordered_backward",
     "ts_group_softmax_workspace_bytes", "ts_group_softmax", "ts_group_softmax_backward",
     "ts_group_order_bytes", "ts_group_order_workspace_bytes", "ts_group_softmax_ordered", "ts_group_softmax_ordered_backward",
     "ts_group_rows_order_bytes", "ts_group_rows_workspace_bytes", "ts_group_reduce_ordered", "ts_group_reduce_ordered_backward",
@@ -62,6 +63,8 @@ def lib() -> ctypes.CDLL:
         _lib.ts_group_softmax_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_group_order_bytes.restype = ctypes.c_size_t
         _lib.ts_group_order_workspace_bytes.restype = ctypes.c_size_t
+        _lib.ts_scatter_order_bytes.restype = ctypes.c_size_t
+        _lib.ts_scatter_order_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_group_rows_order_bytes.restype = ctypes.c_size_t
         _lib.ts_group_rows_workspace_bytes.restype = ctypes.c_size_t
         _lib.ts_indptr_to_index_workspace_bytes.restype = ctypes.c_size_t

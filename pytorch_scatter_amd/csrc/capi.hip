@@ -801,7 +801,98 @@ int scatter_ws_impl(const void *src, const int64_t *index, void *out, int64_t *a
   return dispatch_scatter(dtype, a, reduce, vec, s);
 }
 }  // namespace
+namespace {
+// Scatter with wide rows whose order stays for the backward pass. us forward and backward, without / with the order:
+//   sums   the gradients' rows in whole lines, from 32 MB of them: 2.3 M x 128 bf16 onto 268 k rows 361 / 304, 603 k x 128 floats
+//          onto 176 k 194 / 163, 1.9 M x 32 floats onto 1.05 M 201 / 186. What the L2 holds is gathered faster than entries' rows are
+//          written in no order: 9.7 M x 16 floats onto 65 k 386 / 541; so are rows that are not whole lines, 742 k x 100 doubles 290 / 357
+//   min / max   from 366 MB of entries, beyond the memory-side cache: 2.3 M x 64 floats onto 282 k rows 454 / 381, 678 k x 256 floats
+//          onto 19 k 511 / 304, 678 k x 128 doubles onto 1.4 k 336 / 300; with up to eight entries a row from 32 MB: 3.2 M x 32 floats
+//          onto 1.1 M 618 / 430, 3.4 M x 8 doubles onto 429 k 234 / 210. Else a fill and a scatter of single elements: 525 k x 128
+//          floats onto 2.4 k 147 / 160; 240 k x 100 floats under a hub 112 / 128 (rows that are not whole 64 bytes)
+// TS_SCATTER_ORDER (tuning aid): 0 never, 2 wherever the entries are sorted.
+bool scatter_order_ok(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce, RowsRoute &rr) {
+  if (!valid_dtype(dtype) || !is_float_dtype(dtype) || !sizes_ok(B, N, E, K) || B * E * K == 0 || N == 0) return false;
+  if (reduce != TS_SUM && reduce != TS_MIN && reduce != TS_MAX) return false;
+  const int mode = env_int("TS_SCATTER_ORDER", 1);
+  const int64_t row_bytes = K * kElemBytes[dtype], MB = (int64_t)1 << 20;
+  if (mode == 0 || (reduce != TS_SUM && row_bytes % kVecBytes != 0)) return false;
+  if (mode != 2) {
+    if (reduce == TS_SUM && (row_bytes % 128 != 0 || B * N * row_bytes < 32 * MB)) return false;
+    if (reduce != TS_SUM && (row_bytes % 64 != 0 || B * E * row_bytes < (E > 8 * N ? 366 * MB : 32 * MB))) return false;
+  }
+  rr = rows_route(B, E, K, N, dtype, reduce);
+  return rr.ok;
+}
+}  // namespace
 extern "C" {
+
+size_t ts_scatter_order_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce) {
+  RowsRoute rr;
+  return scatter_order_ok(B, E, K, N, dtype, reduce, rr) ? row_sort_plan(B, E, N, nullptr, 0, true).kept_bytes : 0;
+}
+
+size_t ts_scatter_order_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce) {
+  RowsRoute rr;
+  if (!scatter_order_ok(B, E, K, N, dtype, reduce, rr)) return 0;
+  const RowSortPlan sp = row_sort_plan(B, E, N, nullptr, 0, true);
+  return sp.bytes - sp.kept_bytes + rr.csr_bytes + kStatusBytes;
+}
+
+int ts_scatter_ordered(const void *src, const int64_t *index, void *out, int64_t *arg_out, int32_t *count, int64_t B, int64_t E,
+                       int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype, int reduce, int out_given,
+                       void *order, size_t order_bytes, void *workspace, size_t workspace_bytes, ts_stream_t stream) {
+  RowsRoute rr;
+  if (!scatter_order_ok(B, E, K, N, dtype, reduce, rr)) return TS_ERR_UNSUPPORTED;
+  ts_note_scatter_route(TS_ROUTE_NONE);
+  if (!src || !index || !out || (reduce != TS_SUM && !arg_out)) return TS_ERR_BAD_ARG;
+  if (!order || !aligned16(order) || !workspace || !aligned16(workspace)) return TS_ERR_WORKSPACE;
+  const size_t kept = row_sort_plan(B, E, N, nullptr, 0, true).kept_bytes;
+  const size_t sort = row_sort_plan(B, E, N, nullptr, 0, true).bytes - kept;
+  if (order_bytes < kept || workspace_bytes < sort + rr.csr_bytes + kStatusBytes) return TS_ERR_WORKSPACE;
+  const RowSortPlan sp = row_sort_plan(B, E, N, workspace, sort, true, order);
+  if (!sp.ok) return TS_ERR_WORKSPACE;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  ts_note_scatter_route(reduce == TS_SUM ? TS_ROUTE_SUM_BUCKETS_OR_SEGMENTED : TS_ROUTE_MINMAX_BUCKETS_OR_SEGMENTED);
+  int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, false, next_nonce(), s);
+  if (rc != TS_OK) return rc;
+  rc = run_rows_reduce(src, sp.p, out, arg_out, B, E, K, N, dtype, reduce, out_given,
+                       static_cast<char *>(workspace) + sort, rr.csr_bytes, next_nonce(), s);
+  if (rc != TS_OK || count == nullptr) return rc;
+  hipLaunchKernelGGL(row_lengths_kernel, dim3(grid_for(B * N)), dim3(kBlock), 0, s, sp.p.ptr, count, B * N);
+  return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
+}
+
+int ts_scatter_ordered_backward(const void *grad_out, const int64_t *arg, const int64_t *index, void *grad_in, int64_t B,
+                                int64_t E, int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e, int dtype,
+                                int mean, const void *order, size_t order_bytes, ts_stream_t stream) {
+  RowsRoute rr;
+  // (minimum and maximum take their order at the same sizes)
+  if (!scatter_order_ok(B, E, K, N, dtype, arg != nullptr ? TS_MAX : TS_SUM, rr)) return TS_ERR_UNSUPPORTED;
+  if (!grad_out || !index || !grad_in) return TS_ERR_BAD_ARG;
+  RowSortPlan sp = row_sort_plan(B, E, N, nullptr, 0, true, const_cast<void *>(order));
+  if (!order || !aligned16(order) || order_bytes < sp.kept_bytes || !sp.ok) return TS_ERR_WORKSPACE;
+  RowSortArgs p = sp.p;
+  p.index = index;
+  p.sb = index_stride_b;
+  p.se = index_stride_e;
+  p.flat = B == 1 && index_stride_e == 1;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (arg != nullptr) {
+    if (!aligned16(grad_out) || !aligned16(arg) || !aligned16(grad_in)) return TS_ERR_UNSUPPORTED;
+    switch (kElemBytes[dtype]) {
+    case 2: return launch_arg_rows<uint16_t, 8>(p, grad_out, arg, grad_in, K, s);
+    case 4: return launch_arg_rows<uint32_t, 4>(p, grad_out, arg, grad_in, K, s);
+    default: return launch_arg_rows<uint64_t, 2>(p, grad_out, arg, grad_in, K, s);
+    }
+  }
+  switch (dtype) {
+  case TS_F32: return launch_rows_spread<float>(p, grad_out, grad_in, K, mean != 0, s);
+  case TS_F64: return launch_rows_spread<double>(p, grad_out, grad_in, K, mean != 0, s);
+  case TS_F16: return launch_rows_spread<f16_t>(p, grad_out, grad_in, K, mean != 0, s);
+  default: return launch_rows_spread<bf16_t>(p, grad_out, grad_in, K, mean != 0, s);
+  }
+}
 
 int ts_scatter_with_workspace(const void *src, const int64_t *index, void *out, int64_t *arg_out, int64_t B,
                               int64_t E, int64_t K, int64_t N, int64_t index_stride_b, int64_t index_stride_e,
@@ -1069,7 +1160,7 @@ int ts_arg_backward_rows(const void *grad_out, const int64_t *arg, const int64_t
   RowSortPlan sp = row_sort_plan(B, E, N, workspace, workspace_bytes, true);
   if (!sp.ok) return TS_ERR_WORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, true, next_nonce(), s);
+  const int rc = launch_row_sort(sp.p, index, index_stride_b, index_stride_e, false, next_nonce(), s);
   if (rc != TS_OK) return rc;
   RowSortArgs p = sp.p;
   p.index = index;

@@ -877,6 +877,81 @@ __global__ __launch_bounds__(kRowsBlock) void group_rows_map_kernel(GroupArgs g,
   }
 }
 
+// Backward of a scatter sum or mean over the order of its forward pass: every entry's gradient is its row's (divided by the row's
+// entries). Places of a row read it together, and only the entries' rows are written in no order, in whole pieces: 2.3 M x 128 bf16
+// onto 268 k rows, 115 us (5.7 TB/s) against 165 for a gather in the order of memory, which fetches every row from anywhere.
+struct RowsSpreadArgs {
+  const void *grad;  // [rows, K]
+  void *grad_in;     // [n, K]
+  int64_t K;
+  int lanes, workers;
+  uint32_t inv;
+  int kcols, stream;
+};
+template <typename T, int VEC, bool DIV>
+__global__ __launch_bounds__(kBlock) void rows_spread_kernel(RowSortArgs p, RowsSpreadArgs a) {
+  typedef Vec<T, VEC> V;
+  constexpr int Q = 4;
+  typedef int32_t i4 __attribute__((ext_vector_type(4)));
+  const int tid = threadIdx.x, K = (int)a.K, L = a.lanes;
+  const int w = (int)(((uint32_t)tid * a.inv) >> 16), l = tid - w * L;
+  const int64_t n = p.ptr[p.rows], w0 = (int64_t)blockIdx.x * (a.workers * Q);
+  const int k_first = (int)blockIdx.y * a.kcols, k_end = K - k_first < a.kcols ? K : k_first + a.kcols;
+  T *out = static_cast<T *>(a.grad_in);
+  if (n != p.n) {  // zeros for the entries outside [0, N)
+    for (int64_t e = w0 + tid / kWave; e < p.n && e < w0 + a.workers * Q; e += kBlock / kWave) {
+      if (rs_node(p, e) >= 0) continue;
+      for (int k = k_first + (tid & (kWave - 1)); k < k_end; k += kWave) out[e * K + k] = zero_elem<T>();
+    }
+  }
+  const int first = k_first + l * VEC;
+  const int64_t p0 = w0 + w * Q;
+  if (w >= a.workers || first >= k_end || p0 >= n) return;
+  const int col = first + VEC <= K ? first : K - VEC;  // (the last lane: columns that its neighbour has as well)
+  const i4 row = *reinterpret_cast<const i4 *>(p.perm_row + p0);  // (the arrays end on whole 256 bytes)
+  i4 entry = {(int)p0, (int)p0 + 1, (int)p0 + 2, (int)p0 + 3};
+  if (p.state[0] != 0) entry = *reinterpret_cast<const i4 *>(p.perm + p0);
+  V g[Q];
+  int64_t len[DIV ? Q : 1];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int64_t r = p0 + q < n ? row[q] : row[0];
+    g[q] = rows_load<T, VEC>(static_cast<const T *>(a.grad) + r * K + col);
+    if constexpr (DIV) len[q] = p.ptr[r + 1] - p.ptr[r];
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    if (p0 + q >= n) continue;
+    if constexpr (DIV) {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) g[q].v[v] = div_elem<T>(g[q].v[v], count_as<T>(len[q]));
+    }
+    rows_store<T, VEC>(out + (int64_t)entry[q] * K + col, g[q], a.stream != 0);
+  }
+}
+template <typename T> int launch_rows_spread(const RowSortArgs &p, const void *grad, void *grad_in, int64_t K, bool mean, hipStream_t stream);
+template <typename T> int launch_rows_spread_t(const RowSortArgs &p, const void *grad, void *grad_in, int64_t K, bool mean, hipStream_t stream) {
+  constexpr int VEC = kVecBytes / (int)sizeof(T);
+  RowsSpreadArgs a;
+  a.grad = grad;
+  a.grad_in = grad_in;
+  a.K = K;
+  const int64_t all = (K + VEC - 1) / VEC, slices = (all + kWave - 1) / kWave;
+  if (K < VEC || slices > 65535 || K > 0x7FFFFFFFll) return TS_ERR_UNSUPPORTED;
+  a.lanes = (int)((all + slices - 1) / slices);
+  a.workers = kBlock / a.lanes;
+  a.inv = 65536u / (uint32_t)a.lanes + 1;
+  a.kcols = a.lanes * VEC;
+  a.stream = K * (int64_t)sizeof(T) % 128 == 0 && (reinterpret_cast<uintptr_t>(grad_in) & 127) == 0;
+  const int64_t per = (int64_t)a.workers * 4;
+  const dim3 grid((unsigned)((p.n + per - 1) / per), (unsigned)((all + a.lanes - 1) / a.lanes));
+  if (mean)
+    hipLaunchKernelGGL((rows_spread_kernel<T, VEC, true>), grid, dim3(kBlock), 0, stream, p, a);
+  else
+    hipLaunchKernelGGL((rows_spread_kernel<T, VEC, false>), grid, dim3(kBlock), 0, stream, p, a);
+  return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
+}
+
 template <typename T, int VEC, int MODE> int launch_group_rows_m(const GroupArgs &g, const GroupRowsArgs &f, hipStream_t stream) {
   constexpr bool kReduce = MODE == GS_LSE || MODE == GS_STD;
   if constexpr (MODE == GS_STD_BWD || MODE == GS_LSE_BWD) {
@@ -912,6 +987,10 @@ template <typename T> int launch_group_rows(const GroupArgs &g, const GroupRowsA
   template <> int launch_group_rows<T>(const GroupArgs &g, const GroupRowsArgs &f, int mode, hipStream_t stream) { \
     if (g.K >= group_rows_full<T>()) return launch_group_rows_v<T, group_rows_full<T>()>(g, f, mode, stream);     \
     return launch_group_rows_v<T, 1>(g, f, mode, stream);                                                         \
+  }                                                                                                               \
+  template <> int launch_rows_spread<T>(const RowSortArgs &p, const void *grad, void *grad_in, int64_t K, bool mean, \
+                                        hipStream_t stream) {                                                     \
+    return launch_rows_spread_t<T>(p, grad, grad_in, K, mean, stream);                                            \
   }
 
 }  // namespace ts

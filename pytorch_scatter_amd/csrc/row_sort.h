@@ -692,32 +692,52 @@ static __global__ __launch_bounds__(kBlock) void row_lengths_kernel(const int64_
 // Backward of scatter min / max over entries sorted by row: grad_in[e, k] = grad[row, k] where arg[row, k] == e, else 0.
 // Every row of grad_in is written once, in one piece, and the entries of a row read its gradient and positions from the
 // vector L1. (A fill of grad_in and a scatter of single elements into it writes the buffer twice: 2.3 M x 64 floats onto
-// 282 k rows 368 us, of which the scatter 260; this kernel 210 and the sort 33, 3.9 TB/s in rows of 256 bytes in no order.)
-// U: bits of an element. A workgroup takes 4 positions per worker.
+// 282 k rows 368 us, of which the scatter 260; this kernel 173, 4.7 TB/s in rows of 256 bytes in no order.)
+// U: bits of an element. A worker takes 4 neighbouring places.
 template <typename U, int VEC>
 static __global__ __launch_bounds__(kBlock) void rs_arg_rows_kernel(RowSortArgs p, const U *__restrict__ grad,
                                                                     const int64_t *__restrict__ arg,
                                                                     U *__restrict__ grad_in, int64_t K, int G) {
   constexpr int Q = 4;
+  typedef int32_t i4 __attribute__((ext_vector_type(4)));
   const int W = kBlock / G, w = threadIdx.x / G, lg = threadIdx.x - w * G;
   const int64_t col = ((int64_t)blockIdx.y * G + lg) * VEC;
-  if (col >= K) return;
   const int64_t n = p.ptr[p.rows];  // entries inside [0, N)
-  const int64_t base = (int64_t)blockIdx.x * W * Q + w;
-  int32_t e[Q], row[Q];
+  const int64_t p0 = ((int64_t)blockIdx.x * W + w) * Q;
+  if (col >= K || p0 >= n) return;
+  const int cnt = n - p0 < Q ? (int)(n - p0) : Q;
+  i4 row = *reinterpret_cast<const i4 *>(p.perm_row + p0);  // (the arrays end on whole 256 bytes)
+  i4 e = {(int)p0, (int)p0 + 1, (int)p0 + 2, (int)p0 + 3};
+  if (p.state[0] != 0) e = *reinterpret_cast<const i4 *>(p.perm + p0);
 #pragma unroll
-  for (int q = 0; q < Q; ++q) e[q] = base + (int64_t)q * W < n ? p.perm[base + (int64_t)q * W] : -1;
+  for (int q = 1; q < Q; ++q) row[q] = q < cnt ? row[q] : row[0];
+  // neighbouring places mostly share a row or two: those of the first and the last are on the way together, a third one's behind a
+  // condition (2.3 M x 64 floats onto 282 k rows 173 us; with a row's loads for every place 207: twice as much from the vector L1)
+  Vec<int64_t, VEC> a[2];
+  Vec<U, VEC> g[2];
 #pragma unroll
-  for (int q = 0; q < Q; ++q) row[q] = e[q] >= 0 ? p.perm_row[base + (int64_t)q * W] : 0;
+  for (int i = 0; i < 2; ++i) {
+    const int64_t at = (int64_t)row[i == 0 ? 0 : Q - 1] * K + col;
+    a[i] = load_vec<int64_t, VEC>(arg + at);
+    g[i] = load_vec<U, VEC>(grad + at);
+  }
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    if (e[q] < 0) continue;
-    const Vec<int64_t, VEC> a = load_vec<int64_t, VEC>(arg + (int64_t)row[q] * K + col);
-    const Vec<U, VEC> g = load_vec<U, VEC>(grad + (int64_t)row[q] * K + col);
-    const int64_t at = p.B > 1 ? (int64_t)((uint32_t)e[q] % (uint32_t)p.E) : (int64_t)e[q];  // inside its batch
+    if (q >= cnt) continue;
+    if (q > 0 && row[q] != row[0]) {
+      if (row[q] == row[Q - 1]) {
+        a[0] = a[1];
+        g[0] = g[1];
+      } else {
+        a[0] = load_vec<int64_t, VEC>(arg + (int64_t)row[q] * K + col);
+        g[0] = load_vec<U, VEC>(grad + (int64_t)row[q] * K + col);
+      }
+      row[0] = row[q];
+    }
+    const uint32_t pos = p.B > 1 ? (uint32_t)e[q] % (uint32_t)p.E : (uint32_t)e[q];  // inside its batch
     Vec<U, VEC> o;
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) o.v[v] = a.v[v] == at ? g.v[v] : (U)0;
+    for (int v = 0; v < VEC; ++v) o.v[v] = (uint32_t)a[0].v[v] == pos ? g[0].v[v] : (U)0;  // (positions fit 31 bits)
     store_vec_stream<U, VEC>(grad_in + (int64_t)e[q] * K + col, o);
   }
 }

@@ -194,13 +194,14 @@ BatchedIndex batched_index(const Tensor &idx) {
 // are left here; else it stays undefined
 // small_mean (sum only): a small call divides by the count in the launch that adds; *divided then reads true and, with
 // counted, *small_count holds the divisor in the element type [B * N]
+// order (may be null): where the entries are sorted by row, their order is left here for the backward pass
 struct SmallMean {
   bool counted = false, divided = false;
   Tensor count;
 };
 std::tuple<Tensor, OptTensor> scatter_hip(Tensor src, Tensor index, int64_t dim, OptTensor optional_out,
                                           OptInt dim_size, int reduce, Tensor *mean_count = nullptr,
-                                          SmallMean *small_mean = nullptr) {
+                                          SmallMean *small_mean = nullptr, Tensor *order = nullptr) {
   check_device(src, "src");
   check_device(index, "index");
   if (optional_out.has_value()) check_device(optional_out.value(), "out");
@@ -278,6 +279,21 @@ std::tuple<Tensor, OptTensor> scatter_hip(Tensor src, Tensor index, int64_t dim,
                                   dtype_code(src), small_reduce, optional_out.has_value() ? 1 : 0, stream_of(src)),
                  "scatter");
     if (mean) small_mean->divided = true;
+    return std::make_tuple(out, arg_out);
+  }
+  const size_t order_bytes = order != nullptr && sk.value() == 0 ? ts_scatter_order_bytes(B, E, K, N, dtype_code(src), reduce) : 0;
+  if (order_bytes > 0) {
+    *order = workspace(order_bytes, src);
+    const size_t bytes = ts_scatter_order_workspace_bytes(B, E, K, N, dtype_code(src), reduce);
+    Tensor ows = workspace(bytes, src), count;
+    if (mean_count != nullptr) count = *mean_count = at::empty({B * N}, src.options().dtype(at::kInt));
+    check_status(ts_scatter_ordered(src.data_ptr(), index.data_ptr<int64_t>(), out.data_ptr(),
+                                    minmax ? arg_out.value().data_ptr<int64_t>() : nullptr,
+                                    count.defined() ? count.data_ptr<int32_t>() : nullptr, B, E, K, N, sb.value(), se,
+                                    dtype_code(src), reduce, optional_out.has_value() ? 1 : 0, order->data_ptr(), order_bytes,
+                                    ows.data_ptr(), bytes, stream_of(src)),
+                 "scatter");
+    maybe_check_status_words(ows, bytes, "scatter", "the bounded wait for the tiles before it ran out");
     return std::make_tuple(out, arg_out);
   }
   if (mean_count != nullptr && reduce == TS_SUM && sk.value() == 0 && B * N < 0x7FFFFFFFll) {
@@ -620,6 +636,28 @@ Tensor gather_grad_rows(const Tensor &grad_out, const Tensor &index, int64_t dim
   return gather_coo_hip(grad_out.contiguous(), rows, std::nullopt, count_rows);
 }
 
+// Backward of a scatter over the order that its forward pass left; undefined where there is none (or hooks have moved what was
+// saved off its border, or the index has become another layout).
+Tensor ordered_backward(Tensor grad_out, const Tensor &arg_out, const std::vector<int64_t> &src_shape, int64_t dim,
+                        const Tensor &index, bool mean, const Tensor &order) {
+  if (!order.defined() || !on_16_bytes(order) || index.sizes() != at::IntArrayRef(src_shape)) return Tensor();
+  c10::DeviceGuard guard(grad_out.device());
+  const int64_t B = prod(src_shape, 0, dim), E = src_shape[dim], N = grad_out.size(dim);
+  const int64_t K = prod(src_shape, dim + 1, static_cast<int64_t>(src_shape.size()));
+  auto sb = collapsed_stride(index, 0, dim);
+  if (!sb.has_value()) return Tensor();
+  grad_out = grad_out.contiguous();
+  Tensor arg = arg_out.defined() ? arg_out.contiguous() : Tensor();
+  if (arg.defined() && (!on_16_bytes(arg) || !on_16_bytes(grad_out))) return Tensor();
+  Tensor grad_in = at::empty(src_shape, grad_out.options());
+  check_status(ts_scatter_ordered_backward(grad_out.data_ptr(), arg.defined() ? arg.data_ptr<int64_t>() : nullptr,
+                                           index.data_ptr<int64_t>(), grad_in.data_ptr(), B, E, K, N, sb.value(), index.stride(dim),
+                                           dtype_code(grad_out), mean ? 1 : 0, order.data_ptr(),
+                                           static_cast<size_t>(order.numel()), stream_of(grad_out)),
+               "scatter backward");
+  return grad_in;
+}
+
 // ------------------------------------------------------- autograd: scatter
 // one Function per reduction, wired as ScatterSum/Mul/Mean/Min/Max in csrc/scatter.cpp:54-233
 template <int REDUCE> struct ScatterFn : public torch::autograd::Function<ScatterFn<REDUCE>> {
@@ -631,17 +669,19 @@ template <int REDUCE> struct ScatterFn : public torch::autograd::Function<Scatte
     Variable old_index = index;
     index = broadcast(index, src, dim);
     Tensor fused_count;  // mean of single values: counted together with the sum
+    Tensor order;        // of the entries by row, where the call makes one and src needs a gradient
     // mean with one index per row (a 1-D index along dim 0, or an index shaped like src's leading dims)
     bool per_row = REDUCE == TS_MEAN && old_index.dim() == dim + 1 && src.numel() > 0 && old_index.size(dim) == src.size(dim);
     for (int64_t i = 0; per_row && i < dim; i++) per_row = old_index.size(i) == src.size(i);
     SmallMean small;
     small.counted = per_row && src.requires_grad();  // for the backward pass
     auto result = scatter_hip(src, index, dim, optional_out, dim_size, REDUCE == TS_MEAN ? TS_SUM : REDUCE,
-                              REDUCE == TS_MEAN ? &fused_count : nullptr, per_row ? &small : nullptr);
+                              REDUCE == TS_MEAN ? &fused_count : nullptr, per_row ? &small : nullptr,
+                              src.requires_grad() && (REDUCE != TS_MEAN || per_row) ? &order : nullptr);
     Variable out = std::get<0>(result);
     if (optional_out.has_value()) ctx->mark_dirty({optional_out.value()});
     if (REDUCE == TS_SUM) {
-      ctx->save_for_backward({index});
+      ctx->save_for_backward({index, Variable(), order});
       return {out};
     }
     if (REDUCE == TS_MUL) {
@@ -687,7 +727,7 @@ template <int REDUCE> struct ScatterFn : public torch::autograd::Function<Scatte
           auto count_sizes = out.sizes().vec();
           count_sizes.resize(dim + 1);
           Variable count = broadcast(count_f.clamp_min_(1).to(src.scalar_type()).view(count_sizes), out, dim);
-          ctx->save_for_backward({index, count});
+          ctx->save_for_backward({index, count, order});
         }
         return {out};
       }
@@ -704,7 +744,7 @@ template <int REDUCE> struct ScatterFn : public torch::autograd::Function<Scatte
       return {out};
     }
     Variable arg_out = std::get<1>(result).value();
-    ctx->save_for_backward({index, arg_out});
+    ctx->save_for_backward({index, arg_out, order});
     ctx->mark_non_differentiable({arg_out});
     ctx->set_materialize_grads(false);  // no zeros [.., N, ..] in the place of a gradient of the positions
     ctx->saved_data["src_dtype"] = static_cast<int64_t>(src.scalar_type());
@@ -720,6 +760,9 @@ template <int REDUCE> struct ScatterFn : public torch::autograd::Function<Scatte
     } else if (!grad_out.defined()) {  // (min / max: whoever used the values handed no gradient back) zeros, as everywhere else
       const auto dtype = static_cast<at::ScalarType>(ctx->saved_data["src_dtype"].toInt());
       grad_in = at::zeros(saved_shape(ctx), saved[1].options().dtype(dtype));
+    } else if (saved.size() > 2 && REDUCE != TS_MUL &&
+               (grad_in = ordered_backward(grad_out, REDUCE == TS_MIN || REDUCE == TS_MAX ? saved[1] : Tensor(), saved_shape(ctx), dim,
+                                           saved[0], REDUCE == TS_MEAN, saved[2])).defined()) {
     } else if (REDUCE == TS_SUM) {
       grad_in = gather_grad_rows(grad_out, saved[0], dim, std::nullopt);
     } else if (REDUCE == TS_MUL) {
