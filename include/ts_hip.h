@@ -295,7 +295,8 @@ enum ts_scatter_route {
                                             output row counted by the same launch */
   TS_ROUTE_SUM_SLABS = 20,               /* workspace, one 4-byte value per entry, 2^19 to 2^21 entries: a table per workgroup,
                                             handed over in slabs (no atomics for the write-back) */
-  TS_ROUTE_SMALL = 21                    /* ts_scatter_small: sum, mean, min or max of a small input in one launch */
+  TS_ROUTE_SMALL = 21,                   /* ts_scatter_small: sum, mean, min or max of a small input in one launch */
+  TS_ROUTE_SUM_NARROW_SORTED = 22        /* workspace, rows below 64 bytes: entries sorted by row, sums in registers */
 };
 /* Self-test of the fixed-pattern cross-lane helpers the kernels use (DPP row shifts, wave_shr:1,
  * v_permlane16_swap / v_permlane32_swap: csrc/dpp.h): one wavefront applies each helper to x = 3 * lane + 1 and

@@ -429,7 +429,7 @@ const char *ts_scatter_route_name(int route) {
       "min/max: slabs, one value per entry", "min/max: buckets", "min/max: buckets or segmented reduction (index checked)",
       "min/max: 64-bit elements, two passes", "sum: single values in buckets, table or runs (sample)",
       "sum: runs, entries per row counted by the same launch", "sum: single values, tables in slabs",
-      "sum, mean, min or max of a small input: one launch"};
+      "sum, mean, min or max of a small input: one launch", "sum: narrow rows, entries sorted by row"};
   return route >= 0 && route < (int)(sizeof(names) / sizeof(names[0])) ? names[route] : "unknown";
 }
 
@@ -683,6 +683,76 @@ int ts_segment_mean_coo_backward(const void *grad_out, const int64_t *index, con
   return run_coo_gather(dtype, a, p, B, true, static_cast<hipStream_t>(stream));
 }
 
+}  // extern "C"
+namespace {
+// Sums of rows below 64 bytes over sorted entries (group_rows.h), where adding in memory is slowest: 16-bit elements (packed pairs, or
+// one by one in rows of odd width), floats of nine columns and more, from where they outgrow what the launches of the sort cost. us
+// without / with, ten entries a row unless said, in random order | in order | a power law's hubs (p ~ i^-1.2, the sort's worst, memory's
+// best: its hot rows are added up in LDS):
+//   16 bits  10 M x 24  3943 / 448 | 479 / 371 | 3351 / 603      10 M x 8  1393 / 289 | 164 / 166 | 574 / 359
+//            10 M x 5   1317 / 291 | 334 / 162 | 648 / 342       10 M x 3  1012 / 283 | 205 / 152 | 422 / 323
+//            2 M x 16    486 / 81  |  67 / 68  | 276 / 117       2 M x 6    304 / 72  |  57 / 50  | 152 / 97
+//            9.7 M x 24, four a row 4097 / 581; 2.4 M x 16, 14 a row, with the backward pass 671 / 146; 629 k x 15 in order 81 / 35
+//     left   10 M x 4    928 / 279 | 128 / 114 | 291 / 321       2 M x 4    177 / 66  |  39 / 41  |  76 / 99
+//            10 M x 2    922 / 266 |  77 / 120 | 258 / 297       700 k x 6   92 / 40  |  21 / 31  |  57 / 66
+//            and, with fewer than two entries a row, 654 k x 8 83 / 108
+//   floats   10 M x 15  1021 / 403 | 477 / 265 | 615 / 556       10 M x 9   799 / 331 | 453 / 213 | 467 / 439
+//            10 M x 12   787 / 344 | 266 / 217 | 452 / 472       5.8 M x 13, nine a row 624 / 236
+//     left   10 M x 8    502 / 290 | 171 / 164 | 231 / 382       10 M x 5   638 / 307 | 282 / 162 | 291 / 377
+//            2 M x 13    200 / 88  | 120 / 66  | 111 / 127
+// The sums are held in double (the packed adds round to 16 bits every time). TS_SCATTER_NARROW (tuning aid): 0 never, 2 at any size.
+bool scatter_narrow_rule(int64_t B, int64_t E, int64_t K, int64_t N, int dtype) {
+  const int es = kElemBytes[dtype];
+  const int64_t row_bytes = K * es, n = B * E, M = 1000000;
+  if (!is_float_dtype(dtype) || row_bytes >= 64 || n < 1 || B * N < 1) return false;
+  const int mode = env_int("TS_SCATTER_NARROW", 1);
+  if (mode == 0) return false;
+  if (mode == 2) return true;
+  if (E < 2 * N) return false;
+  if (es == 2) return K >= 3 && K != 4 && n * K >= 8 * M;
+  return es == 4 && K >= 9 && n * K >= (row_bytes % kVecBytes == 0 ? 100 * M : 40 * M);
+}
+size_t scatter_narrow_records(int64_t B, int64_t E, int64_t K, int64_t N, int dtype) {
+  return group_rows_plan(B * E, B * N, K, kElemBytes[dtype], nullptr).bytes;
+}
+size_t scatter_narrow_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype) {
+  if (!scatter_narrow_rule(B, E, K, N, dtype)) return 0;
+  const size_t sort = row_sort_plan(B, E, N, nullptr, 0, true).bytes, records = scatter_narrow_records(B, E, K, N, dtype);
+  return sort == 0 || records == 0 ? 0 : sort + records;
+}
+int run_scatter_narrow(const void *src, const int64_t *index, void *out, int64_t B, int64_t E, int64_t K, int64_t N, int64_t sb,
+                       int64_t se, int dtype, void *ws, size_t ws_bytes, int32_t *count_out, hipStream_t s) {
+  const size_t records = scatter_narrow_records(B, E, K, N, dtype);
+  const RowSortPlan sp = row_sort_plan(B, E, N, static_cast<char *>(ws) + records, ws_bytes - records, true);
+  if (!sp.ok) return TS_ERR_WORKSPACE;
+  int rc = launch_row_sort(sp.p, index, sb, se, false, next_nonce(), s);
+  if (rc != TS_OK) return rc;
+  GroupRowsPlan p = group_rows_plan(B * E, B * N, K, kElemBytes[dtype], ws);
+  GroupArgs g = {};
+  g.src = src;
+  g.out = out;
+  g.B = 1;
+  g.E = B * E;
+  g.K = K;
+  g.N = B * N;
+  p.f.state = sp.p.state;
+  p.f.ptr = sp.p.ptr;
+  p.f.perm = sp.p.perm;
+  p.f.group = sp.p.perm_row;
+  p.f.gate = nullptr;
+  p.f.index = index;
+  p.f.sb = sb;
+  p.f.se = se;
+  p.f.E0 = E;
+  p.f.N0 = N;
+  rc = dispatch_group_rows(dtype, g, p.f, GS_SUM, s);
+  if (rc != TS_OK || count_out == nullptr) return rc;
+  hipLaunchKernelGGL(row_lengths_kernel, dim3(grid_for(B * N)), dim3(kBlock), 0, s, sp.p.ptr, count_out, B * N);
+  return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
+}
+}  // namespace
+extern "C" {
+
 size_t ts_scatter_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, int dtype, int reduce) {
   if (!valid_dtype(dtype) || !sizes_ok(B, N, E, K)) return 0;
   const bool any_size = env_int("TS_SCATTER_BINNED", 1) == 2;
@@ -700,6 +770,8 @@ size_t ts_scatter_workspace_bytes(int64_t B, int64_t E, int64_t K, int64_t N, in
   }
   if (reduce == TS_SUM && kAccBytes[dtype] >= 4) {  // table slots: int32 for int32, 8 bytes for the other types
     if (rr.ok) return rr.total();
+    const size_t narrow = scatter_narrow_bytes(B, E, K, N, dtype);
+    if (narrow != 0) return narrow;
     if (env_int("TS_SCATTER_LDS", 1)) {
       // one 4-byte value per entry: (row in bucket, value) words, 8 bytes of scratch per entry
       const size_t payload = bin_plan_payload(B, E, K, N, kElemBytes[dtype], nullptr, 0, any_size).bytes;
@@ -792,6 +864,16 @@ int scatter_ws_impl(const void *src, const int64_t *index, void *out, int64_t *a
       hipLaunchKernelGGL(row_lengths_kernel, dim3(grid_for(B * N)), dim3(kBlock), 0, s, sp.p.ptr, count_out, B * N);
       if (count_done != nullptr) *count_done = 1;
       return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH;
+    }
+  }
+  if (reduce == TS_SUM && !out_given && a.bin_ws != nullptr && index_stride_k == 0 && B * E * K > 0 && aligned16(workspace)) {
+    const size_t need = scatter_narrow_bytes(B, E, K, N, dtype);
+    if (need != 0 && workspace_bytes >= need) {
+      ts_note_scatter_route(TS_ROUTE_SUM_NARROW_SORTED);
+      const int rc = run_scatter_narrow(src, index, out, B, E, K, N, index_stride_b, index_stride_e, dtype, workspace,
+                                        workspace_bytes, count_out, s);
+      if (rc == TS_OK && count_out != nullptr && count_done != nullptr) *count_done = 1;
+      return rc;
     }
   }
   if (reduce == TS_SUM && workspace != nullptr && workspace_bytes >= 256 && aligned16(workspace) &&

@@ -1,7 +1,7 @@
-// Softmax, log-softmax (forward and backward), logsumexp and standard deviation over entries that were sorted by group
+// Softmax, log-softmax (forward and backward), logsumexp, standard deviation and sums of narrow rows over entries that were sorted by group
 // (row_sort.h): rows of the entries in registers, gathered once.
 //
-// A worker of `lanes` lanes holds eight neighbouring places of the order, a lane VEC columns of each of them. It walks its
+// A worker of `lanes` lanes holds four neighbouring places of the order (kRowsHeld), a lane VEC columns of each of them. It walks its
 // places in the order: running maximum, then running sum, reset where a group begins; the value at a group's end is handed
 // back to its places, and the results go out through perm. Only a group that crosses workers meets in LDS: the worker in
 // which it begins puts the parts together. Columns never meet, so a worker is as wide as the row needs (nine lanes for 33
@@ -139,7 +139,7 @@ __device__ __forceinline__ void rows_zero_outside(const GroupArgs &g, const Grou
   }
 }
 
-// A worker's eight places: which are the tile's, where groups begin and end among them.
+// A worker's places: which are the tile's, where groups begin and end among them.
 struct RowsPlaces {
   uint32_t valid, head, end;  // one bit per place
   bool enters, leaves, whole;  // the first place goes on with the worker's before, the last with the worker's behind; both, and no
@@ -482,6 +482,24 @@ __global__ __launch_bounds__(kRowsBlock) void group_rows_kernel(GroupArgs g, Gro
       }
       rows_store<T, VEC>(static_cast<T *>(g.out) + (int64_t)row[i] * K + col, r, f.stream != 0);
     }
+  } else if constexpr (MODE == GS_SUM) {
+    sums([&](int i, int c) { return to_acc<T>(x[i].v[c]); });
+    keep_sums();
+    rows_at_ends<S>(at.end & inside, [&](int i) {
+      const bool back = at.enters && i == fe;
+      int32_t group = gr[1];
+#pragma unroll
+      for (int j = 1; j < S; ++j) group = rows_pick(i == j, gr[j + 1], group);
+      V r;
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) {
+        F s = (F)in[c];
+#pragma unroll
+        for (int j = 0; j < S; ++j) s = rows_pick(i == j && !back, sum[j][c], s);
+        r.v[c] = from_acc<T>(s);
+      }
+      rows_store<T, VEC>(static_cast<T *>(g.out) + (int64_t)group * K + col, r, false);
+    });
   } else if constexpr (MODE == GS_LSE) {
     sums([&](int i, int c) { return round_elem<T>(to_acc<T>(x[i].v[c])); });
     keep_sums();
@@ -603,8 +621,8 @@ __global__ __launch_bounds__(kRowsBlock) void group_rows_kernel(GroupArgs g, Gro
 // sixteen columns of such a group, the workgroup those that cross more than 64 tiles: 64 partials by eight on the way together.
 template <typename T, int MODE>
 __global__ __launch_bounds__(kRowsCombine) void group_rows_combine_kernel(GroupArgs g, GroupRowsArgs f) {
-  constexpr bool kBackward = MODE == GS_SOFTMAX_BWD || MODE == GS_LOG_SOFTMAX_BWD;
-  constexpr bool kReduce = MODE == GS_LSE || MODE == GS_STD;
+  constexpr bool kBackward = MODE == GS_SOFTMAX_BWD || MODE == GS_LOG_SOFTMAX_BWD || MODE == GS_SUM;  // (a sum alone)
+  constexpr bool kReduce = MODE == GS_LSE || MODE == GS_STD || MODE == GS_SUM;
   // the kind of partial: log-softmax as softmax, the backward passes carry a sum alone
   typedef GroupBinPart<T, MODE == GS_STD ? GS_STD : MODE == GS_LSE ? GS_LSE : GS_SOFTMAX> Part;
   __shared__ Part s_part[kRowsCombine];
@@ -619,6 +637,13 @@ __global__ __launch_bounds__(kRowsCombine) void group_rows_combine_kernel(GroupA
       for (int64_t i = (int64_t)blockIdx.x * kRowsCombine + tid; i < (g.N + kWave - 1) / kWave * kWave; i += step) {
         const int64_t len = i < g.N ? f.ptr[i + 1] - f.ptr[i] : 1;
         if (MODE == GS_STD && i < g.N) g.count_w[i] = (int32_t)len;
+        if (g.K <= 16) {  // few columns: a lane its own
+          for (int64_t k = len == 0 ? 0 : g.K; k < g.K; ++k) {
+            out[i * g.K + k] = from_acc<T>((typename Acc<T>::type)0);
+            if (MODE == GS_STD) total[i * g.K + k] = from_acc<T>((typename Acc<T>::type)0);
+          }
+          continue;
+        }
         uint64_t empty = __ballot(len == 0);
         const int64_t base = i - (tid & (kWave - 1));
         while (empty != 0) {  // the wavefront's empty groups, one after the other
@@ -664,7 +689,9 @@ __global__ __launch_bounds__(kRowsCombine) void group_rows_combine_kernel(GroupA
   };
   auto leave = [&](int64_t t, int32_t group, const Part &r) {
     if (!col_on) return;
-    if constexpr (MODE == GS_STD || MODE == GS_LSE) {
+    if constexpr (MODE == GS_SUM) {
+      static_cast<T *>(g.out)[(int64_t)group * K + k] = from_acc<T>((typename Acc<T>::type)r.b);
+    } else if constexpr (MODE == GS_STD || MODE == GS_LSE) {
       group_bin_emit<T, MODE>(g, (int64_t)group * K + k, group, k, r);
     } else {
       const int64_t at = (t * 2 + 1) * K + k;
@@ -953,7 +980,7 @@ template <typename T> int launch_rows_spread_t(const RowSortArgs &p, const void 
 }
 
 template <typename T, int VEC, int MODE> int launch_group_rows_m(const GroupArgs &g, const GroupRowsArgs &f, hipStream_t stream) {
-  constexpr bool kReduce = MODE == GS_LSE || MODE == GS_STD;
+  constexpr bool kReduce = MODE == GS_LSE || MODE == GS_STD || MODE == GS_SUM;
   if constexpr (MODE == GS_STD_BWD || MODE == GS_LSE_BWD) {
     const int64_t per = (int64_t)f.workers * kRowsMapHeld;
     hipLaunchKernelGGL((group_rows_map_kernel<T, VEC, MODE>), dim3((unsigned)((g.E + per - 1) / per), (unsigned)f.slices),
@@ -961,7 +988,11 @@ template <typename T, int VEC, int MODE> int launch_group_rows_m(const GroupArgs
   } else {
     const dim3 grid((unsigned)f.nt, (unsigned)f.slices);
     hipLaunchKernelGGL((group_rows_kernel<T, VEC, MODE>), grid, dim3(kRowsBlock), 0, stream, g, f);
-    const int64_t shares = (f.nt + kRowsTeams - 1) / kRowsTeams;
+    int64_t shares = (f.nt + kRowsTeams - 1) / kRowsTeams;
+    if (kReduce) {  // (and a workgroup for 1024 groups, which may be empty: 450 k single values onto 266 k rows, ten workgroups 347 us)
+      const int64_t want = (g.N + kRowsCombine - 1) / kRowsCombine;
+      shares = shares < want ? (want < 2048 ? want : 2048 < shares ? shares : 2048) : shares;
+    }
     hipLaunchKernelGGL((group_rows_combine_kernel<T, MODE>), dim3((unsigned)shares, (unsigned)((g.K + kRowsTeam - 1) / kRowsTeam)),
                        dim3(kRowsCombine), 0, stream, g, f);
     if constexpr (!kReduce) hipLaunchKernelGGL((group_rows_finish_kernel<T, VEC, MODE>), grid, dim3(kRowsBlock), 0, stream, g, f);
@@ -978,6 +1009,7 @@ template <typename T, int VEC> int launch_group_rows_v(const GroupArgs &g, const
   case GS_LSE_BWD: return launch_group_rows_m<T, VEC, GS_LSE_BWD>(g, f, stream);
   case GS_STD: return launch_group_rows_m<T, VEC, GS_STD>(g, f, stream);
   case GS_STD_BWD: return launch_group_rows_m<T, VEC, GS_STD_BWD>(g, f, stream);
+  case GS_SUM: return launch_group_rows_m<T, VEC, GS_SUM>(g, f, stream);
   default: return TS_ERR_BAD_ARG;
   }
 }

@@ -69,7 +69,8 @@ enum {
   GS_SOFTMAX = 0, GS_LOG_SOFTMAX = 1, GS_SOFTMAX_BWD = 2, GS_LOG_SOFTMAX_BWD = 3, GS_LSE = 4, GS_LSE_BWD = 5,
   GS_STD = 6, GS_STD_BWD = 7,
   GS_STD_BINS = 8, GS_LSE_BINS = 9,  // std / logsumexp forward through buckets of groups (group_binned.h)
-  GS_STD_ROWS = 10  // std forward: the sweep of squared deviations over entries sorted by group (row_sort.h, csr_reduce.h)
+  GS_STD_ROWS = 10,  // std forward: the sweep of squared deviations over entries sorted by group (row_sort.h, csr_reduce.h)
+  GS_SUM = 11  // sums of a scatter whose rows the segmented reduction does not hold, over entries sorted by row (group_rows.h)
 };
 
 struct BinArgs;
